@@ -2,8 +2,8 @@
 //
 //   latent_decode_kernel   few query tokens: queries are already in the latent space, all heads share the cached latents
 //                          (read once per row tile), the context is cut into slices; latent_merge_kernel joins them
-//   latent_prefill_kernel  many query tokens: keys and values expanded per head beforehand, flash attention, the output
-//                          gate in the epilogue
+//   prompt_attn_kernel     (pq_prompt_attn.h) many query tokens: keys and values expanded per head beforehand, flash attention,
+//                          the output gate in the epilogue
 //   latent_plain_kernel    any rank, any dtype (float32 runs here), one wavefront per query row
 //
 // Both matrix-core kernels compute the TRANSPOSED score tile, S^T = K Q^T, so that a query row is a tile column, i.e. a
@@ -11,7 +11,7 @@
 // O^T = V^T P^T, takes its right operand in, once the tokens are numbered accordingly (the order of the summed index is
 // free as long as both operands agree).  Scores, their softmax and all sums are float32; latents, queries and weights
 // enter the products in the model's 16-bit dtype.
-#include "pq_mfma.h"
+#include "pq_prompt_attn.h"
 #include "pq_latent_internal.h"
 
 namespace pq {
@@ -353,216 +353,19 @@ int launch_latent_decode_any(const LatentDecodeArgs& a, int dtype, hipStream_t s
 }
 
 // ---- prompt --------------------------------------------------------------------------------------------------------
-// grid (heads, query tiles, sequences): consecutive workgroups are different heads of one query tile, so that with a
-// multiple of 8 heads the query tiles of a head meet in one XCD's L2.  Four wavefronts with 32 query rows each over
-// 64-key tiles, double-buffered in LDS; longest query tiles first.
-// K tile: rows of DKP + 8 elements.  V tile: one row per channel, 64 tokens + 8; inside each 16 tokens the order is
-// 0-3, 8-11, 4-7, 12-15, so that the 8 tokens a lane half needs for one product are one 16-byte read.
-constexpr int kPrefillRows = 128, kPrefillKeys = 64;
-
-template <typename T, int DKP, int DVP>
-__global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void latent_prefill_kernel(LatentPrefillArgs a) {
-    constexpr int KS = DKP / 16, VT = DVP / 32, KROW = DKP + 8, VROW = kPrefillKeys + 8;
-    constexpr int KLOADS = kPrefillKeys * (DKP / 8) / 256, VLOADS = DVP * (kPrefillKeys / 8) / 256;
-    static_assert(KLOADS * 256 == kPrefillKeys * (DKP / 8) && VLOADS * 256 == DVP * (kPrefillKeys / 8), "whole loads");
-    extern __shared__ __attribute__((aligned(16))) uint16_t sm[];
-    constexpr int kTileK = kPrefillKeys * KROW, kTileV = DVP * VROW;      // two K tiles, then two V tiles
-    auto kt = [&](int buf) { return sm + buf * kTileK; };
-    auto vt = [&](int buf) { return sm + 2 * kTileK + buf * kTileV; };
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid / kWave, col = lane & 31, hi = lane >> 5;
-    const int h = blockIdx.x, b = blockIdx.z, D = a.D, Dv = a.Dv, H = a.H;
-    const int tile = static_cast<int>(gridDim.y) - 1 - static_cast<int>(blockIdx.y);
-    const int past = a.Lk - a.L;
-    const int qw = tile * kPrefillRows + wv * 32;                  // the wavefront's first query token
-    const int qi = qw + col;
-    const bool valid = qi < a.L;
-    const int qc = valid ? qi : a.L - 1;
-    const int limit = past + qc;                                   // last key this row sees
-    const int lo = a.start ? a.start[b] : 0;
-    const int q_last = tile * kPrefillRows + kPrefillRows - 1 < a.L - 1 ? tile * kPrefillRows + kPrefillRows - 1 : a.L - 1;
-    const int wave_last = past + (qw + 31 < a.L - 1 ? qw + 31 : a.L - 1);
-    const int it0 = lo / kPrefillKeys, it1 = (past + q_last) / kPrefillKeys + 1;
-
-    u32x4_a q[KS];
-    {
-        const uint16_t* qp = static_cast<const uint16_t*>(a.q) + ((static_cast<size_t>(b) * a.L + qc) * H + h) * D;
-        static_for<KS>([&](auto I) {
-            constexpr int i = decltype(I)::value;
-            const int c = i * 16 + 8 * hi;
-            const u32x4_a t = *reinterpret_cast<const u32x4_a*>(qp + (c < D ? c : 0));
-            q[i] = c < D ? t : u32x4_a{0, 0, 0, 0};
-        });
-    }
-    const uint16_t* kb = static_cast<const uint16_t*>(a.k) + (static_cast<size_t>(b) * a.Lk * H + h) * D;
-    const uint16_t* vb = static_cast<const uint16_t*>(a.vt) + (static_cast<size_t>(b) * H + h) * Dv * a.ldv;
-    u32x4_a ks[KLOADS], vs[VLOADS];
-    const uint32_t k_row = static_cast<uint32_t>(H) * D;
-    auto fetch = [&](int it) {
-        const uint16_t* kbase = kb + static_cast<size_t>(it) * kPrefillKeys * k_row;
-        const int last = a.Lk - 1 - it * kPrefillKeys;             // uniform
-        static_for<KLOADS>([&](auto I) {
-            constexpr int i = decltype(I)::value;
-            const int u = i * 256 + tid, tok = u / (DKP / 8), ch = u % (DKP / 8);
-            // no branch around a load (it would be waited for at the join): keys past the end are a copy with weight zero,
-            // columns past D a copy that meets zeros of q
-            ks[i] = *reinterpret_cast<const u32x4_a*>(kbase + (static_cast<uint32_t>(tok <= last ? tok : last) * k_row + (ch * 8 < D ? ch * 8 : 0)));
-        });
-        static_for<VLOADS>([&](auto I) {
-            constexpr int i = decltype(I)::value;
-            const int u = i * 256 + tid, piece = u % 8, ch = u / 8 < Dv ? u / 8 : Dv - 1;      // (rows past Dv are never stored)
-            vs[i] = *reinterpret_cast<const u32x4_a*>(vb + static_cast<size_t>(ch) * a.ldv + it * kPrefillKeys + piece * 8);
-        });
-    };
-    auto put = [&](int buf) {
-        static_for<KLOADS>([&](auto I) {
-            constexpr int i = decltype(I)::value;
-            const int u = i * 256 + tid, tok = u / (DKP / 8), ch = u % (DKP / 8);
-            *reinterpret_cast<u32x4_a*>(kt(buf) + tok * KROW + ch * 8) = ks[i];
-        });
-        static_for<VLOADS>([&](auto I) {
-            constexpr int i = decltype(I)::value;
-            const int u = i * 256 + tid, ch = u / 8, piece = u % 8;
-            uint16_t* d = vt(buf) + ch * VROW + (piece >> 1) * 16 + (piece & 1) * 4;
-            *reinterpret_cast<u32x2_a*>(d) = u32x2_a{vs[i].x, vs[i].y};
-            *reinterpret_cast<u32x2_a*>(d + 8) = u32x2_a{vs[i].z, vs[i].w};
-        });
-    };
-    floatx16_a o[VT];
-    static_for<VT>([&](auto I) {
-        constexpr int i = decltype(I)::value;
-#pragma unroll
-        for (int j = 0; j < 16; j++) o[i][j] = 0.0f;
-    });
-    float m = kNone, l = 0.0f;
-    const float scale2 = a.scale * kLog2e;
-
-    if (it0 < it1) {
-        fetch(it0);
-        put(it0 & 1);
-    }
-    __syncthreads();
-    for (int it = it0; it < it1; it++) {
-        const int buf = it & 1;
-        if (it + 1 < it1) fetch(it + 1);
-        __builtin_amdgcn_sched_barrier(0);
-        const int key0 = it * kPrefillKeys;
-        if (key0 <= wave_last) {                                   // uniform over the wavefront
-            floatx16_a s[2];
-#pragma unroll
-            for (int u = 0; u < 2; u++)
-#pragma unroll
-                for (int j = 0; j < 16; j++) s[u][j] = 0.0f;
-            const uint16_t* kp = kt(buf) + col * KROW + 8 * hi;
-            static_for<KS>([&](auto I) {
-                constexpr int i = decltype(I)::value;
-                s[0] = mma32<T>(*reinterpret_cast<const u32x4_a*>(kp + i * 16), q[i], s[0]);
-                s[1] = mma32<T>(*reinterpret_cast<const u32x4_a*>(kp + 32 * KROW + i * 16), q[i], s[1]);
-            });
-            // this lane: query qi, keys key0 + 32 u + 8 (j / 4) + 4 hi + j % 4
-            float mx = kNone;
-            if (key0 + kPrefillKeys - 1 > past + qw || key0 < lo) {
-#pragma unroll
-                for (int u = 0; u < 2; u++)
-#pragma unroll
-                    for (int j = 0; j < 16; j++) {
-                        const int key = key0 + 32 * u + 8 * (j >> 2) + 4 * hi + (j & 3);
-                        s[u][j] = (key <= limit && key >= lo) ? s[u][j] * scale2 : -INFINITY;
-                        mx = fmaxf(mx, s[u][j]);
-                    }
-            } else {
-#pragma unroll
-                for (int u = 0; u < 2; u++)
-#pragma unroll
-                    for (int j = 0; j < 16; j++) {
-                        s[u][j] *= scale2;
-                        mx = fmaxf(mx, s[u][j]);
-                    }
-            }
-            mx = fmaxf(mx, __shfl_xor(mx, 32));
-            if (__any(mx > m)) {
-                const float mn = fmaxf(m, mx), al = exp2_hw(m - mn);
-                l *= al;
-                static_for<VT>([&](auto I) {
-                    constexpr int i = decltype(I)::value;
-#pragma unroll
-                    for (int j = 0; j < 16; j++) o[i][j] *= al;
-                });
-                m = mn;
-            }
-            u32x4_a p[4];                                           // right operands of the four 16-token steps
-#pragma unroll
-            for (int u = 0; u < 2; u++)
-#pragma unroll
-                for (int j = 0; j < 16; j += 2) {
-                    const float e0 = exp2_hw(s[u][j] - m), e1 = exp2_hw(s[u][j + 1] - m);
-                    l += e0 + e1;
-                    p[2 * u + (j >> 3)][(j & 7) >> 1] = pack2<T>(e0, e1);
-                }
-            const uint16_t* vp = vt(buf) + col * VROW + 8 * hi;
-            static_for<VT>([&](auto I) {
-                constexpr int i = decltype(I)::value;
-                static_for<4>([&](auto J) {
-                    constexpr int j = decltype(J)::value;
-                    o[i] = mma32<T>(*reinterpret_cast<const u32x4_a*>(vp + i * 32 * VROW + j * 16), p[j], o[i]);
-                });
-            });
-        }
-        if (it + 1 < it1) put(buf ^ 1);
-        __syncthreads();
-    }
-    l += __shfl_xor(l, 32);
-    if (!valid) return;
-    const float sink2 = a.sink[h] * kLog2e, mf = fmaxf(m, sink2);
-    const float al = exp2_hw(m - mf), inv = al / (l * al + exp2_hw(sink2 - mf));
-    const size_t row = static_cast<size_t>(b) * a.L + qi;
-    uint16_t* out = static_cast<uint16_t*>(a.out) + row * H * Dv + static_cast<size_t>(h) * Dv;
-    const uint16_t* gate = a.gate ? static_cast<const uint16_t*>(a.gate) + row * a.gate_row + static_cast<size_t>(h) * Dv : nullptr;
-    const bool quads = Dv % 4 == 0 && (!gate || a.gate_row % 4 == 0);
-    static_for<VT>([&](auto I) {
-        constexpr int i = decltype(I)::value;
-#pragma unroll
-        for (int j4 = 0; j4 < 4; j4++) {
-            const int ch = i * 32 + 8 * j4 + 4 * hi;
-            float v[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = o[i][4 * j4 + j] * inv;
-            if (quads && ch + 4 <= Dv) {
-                if (gate) {
-                    const uint2 gv = *reinterpret_cast<const uint2*>(gate + ch);
-                    const uint32_t gw[2] = {gv.x, gv.y};
-#pragma unroll
-                    for (int j = 0; j < 4; j++) v[j] = v[j] / (1.0f + __expf(-lo2f<T>(static_cast<uint16_t>(gw[j >> 1] >> (16 * (j & 1))))));
-                }
-                *reinterpret_cast<uint2*>(out + ch) = make_uint2(pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3]));
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; j++)
-                    if (ch + j < Dv) out[ch + j] = f2lo<T>(gate ? v[j] / (1.0f + __expf(-lo2f<T>(gate[ch + j]))) : v[j]);
-            }
-        }
-    });
-}
-
-template <typename T, int DKP, int DVP>
-static int prefill_one(const LatentPrefillArgs& a, hipStream_t st) {
-    constexpr size_t bytes = 2 * 2 * (static_cast<size_t>(kPrefillKeys) * (DKP + 8) + static_cast<size_t>(DVP) * (kPrefillKeys + 8));
-    static_assert(bytes <= 160 * 1024, "LDS");
-    if (bytes > 64 * 1024) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_prefill_kernel<T, DKP, DVP>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
-        if (e != hipSuccess) return static_cast<int>(e);
-    }
-    dim3 grid(a.H, (a.L + kPrefillRows - 1) / kPrefillRows, a.B), block(256);
-    hipLaunchKernelGGL((latent_prefill_kernel<T, DKP, DVP>), grid, block, bytes, st, a);
-    return static_cast<int>(hipGetLastError());
-}
-
 template <typename T>
-static int prefill_dims(const LatentPrefillArgs& a, hipStream_t st) {
-    if (a.D <= 64 && a.Dv <= 64) return prefill_one<T, 64, 64>(a, st);
-    if (a.D <= 128 && a.Dv <= 128) return prefill_one<T, 128, 128>(a, st);
-    if (a.D <= 192 && a.Dv <= 128) return prefill_one<T, 192, 128>(a, st);
-    return prefill_one<T, 256, 256>(a, st);
+static int prefill_dims(const LatentPrefillArgs& l, hipStream_t st) {
+    PromptAttnArgs a{};
+    const int64_t kv = static_cast<int64_t>(l.H) * l.D;
+    a.q = l.q; a.q_b = l.L * kv; a.q_t = kv; a.q_h = l.D;
+    a.k = l.k; a.k_b = l.Lk * kv; a.k_t = kv; a.k_h = l.D;
+    a.v = l.vt; a.v_b = static_cast<int64_t>(l.H) * l.Dv * l.ldv; a.v_t = l.ldv; a.v_h = l.Dv * l.ldv;
+    a.sink = l.sink; a.gate = l.gate; a.gate_row = l.gate_row; a.start = l.start; a.out = l.out;
+    a.B = l.B; a.L = l.L; a.Lk = l.Lk; a.H = a.G = l.H; a.D = l.D; a.Dv = l.Dv; a.scale = l.scale;
+    if (l.D <= 64 && l.Dv <= 64) return launch_prompt_attn<T, 64, 64, false>(a, st);
+    if (l.D <= 128 && l.Dv <= 128) return launch_prompt_attn<T, 128, 128, false>(a, st);
+    if (l.D <= 192 && l.Dv <= 128) return launch_prompt_attn<T, 192, 128, false>(a, st);
+    return launch_prompt_attn<T, 256, 256, false>(a, st);
 }
 
 int launch_latent_prefill(const LatentPrefillArgs& a, int dtype, hipStream_t st) {

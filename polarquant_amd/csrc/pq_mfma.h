@@ -13,6 +13,7 @@ typedef __bf16 bf16x8_a __attribute__((ext_vector_type(8)));
 typedef short short4_a __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) short4_a lds_short4;
 typedef __attribute__((address_space(3))) u32x4_a lds_u32x4;
+typedef __attribute__((address_space(3))) u32x2_a lds_u32x2;
 
 template <typename T> __device__ __forceinline__ floatx4_a mma16(u32x4_a a, u32x4_a b, floatx4_a c);
 template <> __device__ __forceinline__ floatx4_a mma16<F16>(u32x4_a a, u32x4_a b, floatx4_a c) {

@@ -1,0 +1,268 @@
+// Causal attention of a prompt (flash attention on the matrix cores), shared by the polar-key and the latent-attention libraries.
+#pragma once
+#include "pq_mfma.h"
+
+namespace pq {
+
+struct PromptAttnArgs {
+    const void *q, *k, *v;                    // q element (b, t, h, d) at b q_b + t q_t + h q_h + d; k likewise with key head h / (H / G)
+    int64_t q_b, q_t, q_h, k_b, k_t, k_h;
+    int64_t v_b, v_t, v_h;                    // a row per token: (b, t, g, c) at b v_b + t v_t + g v_h + c; a row per channel: v_t apart
+    const float* sink;                        // [H] or null
+    const void* gate;                         // [B * L, H * Dv] rows gate_row apart, or null
+    int64_t gate_row;
+    const int32_t* start;                     // [B]: keys before it do not exist; or null
+    void* out;                                // [B, L, H * Dv]
+    int B, L, Lk, H, G, D, Dv;                // the L queries are the last of the Lk tokens
+    float scale;
+};
+
+constexpr int kPromptTileRows = 128, kPromptTileKeys = 64;
+
+// 16 bytes per lane from global memory into 1 KiB of LDS at `lds` (uniform), lane after lane.  Not known to the compiler's count
+// of loads in flight: wait_lds_loads() before the barrier behind which the data is read.
+__device__ __forceinline__ void load_to_lds(const void* p, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "s"(lds) : "memory");
+}
+__device__ __forceinline__ void wait_lds_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+typedef float floatx2_a __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_a __attribute__((ext_vector_type(2)));
+typedef _Float16 halfx2_a __attribute__((ext_vector_type(2)));
+template <typename T> __device__ __forceinline__ uint32_t pack_pair(float a, float b);
+template <> __device__ __forceinline__ uint32_t pack_pair<BF16>(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2_a{a, b}, bf16x2_a));
+}
+template <> __device__ __forceinline__ uint32_t pack_pair<F16>(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2_a{a, b}, halfx2_a));
+}
+
+// grid (heads, query tiles, sequences), longest query tiles first.  Four wavefronts with 32 query rows each over 64-key tiles of K
+// and V that are double-buffered in LDS.  The transposed score tile S^T = K Q^T makes a query a lane, its softmax state a
+// register, and P^T the right operand of O^T = V^T P^T as it stands.  TOKEN_ROWS: V has a row per token and is transposed on the
+// way out of LDS; otherwise a row per channel, as a product with the weights on the left leaves it.
+//
+// What bounds it: the vector unit and the matrix cores need about the same time per tile (32 exponentials at a quarter of the rate and
+// 112 other vector instructions a lane; 32 products of 32 cycles), the LDS half of it, so the two wavefronts of a SIMD have to
+// overlap.  Tiles therefore go to LDS directly (no registers, no store instructions, the swizzle that keeps reads free of
+// conflicts is in the addresses that the lanes load from), the scale is part of the exponential's multiply-add, and the maximum is
+// raised only when exceeded by 2^8.  Measured at 8192 tokens, 32 heads of 128, bf16: 557 us (987 TFLOP/s) with a row per
+// channel, 570 us with a row per token; 724 us with tiles passed through registers and a maximum raised at each excess.  A step that
+// makes the next tile's scores beside this tile's weights needs more registers than two wavefronts have (830 us); raised
+// wavefront priority around the products changes nothing.
+template <typename T, int DKP, int DVP, bool TOKEN_ROWS>
+__global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(PromptAttnArgs a) {
+    constexpr int KS = DKP / 16, VT = DVP / 32, KC = DKP / 8, VC = TOKEN_ROWS ? DVP / 8 : 8;        // 16-byte chunks of a row of K, of V
+    constexpr int KBYTES = kPromptTileKeys * DKP * 2, VBYTES = kPromptTileKeys * DVP * 2;
+    constexpr int KL = KBYTES / 4096, VL = VBYTES / 4096;                                          // loads per lane and tile
+    static_assert(!TOKEN_ROWS || DVP == 128, "swizzle of token rows");
+    extern __shared__ __attribute__((aligned(1024))) uint8_t sm[];                                // two K tiles, then two V tiles
+    const uint32_t lds0 = lds_addr(sm);
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 31, hi = lane >> 5;
+    const int H = a.H, D = a.D, Dv = a.Dv, b = blockIdx.z;
+        const int h = blockIdx.x, g = h / (H / a.G);
+    const int tile = static_cast<int>(gridDim.y) - 1 - static_cast<int>(blockIdx.y);
+    const int past = a.Lk - a.L;
+    const int qw = tile * kPromptTileRows + wv * 32, qi = qw + col;                 // the wavefront's first query token; this lane's
+    const bool valid = qi < a.L;
+    const int qc = valid ? qi : a.L - 1, limit = past + qc;                         // last key this row sees
+    const int lo = a.start ? a.start[b] : 0;
+    const int q_last = tile * kPromptTileRows + kPromptTileRows - 1 < a.L - 1 ? tile * kPromptTileRows + kPromptTileRows - 1 : a.L - 1;
+    const int wave_last = past + (qw + 31 < a.L - 1 ? qw + 31 : a.L - 1);
+    const int it0 = lo / kPromptTileKeys, it1 = (past + q_last) / kPromptTileKeys + 1;
+    const float scale2 = a.scale != 0.0f ? fabsf(a.scale) * kLog2e : 1.0e-30f;      // (a masked score, -inf, stays one)
+
+    u32x4_a q[KS];
+    {
+        const uint16_t* qp = static_cast<const uint16_t*>(a.q) + b * a.q_b + qc * a.q_t + h * a.q_h;
+        const uint32_t flip = a.scale < 0.0f ? 0x80008000u : 0u;
+        static_for<KS>([&](auto I) {
+            constexpr int i = decltype(I)::value;
+            const int c = i * 16 + 8 * hi;
+            const u32x4_a t = *reinterpret_cast<const u32x4_a*>(qp + (c < D ? c : 0));
+            q[i] = c < D ? u32x4_a{t.x ^ flip, t.y ^ flip, t.z ^ flip, t.w ^ flip} : u32x4_a{0, 0, 0, 0};
+        });
+    }
+    // where this lane's 16 bytes of each load come from: load i of a wavefront fills chunks (wv KL + i) 64 .. + 63 of a tile
+    const uint16_t* kb = static_cast<const uint16_t*>(a.k) + b * a.k_b + g * a.k_h;
+    const uint16_t* vb = static_cast<const uint16_t*>(a.v) + b * a.v_b + g * a.v_h;
+    auto k_swz = [](int row) { return DKP == 64 ? (row >> 1) & 7 : row & 7; };
+    auto v_swz = [](int row) { return TOKEN_ROWS ? (row & 7) << 1 : (row >> 1) & 7; };
+    auto k_src = [&](int i, int first, int last) {
+        const int u = (wv * KL + i) * 64 + lane, row = u / KC, c = ((u % KC) ^ k_swz(row)) * 8;
+        return kb + static_cast<int64_t>(first + (row < last ? row : last)) * a.k_t + (c < D ? c : 0);
+    };
+    auto v_src = [&](int i, int first, int last) {
+        const int u = (wv * VL + i) * 64 + lane, row = u / VC, c = ((u % VC) ^ v_swz(row)) * 8;
+        if (TOKEN_ROWS) return vb + static_cast<int64_t>(first + (row < last ? row : last)) * a.v_t + (c < Dv ? c : 0);
+        return vb + static_cast<int64_t>(row < Dv ? row : Dv - 1) * a.v_t + first + c;
+    };
+    const uint16_t *ks[KL], *vs[VL];
+    static_for<KL>([&](auto I) { ks[I] = k_src(I, it0 * kPromptTileKeys, kPromptTileKeys - 1); });
+    static_for<VL>([&](auto I) { vs[I] = v_src(I, it0 * kPromptTileKeys, kPromptTileKeys - 1); });
+    auto fetch = [&](int it, auto BUF) {
+        constexpr int buf = decltype(BUF)::value;
+        const int last = a.Lk - 1 - it * kPromptTileKeys;          // rows past the end: copies of the last one, with weight zero
+        if (last < kPromptTileKeys - 1) {
+            static_for<KL>([&](auto I) { ks[I] = k_src(I, it * kPromptTileKeys, last); });
+            if (TOKEN_ROWS) static_for<VL>([&](auto I) { vs[I] = v_src(I, it * kPromptTileKeys, last); });
+        }
+        static_for<KL>([&](auto I) {
+            load_to_lds(ks[I], lds0 + buf * KBYTES + (wv * KL + I) * 1024);
+            ks[I] += kPromptTileKeys * a.k_t;
+        });
+        static_for<VL>([&](auto I) {
+            load_to_lds(vs[I], lds0 + 2 * KBYTES + buf * VBYTES + (wv * VL + I) * 1024);
+            vs[I] += TOKEN_ROWS ? kPromptTileKeys * a.v_t : kPromptTileKeys;
+        });
+    };
+    floatx16_a o[VT];
+    static_for<VT>([&](auto I) {
+#pragma unroll
+        for (int j = 0; j < 16; j++) o[decltype(I)::value][j] = 0.0f;
+    });
+    float m = kNone, l = 0.0f;
+
+    // LDS addresses of this lane's reads: row `col` of K, chunk 2 i + hi
+    uint32_t ka[KS], va[VT];
+    static_for<KS>([&](auto I) { ka[I] = lds0 + col * (DKP * 2) + ((2 * I + hi) ^ k_swz(col)) * 16; });
+    static_for<VT>([&](auto I) {
+        constexpr int i = decltype(I)::value;
+        if (TOKEN_ROWS) {           // 16 lanes read 4 tokens x 16 channels and get them transposed
+            const int row = 4 * hi + ((lane & 15) >> 2), chunk = 4 * i + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
+            va[i] = lds0 + 2 * KBYTES + row * (DVP * 2) + (chunk ^ v_swz(row)) * 16 + (lane & 1) * 8;
+        } else {
+            va[i] = lds0 + 2 * KBYTES + (32 * i + col) * 128 + hi * 8;
+        }
+    });
+    auto step = [&](int it, auto BUF) {
+        constexpr int buf = decltype(BUF)::value;
+        if (it + 1 < it1) fetch(it + 1, IC<buf ^ 1>{});
+        const int key0 = it * kPromptTileKeys;
+        if (key0 <= wave_last) {                                   // uniform over the wavefront
+            floatx16_a s[2];
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+#pragma unroll
+                for (int j = 0; j < 16; j++) s[u][j] = 0.0f;
+            static_for<KS>([&](auto I) {
+                constexpr int i = decltype(I)::value;
+                s[0] = mma32<T>(*lds_ptr<lds_u32x4>(ka[i] + buf * KBYTES), q[i], s[0]);
+                s[1] = mma32<T>(*lds_ptr<lds_u32x4>(ka[i] + buf * KBYTES + 32 * DKP * 2), q[i], s[1]);
+            });
+            // this lane: query qi, keys key0 + 32 u + 8 (j / 4) + 4 hi + j % 4
+            if (key0 + kPromptTileKeys - 1 > past + qw || key0 < lo) {
+                const int last = limit - key0 - 4 * hi, first = lo - key0 - 4 * hi;
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+#pragma unroll
+                    for (int j = 0; j < 16; j++) {
+                        const int e = 32 * u + 8 * (j >> 2) + (j & 3);
+                        s[u][j] = (e <= last && e >= first) ? s[u][j] : -INFINITY;
+                    }
+            }
+            float mx = fmaxf(s[0][0], s[1][0]);
+#pragma unroll
+            for (int j = 1; j < 16; j++) mx = fmaxf(fmaxf(mx, s[0][j]), s[1][j]);
+            mx = fmaxf(mx, __shfl_xor(mx, 32)) * scale2;
+            // the maximum is raised only when it is exceeded by a factor of 2^8: weights stay below 2^8 of the reference point
+            if (__any(mx > m + 8.0f)) {
+                const float mn = fmaxf(m, mx), al = exp2_hw(m - mn);
+                l *= al;
+                static_for<VT>([&](auto I) {
+#pragma unroll
+                    for (int j = 0; j < 16; j++) o[decltype(I)::value][j] *= al;
+                });
+                m = mn;
+            }
+            u32x4_a p[4];                                           // right operands of the four 16-token steps
+            float sum[2] = {0.0f, 0.0f};
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+#pragma unroll
+                for (int j = 0; j < 16; j += 2) {
+                    const float e0 = exp2_hw(__builtin_fmaf(s[u][j], scale2, -m)), e1 = exp2_hw(__builtin_fmaf(s[u][j + 1], scale2, -m));
+                    sum[0] += e0;
+                    sum[1] += e1;
+                    p[2 * u + (j >> 3)][(j & 7) >> 1] = pack_pair<T>(e0, e1);
+                }
+            l += sum[0] + sum[1];
+            static_for<4>([&](auto J) {
+                constexpr int j = decltype(J)::value;
+                static_for<VT>([&](auto I) {
+                    constexpr int i = decltype(I)::value;
+                    u32x2_a w0, w1;
+                    if constexpr (TOKEN_ROWS) {
+                        const uint32_t at = va[i] + buf * VBYTES + j * 16 * DVP * 2;
+                        w0 = __builtin_bit_cast(u32x2_a, __builtin_amdgcn_ds_read_tr16_b64_v4i16(lds_ptr<lds_short4>(at)));
+                        w1 = __builtin_bit_cast(u32x2_a, __builtin_amdgcn_ds_read_tr16_b64_v4i16(lds_ptr<lds_short4>(at + 8 * DVP * 2)));
+                    } else {
+                        const uint32_t at = va[i] + buf * VBYTES;
+                        w0 = *lds_ptr<lds_u32x2>(at + ((2 * j) ^ v_swz(col)) * 16);
+                        w1 = *lds_ptr<lds_u32x2>(at + ((2 * j + 1) ^ v_swz(col)) * 16);
+                    }
+                    o[i] = mma32<T>(u32x4_a{w0.x, w0.y, w1.x, w1.y}, p[j], o[i]);
+                });
+            });
+        }
+        wait_lds_loads();
+        __syncthreads();
+    };
+    if (it0 < it1) fetch(it0, IC<0>{});
+    wait_lds_loads();
+    __syncthreads();
+    for (int it = it0; it < it1; it += 2) {
+        step(it, IC<0>{});
+        if (it + 1 < it1) step(it + 1, IC<1>{});
+    }
+    l += __shfl_xor(l, 32);
+    if (!valid) return;
+    float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    if (a.sink) {
+        const float sink2 = a.sink[h] * kLog2e, mf = fmaxf(m, sink2), al = exp2_hw(m - mf);
+        inv = al / (l * al + exp2_hw(sink2 - mf));
+    }
+    const size_t row = static_cast<size_t>(b) * a.L + qi;
+    uint16_t* out = static_cast<uint16_t*>(a.out) + row * H * Dv + static_cast<size_t>(h) * Dv;
+    const uint16_t* gate = a.gate ? static_cast<const uint16_t*>(a.gate) + row * a.gate_row + static_cast<size_t>(h) * Dv : nullptr;
+    const bool quads = Dv % 4 == 0 && (!gate || a.gate_row % 4 == 0);
+    static_for<VT>([&](auto I) {
+        constexpr int i = decltype(I)::value;
+#pragma unroll
+        for (int j4 = 0; j4 < 4; j4++) {
+            const int ch = i * 32 + 8 * j4 + 4 * hi;
+            float v[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = o[i][4 * j4 + j] * inv;
+            if (quads && ch + 4 <= Dv) {
+                if (gate) {
+                    const uint2 gv = *reinterpret_cast<const uint2*>(gate + ch);
+                    const uint32_t gw[2] = {gv.x, gv.y};
+#pragma unroll
+                    for (int j = 0; j < 4; j++) v[j] = v[j] / (1.0f + __expf(-lo2f<T>(static_cast<uint16_t>(gw[j >> 1] >> (16 * (j & 1))))));
+                }
+                *reinterpret_cast<uint2*>(out + ch) = make_uint2(pack_pair<T>(v[0], v[1]), pack_pair<T>(v[2], v[3]));
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    if (ch + j < Dv) out[ch + j] = f2lo<T>(gate ? v[j] / (1.0f + __expf(-lo2f<T>(gate[ch + j]))) : v[j]);
+            }
+        }
+    });
+}
+
+template <typename T, int DKP, int DVP, bool TOKEN_ROWS>
+static int launch_prompt_attn(const PromptAttnArgs& a, hipStream_t st) {
+    constexpr size_t bytes = 2 * 2 * static_cast<size_t>(kPromptTileKeys) * (DKP + DVP);
+    static_assert(bytes <= 160 * 1024, "LDS");
+    if (bytes > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&prompt_attn_kernel<T, DKP, DVP, TOKEN_ROWS>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
+        if (e != hipSuccess) return static_cast<int>(e);
+    }
+    dim3 grid(a.H, (a.L + kPromptTileRows - 1) / kPromptTileRows, a.B), block(256);
+    hipLaunchKernelGGL((prompt_attn_kernel<T, DKP, DVP, TOKEN_ROWS>), grid, block, bytes, st, a);
+    return static_cast<int>(hipGetLastError());
+}
+
+}  // namespace pq

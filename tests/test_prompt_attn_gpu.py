@@ -1,0 +1,48 @@
+"""Causal attention of a prompt (prompt_attn_kernel) against float64, at the edges of its tiles (128 queries, 64 keys, 16-byte pieces of
+a row).
+
+Tolerance: weights and result are rounded to the dtype, each by at most half a unit in the last place u (2^-8 bf16, 2^-11 fp16); the
+errors of a row's weights are independent, so the relative 2-norm error stays below u."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+UNIT = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+
+
+def reference(q, k, v, scale, start=None, sink=None):
+    """q [B, L, H, D], k [B, Lk, G, D], v [B, Lk, G, Dv] -> [B, L, H, Dv]; the queries are the last of the keys' tokens."""
+    (B, L, H, _), (Lk, G) = q.shape, k.shape[1:3]
+    q, k, v = [t.double().transpose(1, 2) for t in (q, k, v)]
+    k, v = k.repeat_interleave(H // G, 1), v.repeat_interleave(H // G, 1)
+    s = torch.matmul(q, k.transpose(2, 3).contiguous()) * scale
+    i, j = torch.arange(L, device=q.device)[:, None] + (Lk - L), torch.arange(Lk, device=q.device)
+    hidden = (j > i)[None, None].expand(B, 1, L, Lk)
+    if start is not None:
+        hidden = hidden | (j < start[:, None, None, None])
+    s = s.masked_fill(hidden, -math.inf)
+    if sink is not None:
+        s = torch.cat([s, sink.double()[None, :, None, None].expand(B, H, L, 1)], -1)
+    return torch.matmul(s.softmax(-1)[..., :Lk], v).transpose(1, 2)
+
+
+def off(got, want):
+    return float((got.double() - want).norm() / want.norm())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,L,Lk,H,D,Dv,scale", [
+    (1, 1, 1, 1, 128, 128, 0.1), (2, 63, 63, 8, 128, 128, 0.09), (1, 64, 64, 3, 64, 64, 0.2), (1, 65, 65, 8, 128, 128, -0.09), (1, 127, 255, 2, 128, 128, 0.0),
+    (1, 129, 129, 16, 128, 128, 1.0), (2, 200, 333, 5, 72, 40, 0.1), (1, 257, 257, 2, 192, 128, 0.07), (1, 130, 449, 2, 256, 256, 0.06)])
+def test_values_by_channel(B, L, Lk, H, D, Dv, scale, dtype):
+    from polarquant_amd.latent_ops import latent_prefill_attention
+    g = torch.Generator(device="cuda").manual_seed(L + Lk)
+    q, k, v = [torch.randn(B, n, H, d, generator=g, device="cuda").to(dtype) for n, d in ((L, D), (Lk, D), (Lk, Dv))]
+    sink = torch.randn(H, generator=g, device="cuda")
+    start = torch.tensor([0] * (B - 1) + [(Lk - L) // 2], dtype=torch.int32, device="cuda")
+    vt = torch.zeros(B, H, Dv, -(-Lk // 64) * 64, dtype=dtype, device="cuda")
+    vt[..., :Lk] = v.permute(0, 2, 3, 1)
+    got = latent_prefill_attention(q, k, vt, sink, scale, None, start).view(B, L, H, Dv)
+    assert off(got, reference(q, k, v, scale, start, sink)) < UNIT[dtype]
