@@ -393,6 +393,16 @@ int pq_rope_qk(const void *q_lin, int64_t q_token_stride, const void *k_lin, int
                const void *sin_rows, int64_t cos_sin_batch_stride, void *q_out, void *k_out, int B, int L, int N, int Nk,
                int dtype, void *stream);
 
+/* Causal attention of a prompt over half-precision keys and values, the flash-attention call of the prompt pass
+ * (models/modeling_llama_polar.py:106-114): softmax(sm_scale q k^T) v, query l over keys 0 .. l.  q [B, N, L, 128], k, v
+ * [B, Nk, L, 128]; strides: 9 element strides, (batch, head, token) of q, of k, of v, each a multiple of 8 with unit stride
+ * inside a row (transposed views of [B, L, heads, 128] and slices of one projection's output are such tensors); out
+ * [B, L, N, 128] contiguous.  Scores, softmax and sums are float32, the weights enter the second product in the dtype. */
+int pq_prompt_attn(const void *q, const void *k, const void *v, const int64_t *strides, void *out, float sm_scale, int B, int L,
+                   int N, int Nk, int dtype, void *stream);
+int pq_validate_prompt_attn(const void *q, const void *k, const void *v, const int64_t *strides, const void *out, int B, int L,
+                            int N, int Nk, int dtype);
+
 /* ---------------------------------------------------------------------------
  * A — the elementwise steps around the attention call of one decode step, each a
  * chain of 8-12 eager launches on a [B,1,hidden] activation in the reference.

@@ -75,6 +75,8 @@ SIGNATURES = {
     "pq_validate_linear_small_m": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int]),
     "pq_rope_qk": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_void_p,
                            c_int, c_int, c_int, c_int, c_int, c_void_p]),
+    "pq_prompt_attn": (c_int, [c_void_p] * 5 + [c_float] + [c_int] * 5 + [c_void_p]),
+    "pq_validate_prompt_attn": (c_int, [c_void_p] * 5 + [c_int] * 5),
     "pq_qkv_rope_append": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_int64,
                                    c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_int, c_int, c_void_p]),
     "pq_validate_qkv_rope_append": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_int64,

@@ -6,6 +6,7 @@ LlamaPolarGroupAttention.forward computes between RoPE and o_proj
 """
 from __future__ import annotations
 
+import ctypes
 import math
 from typing import Optional
 
@@ -252,4 +253,27 @@ def polar_decode_attention_v4(
             value_resid.data_ptr(), *vptr, v4_cap, mptr, mstride, float(sm_scale), B, N, Nk, rbits, tbits, dt,
             n_splits, min_groups_per_split, ws.data_ptr(), ws.numel() * 4, out.data_ptr(), flags, sptr, _stream_ptr(dev))
     _ffi.check(rc, "pq_decode_attn_v4")
+    return out
+
+
+def prompt_attention_takes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
+    """Whether `prompt_attention` can read these [B, heads, L, 128] tensors as they lie."""
+    return (q.is_cuda and q.dtype in (torch.float16, torch.bfloat16) and q.dtype == k.dtype == v.dtype and q.shape[-1] == 128 and q.shape[2] > 0
+            and k.shape == v.shape == (q.shape[0], k.shape[1], q.shape[2], 128) and 0 < q.shape[0] <= 65535 and q.shape[1] % k.shape[1] == 0
+            and all(t.device == q.device and t.stride(3) == 1 and all(s % 8 == 0 for s in t.stride()[:3]) and t.data_ptr() % 16 == 0 for t in (q, k, v)))
+
+
+def prompt_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sm_scale: Optional[float] = None) -> torch.Tensor:
+    """Causal attention of a prompt: q [B, N, L, 128], k, v [B, Nk, L, 128] (any strides that are multiples of 8, unit stride inside
+    a row) -> [B, L, N, 128], what the reference's flash-attention call returns (models/modeling_llama_polar.py:106-114)."""
+    if not prompt_attention_takes(q, k, v):
+        raise ValueError("polarquant_amd: prompt attention takes half-precision [B, heads, L, 128] tensors on one GPU, strides multiples of 8")
+    B, N, L, _ = q.shape
+    out = torch.empty((B, L, N, 128), dtype=q.dtype, device=q.device)
+    strides = (ctypes.c_int64 * 9)(*q.stride()[:3], *k.stride()[:3], *v.stride()[:3])
+    with torch.cuda.device(q.device):
+        rc = _ffi.lib().pq_prompt_attn(q.data_ptr(), k.data_ptr(), v.data_ptr(), ctypes.cast(strides, ctypes.c_void_p), out.data_ptr(),
+                                       float(sm_scale if sm_scale is not None else 1.0 / math.sqrt(128)), B, L, N, k.shape[1], _dtype_code(q),
+                                       _stream_ptr(q.device))
+    _ffi.check(rc, "pq_prompt_attn")
     return out

@@ -397,6 +397,24 @@ int pq_rope_qk(const void* q_lin, int64_t q_token_stride, const void* k_lin, int
     return err == 0 ? PQ_OK : PQ_ERR_LAUNCH;
 }
 
+int pq_validate_prompt_attn(const void* q, const void* k, const void* v, const int64_t* strides, const void* out, int B, int L,
+                            int N, int Nk, int dtype) {
+    if (!q || !k || !v || !strides || !out) return PQ_ERR_NULL_POINTER;
+    if (B <= 0 || B > 65535 || L <= 0 || (L + 127) / 128 > 65535 || N <= 0 || Nk <= 0 || N > 65535 || N % Nk) return PQ_ERR_BAD_SHAPE;
+    if (dtype != PQ_F16 && dtype != PQ_BF16) return PQ_ERR_BAD_DTYPE;
+    for (int i = 0; i < 9; i++)
+        if (strides[i] < 0 || strides[i] % 8) return PQ_ERR_BAD_STRIDE;
+    if (!aligned(q, 16) || !aligned(k, 16) || !aligned(v, 16) || !aligned(out, 16)) return PQ_ERR_MISALIGNED;
+    return PQ_OK;
+}
+
+int pq_prompt_attn(const void* q, const void* k, const void* v, const int64_t* strides, void* out, float sm_scale, int B, int L,
+                   int N, int Nk, int dtype, void* stream) {
+    if (int rc = pq_validate_prompt_attn(q, k, v, strides, out, B, L, N, Nk, dtype)) return rc;
+    const int err = pq::launch_prompt_attn(q, k, v, strides, out, B, L, N, Nk, sm_scale, dtype, static_cast<hipStream_t>(stream));
+    return err == 0 ? PQ_OK : PQ_ERR_LAUNCH;
+}
+
 int pq_rmsnorm(const void* x, const void* residual, const void* weight, void* y, void* sum_out, int rows, int hidden,
                float eps, int dtype, void* stream) {
     if (!x || !weight || !y) return PQ_ERR_NULL_POINTER;

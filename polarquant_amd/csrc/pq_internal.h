@@ -19,6 +19,9 @@ int launch_selftest(int dtype, unsigned long long* counters, hipStream_t st);
 int launch_quantize_values(const void* v, const int64_t* strides, int dtype, int B, int Nk, int T,
                            int32_t* codes, void* scale, void* mn, int64_t cap, int64_t off, hipStream_t st);
 
+// strides: (batch, head, token) of q, k, v, in elements
+int launch_prompt_attn(const void* q, const void* k, const void* v, const int64_t* strides, void* out, int B, int L, int N, int Nk,
+                       float scale, int dtype, hipStream_t st);
 int launch_rope_qk(const void* q_lin, int64_t q_stride, const void* k_lin, int64_t k_stride, const void* cos_t,
                    const void* sin_t, int64_t cs_batch_stride, void* q_out, void* k_out, int B, int L, int N, int Nk,
                    int dtype, hipStream_t st);

@@ -30,7 +30,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .attention import polar_decode_attention, polar_decode_attention_v4
+from .attention import polar_decode_attention, polar_decode_attention_v4, prompt_attention, prompt_attention_takes
 from .quantize import quantize_and_pack_nbit
 from .values import quantize_values
 
@@ -593,6 +593,10 @@ def _prefill_attention(q, k, v, attention_mask, n_rep, is_causal):
     `attention_mask` [B, L] of {0,1} marks left padding."""
     B, N, L, hd = q.shape
     if attention_mask is None or bool((attention_mask != 0).all()):
+        # the library's flash attention takes twice the time from 512 tokens on (32 heads, 512 / 8192 / 16384 tokens: 34, 1270, 4484
+        # against 18, 564, 2121 us) and the same below; it stays for what the kernel does not take: float32, tensors on the host, gradients
+        if is_causal and not torch.is_grad_enabled() and prompt_attention_takes(q, k, v):
+            return prompt_attention(q, k, v)
         out = F.scaled_dot_product_attention(q, k, v, is_causal=is_causal and L > 1, enable_gqa=n_rep > 1)
     else:
         keep = (attention_mask != 0)[:, None, None, :]

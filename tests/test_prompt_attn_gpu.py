@@ -46,3 +46,38 @@ def test_values_by_channel(B, L, Lk, H, D, Dv, scale, dtype):
     vt[..., :Lk] = v.permute(0, 2, 3, 1)
     got = latent_prefill_attention(q, k, vt, sink, scale, None, start).view(B, L, H, Dv)
     assert off(got, reference(q, k, v, scale, start, sink)) < UNIT[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,L,N,Nk,layout", [(1, 1, 4, 4, "tokens"), (2, 63, 8, 2, "heads"), (1, 64, 7, 1, "tokens"), (3, 65, 28, 4, "slices"),
+                                             (1, 128, 32, 8, "slices"), (2, 129, 5, 5, "expanded"), (1, 515, 16, 8, "tokens")])
+def test_values_by_token(B, L, N, Nk, layout, dtype):
+    """The strides that callers have: transposed views of [B, L, heads, 128], contiguous heads, slices of one projection, a batch that
+    is one expanded sequence."""
+    from polarquant_amd.attention import prompt_attention, prompt_attention_takes
+    g = torch.Generator(device="cuda").manual_seed(7 * L)
+    if layout == "slices":
+        p = torch.randn(B, L, N + 2 * Nk, 128, generator=g, device="cuda").to(dtype).transpose(1, 2)
+        q, k, v = p[:, :N], p[:, N:N + Nk], p[:, N + Nk:]
+    else:
+        q, k, v = [torch.randn(1 if layout == "expanded" else B, L, n, 128, generator=g, device="cuda").to(dtype).transpose(1, 2) for n in (N, Nk, Nk)]
+        if layout == "heads":
+            q, k, v = [t.contiguous() for t in (q, k, v)]
+        if layout == "expanded":
+            q, k, v = [t.expand(B, -1, -1, -1) for t in (q, k, v)]
+    assert prompt_attention_takes(q, k, v)
+    got = prompt_attention(q, k, v)
+    assert got.shape == (B, L, N, 128) and off(got, reference(*[t.transpose(1, 2) for t in (q, k, v)], 128 ** -0.5)) < UNIT[dtype]
+
+
+def test_what_prompt_attention_refuses():
+    from polarquant_amd.attention import prompt_attention_takes
+    x = torch.randn(2, 4, 70, 128, device="cuda").bfloat16()
+    assert prompt_attention_takes(x, x[:, :2], x[:, :2])
+    assert not prompt_attention_takes(x, x[:, :3], x[:, :3])                       # heads that do not share evenly
+    assert not prompt_attention_takes(x.float(), x.float(), x.float())
+    assert not prompt_attention_takes(x[..., :64], x[..., :64], x[..., :64])
+    y = torch.randn(2 * 4 * 70 * 132, device="cuda").bfloat16().view(2, 4, 70, 132)
+    assert not prompt_attention_takes(y[..., :128], x, x)                          # rows 132 apart
+    z = torch.randn(2 * 4 * 70 * 128 + 4, device="cuda").bfloat16()[4:].view(2, 4, 70, 128)
+    assert not prompt_attention_takes(z, x, x)                                     # 8-byte aligned
