@@ -10,25 +10,32 @@ int launch_head_linear_mfma(const HeadLinearArgs& a, int dtype, hipStream_t st) 
     const int kstep = m8 ? 64 : 32;
     int ks = (m8 && a.K >= 8192) ? 8 : 4;
     while (ks > 1 && ((a.K % (kstep * ks)) != 0 || a.K / (kstep * ks) < 2)) ks >>= 1;
-    dim3 grid(a.N / 16, a.heads), block(kWave * ks);
+    const int nt = m8 && a.heads == 1 ? small_m8_row_tiles(a.N, ks, 1) : 2;      // (several heads: their K is short, nothing is gained)
+    dim3 grid(a.N / (8 * nt), a.heads), block(kWave * ks);
     const HeadEpi he{a.x_head, static_cast<int64_t>(a.N) * a.K, a.y_head, static_cast<const uint16_t*>(a.gate), a.gate_row};
-#define PQ_H(KERNEL, T, KS, S, E)                                                                                    \
-    hipLaunchKernelGGL((KERNEL<T, KS, false, S, 1 + E>), grid, block, 0, st, (const uint16_t*)a.x, a.x_row,          \
+#define PQ_H(KERNEL)                                                                                                 \
+    hipLaunchKernelGGL((KERNEL), grid, block, 0, st, (const uint16_t*)a.x, a.x_row,                                  \
                        (const uint16_t*)a.w, nullptr, nullptr, (uint16_t*)a.y, a.y_row, a.M, a.K, he)
-#define PQ_H8(T, E)                                                                                                  \
+#define PQ_HN(T, E, NT)                                                                                              \
     do {                                                                                                             \
-        if (ks == 8) PQ_H(small_m8_linear_kernel, T, 8, 2, E);                                                       \
-        else if (ks == 4) PQ_H(small_m8_linear_kernel, T, 4, 1, E);                                                  \
-        else if (ks == 2) PQ_H(small_m8_linear_kernel, T, 2, 1, E);                                                  \
-        else PQ_H(small_m8_linear_kernel, T, 1, 1, E);                                                               \
+        if (ks == 8) PQ_H((small_m8_linear_kernel<T, 8, false, NT == 2 ? 2 : 1, 1 + E, NT>));                        \
+        else if (ks == 4) PQ_H((small_m8_linear_kernel<T, 4, false, 1, 1 + E, NT>));                                 \
+        else if (ks == 2) PQ_H((small_m8_linear_kernel<T, 2, false, 1, 1 + E, NT>));                                 \
+        else PQ_H((small_m8_linear_kernel<T, 1, false, 1, 1 + E, NT>));                                              \
     } while (0)
 #define PQ_H16(T, E)                                                                                                 \
     do {                                                                                                             \
-        if (ks == 4) PQ_H(small_m_linear_kernel, T, 4, 4, E);                                                        \
-        else if (ks == 2) PQ_H(small_m_linear_kernel, T, 2, 4, E);                                                   \
-        else PQ_H(small_m_linear_kernel, T, 1, 4, E);                                                                \
+        if (ks == 4) PQ_H((small_m_linear_kernel<T, 4, false, 4, 1 + E>));                                           \
+        else if (ks == 2) PQ_H((small_m_linear_kernel<T, 2, false, 4, 1 + E>));                                      \
+        else PQ_H((small_m_linear_kernel<T, 1, false, 4, 1 + E>));                                                   \
     } while (0)
-#define PQ_HE(T, E) do { if (m8) PQ_H8(T, E); else PQ_H16(T, E); } while (0)
+#define PQ_HE(T, E)                                                                                                  \
+    do {                                                                                                             \
+        if (!m8) PQ_H16(T, E);                                                                                       \
+        else if (nt == 8) PQ_HN(T, E, 8);                                                                            \
+        else if (nt == 4) PQ_HN(T, E, 4);                                                                            \
+        else PQ_HN(T, E, 2);                                                                                         \
+    } while (0)
 #define PQ_HT(T)                                                                                                     \
     do {                                                                                                             \
         if (a.epilogue == kEpiReluSq) PQ_HE(T, kEpiReluSq);                                                          \
@@ -40,7 +47,7 @@ int launch_head_linear_mfma(const HeadLinearArgs& a, int dtype, hipStream_t st) 
 #undef PQ_HT
 #undef PQ_HE
 #undef PQ_H16
-#undef PQ_H8
+#undef PQ_HN
 #undef PQ_H
     return static_cast<int>(hipGetLastError());
 }

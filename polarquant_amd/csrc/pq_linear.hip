@@ -44,7 +44,7 @@ __global__ __launch_bounds__(kWave * KSPLIT) void qkv_rope_append_kernel(
 
     floatx4_l acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
     auto ldw = [](const uint16_t* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4_l*>(p)); };
-    auto load = [&](Stage8T<false, kStage>& st, int s0) {
+    auto load = [&](Stage8T<false, 2, kStage>& st, int s0) {
         static_for<kStage>([&](auto U) {
             constexpr int u = decltype(U)::value;
             st.w[0][u] = ldw(wp + (s0 + u) * 64);
@@ -52,7 +52,7 @@ __global__ __launch_bounds__(kWave * KSPLIT) void qkv_rope_append_kernel(
             st.x[u] = *reinterpret_cast<const u32x4_l*>(xp + (s0 + u) * 64);
         });
     };
-    auto compute = [&](const Stage8T<false, kStage>& st) {
+    auto compute = [&](const Stage8T<false, 2, kStage>& st) {
         static_for<kStage>([&](auto U) {
             constexpr int u = decltype(U)::value;
             acc[0] = mfma32<T>(st.w[0][u], st.x[u], acc[0]);
@@ -61,7 +61,7 @@ __global__ __launch_bounds__(kWave * KSPLIT) void qkv_rope_append_kernel(
     };
     const int full = steps / kStage;
     if (full > 0) {
-        Stage8T<false, kStage> sa, sb;
+        Stage8T<false, 2, kStage> sa, sb;
         load(sa, 0);
         int st = 0;
         while (st + 2 < full) {
@@ -170,8 +170,8 @@ int launch_qkv_rope_append(const void* x, int64_t x_stride, const void* w, const
 
 // Launch shapes measured at the decode shapes of Llama-3-8B (K-split 4 / 8 / 16 and stages of 1 / 2 / 4 / 8
 // loads were swept): the 16-row kernel runs four wavefronts per workgroup with stages of 4 (2 when gated); the
-// M <= 8 kernel four wavefronts with stages of 1, or eight with stages of 2 when K >= 8192 (down_proj).
-// K / KSPLIT must stay a whole number of k-steps.
+// M <= 8 kernel four wavefronts, or eight when K >= 8192 (down_proj), with stages of 1 (2 with eight wavefronts on two row tiles).
+// K / KSPLIT must stay a whole number of k-steps.  The split of K, and with it every sum's order, depends on K alone.
 int launch_small_m_linear(const void* x, int64_t x_stride, const void* w, const void* w_up, const void* bias, void* y,
                           int64_t y_stride, int M, int N, int K, int dtype, hipStream_t st) {
     const bool gated = w_up != nullptr;
@@ -179,33 +179,35 @@ int launch_small_m_linear(const void* x, int64_t x_stride, const void* w, const 
     const int kstep = m8 ? 64 : 32;
     int ks = (m8 && K >= 8192) ? 8 : 4;
     while (ks > 1 && (K % (kstep * ks)) != 0) ks >>= 1;
-    dim3 grid(N / 16), block(kWave * ks);
-#define PQ_LAUNCH_L(KERNEL, T, KS, G, S)                                                                             \
-    hipLaunchKernelGGL((KERNEL<T, KS, G, S>), grid, block, 0, st, (const uint16_t*)x, x_stride,                      \
+    const int nt = m8 ? small_m8_row_tiles(N, ks, gated ? 2 : 1) : 2;
+    dim3 grid(N / (8 * nt)), block(kWave * ks);
+#define PQ_LAUNCH_L(KERNEL)                                                                                          \
+    hipLaunchKernelGGL((KERNEL), grid, block, 0, st, (const uint16_t*)x, x_stride,                                   \
                        (const uint16_t*)w, (const uint16_t*)w_up, (const uint16_t*)bias, (uint16_t*)y, y_stride, M, K, HeadEpi{})
-#define PQ_LAUNCH_M8(T, G)                                                                                           \
+#define PQ_LAUNCH_N(T, G, NT)                                                                                        \
     do {                                                                                                             \
-        if (ks == 8) PQ_LAUNCH_L(small_m8_linear_kernel, T, 8, G, 2);                                                \
-        else if (ks == 4) PQ_LAUNCH_L(small_m8_linear_kernel, T, 4, G, 1);                                           \
-        else if (ks == 2) PQ_LAUNCH_L(small_m8_linear_kernel, T, 2, G, 1);                                           \
-        else PQ_LAUNCH_L(small_m8_linear_kernel, T, 1, G, 1);                                                        \
+        if (ks == 8) PQ_LAUNCH_L((small_m8_linear_kernel<T, 8, G, NT == 2 ? 2 : 1, 0, NT>));                         \
+        else if (ks == 4) PQ_LAUNCH_L((small_m8_linear_kernel<T, 4, G, 1, 0, NT>));                                  \
+        else if (ks == 2) PQ_LAUNCH_L((small_m8_linear_kernel<T, 2, G, 1, 0, NT>));                                  \
+        else PQ_LAUNCH_L((small_m8_linear_kernel<T, 1, G, 1, 0, NT>));                                               \
     } while (0)
 #define PQ_LAUNCH_M16(T, G, S)                                                                                       \
     do {                                                                                                             \
-        if (ks == 4) PQ_LAUNCH_L(small_m_linear_kernel, T, 4, G, S);                                                 \
-        else if (ks == 2) PQ_LAUNCH_L(small_m_linear_kernel, T, 2, G, S);                                            \
-        else PQ_LAUNCH_L(small_m_linear_kernel, T, 1, G, S);                                                         \
+        if (ks == 4) PQ_LAUNCH_L((small_m_linear_kernel<T, 4, G, S>));                                               \
+        else if (ks == 2) PQ_LAUNCH_L((small_m_linear_kernel<T, 2, G, S>));                                          \
+        else PQ_LAUNCH_L((small_m_linear_kernel<T, 1, G, S>));                                                       \
     } while (0)
 #define PQ_LAUNCH_LM(T)                                                                                              \
     do {                                                                                                             \
-        if (m8) { if (gated) PQ_LAUNCH_M8(T, true); else PQ_LAUNCH_M8(T, false); }                                   \
-        else    { if (gated) PQ_LAUNCH_M16(T, true, 2); else PQ_LAUNCH_M16(T, false, 4); }                           \
+        if (m8 && gated) { if (nt == 4) PQ_LAUNCH_N(T, true, 4); else PQ_LAUNCH_N(T, true, 2); }                     \
+        else if (m8)     { if (nt == 8) PQ_LAUNCH_N(T, false, 8); else if (nt == 4) PQ_LAUNCH_N(T, false, 4); else PQ_LAUNCH_N(T, false, 2); } \
+        else             { if (gated) PQ_LAUNCH_M16(T, true, 2); else PQ_LAUNCH_M16(T, false, 4); }                  \
     } while (0)
     if (dtype == 0) PQ_LAUNCH_LM(F16);
     else PQ_LAUNCH_LM(BF16);
 #undef PQ_LAUNCH_LM
 #undef PQ_LAUNCH_M16
-#undef PQ_LAUNCH_M8
+#undef PQ_LAUNCH_N
 #undef PQ_LAUNCH_L
     return static_cast<int>(hipGetLastError());
 }

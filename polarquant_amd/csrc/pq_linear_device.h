@@ -190,14 +190,36 @@ __global__ __launch_bounds__(kWave * KSPLIT) void small_m_linear_kernel(
 // y[m][n] = C[n][m] + C[n + 8][m + 8] and the off-diagonal quarters are ignored.  No lane loads a
 // duplicate row of x, a wavefront load of W covers 8 rows x 128 contiguous bytes (whole cache lines,
 // which is what lets the weight stream carry the non-temporal hint: with half lines the hint drops a
-// line before its second half is asked for), and the workgroup's 16 rows of W are two such tiles that
-// share one x operand: per 64-wide step two W loads and one x load instead of four and four.
-template <bool GATED, int kStage>
+// line before its second half is asked for), and the workgroup's 8 NT rows of W are NT such tiles that
+// share one x operand.
+//
+// NT: what a compute unit can have on its way from memory is about its share of the HBM rate, so the unit with the most rows sets
+// the time, and x, which every workgroup reads from L2, comes on top (without the x loads 28672 x 4096 takes 37.4 us, the plain
+// stream's time).  small_m8_row_tiles therefore takes the NT for which the fullest unit's W and x bytes are least.  Measured in a
+// chain of calls, 8 rows, NT 2 / 4 / 8 in us: 6144 x 4096 13.5 / 12.3 / 23.9; 10240 x 4096 20.7 / 22.6 / 24.9; 21504 x 4096
+// 37.6 / 34.9 / 38.6; 43136 x 4096 65.6 / 62.3 / 59.1; 32768 x 4096 50.3 / 45.8 / 44.8.  (x kept in registers by persistent
+// workgroups: 41 / 59 us at N 28672 / 43136, and 10.2 instead of 8.8 at 4096.)
+inline int small_m8_row_tiles(int N, int ksplit, int matrices) {
+    constexpr int kUnits = 256;
+    int best = 2;
+    double least = 0.0;
+    for (int nt = 2; nt * matrices <= 8; nt *= 2) {
+        if (N % (8 * nt)) break;
+        const int groups = N / (8 * nt);
+        // too few wavefronts to keep loads on the way: 3 per unit with four tiles' loads each, 7 with eight
+        if (nt > 2 && groups * ksplit < (nt * matrices == 8 ? 7 : 3) * kUnits) break;
+        const double cost = ((groups + kUnits - 1) / kUnits) * nt * (1.0 + 0.42 / (nt * matrices));
+        if (nt == 2 || cost < least) { best = nt; least = cost; }
+    }
+    return best;
+}
+
+template <bool GATED, int NT, int kStage>
 struct Stage8T {
-    u32x4_l w[2][kStage], x[kStage], u[GATED ? 2 : 1][GATED ? kStage : 1];
+    u32x4_l w[NT][kStage], x[kStage], u[GATED ? NT : 1][GATED ? kStage : 1];
 };
 
-template <typename T, int KSPLIT, bool GATED, int kStage, int EPI = 0>
+template <typename T, int KSPLIT, bool GATED, int kStage, int EPI = 0, int NT = 2>
 __global__ __launch_bounds__(kWave * KSPLIT) void small_m8_linear_kernel(
     const uint16_t* __restrict__ x, int64_t x_stride, const uint16_t* __restrict__ w, const uint16_t* __restrict__ w_up,
     const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, int64_t y_stride, int M, int K, HeadEpi he) {
@@ -205,47 +227,45 @@ __global__ __launch_bounds__(kWave * KSPLIT) void small_m8_linear_kernel(
         x += blockIdx.y * he.x_head;
         w += blockIdx.y * he.w_head;
     }
-    __shared__ float part[KSPLIT][GATED ? 4 : 2][4][kWave];
+    __shared__ float part[KSPLIT][(GATED ? 2 : 1) * NT][4][kWave];
     const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
     const int r = lane & 15, g = lane >> 4;
     const int row = r & 7, chunk = (r >> 3) * 4 + g;       // W row inside an 8-row tile == x row; 16-byte piece of the step
-    const int n0 = blockIdx.x * 16;
+    const int n0 = blockIdx.x * 8 * NT;
     const int klen = K / KSPLIT, steps = klen / 64;
     const int m = row < M ? row : 0;                       // tile columns >= M repeat row 0 and are never stored
     const size_t koff = static_cast<size_t>(wv) * klen + 8 * chunk;
     const uint16_t* wp = w + static_cast<size_t>(n0 + row) * K + koff;
     const uint16_t* up = GATED ? w_up + static_cast<size_t>(n0 + row) * K + koff : nullptr;
     const uint16_t* xp = x + static_cast<size_t>(m) * x_stride + koff;
-    const size_t half_tile = static_cast<size_t>(8) * K;   // rows n0 + 8 .. n0 + 15
+    const size_t tile = static_cast<size_t>(8) * K;
 
-    floatx4_l acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}}, acu[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+    floatx4_l acc[NT], acu[GATED ? NT : 1];
+    static_for<NT>([&](auto I) {
+        acc[I] = floatx4_l{0, 0, 0, 0};
+        if constexpr (GATED) acu[I] = floatx4_l{0, 0, 0, 0};
+    });
     auto ldw = [](const uint16_t* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4_l*>(p)); };
-    auto load = [&](Stage8T<GATED, kStage>& st, int s0) {          // branch-free, see small_m_linear_kernel
+    auto load = [&](Stage8T<GATED, NT, kStage>& st, int s0) {      // branch-free, see small_m_linear_kernel
         static_for<kStage>([&](auto U) {
             constexpr int u = decltype(U)::value;
-            st.w[0][u] = ldw(wp + (s0 + u) * 64);
-            st.w[1][u] = ldw(wp + half_tile + (s0 + u) * 64);
-            if constexpr (GATED) {
-                st.u[0][u] = ldw(up + (s0 + u) * 64);
-                st.u[1][u] = ldw(up + half_tile + (s0 + u) * 64);
-            }
+            static_for<NT>([&](auto I) { st.w[I][u] = ldw(wp + I * tile + (s0 + u) * 64); });
+            if constexpr (GATED) static_for<NT>([&](auto I) { st.u[I][u] = ldw(up + I * tile + (s0 + u) * 64); });
             st.x[u] = *reinterpret_cast<const u32x4_l*>(xp + (s0 + u) * 64);
         });
     };
-    auto compute = [&](const Stage8T<GATED, kStage>& st) {
+    auto compute = [&](const Stage8T<GATED, NT, kStage>& st) {
         static_for<kStage>([&](auto U) {
             constexpr int u = decltype(U)::value;
-            acc[0] = mfma32<T>(st.w[0][u], st.x[u], acc[0]);
-            acc[1] = mfma32<T>(st.w[1][u], st.x[u], acc[1]);
-            if constexpr (GATED) {
-                acu[0] = mfma32<T>(st.u[0][u], st.x[u], acu[0]);
-                acu[1] = mfma32<T>(st.u[1][u], st.x[u], acu[1]);
-            }
+            static_for<NT>([&](auto I) {
+                acc[I] = mfma32<T>(st.w[I][u], st.x[u], acc[I]);
+                if constexpr (GATED) acu[I] = mfma32<T>(st.u[I][u], st.x[u], acu[I]);
+            });
         });
     };
     const int full = steps / kStage;
     if (full > 0) {
-        Stage8T<GATED, kStage> sa, sb;
+        Stage8T<GATED, NT, kStage> sa, sb;
         load(sa, 0);
         int st = 0;
         while (st + 2 < full) {
@@ -265,25 +285,23 @@ __global__ __launch_bounds__(kWave * KSPLIT) void small_m8_linear_kernel(
     }
     for (int s1 = full * kStage; s1 < steps; s1++) {
         const u32x4_l xv1 = *reinterpret_cast<const u32x4_l*>(xp + s1 * 64);
-        acc[0] = mfma32<T>(ldw(wp + s1 * 64), xv1, acc[0]);
-        acc[1] = mfma32<T>(ldw(wp + half_tile + s1 * 64), xv1, acc[1]);
-        if constexpr (GATED) {
-            acu[0] = mfma32<T>(ldw(up + s1 * 64), xv1, acu[0]);
-            acu[1] = mfma32<T>(ldw(up + half_tile + s1 * 64), xv1, acu[1]);
-        }
+        static_for<NT>([&](auto I) {
+            acc[I] = mfma32<T>(ldw(wp + I * tile + s1 * 64), xv1, acc[I]);
+            if constexpr (GATED) acu[I] = mfma32<T>(ldw(up + I * tile + s1 * 64), xv1, acu[I]);
+        });
     }
+    static_for<NT>([&](auto I) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        part[wv][0][i][lane] = acc[0][i];
-        part[wv][1][i][lane] = acc[1][i];
-        if constexpr (GATED) { part[wv][2][i][lane] = acu[0][i]; part[wv][3][i][lane] = acu[1][i]; }
-    }
+        for (int i = 0; i < 4; i++) {
+            part[wv][I][i][lane] = acc[I][i];
+            if constexpr (GATED) part[wv][NT + I][i][lane] = acu[I][i];
+        }
+    });
     __syncthreads();
     // lane (r < 8, g < 2) owns outputs y[r][n0 + 8h + 4g + i] (h: which 8-row tile), each the sum of the tile's
     // entry (row 4g + i, column r) and its diagonal partner (row + 8, column + 8), which lane + 40 holds
-    if (wv != 0 || r >= 8 || r >= M || g >= 2) return;
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
+    if (r >= 8 || r >= M || g >= 2) return;
+    for (int h = wv; h < NT; h += KSPLIT) {
         if constexpr (EPI != 0) {
             float s4[4];
 #pragma unroll
@@ -292,7 +310,7 @@ __global__ __launch_bounds__(kWave * KSPLIT) void small_m8_linear_kernel(
 #pragma unroll
                 for (int k = 0; k < KSPLIT; k++) s4[i] += part[k][h][i][lane] + part[k][h][i][lane + 40];
             }
-            store_head<T, EPI>(s4, y, y_stride, r, n0 + 8 * h + 4 * g, static_cast<int>(gridDim.x) * 16, he);
+            store_head<T, EPI>(s4, y, y_stride, r, n0 + 8 * h + 4 * g, static_cast<int>(gridDim.x) * 8 * NT, he);
             continue;
         }
         uint16_t out[4];
@@ -302,7 +320,7 @@ __global__ __launch_bounds__(kWave * KSPLIT) void small_m8_linear_kernel(
 #pragma unroll
             for (int k = 0; k < KSPLIT; k++) {
                 s += part[k][h][i][lane] + part[k][h][i][lane + 40];
-                if constexpr (GATED) t += part[k][2 + h][i][lane] + part[k][2 + h][i][lane + 40];
+                if constexpr (GATED) t += part[k][NT + h][i][lane] + part[k][NT + h][i][lane + 40];
             }
             if constexpr (GATED) {
                 const float gv = rnd_l<T>(s), uv = rnd_l<T>(t);

@@ -149,3 +149,36 @@ def test_qkv_rope_append_equals_projection_then_rotation(gpu, dtype, B, N, Nk, K
     k3, v3 = fill.clone(), fillv.clone()
     assert torch.equal(qkv_rope_append(wide[..., :K], w, b, cos, sin, pos, k3, k_row, v3, pos, N, Nk), q_ref)
     assert torch.equal(k3, k1) and torch.equal(v3, v1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(8, 6144, 256), (3, 10240, 512), (8, 28672, 256), (1, 28704, 256), (8, 28688, 320), (5, 28672, 8192)])
+def test_rows_per_workgroup_do_not_change_the_sums(gpu, dtype, M, N, K):
+    """16, 32 and 64 rows of W per workgroup (by N): a row's sum is the same as in a product of the first 512 rows alone."""
+    g = torch.Generator(device=gpu).manual_seed(N + K)
+    x = torch.randn(M, K, generator=g, device=gpu).to(dtype)
+    w = (torch.randn(N, K, generator=g, device=gpu) * 0.05).to(dtype)
+    b = torch.randn(N, generator=g, device=gpu).to(dtype)
+    y = linear_small_m(x, w, b)
+    for n in (0, N // 2 // 16 * 16, N - 512):
+        assert torch.equal(y[:, n:n + 512], linear_small_m(x, w[n:n + 512], b[n:n + 512]))
+    _check(y, F.linear(x.double(), w.double(), b.double()), dtype)
+    up = (torch.randn(N, K, generator=g, device=gpu) * 0.05).to(dtype)
+    z = linear_small_m(x, w, up_weight=up)
+    assert torch.equal(z[:, -512:], linear_small_m(x, w[-512:], up_weight=up[-512:]))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_linear_module_takes_the_kernel_only_where_it_may(gpu, dtype):
+    """The module's result is the kernel's for few rows in half precision without gradients, torch's otherwise."""
+    from polarquant_amd.modeling_common import Linear
+    g = torch.Generator(device=gpu).manual_seed(3)
+    lin = Linear(160, 64, bias=True).to(gpu, dtype)
+    wide = torch.randn(2, 9, 168, generator=g, device=gpu).to(dtype)
+    with torch.no_grad():
+        for x in (wide[:, :8, :160], wide[:1, :, 8:], wide[:, -1:, 4:164], wide[:, :, :160], wide[0, 0, :160]):     # 16, 9, 2 (8-byte aligned), 18, 1 rows
+            _check(lin(x), F.linear(x.double(), lin.weight.double(), lin.bias.double()), dtype)
+        assert torch.equal(lin(wide[:1, :, :160].contiguous()), linear_small_m(wide[:1, :, :160].contiguous(), lin.weight, lin.bias))
+        assert lin(wide[:0, :, :160]).shape == (0, 9, 64)
+    assert lin(wide[:1, :, :160].clone().requires_grad_()).requires_grad
+    assert Linear(160, 64)(torch.randn(3, 160)).shape == (3, 64)
