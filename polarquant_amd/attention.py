@@ -159,6 +159,8 @@ def polar_decode_attention(
         min_gps = min_groups_per_split
     if n_splits is None:
         n_splits = plan_splits(B, Nk, max_groups, dev)
+        if 1 < n_splits == max_groups:
+            n_splits += 1                  # one group per slice: the residual keys get a slice of their own too
     ws = _pick_workspace(workspace, B, N, n_splits, dev)
     if out is None:
         out = torch.empty((B, N, 1, hd), dtype=query_states.dtype, device=dev)
@@ -237,6 +239,8 @@ def polar_decode_attention_v4(
             n_splits = balanced_slots(B, Nk, max_groups, total_groups, (8 if N // Nk <= 4 else 4) * _num_cus(dev), r_cap)
     if n_splits is None:
         n_splits = _ffi.lib().pq_decode_attn_v4_plan(B, N, Nk, max(max_groups, 1), _num_cus(dev))
+        if 1 < n_splits == max_groups:
+            n_splits += 1
     sptr = None
     if status is not None:
         if status.dtype != torch.int32 or status.device != dev or status.numel() != 1:

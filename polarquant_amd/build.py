@@ -25,6 +25,7 @@ LIB = os.path.join(HERE, "libpolarquant_hip.so")
 # many template instantiations build side by side
 UNITS = [("pq_attn.hip", ("PQ_DTYPE=0",), ".f16"), ("pq_attn.hip", ("PQ_DTYPE=1",), ".bf16"),
          ("pq_attn_pair.hip", ("PQ_DTYPE=0",), ".f16"), ("pq_attn_pair.hip", ("PQ_DTYPE=1",), ".bf16"),
+         ("pq_attn_group.hip", ("PQ_DTYPE=0",), ".f16"), ("pq_attn_group.hip", ("PQ_DTYPE=1",), ".bf16"),
          ("pq_scores.hip", (), ""), ("pq_quantize.hip", (), ""), ("pq_linear.hip", (), ""), ("pq_attn_common.hip", (), ""),
          ("pq_capi.hip", (), ""), ("pq_values.hip", (), ""), ("pq_decode_ops.hip", (), ""), ("pq_prompt_attn.hip", (), "")]
 SOURCES = sorted({u[0] for u in UNITS})

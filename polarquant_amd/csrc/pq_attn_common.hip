@@ -97,8 +97,19 @@ static int device_compute_units() {
     return cus[dev];
 }
 
+// Calls of few, short slices run eight wavefronts per slice.  Both sides, attention kernel alone, us (pairs / groups): 120 slices of one
+// group 11.3 / 8.6, 248 slices 11.4 / 8.8, with 7 heads per KV head 64 slices 13.4 / 10.4, 252 slices 13.6 / 11.3; 504 slices 11.7 /
+// 11.9, 744 slices 12.2 / 15.8 (a unit then has more workgroups than it holds); a slice of three groups 12 / 12.
+constexpr long long kGroupSlices = 320;
+static bool runs_groups(const AttnArgs& a) {
+    if (a.tbits > 4 || a.single_wave || a.silent_scorer || static_cast<long long>(a.n_splits) * a.B * a.Nk > kGroupSlices) return false;
+    const int groups = a.n_groups_per_seq ? a.group_capacity : a.n_groups < a.group_capacity ? a.n_groups : a.group_capacity;
+    return groups <= 2 * a.n_splits && a.min_groups_per_split <= 2;
+}
+
 int launch_attn_partials(const AttnArgs& a, hipStream_t st) {
     const int rep = a.N / a.Nk;
+    if (runs_groups(a)) return a.dtype == 0 ? launch_attn_group_f16(a, st) : launch_attn_group_bf16(a, st);
     // half-precision values and at most 16 angle bins: a scorer / accumulator pair of wavefronts per slice or segment.
     // (4-bit values stay with one wavefront per slice, two per SIMD: a paired form of that kernel at four wavefronts per
     // SIMD was measured no faster -- the vector ALU's total work bounds it, however it is spread over wavefronts.)

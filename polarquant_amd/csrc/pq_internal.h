@@ -79,6 +79,9 @@ int launch_attn_merge(const float* ws, int B, int N, int n_splits, int dtype, vo
 //   pq_attn_pair.hip: a scorer / accumulator pair of wavefronts per slice, the default for half-precision values
 int launch_attn_pair_f16(const AttnArgs& a, int total, hipStream_t st);
 int launch_attn_pair_bf16(const AttnArgs& a, int total, hipStream_t st);
+//   pq_attn_group.hip: eight wavefronts per slice, for calls of few slices
+int launch_attn_group_f16(const AttnArgs& a, hipStream_t st);
+int launch_attn_group_bf16(const AttnArgs& a, hipStream_t st);
 //   pq_attn.hip: one wavefront per slice (PQ_SINGLE_WAVEFRONT, 4-bit values, more than 16 angle bins)
 int launch_attn_one_f16(const AttnArgs& a, int total, hipStream_t st);
 int launch_attn_one_bf16(const AttnArgs& a, int total, hipStream_t st);

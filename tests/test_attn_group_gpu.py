@@ -1,0 +1,101 @@
+"""Decode attention of few slices (attn_group_kernel: eight wavefronts per slice) at its edges, against the float64 oracle and against
+the kernels that serve larger calls, which the same inputs reach through more slots than that kernel takes."""
+import pytest
+import torch
+
+from oracle import polar_oracle as po
+from polarquant_amd import workloads as wl
+from polarquant_amd.attention import polar_decode_attention, polar_decode_attention_v4
+from polarquant_amd.quantize import convert_codes6
+
+pytestmark = pytest.mark.gpu
+FEW = 320                   # slices the kernel takes (kGroupSlices)
+
+
+def inputs(B, N, Nk, groups, resid, rbits, tbits, dtype, seed, cap=128):
+    g = torch.Generator().manual_seed(seed)
+    L = groups * 128 + resid
+    k = wl.make_keys(B, Nk, L, 5e5, g, dtype) if L else torch.zeros(B, Nk, 0, 128, dtype=dtype)
+    q, v = wl.make_half((B, N, 1, 128), g, dtype), wl.make_half((B, Nk, L, 128), g, dtype)
+    codes = po.quantize_and_pack_nbit(k[:, :, :groups * 128].contiguous(), rbits, tbits) if groups else None
+    kres = torch.zeros(B, Nk, cap, 128, dtype=dtype)
+    kres[:, :, :resid] = k[:, :, groups * 128:]
+    return q, codes, kres, v
+
+
+def close(got, want, dtype):
+    """fp16: the parity bar.  bf16: a window key's score is rounded to the dtype before it is scaled; scores reach 100 here, where half a
+    unit is 0.25, so that a weight is off by up to 0.25 / sqrt(128) = 2.2 %, beside the roundings of weight and result (2^-9 each)."""
+    got, want = got.double().cpu(), want.double()
+    if dtype == torch.float16:
+        return bool(((got - want).abs() <= 1e-3 + 1e-2 * want.abs()).all())
+    return float((got - want).norm() / want.norm()) < 2.6e-2
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,N,Nk,groups,resid,rbits,tbits,masked", [
+    (1, 8, 8, 0, 1, 4, 4, False), (2, 8, 2, 0, 128, 4, 4, True), (1, 7, 1, 1, 0, 4, 4, False), (1, 28, 4, 1, 17, 3, 3, True), (2, 16, 8, 2, 128, 4, 4, False),
+    (1, 15, 3, 3, 127, 5, 2, True), (1, 12, 2, 5, 16, 6, 1, False), (3, 24, 3, 4, 15, 4, 4, True), (1, 32, 8, 9, 65, 4, 3, False)])
+def test_against_the_oracle_and_the_other_kernels(gpu, dtype, B, N, Nk, groups, resid, rbits, tbits, masked):
+    q, codes, kres, v = inputs(B, N, Nk, groups, resid, rbits, tbits, dtype, 10 * groups + resid)
+    L = groups * 128 + resid
+    mask = None
+    if masked:
+        mask = torch.ones(B, L, dtype=torch.uint8)
+        mask[0, :L // 3] = 0
+        mask[-1, L - 1:] = 1
+    want = po.decode_attention_exact(q, kres[:, :, :resid], *(codes or [None] * 5), v, attention_mask=mask, rbits=rbits, tbits=tbits)
+    dev = lambda t: None if t is None else t.to(gpu)
+    cache = [dev(t) for t in codes] if codes else [None] * 5
+    run = lambda **kw: polar_decode_attention(q.to(gpu), *cache, kres.to(gpu), v.to(gpu), groups, resid, attention_mask=dev(mask), rbits=rbits, tbits=tbits, **kw)
+    few, many = FEW // (B * Nk), FEW // (B * Nk) + 1
+    for name, got in (("default", run()), ("one slice", run(n_splits=1)), ("two groups a slice", run(n_splits=max(1, groups // 2))), ("empty slots", run(n_splits=few)),
+                      ("pairs", run(n_splits=many)), ("single wavefront", run(single_wavefront=True)),
+                      ("balanced", run(n_groups_per_seq=torch.full((B,), groups, dtype=torch.int32, device=gpu),
+                                       n_resid_per_seq=torch.full((B,), resid, dtype=torch.int32, device=gpu)))):
+        assert close(got, want, dtype), name
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_ragged_counts_and_a_long_window(gpu, dtype):
+    """Per-sequence counts from nothing quantized to the capacity, and a window of more than 128 residual keys."""
+    B, N, Nk, groups, cap = 4, 8, 2, 3, 300
+    q, codes, _, v = inputs(B, N, Nk, groups, 0, 4, 4, dtype, 5)
+    g = torch.Generator().manual_seed(6)
+    kres = wl.make_half((B, Nk, cap, 128), g, dtype)
+    v = torch.cat([v, wl.make_half((B, Nk, cap, 128), g, dtype)], 2).contiguous()
+    nb, nr = [0, 1, 3, 2], [300, 1, 0, 129]
+    got = polar_decode_attention(q.to(gpu), *[t.to(gpu) for t in codes], kres.to(gpu), v.to(gpu), 0, 0,
+                                 n_groups_per_seq=torch.tensor(nb, dtype=torch.int32, device=gpu), n_resid_per_seq=torch.tensor(nr, dtype=torch.int32, device=gpu))
+    for b in range(B):
+        n, r = nb[b], nr[b]
+        one = [t[b:b + 1, :, :n] for t in codes] if n else [None] * 5
+        want = po.decode_attention_exact(q[b:b + 1], kres[b:b + 1, :, :r], *one, v[b:b + 1, :, :n * 128 + r])
+        assert close(got[b:b + 1], want, dtype), b
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,N,Nk,groups,resid,packed", [(1, 8, 2, 1, 128, False), (2, 28, 4, 3, 17, True), (1, 8, 8, 2, 1, False), (1, 8, 1, 5, 0, True)])
+def test_four_bit_values(gpu, dtype, B, N, Nk, groups, resid, packed):
+    bits = 3 if packed else 4
+    q, codes, kres, v = inputs(B, N, Nk, groups, resid, bits, bits, dtype, 3 * groups)
+    vq = po.quantize_values_along_last_dim(v[:, :, :groups * 128].contiguous())
+    vres = torch.zeros_like(kres)
+    vres[:, :, :resid] = v[:, :, groups * 128:]
+    want = po.decode_attention_mixed_exact(q, kres[:, :, :resid], *codes, vres[:, :, :resid], *vq, rbits=bits, tbits=bits)
+    cache = [t.to(gpu) for t in codes]
+    if packed:
+        cache[0] = convert_codes6(cache[0], pack=True)
+    run = lambda **kw: polar_decode_attention_v4(q.to(gpu), *cache, kres.to(gpu), vres.to(gpu), *[t.to(gpu) for t in vq], groups, resid, rbits=bits, tbits=bits, **kw)
+    for got in (run(), run(n_splits=1), run(n_splits=FEW // (B * Nk)), run(single_wavefront=True)):
+        assert close(got, want, dtype)
+
+
+def test_nan_scores_stay_visible(gpu):
+    """A NaN in a query reaches the head's output and no other, a masked-out sequence gives zeros."""
+    q, codes, kres, v = inputs(1, 8, 2, 2, 5, 4, 4, torch.float16, 1)
+    q[0, 3, 0, 7] = float("nan")
+    run = lambda qq, m=None, **kw: polar_decode_attention(qq.to(gpu), *[t.to(gpu) for t in codes], kres.to(gpu), v.to(gpu), 2, 5, attention_mask=m, **kw)
+    got = run(q, n_splits=1).cpu()
+    assert torch.isnan(got[0, 3]).all() and not torch.isnan(got[0, [0, 1, 2, 4, 5, 6, 7]]).any()
+    assert not run(torch.zeros_like(q), torch.zeros(1, 261, dtype=torch.uint8, device=gpu)).any()
