@@ -7,18 +7,20 @@ LlamaPolarGroupAttention.forward computes between RoPE and o_proj
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 from typing import Optional
 
 import torch
 
 from . import _ffi
-from .kernel4group import _dtype_code, _stream_ptr
+from .kernel4group import _dtype_code, _on_device, _stream_ptr
 
 GROUP = 128
 _WORKSPACES = {}
 
 
+@functools.lru_cache(maxsize=None)
 def _num_cus(device: torch.device) -> int:
     return torch.cuda.get_device_properties(device).multi_processor_count
 
@@ -44,7 +46,7 @@ def workspace_for(B: int, N: int, n_splits: int, device: torch.device) -> torch.
     replaced buffer goes back to torch's allocator, which hands it out again only behind the work
     already queued on that stream."""
     need = workspace_bytes(B, N, n_splits)
-    key = (device.type, device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (device.type, device.index, _stream_ptr(device))
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() * 4 < need:
         ws = torch.empty((need + 3) // 4, dtype=torch.float32, device=device)
@@ -114,9 +116,9 @@ def polar_decode_attention(
     Nk = value_states.shape[1]
     assert hd == 128
     dt = _dtype_code(query_states)
-    q = query_states.reshape(B, N, hd)
+    q = query_states
     if not q.is_contiguous() or q.data_ptr() % 16:
-        q = q.clone(memory_format=torch.contiguous_format)
+        q = q.reshape(B, N, hd).clone(memory_format=torch.contiguous_format)
     assert value_states.is_contiguous() and value_states.dtype == query_states.dtype
     v_cap = value_states.shape[2]
     if indices is not None:
@@ -171,7 +173,7 @@ def polar_decode_attention(
         if status.dtype != torch.int32 or status.device != dev or status.numel() != 1:
             raise ValueError("polarquant_amd: status must be one int32 on %s" % dev)
         sptr = status.data_ptr()
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         rc = _ffi.lib().pq_decode_attn(
             q.data_ptr(), *cptr, g_cap, n_groups, gps, kptr, r_cap, n_resid, rps,
             value_states.data_ptr(), v_cap, mptr, mstride, float(sm_scale), B, N, Nk, rbits, tbits, dt,
@@ -207,9 +209,9 @@ def polar_decode_attention_v4(
     Nk = key_resid.shape[1]
     assert hd == 128
     dt = _dtype_code(query_states)
-    q = query_states.reshape(B, N, hd)
+    q = query_states
     if not q.is_contiguous() or q.data_ptr() % 16:
-        q = q.clone(memory_format=torch.contiguous_format)
+        q = q.reshape(B, N, hd).clone(memory_format=torch.contiguous_format)
     assert key_resid.is_contiguous() and value_resid.is_contiguous() and key_resid.shape == value_resid.shape
     assert key_resid.dtype == query_states.dtype == value_resid.dtype
     r_cap = key_resid.shape[2]
@@ -251,7 +253,7 @@ def polar_decode_attention_v4(
         out = torch.empty((B, N, 1, hd), dtype=query_states.dtype, device=dev)
     gps = n_groups_per_seq.data_ptr() if n_groups_per_seq is not None else None
     rps = n_resid_per_seq.data_ptr() if n_resid_per_seq is not None else None
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         rc = _ffi.lib().pq_decode_attn_v4(
             q.data_ptr(), *cptr, g_cap, n_groups, gps, key_resid.data_ptr(), r_cap, n_resid, rps,
             value_resid.data_ptr(), *vptr, v4_cap, mptr, mstride, float(sm_scale), B, N, Nk, rbits, tbits, dt,
@@ -275,7 +277,7 @@ def prompt_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sm_scale
     B, N, L, _ = q.shape
     out = torch.empty((B, L, N, 128), dtype=q.dtype, device=q.device)
     strides = (ctypes.c_int64 * 9)(*q.stride()[:3], *k.stride()[:3], *v.stride()[:3])
-    with torch.cuda.device(q.device):
+    with _on_device(q.device):
         rc = _ffi.lib().pq_prompt_attn(q.data_ptr(), k.data_ptr(), v.data_ptr(), ctypes.cast(strides, ctypes.c_void_p), out.data_ptr(),
                                        float(sm_scale if sm_scale is not None else 1.0 / math.sqrt(128)), B, L, N, k.shape[1], _dtype_code(q),
                                        _stream_ptr(q.device))

@@ -8,7 +8,7 @@ from typing import Optional
 import torch
 
 from . import _ffi
-from .kernel4group import _dtype_code, _stream_ptr
+from .kernel4group import _dtype_code, _on_device, _stream_ptr
 
 
 def _gpu(t: torch.Tensor):
@@ -33,7 +33,7 @@ def rope_append(q_lin: torch.Tensor, k_lin: torch.Tensor, v_lin: torch.Tensor, c
     assert q_lin.shape[-1] == n_heads * 128 and k_lin.shape[-1] == n_kv_heads * 128 == v_lin.shape[-1] and q_lin.numel() == B * n_heads * 128
     assert k_dst.shape[:2] == (B, n_kv_heads) == v_dst.shape[:2] and k_dst.shape[3] == 128 == v_dst.shape[3]
     q_out = torch.empty((B, n_heads, 1, 128), dtype=q_lin.dtype, device=q_lin.device)
-    with torch.cuda.device(q_lin.device):
+    with _on_device(q_lin.device):
         rc = _ffi.lib().pq_rope_append(q_lin.data_ptr(), k_lin.data_ptr(), v_lin.data_ptr(), cos_table.data_ptr(),
                                        sin_table.data_ptr(), cos_table.shape[0], pos.data_ptr(), q_out.data_ptr(),
                                        k_dst.data_ptr(), k_dst.shape[2], k_row.data_ptr(), v_dst.data_ptr(), v_dst.shape[2],
@@ -55,7 +55,7 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, residual: Optiona
     if sum_out is not None:
         assert sum_out.is_contiguous() and sum_out.shape == x.shape and sum_out.dtype == x.dtype
     y = torch.empty_like(x)
-    with torch.cuda.device(x.device):
+    with _on_device(x.device):
         rc = _ffi.lib().pq_rmsnorm(x.data_ptr(), None if residual is None else residual.data_ptr(), weight.data_ptr(),
                                    y.data_ptr(), None if sum_out is None else sum_out.data_ptr(), x.numel() // hidden, hidden,
                                    float(eps), _dtype_code(x), _stream_ptr(x.device))
@@ -76,7 +76,7 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
         "rows must be evenly spaced"
     y = torch.empty(gate.shape, dtype=gate.dtype, device=gate.device)
     esz = gate.element_size()
-    with torch.cuda.device(gate.device):
+    with _on_device(gate.device):
         for r0 in range(0, rows, 65535):          # one launch covers at most 65535 rows (a prompt has more)
             n = min(65535, rows - r0)
             rc = _ffi.lib().pq_silu_mul(gate.data_ptr() + r0 * stride * esz, up.data_ptr() + r0 * stride * esz,
@@ -102,7 +102,7 @@ def linear_small_m(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
     if bias is not None:
         assert bias.is_contiguous() and bias.numel() == N and bias.dtype == x.dtype
     y = torch.empty(x.shape[:-1] + (N,), dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on_device(x.device):
         rc = _ffi.lib().pq_linear_small_m(x2.data_ptr(), x2.stride(0) if M > 1 else K, weight.data_ptr(),
                                           None if up_weight is None else up_weight.data_ptr(),
                                           None if bias is None else bias.data_ptr(), y.data_ptr(), N, M, N, K,
@@ -127,7 +127,7 @@ def qkv_rope_append(x: torch.Tensor, w_qkv: torch.Tensor, b_qkv: Optional[torch.
     assert pos.dtype == k_row.dtype == v_row.dtype == torch.int64
     assert k_dst.shape[:2] == (B, n_kv_heads) == v_dst.shape[:2] and k_dst.shape[3] == 128 == v_dst.shape[3]
     q_out = torch.empty((B, n_heads, 1, 128), dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on_device(x.device):
         rc = _ffi.lib().pq_qkv_rope_append(x2.data_ptr(), x2.stride(0) if B > 1 else K, w_qkv.data_ptr(),
                                            None if b_qkv is None else b_qkv.data_ptr(), B, K, _dtype_code(x),
                                            cos_table.data_ptr(), sin_table.data_ptr(), cos_table.shape[0], pos.data_ptr(),
@@ -160,7 +160,7 @@ def rope_qk(q_lin: torch.Tensor, k_lin: torch.Tensor, cos: torch.Tensor, sin: to
     cos, sin = cos.contiguous(), sin.contiguous()
     q_out = torch.empty((B, L, n_heads, 128), dtype=q_lin.dtype, device=q_lin.device)
     k_out = torch.empty((B, L, n_kv_heads, 128), dtype=q_lin.dtype, device=q_lin.device)
-    with torch.cuda.device(q_lin.device):
+    with _on_device(q_lin.device):
         rc = _ffi.lib().pq_rope_qk(q_lin.data_ptr(), qs, k_lin.data_ptr(), ks, cos.data_ptr(), sin.data_ptr(),
                                    0 if cos.shape[0] == 1 else L * 128, q_out.data_ptr(), k_out.data_ptr(), B, L, n_heads,
                                    n_kv_heads, _dtype_code(q_lin), _stream_ptr(q_lin.device))

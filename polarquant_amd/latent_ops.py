@@ -8,7 +8,7 @@ import torch
 
 from . import _ffi
 from .attention import _num_cus
-from .kernel4group import _stream_ptr
+from .kernel4group import _on_device, _stream_ptr
 
 from .layer_ops import (_DTYPES, _code, _ptr, ConvState, IN_PLACE_TOKENS, SMALL_M, head_linear, linear, linear_f32,  # noqa: F401
                         norm_conv, relu_sq, streams)
@@ -24,7 +24,7 @@ def latent_norm(p: torch.Tensor, w_q: torch.Tensor, w_kv: Optional[torch.Tensor]
     assert cache is None or (cache.is_contiguous() and cache.shape[0] == B and (w_kv is None or cache.shape[2] == w_kv.numel()))
     qr = w_q.numel()
     out = torch.empty(B, L, qr, dtype=p.dtype, device=p.device)
-    with torch.cuda.device(p.device):
+    with _on_device(p.device):
         rc = _ffi.latent_lib().pq_latent_norm(_ptr(p), ld, _ptr(w_q), _ptr(w_kv), _ptr(out), _ptr(cache) if w_kv is not None else None,
                                               cache.shape[1] if w_kv is not None else 0, _ptr(pos_dev), pos, B, L, qr,
                                               w_kv.numel() if w_kv is not None else 1, float(eps), dt, _stream_ptr(p.device))
@@ -53,7 +53,7 @@ def latent_decode_attention(q: torch.Tensor, cache: torch.Tensor, sink: torch.Te
     nbytes = lib.pq_latent_decode_workspace_bytes(B, L, H, R, n_splits)
     ws = torch.empty(nbytes // 4, dtype=torch.float32, device=q.device) if dt != _ffi.PQ_F32 else None
     out = torch.empty_like(q)
-    with torch.cuda.device(q.device):
+    with _on_device(q.device):
         rc = lib.pq_latent_decode(_ptr(q), _ptr(cache), cache.shape[1], _ptr(sink), _ptr(start), _ptr(pos_dev), pos, _ptr(out), B, L, H,
                                   R, float(scale), n_splits, _ptr(ws), nbytes if ws is not None else 0, dt, _stream_ptr(q.device))
     _ffi.check(rc, "pq_latent_decode")
@@ -78,7 +78,7 @@ def latent_prefill_attention(q: torch.Tensor, k: torch.Tensor, vt: torch.Tensor,
         if gate.data_ptr() % 8:
             gate = gate.contiguous()
     out = torch.empty(B, L, H * Dv, dtype=q.dtype, device=q.device)
-    with torch.cuda.device(q.device):
+    with _on_device(q.device):
         rc = _ffi.latent_lib().pq_latent_prefill(_ptr(q), _ptr(k), _ptr(vt), ld, _ptr(sink), _ptr(gate), 0 if gate is None else gate.stride(0),
                                                  _ptr(start), _ptr(out), B, L, Lk, H, D, Dv, float(scale), dt, _stream_ptr(q.device))
     _ffi.check(rc, "pq_latent_prefill")

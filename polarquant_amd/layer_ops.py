@@ -8,7 +8,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _ffi
-from .kernel4group import _stream_ptr
+from .kernel4group import _on_device, _stream_ptr
 
 _DTYPES = {torch.float16: _ffi.PQ_F16, torch.bfloat16: _ffi.PQ_BF16, torch.float32: _ffi.PQ_F32}
 IN_PLACE_TOKENS = 32        # longer calls are cut into strips that read what others of the launch write
@@ -69,7 +69,7 @@ def norm_conv(x: torch.Tensor, w_pre: torch.Tensor, groups: int, eps: float, y: 
         s_in, s_out = state.targets(L)
         assert s_in.shape == (B, taps - 1, W)
     h = torch.empty(B, L, W, dtype=w_pre.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on_device(x.device):
         rc = _ffi.steps_lib().pq_norm_conv(
             _ptr(x), _ptr(y), _ptr(w_post) if y is not None else None, _ptr(x_out), _ptr(w_pre), _ptr(conv_w),
             _ptr(s_in) if taps > 1 else None, _ptr(s_out) if taps > 1 else None, _ptr(h), _ptr(start), _ptr(pos_dev), pos, B, L, W,
@@ -82,7 +82,7 @@ def relu_sq(x: torch.Tensor) -> torch.Tensor:
     """max(x, 0)^2, in place."""
     dt = _code(x)
     assert x.is_contiguous()
-    with torch.cuda.device(x.device):
+    with _on_device(x.device):
         rc = _ffi.steps_lib().pq_relu_sq(_ptr(x), _ptr(x), x.numel(), dt, _stream_ptr(x.device))
     _ffi.check(rc, "pq_relu_sq")
     return x
@@ -95,7 +95,7 @@ def gelu_mul(gate: torch.Tensor, up: torch.Tensor, out: Optional[torch.Tensor] =
     out = torch.empty(M, N, dtype=gate.dtype, device=gate.device) if out is None else out
     assert up.shape == out.shape == (M, N) and gate.stride() == up.stride() and gate.stride(1) == out.stride(1) == 1
     assert up.dtype == out.dtype == gate.dtype
-    with torch.cuda.device(gate.device):
+    with _on_device(gate.device):
         rc = _ffi.steps_lib().pq_gelu_mul(_ptr(gate), _ptr(up), gate.stride(0), _ptr(out), out.stride(0), M, N, dt, _stream_ptr(gate.device))
     _ffi.check(rc, "pq_gelu_mul")
     return out
@@ -113,7 +113,7 @@ def stream_add(x: torch.Tensor, y: Optional[torch.Tensor] = None, e: Optional[to
     assert v is None or (v.is_contiguous() and v.numel() == W and v.dtype == dtype)
     _code(x)
     out = torch.empty_like(x)
-    with torch.cuda.device(x.device):
+    with _on_device(x.device):
         rc = _ffi.steps_lib().pq_stream_add(_ptr(x), _ptr(y), _ptr(e), _ptr(v), _ptr(out), x.numel() // W, W, _DTYPES[dtype], _stream_ptr(x.device))
     _ffi.check(rc, "pq_stream_add")
     return out
@@ -125,7 +125,7 @@ def embed_rows(table: torch.Tensor, ids: torch.Tensor, scale: float = 1.0) -> to
     ids = ids.contiguous()
     assert table.is_contiguous() and ids.dtype == torch.int64 and ids.is_cuda
     out = torch.empty(tuple(ids.shape) + (table.shape[1],), dtype=torch.float32, device=table.device)
-    with torch.cuda.device(table.device):
+    with _on_device(table.device):
         rc = _ffi.steps_lib().pq_embed_rows(_ptr(table), _ptr(ids), float(scale), _ptr(out), ids.numel(), table.shape[1], table.shape[0], dt,
                                             _stream_ptr(table.device))
     _ffi.check(rc, "pq_embed_rows")
@@ -136,7 +136,7 @@ def softcap(x: torch.Tensor, scale: float, cap: Optional[float]) -> torch.Tensor
     """cap * tanh(x * scale / cap) in place, float32; without a cap x * scale."""
     _code(x)
     assert x.is_contiguous() and x.dtype == torch.float32
-    with torch.cuda.device(x.device):
+    with _on_device(x.device):
         rc = _ffi.steps_lib().pq_softcap(_ptr(x), x.numel(), float(scale), float(cap or 0.0), _stream_ptr(x.device))
     _ffi.check(rc, "pq_softcap")
     return x
@@ -154,7 +154,7 @@ def head_linear(x: torch.Tensor, w: torch.Tensor, gate: Optional[torch.Tensor] =
         epilogue = _ffi.PQ_EPI_SIGMOID_GATE
     y = torch.empty(M, H, N, dtype=torch.float32 if epilogue == _ffi.PQ_EPI_F32 else x.dtype, device=x.device)
     rows = SMALL_M if (dt != _ffi.PQ_F32 and N % 16 == 0 and K % 32 == 0) else 65535
-    with torch.cuda.device(x.device):
+    with _on_device(x.device):
         for m in range(0, M, rows):
             xs, ys, gs = x[m:m + rows], y[m:m + rows], None if gate is None else gate[m:m + rows]
             rc = _ffi.steps_lib().pq_head_linear(_ptr(xs), x.stride(0), x.stride(1), _ptr(w), _ptr(gs), 0 if gate is None else gate.stride(0),

@@ -8,7 +8,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _ffi
-from .kernel4group import _dtype_code, _stream_ptr
+from .kernel4group import _dtype_code, _on_device, _stream_ptr
 
 GROUP = 128
 PAIRS = 64
@@ -60,7 +60,7 @@ def quantize_and_pack_nbit(key_states: torch.Tensor, rbits: int = 4, tbits: int 
         cap, off = codes.shape[2], group_offset
         assert codes.is_contiguous() and all(m.is_contiguous() for m in meta) and codes.shape[-1] == row
     strides = (ctypes.c_int64 * 4)(*key_states.stride())
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         rc = _ffi.lib().pq_quantize_groups(key_states.data_ptr(), ctypes.cast(strides, ctypes.c_void_p), dt, B, Nk, Nb,
                                            rbits, tbits, (_ffi.PQ_WRAP_FP32 if wrap_fp32 or eager_gpu else 0)
                                            | (_ffi.PQ_DEVICE_ATAN2 if device_atan2 or eager_gpu else 0)
@@ -83,7 +83,7 @@ def convert_codes6(indices: torch.Tensor, pack: bool) -> torch.Tensor:
     assert indices.dtype == torch.uint8 and indices.shape[-1] == src_row
     src = indices.contiguous()
     dst = torch.empty(src.shape[:-1] + (dst_row,), dtype=torch.uint8, device=src.device)
-    with torch.cuda.device(src.device):
+    with _on_device(src.device):
         rc = _ffi.lib().pq_convert_codes6(src.data_ptr(), dst.data_ptr(), src.numel() // src_row, int(pack), _stream_ptr(src.device))
     _ffi.check(rc, "pq_convert_codes6")
     return dst

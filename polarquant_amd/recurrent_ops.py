@@ -10,7 +10,7 @@ import torch
 
 from . import _ffi
 from .attention import _num_cus
-from .kernel4group import _stream_ptr
+from .kernel4group import _on_device, _stream_ptr
 from .layer_ops import _DTYPES, ConvState, _code, _ptr
 
 WINDOW_SMALL = 16          # new tokens per sequence up to which keys go to the ring before they are read
@@ -34,7 +34,7 @@ def _rows(t: torch.Tensor, M: int, n: int, dtype: torch.dtype) -> None:
 
 
 def _run(lib_fn, name: str, device, *args) -> None:
-    with torch.cuda.device(device):
+    with _on_device(device):
         rc = lib_fn(*args, _stream_ptr(device))
     _ffi.check(rc, name)
 

@@ -9,7 +9,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _ffi
-from .kernel4group import _dtype_code, _stream_ptr
+from .kernel4group import _dtype_code, _on_device, _stream_ptr
 
 HEAD_DIM = 128
 WORDS = 16          # int32 words per token row: 8 four-bit codes each
@@ -40,7 +40,7 @@ def quantize_values(value_states: torch.Tensor, group_size: int = HEAD_DIM, bits
         cap, off = code.shape[2], token_offset
         assert code.is_contiguous() and scale.is_contiguous() and mn.is_contiguous() and code.dtype == torch.int32
     strides = (ctypes.c_int64 * 4)(*value_states.stride())
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         rc = _ffi.lib().pq_quantize_values(value_states.data_ptr(), ctypes.cast(strides, ctypes.c_void_p), dt, B, Nk, T,
                                            code.data_ptr(), scale.data_ptr(), mn.data_ptr(), cap, off, _stream_ptr(dev))
     _ffi.check(rc, "pq_quantize_values")
