@@ -257,7 +257,14 @@ int launch_norm_conv(const NormConvArgs& args, int dtype, hipStream_t st) {
     const int per = (pieces + nthr - 1) / nthr;
     const int NC = per <= 1 ? 1 : per <= 2 ? 2 : per <= 4 ? 4 : 8;
     if (per > 8) return static_cast<int>(hipErrorInvalidValue);
-    a.strip = a.L <= kConvInPlaceTokens ? a.L : 32;
+    // Strips as long as the device stays full with them: every strip recomputes taps - 1 norms, and its tokens follow each other
+    // (2.2 us a token).  Full is one workgroup per unit, two where a thread has one piece.  8192 tokens of 4096, taps 4, strips
+    // of 32 / 16 / 8: 103 / 108 / 126 us; 2048 tokens 77 / 46 / 31; 512 tokens, down to strips of 4: 71 / 41 / 26 / 18.
+    constexpr int64_t kUnits = 256;
+    const int64_t full = NC == 1 ? 2 * kUnits : kUnits, tokens = static_cast<int64_t>(a.B) * a.L;
+    a.strip = 32;
+    while (a.strip > 4 && a.strip / 2 >= a.taps && tokens / (a.strip / 2) <= full) a.strip /= 2;
+    if (a.L <= kConvInPlaceTokens) a.strip = a.L;
     const size_t shared = (static_cast<size_t>(NC) * nthr + a.groups) * sizeof(float);
     if (shared > 64 * 1024) return static_cast<int>(hipErrorInvalidValue);
     dim3 grid(static_cast<unsigned>((a.L + a.strip - 1) / a.strip), static_cast<unsigned>(a.B)), block(nthr);

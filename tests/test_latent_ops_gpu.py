@@ -214,3 +214,21 @@ def test_latent_prefill(gpu, D, Dv):
                     full = do.attend(q[b].double(), k[b].double(), v[b].double(), sink.double(), scale, s)
                 want = full * torch.sigmoid(gate[b * L:(b + 1) * L].double())
                 assert err(got[b], want) < {"bf16": 1.2e-2, "f16": 2e-3}[dt], (dt, L, past, b)
+
+
+@pytest.mark.parametrize("W,groups,taps", [(256, 2, 4), (2048, 1, 4), (4096, 4, 3), (300, 3, 16), (512, 1, 0)])
+@pytest.mark.parametrize("B,L", [(1, 33), (1, 64), (2, 70), (1, 1030), (3, 700), (1, 2100), (1, 4200)])
+def test_norm_conv_strips_give_the_bits_of_shorter_calls(W, groups, taps, B, L):
+    """However a call is cut into strips (by its length, width and filter), its rows and the state it leaves are those of calls of up to
+    32 tokens, which one workgroup per sequence works through."""
+    g = torch.Generator(device="cuda").manual_seed(L + W)
+    x = torch.randn(B, L, W, generator=g, device="cuda")
+    y = torch.randn(B, L, W, generator=g, device="cuda").bfloat16()
+    w = torch.randn(W, generator=g, device="cuda").bfloat16()
+    cw = (torch.randn(W, taps, generator=g, device="cuda") * 0.4).bfloat16() if taps else None
+    conv = dict(conv_w=cw) if taps else {}
+    whole, parts = [ops.ConvState(B, taps, W, "cuda") if taps else None for _ in range(2)]
+    xs, hs = ops.norm_conv(x.clone(), w, groups, 1e-5, y, w, state=whole, **conv)
+    got = [ops.norm_conv(x[:, i:i + 32].contiguous(), w, groups, 1e-5, y[:, i:i + 32].contiguous(), w, state=parts, **conv) for i in range(0, L, 32)]
+    assert torch.equal(xs, torch.cat([a for a, _ in got], 1)) and torch.equal(hs, torch.cat([b for _, b in got], 1))
+    assert not taps or torch.equal(whole.rows, parts.rows)
