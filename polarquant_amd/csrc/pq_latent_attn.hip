@@ -360,7 +360,7 @@ static int prefill_dims(const LatentPrefillArgs& l, hipStream_t st) {
     a.q = l.q; a.q_b = l.L * kv; a.q_t = kv; a.q_h = l.D;
     a.k = l.k; a.k_b = l.Lk * kv; a.k_t = kv; a.k_h = l.D;
     a.v = l.vt; a.v_b = static_cast<int64_t>(l.H) * l.Dv * l.ldv; a.v_t = l.ldv; a.v_h = l.Dv * l.ldv;
-    a.sink = l.sink; a.gate = l.gate; a.gate_row = l.gate_row; a.start = l.start; a.out = l.out;
+    a.sink = l.sink; a.gate = l.gate; a.gate_row = l.gate_row; a.start = l.start; a.out = l.out; a.out_row = static_cast<int64_t>(l.H) * l.Dv;
     a.B = l.B; a.L = l.L; a.Lk = l.Lk; a.H = a.G = l.H; a.D = l.D; a.Dv = l.Dv; a.scale = l.scale;
     if (l.D <= 64 && l.Dv <= 64) return launch_prompt_attn<T, 64, 64, false>(a, st);
     if (l.D <= 128 && l.Dv <= 128) return launch_prompt_attn<T, 128, 128, false>(a, st);

@@ -12,9 +12,15 @@ struct PromptAttnArgs {
     const void* gate;                         // [B * L, H * Dv] rows gate_row apart, or null
     int64_t gate_row;
     const int32_t* start;                     // [B]: keys before it do not exist; or null
-    void* out;                                // [B, L, H * Dv]
+    void* out;                                // [B * L, H * Dv] rows out_row apart
+    int64_t out_row;
     int B, L, Lk, H, G, D, Dv;                // the L queries are the last of the Lk tokens
     float scale;
+    // of a sliding window (WINDOW): k and v hold the call's own tokens, those before it are row (position % cap) of [B, G, cap, ..] rings
+    const void *k_ring, *v_ring;
+    const float* slopes;                      // [H] taken off a score per position of distance, or null
+    int cap, window;
+    float out_scale;                          // (times the result)
 };
 
 constexpr int kPromptTileRows = 128, kPromptTileKeys = 64;
@@ -50,17 +56,22 @@ template <> __device__ __forceinline__ uint32_t pack_pair<F16>(float a, float b)
 // channel, 570 us with a row per token; 724 us with tiles passed through registers and a maximum raised at each excess.  A step that
 // makes the next tile's scores beside this tile's weights needs more registers than two wavefronts have (830 us); raised
 // wavefront priority around the products changes nothing.
-template <typename T, int DKP, int DVP, bool TOKEN_ROWS>
+// WINDOW: a query sees the last `window` positions, with a bias per position of distance; tiles that a workgroup's windows do not touch
+// are not visited, those before the call come from a ring, or from both where the call begins inside a tile.  8192 tokens, window
+// 2048, 32 query and 8 KV heads of 128: 440 -> 370 us against tiles passed through registers (16 heads of 256: 640 -> 580).  The
+// bias is where a score's accumulator starts, in units of an unscaled score (with a second multiply-add per score: 385 us); rows
+// come from ring or call by selection (with branches: 436 -> 448 us at 5000 tokens before the call).
+template <typename T, int DKP, int DVP, bool TOKEN_ROWS, bool WINDOW = false>
 __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(PromptAttnArgs a) {
     constexpr int KS = DKP / 16, VT = DVP / 32, KC = DKP / 8, VC = TOKEN_ROWS ? DVP / 8 : 8;        // 16-byte chunks of a row of K, of V
     constexpr int KBYTES = kPromptTileKeys * DKP * 2, VBYTES = kPromptTileKeys * DVP * 2;
     constexpr int KL = KBYTES / 4096, VL = VBYTES / 4096;                                          // loads per lane and tile
-    static_assert(!TOKEN_ROWS || DVP == 128, "swizzle of token rows");
+    static_assert(TOKEN_ROWS || !WINDOW, "a ring has a row per token");
     extern __shared__ __attribute__((aligned(1024))) uint8_t sm[];                                // two K tiles, then two V tiles
     const uint32_t lds0 = lds_addr(sm);
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 31, hi = lane >> 5;
     const int H = a.H, D = a.D, Dv = a.Dv, b = blockIdx.z;
-        const int h = blockIdx.x, g = h / (H / a.G);
+    const int h = blockIdx.x, g = h / (H / a.G);
     const int tile = static_cast<int>(gridDim.y) - 1 - static_cast<int>(blockIdx.y);
     const int past = a.Lk - a.L;
     const int qw = tile * kPromptTileRows + wv * 32, qi = qw + col;                 // the wavefront's first query token; this lane's
@@ -69,8 +80,15 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
     const int lo = a.start ? a.start[b] : 0;
     const int q_last = tile * kPromptTileRows + kPromptTileRows - 1 < a.L - 1 ? tile * kPromptTileRows + kPromptTileRows - 1 : a.L - 1;
     const int wave_last = past + (qw + 31 < a.L - 1 ? qw + 31 : a.L - 1);
-    const int it0 = lo / kPromptTileKeys, it1 = (past + q_last) / kPromptTileKeys + 1;
-    const float scale2 = a.scale != 0.0f ? fabsf(a.scale) * kLog2e : 1.0e-30f;      // (a masked score, -inf, stays one)
+    const int wave_first = past + (qw < a.L - 1 ? qw : a.L - 1);
+    // the first key that any row of the workgroup sees
+    int key_lo = WINDOW ? past + tile * kPromptTileRows - a.window + 1 : lo;
+    key_lo = key_lo > lo ? key_lo : lo;
+    key_lo = !WINDOW || key_lo > 0 ? key_lo : 0;
+    const int it0 = key_lo / kPromptTileKeys, it1 = (past + q_last) / kPromptTileKeys + 1;
+    // a scale of zero: the scores of zero queries, times one (a masked score, -inf, stays one)
+    const float scale2 = a.scale != 0.0f ? fabsf(a.scale) * kLog2e : 1.0f;
+    const float slope = WINDOW && a.slopes ? a.slopes[h] * kLog2e / scale2 : 0.0f;      // (of a score before it is scaled)
 
     u32x4_a q[KS];
     {
@@ -80,32 +98,45 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
             constexpr int i = decltype(I)::value;
             const int c = i * 16 + 8 * hi;
             const u32x4_a t = *reinterpret_cast<const u32x4_a*>(qp + (c < D ? c : 0));
-            q[i] = c < D ? u32x4_a{t.x ^ flip, t.y ^ flip, t.z ^ flip, t.w ^ flip} : u32x4_a{0, 0, 0, 0};
+            q[i] = c < D && a.scale != 0.0f ? u32x4_a{t.x ^ flip, t.y ^ flip, t.z ^ flip, t.w ^ flip} : u32x4_a{0, 0, 0, 0};
         });
     }
     // where this lane's 16 bytes of each load come from: load i of a wavefront fills chunks (wv KL + i) 64 .. + 63 of a tile
     const uint16_t* kb = static_cast<const uint16_t*>(a.k) + b * a.k_b + g * a.k_h;
     const uint16_t* vb = static_cast<const uint16_t*>(a.v) + b * a.v_b + g * a.v_h;
     auto k_swz = [](int row) { return DKP == 64 ? (row >> 1) & 7 : row & 7; };
-    auto v_swz = [](int row) { return TOKEN_ROWS ? (row & 7) << 1 : (row >> 1) & 7; };
-    auto k_src = [&](int i, int first, int last) {
-        const int u = (wv * KL + i) * 64 + lane, row = u / KC, c = ((u % KC) ^ k_swz(row)) * 8;
-        return kb + static_cast<int64_t>(first + (row < last ? row : last)) * a.k_t + (c < D ? c : 0);
+    auto v_swz = [](int row) { return TOKEN_ROWS ? (DVP == 64 ? ((row >> 1) & 3) << 1 : (row & 7) << 1) : (row >> 1) & 7; };
+    // with WINDOW, row (first + row) of the sequence: the ring's before this call's own
+    auto either = [&](const uint16_t* own, int64_t own_t, const void* ring, int width, int first, int slot, int row, int last) {
+        const int key = first + (row < last ? row : last);
+        const bool past_key = key < past;                           // (selected, not branched on)
+        return (past_key ? static_cast<const uint16_t*>(ring) + (static_cast<int64_t>(b) * a.G + g) * a.cap * width : own) +
+               static_cast<int64_t>(past_key ? slot + row : key - past) * (past_key ? width : own_t);
     };
-    auto v_src = [&](int i, int first, int last) {
+    auto k_src = [&](int i, int first, int slot, int last) {
+        const int u = (wv * KL + i) * 64 + lane, row = u / KC, c = ((u % KC) ^ k_swz(row)) * 8;
+        const uint16_t* at = WINDOW ? either(kb, a.k_t, a.k_ring, D, first, slot, row, last) : kb + static_cast<int64_t>(first + (row < last ? row : last)) * a.k_t;
+        return at + (c < D ? c : 0);
+    };
+    auto v_src = [&](int i, int first, int slot, int last) {
         const int u = (wv * VL + i) * 64 + lane, row = u / VC, c = ((u % VC) ^ v_swz(row)) * 8;
-        if (TOKEN_ROWS) return vb + static_cast<int64_t>(first + (row < last ? row : last)) * a.v_t + (c < Dv ? c : 0);
-        return vb + static_cast<int64_t>(row < Dv ? row : Dv - 1) * a.v_t + first + c;
+        if (!TOKEN_ROWS) return vb + static_cast<int64_t>(row < Dv ? row : Dv - 1) * a.v_t + first + c;
+        const uint16_t* at = WINDOW ? either(vb, a.v_t, a.v_ring, Dv, first, slot, row, last) : vb + static_cast<int64_t>(first + (row < last ? row : last)) * a.v_t;
+        return at + (c < Dv ? c : 0);
     };
     const uint16_t *ks[KL], *vs[VL];
-    static_for<KL>([&](auto I) { ks[I] = k_src(I, it0 * kPromptTileKeys, kPromptTileKeys - 1); });
-    static_for<VL>([&](auto I) { vs[I] = v_src(I, it0 * kPromptTileKeys, kPromptTileKeys - 1); });
+    if (!WINDOW) {
+        static_for<KL>([&](auto I) { ks[I] = k_src(I, it0 * kPromptTileKeys, 0, kPromptTileKeys - 1); });
+        static_for<VL>([&](auto I) { vs[I] = v_src(I, it0 * kPromptTileKeys, 0, kPromptTileKeys - 1); });
+    }
     auto fetch = [&](int it, auto BUF) {
         constexpr int buf = decltype(BUF)::value;
         const int last = a.Lk - 1 - it * kPromptTileKeys;          // rows past the end: copies of the last one, with weight zero
-        if (last < kPromptTileKeys - 1) {
-            static_for<KL>([&](auto I) { ks[I] = k_src(I, it * kPromptTileKeys, last); });
-            if (TOKEN_ROWS) static_for<VL>([&](auto I) { vs[I] = v_src(I, it * kPromptTileKeys, last); });
+        // (the addresses of whole tiles of this call's tokens only advance)
+        if (last < kPromptTileKeys - 1 || (WINDOW && (it == it0 || (it - 1) * kPromptTileKeys < past))) {
+            const int first = it * kPromptTileKeys, slot = WINDOW ? first % a.cap : 0;
+            static_for<KL>([&](auto I) { ks[I] = k_src(I, first, slot, last); });
+            if (TOKEN_ROWS) static_for<VL>([&](auto I) { vs[I] = v_src(I, first, slot, last); });
         }
         static_for<KL>([&](auto I) {
             load_to_lds(ks[I], lds0 + buf * KBYTES + (wv * KL + I) * 1024);
@@ -139,20 +170,22 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
         constexpr int buf = decltype(BUF)::value;
         if (it + 1 < it1) fetch(it + 1, IC<buf ^ 1>{});
         const int key0 = it * kPromptTileKeys;
-        if (key0 <= wave_last) {                                   // uniform over the wavefront
+        if (key0 <= wave_last && (!WINDOW || key0 + kPromptTileKeys - 1 > wave_first - a.window)) {        // uniform over the wavefront
             floatx16_a s[2];
+            // (this lane: query qi, keys key0 + 32 u + 8 (j / 4) + 4 hi + j % 4)
+            const float base = WINDOW ? -slope * static_cast<float>(limit - key0 - 4 * hi) : 0.0f;
 #pragma unroll
             for (int u = 0; u < 2; u++)
 #pragma unroll
-                for (int j = 0; j < 16; j++) s[u][j] = 0.0f;
+                for (int j = 0; j < 16; j++) s[u][j] = WINDOW ? __builtin_fmaf(slope, static_cast<float>(32 * u + 8 * (j >> 2) + (j & 3)), base) : 0.0f;
             static_for<KS>([&](auto I) {
                 constexpr int i = decltype(I)::value;
                 s[0] = mma32<T>(*lds_ptr<lds_u32x4>(ka[i] + buf * KBYTES), q[i], s[0]);
                 s[1] = mma32<T>(*lds_ptr<lds_u32x4>(ka[i] + buf * KBYTES + 32 * DKP * 2), q[i], s[1]);
             });
-            // this lane: query qi, keys key0 + 32 u + 8 (j / 4) + 4 hi + j % 4
-            if (key0 + kPromptTileKeys - 1 > past + qw || key0 < lo) {
-                const int last = limit - key0 - 4 * hi, first = lo - key0 - 4 * hi;
+            if (key0 + kPromptTileKeys - 1 > past + qw || key0 < lo || (WINDOW && key0 <= wave_last - a.window)) {
+                const int oldest = WINDOW && limit - a.window + 1 > lo ? limit - a.window + 1 : lo;
+                const int last = limit - key0 - 4 * hi, first = oldest - key0 - 4 * hi;
 #pragma unroll
                 for (int u = 0; u < 2; u++)
 #pragma unroll
@@ -217,15 +250,15 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
     }
     l += __shfl_xor(l, 32);
     if (!valid) return;
-    float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    if (a.sink) {
+    float inv = l > 0.0f ? (WINDOW ? a.out_scale : 1.0f) / l : 0.0f;
+    if (!WINDOW && a.sink) {
         const float sink2 = a.sink[h] * kLog2e, mf = fmaxf(m, sink2), al = exp2_hw(m - mf);
         inv = al / (l * al + exp2_hw(sink2 - mf));
     }
     const size_t row = static_cast<size_t>(b) * a.L + qi;
-    uint16_t* out = static_cast<uint16_t*>(a.out) + row * H * Dv + static_cast<size_t>(h) * Dv;
-    const uint16_t* gate = a.gate ? static_cast<const uint16_t*>(a.gate) + row * a.gate_row + static_cast<size_t>(h) * Dv : nullptr;
-    const bool quads = Dv % 4 == 0 && (!gate || a.gate_row % 4 == 0);
+    uint16_t* out = static_cast<uint16_t*>(a.out) + row * a.out_row + static_cast<size_t>(h) * Dv;
+    const uint16_t* gate = !WINDOW && a.gate ? static_cast<const uint16_t*>(a.gate) + row * a.gate_row + static_cast<size_t>(h) * Dv : nullptr;
+    const bool quads = WINDOW || (Dv % 4 == 0 && a.out_row % 4 == 0 && (!gate || a.gate_row % 4 == 0));
     static_for<VT>([&](auto I) {
         constexpr int i = decltype(I)::value;
 #pragma unroll
@@ -251,17 +284,17 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
     });
 }
 
-template <typename T, int DKP, int DVP, bool TOKEN_ROWS>
+template <typename T, int DKP, int DVP, bool TOKEN_ROWS, bool WINDOW = false>
 static int launch_prompt_attn(const PromptAttnArgs& a, hipStream_t st) {
     constexpr size_t bytes = 2 * 2 * static_cast<size_t>(kPromptTileKeys) * (DKP + DVP);
     static_assert(bytes <= 160 * 1024, "LDS");
     if (bytes > 64 * 1024) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&prompt_attn_kernel<T, DKP, DVP, TOKEN_ROWS>),
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&prompt_attn_kernel<T, DKP, DVP, TOKEN_ROWS, WINDOW>),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
         if (e != hipSuccess) return static_cast<int>(e);
     }
     dim3 grid(a.H, (a.L + kPromptTileRows - 1) / kPromptTileRows, a.B), block(256);
-    hipLaunchKernelGGL((prompt_attn_kernel<T, DKP, DVP, TOKEN_ROWS>), grid, block, bytes, st, a);
+    hipLaunchKernelGGL((prompt_attn_kernel<T, DKP, DVP, TOKEN_ROWS, WINDOW>), grid, block, bytes, st, a);
     return static_cast<int>(hipGetLastError());
 }
 

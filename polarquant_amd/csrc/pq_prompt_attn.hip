@@ -11,7 +11,7 @@ int launch_prompt_attn(const void* q, const void* k, const void* v, const int64_
     a.q = q; a.q_b = s[0]; a.q_h = s[1]; a.q_t = s[2];
     a.k = k; a.k_b = s[3]; a.k_h = s[4]; a.k_t = s[5];
     a.v = v; a.v_b = s[6]; a.v_h = s[7]; a.v_t = s[8];
-    a.out = out;
+    a.out = out; a.out_row = static_cast<int64_t>(N) * kHeadDim;
     a.B = B; a.L = a.Lk = L; a.H = N; a.G = Nk; a.D = a.Dv = kHeadDim; a.scale = scale;
     return dtype == 0 ? launch_prompt_attn<F16, 128, 128, true>(a, st) : launch_prompt_attn<BF16, 128, 128, true>(a, st);
 }

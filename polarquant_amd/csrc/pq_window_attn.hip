@@ -4,13 +4,13 @@
 //   qk_norm_kernel         norms of q and of k, the latter and v written to the ring (short calls) or k to a buffer
 //   ring_append_kernel     the last keys and values of a long call, into the ring
 //   window_decode_kernel   few query tokens, from the ring: the window cut into slices; window_merge_kernel joins them
-//   window_prefill_kernel  many query tokens: flash attention over ring and new keys
+//   prompt_attn_kernel     (pq_prompt_attn.h) many query tokens: flash attention over ring and new keys
 //   window_plain_kernel    any size, any dtype (float32 runs here), one wavefront per query row
 //
 // The matrix-core kernels compute S^T = K Q^T, so that a query row is a lane: its softmax state is one register, and the weights
 // P^T leave the first product in the layout in which the second one, O^T = V^T P^T, takes its right operand.  Scores,
 // bias, softmax and all sums are float32; q, k, v and the weights enter the products in the model's 16-bit dtype.
-#include "pq_mfma.h"
+#include "pq_prompt_attn.h"
 #include "pq_recurrent_internal.h"
 
 namespace pq {
@@ -123,7 +123,7 @@ __device__ __forceinline__ size_t window_pairs(const WindowAttnArgs& a) {      /
 template <typename T, int DKP, int DVP>
 __global__ __launch_bounds__(kWave * decode_waves(DVP), 1) void window_decode_kernel(WindowAttnArgs a) {
     constexpr int kDecodeWaves = decode_waves(DVP), KS = DKP / 32, CT = DVP / 16, CH = DVP / 8, LPT = kTile * CH / kWave, VROW = DVP + kVPad;
-    extern __shared__ __attribute__((aligned(16))) uint16_t sm[];
+    extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
     __shared__ float wm[kDecodeWaves][16], wl[kDecodeWaves][16];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid / kWave, r16 = lane & 15, g4 = lane >> 4;
     const int rep = a.H / a.G, rows = a.L * rep, row_tiles = (rows + 15) / 16;
@@ -139,7 +139,7 @@ __global__ __launch_bounds__(kWave * decode_waves(DVP), 1) void window_decode_ke
     const size_t head = static_cast<size_t>(b) * a.G + g;
     const uint16_t* kr = static_cast<const uint16_t*>(a.k_ring) + head * a.cap * D;
     const uint16_t* vr = static_cast<const uint16_t*>(a.v_ring) + head * a.cap * Dv;
-    uint16_t* vt = sm + wv * kTile * VROW;
+    uint16_t* vt = lds + wv * kTile * VROW;
 
     u32x4_a q[KS], k[2][KS], stage[LPT];
     const uint16_t* qp = static_cast<const uint16_t*>(a.q) + ((static_cast<size_t>(b) * a.L + n / rep) * a.H + h) * D;
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(kWave * decode_waves(DVP), 1) void window_decode_ke
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
     __syncthreads();                                                 // the tiles' memory takes the wavefronts' results
-    float* acc = reinterpret_cast<float*>(sm);                       // [wavefront][row][DVP]
+    float* acc = reinterpret_cast<float*>(lds);                       // [wavefront][row][DVP]
     if (g4 == 0) { wm[wv][r16] = m; wl[wv][r16] = l; }
     static_for<CT>([&](auto I) {
         constexpr int i = decltype(I)::value;
@@ -363,206 +363,18 @@ int launch_window_plain(const WindowAttnArgs& a, int dtype, hipStream_t st) {
 }
 
 // ---- prompt --------------------------------------------------------------------------------------------------------------
-// grid (heads, query tiles, sequences).  Four wavefronts with 32 query rows each over 64-key tiles, double-buffered in LDS; a
-// wavefront passes over tiles that its rows' windows do not touch.  A key of an earlier call comes from the ring, one of this
-// call from its own buffer.
-constexpr int kPromptRows = 128, kPromptKeys = 64;
-
-template <typename T, int DKP, int DVP>
-__global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void window_prefill_kernel(WindowAttnArgs a) {
-    constexpr int KS = DKP / 16, VT = DVP / 32, KROW = DKP + 8, VROW = DVP + 16, KCH = DKP / 8, VCH = DVP / 8;
-    constexpr int KLOADS = kPromptKeys * KCH / 256, VLOADS = kPromptKeys * VCH / 256;
-    static_assert(KLOADS * 256 == kPromptKeys * KCH && VLOADS * 256 == kPromptKeys * VCH, "whole loads");
-    extern __shared__ __attribute__((aligned(16))) uint16_t sm[];
-    auto kt = [&](int buf) { return sm + buf * (kPromptKeys * KROW); };
-    auto vt = [&](int buf) { return sm + 2 * (kPromptKeys * KROW) + buf * (kPromptKeys * VROW); };
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid / kWave, col = lane & 31, hi = lane >> 5;
-    const int h = blockIdx.x, b = blockIdx.z, D = a.D, Dv = a.Dv, H = a.H, g = h / (H / a.G), window = a.window, past = a.pos;
-    const int q_tile = blockIdx.y * kPromptRows, qw = q_tile + wv * 32;                 // first query tokens of workgroup and wavefront
-    const int qi = qw + col;
-    const bool valid = qi < a.L;
-    const int qc = valid ? qi : a.L - 1, limit = past + qc;                             // this row's position
-    const int lo = a.start ? a.start[b] : 0;
-    const int q_last = q_tile + kPromptRows - 1 < a.L - 1 ? q_tile + kPromptRows - 1 : a.L - 1;
-    const int wave_last = past + (qw + 31 < a.L - 1 ? qw + 31 : a.L - 1), wave_first = past + (qw < a.L - 1 ? qw : a.L - 1);
-    int key_lo = past + q_tile - window + 1;
-    key_lo = key_lo > lo ? key_lo : lo;
-    key_lo = key_lo > 0 ? key_lo : 0;
-    const int it0 = key_lo / kPromptKeys, it1 = (past + q_last) / kPromptKeys + 1, key_end = past + a.L - 1;
-
-    u32x4_a q[KS];
-    {
-        const uint16_t* qp = static_cast<const uint16_t*>(a.q) + ((static_cast<size_t>(b) * a.L + qc) * H + h) * D;
-        static_for<KS>([&](auto I) {
-            constexpr int i = decltype(I)::value;
-            const int c = i * 16 + 8 * hi;
-            const u32x4_a t = *reinterpret_cast<const u32x4_a*>(qp + (c < D ? c : 0));
-            q[i] = c < D ? t : u32x4_a{0, 0, 0, 0};
-        });
-    }
-    const size_t head = static_cast<size_t>(b) * a.G + g;
-    const uint16_t* kr = static_cast<const uint16_t*>(a.k_ring) + head * a.cap * D;
-    const uint16_t* vr = static_cast<const uint16_t*>(a.v_ring) + head * a.cap * Dv;
-    const uint16_t* kn = static_cast<const uint16_t*>(a.k_new) + static_cast<size_t>(b) * a.L * a.k_row + static_cast<size_t>(g) * D;
-    const uint16_t* vn = static_cast<const uint16_t*>(a.v_new) + static_cast<size_t>(b) * a.L * a.v_row + static_cast<size_t>(g) * Dv;
-    u32x4_a ks[KLOADS], vs[VLOADS];
-    auto fetch = [&](int it) {
-        const int key0 = it * kPromptKeys, slot0 = key0 % a.cap;
-        // no branch around a load (it would be waited for at the join): keys past the end are a copy with weight zero, columns
-        // past D a copy that meets zeros of q, columns past Dv a copy that is never stored
-        auto row = [&](int tok, const uint16_t* ring, int width, const uint16_t* fresh, int64_t fresh_row) {
-            const int key = key0 + tok < key_end ? key0 + tok : key_end;
-            return key < past ? ring + static_cast<size_t>(slot0 + tok) * width : fresh + static_cast<size_t>(key - past) * fresh_row;
-        };
-        static_for<KLOADS>([&](auto I) {
-            constexpr int i = decltype(I)::value;
-            const int u = i * 256 + tid, tok = u / KCH, c = (u % KCH) * 8;
-            ks[i] = *reinterpret_cast<const u32x4_a*>(row(tok, kr, D, kn, a.k_row) + (c < D ? c : 0));
-        });
-        static_for<VLOADS>([&](auto I) {
-            constexpr int i = decltype(I)::value;
-            const int u = i * 256 + tid, tok = u / VCH, c = (u % VCH) * 8;
-            vs[i] = *reinterpret_cast<const u32x4_a*>(row(tok, vr, Dv, vn, a.v_row) + (c < Dv ? c : 0));
-        });
-    };
-    auto put = [&](int buf) {
-        static_for<KLOADS>([&](auto I) {
-            constexpr int i = decltype(I)::value;
-            const int u = i * 256 + tid;
-            *reinterpret_cast<u32x4_a*>(kt(buf) + (u / KCH) * KROW + (u % KCH) * 8) = ks[i];
-        });
-        static_for<VLOADS>([&](auto I) {
-            constexpr int i = decltype(I)::value;
-            const int u = i * 256 + tid;
-            *reinterpret_cast<u32x4_a*>(vt(buf) + (u / VCH) * VROW + (u % VCH) * 8) = vs[i];
-        });
-    };
-    floatx16_a o[VT];
-    static_for<VT>([&](auto I) {
-        constexpr int i = decltype(I)::value;
-#pragma unroll
-        for (int j = 0; j < 16; j++) o[i][j] = 0.0f;
-    });
-    float m = kNone, l = 0.0f;
-    const float scale2 = a.scale * kLog2e, slope2 = a.slopes ? a.slopes[h] * kLog2e : 0.0f;
-
-    if (it0 < it1) {
-        fetch(it0);
-        put(it0 & 1);
-    }
-    __syncthreads();
-    for (int it = it0; it < it1; it++) {
-        const int buf = it & 1;
-        if (it + 1 < it1) fetch(it + 1);
-        __builtin_amdgcn_sched_barrier(0);
-        const int key0 = it * kPromptKeys;
-        if (key0 <= wave_last && key0 + kPromptKeys - 1 > wave_first - window) {        // uniform over the wavefront
-            floatx16_a s[2];
-#pragma unroll
-            for (int u = 0; u < 2; u++)
-#pragma unroll
-                for (int j = 0; j < 16; j++) s[u][j] = 0.0f;
-            const uint16_t* kp = kt(buf) + col * KROW + 8 * hi;
-            static_for<KS>([&](auto I) {
-                constexpr int i = decltype(I)::value;
-                s[0] = mma32<T>(*reinterpret_cast<const u32x4_a*>(kp + i * 16), q[i], s[0]);
-                s[1] = mma32<T>(*reinterpret_cast<const u32x4_a*>(kp + 32 * KROW + i * 16), q[i], s[1]);
-            });
-            // this lane: query qi, keys key0 + 32 u + 8 (j / 4) + 4 hi + j % 4
-            float mx = kNone;
-            const float base = -slope2 * static_cast<float>(limit - key0 - 4 * hi);
-            const bool whole = key0 + kPromptKeys - 1 <= wave_first && key0 > wave_last - window && key0 >= lo;
-#pragma unroll
-            for (int u = 0; u < 2; u++)
-#pragma unroll
-                for (int j = 0; j < 16; j++) {
-                    const int e = 32 * u + 8 * (j >> 2) + (j & 3);
-                    s[u][j] = __builtin_fmaf(s[u][j], scale2, __builtin_fmaf(slope2, static_cast<float>(e), base));
-                }
-            if (!whole) {
-#pragma unroll
-                for (int u = 0; u < 2; u++)
-#pragma unroll
-                    for (int j = 0; j < 16; j++) {
-                        const int key = key0 + 32 * u + 8 * (j >> 2) + 4 * hi + (j & 3);
-                        if (key > limit || limit - key >= window || key < lo) s[u][j] = -INFINITY;
-                    }
-            }
-#pragma unroll
-            for (int u = 0; u < 2; u++)
-#pragma unroll
-                for (int j = 0; j < 16; j++) mx = fmaxf(mx, s[u][j]);
-            mx = fmaxf(mx, __shfl_xor(mx, 32));
-            if (__any(mx > m)) {
-                const float mn = fmaxf(m, mx), al = exp2_hw(m - mn);
-                l *= al;
-                static_for<VT>([&](auto I) {
-                    constexpr int i = decltype(I)::value;
-#pragma unroll
-                    for (int j = 0; j < 16; j++) o[i][j] *= al;
-                });
-                m = mn;
-            }
-            u32x4_a p[4];                                           // right operands of the four 16-token steps
-#pragma unroll
-            for (int u = 0; u < 2; u++)
-#pragma unroll
-                for (int j = 0; j < 16; j += 2) {
-                    const float e0 = exp2_hw(s[u][j] - m), e1 = exp2_hw(s[u][j + 1] - m);
-                    l += e0 + e1;
-                    p[2 * u + (j >> 3)][(j & 7) >> 1] = pack2<T>(e0, e1);
-                }
-            // 16 lanes read 4 tokens x 16 channels and get them transposed: a lane ends up with its channel's tokens 4 hi .. and
-            // 8 + 4 hi .. of a 16-token step, the order in which p holds them
-            const int r16 = lane & 15;
-            const uint16_t* vp = vt(buf) + (4 * hi + (r16 >> 2)) * VROW + ((lane >> 4) & 1) * 16 + (r16 & 3) * 4;
-            static_for<VT>([&](auto I) {
-                constexpr int i = decltype(I)::value;
-                static_for<4>([&](auto J) {
-                    constexpr int j = decltype(J)::value;
-                    const u32x2_a w0 = __builtin_bit_cast(u32x2_a, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(vp + i * 32 + j * 16 * VROW)));
-                    const u32x2_a w1 = __builtin_bit_cast(u32x2_a, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(vp + i * 32 + (j * 16 + 8) * VROW)));
-                    o[i] = mma32<T>(u32x4_a{w0.x, w0.y, w1.x, w1.y}, p[j], o[i]);
-                });
-            });
-        }
-        if (it + 1 < it1) put(buf ^ 1);
-        __syncthreads();
-    }
-    l += __shfl_xor(l, 32);
-    if (!valid) return;
-    const float inv = l > 0.0f ? a.out_scale / l : 0.0f;
-    uint16_t* out = static_cast<uint16_t*>(a.out) + (static_cast<size_t>(b) * a.L + qi) * a.out_row + static_cast<size_t>(h) * Dv;
-    static_for<VT>([&](auto I) {
-        constexpr int i = decltype(I)::value;
-#pragma unroll
-        for (int j4 = 0; j4 < 4; j4++) {
-            const int ch = i * 32 + 8 * j4 + 4 * hi;
-            if (ch < Dv)
-                *reinterpret_cast<uint2*>(out + ch) = make_uint2(pack2<T>(o[i][4 * j4] * inv, o[i][4 * j4 + 1] * inv),
-                                                                 pack2<T>(o[i][4 * j4 + 2] * inv, o[i][4 * j4 + 3] * inv));
-        }
-    });
-}
-
-template <typename T, int P>
-static int window_prefill_one(const WindowAttnArgs& a, hipStream_t st) {
-    constexpr size_t bytes = 2 * 2 * static_cast<size_t>(kPromptKeys) * ((P + 8) + (P + 16));
-    static_assert(bytes <= 160 * 1024, "LDS");
-    if (bytes > 64 * 1024) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&window_prefill_kernel<T, P, P>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
-        if (e != hipSuccess) return static_cast<int>(e);
-    }
-    dim3 grid(a.H, (a.L + kPromptRows - 1) / kPromptRows, a.B), block(256);
-    hipLaunchKernelGGL((window_prefill_kernel<T, P, P>), grid, block, bytes, st, a);
-    return static_cast<int>(hipGetLastError());
-}
-
 template <typename T>
-static int window_prefill_dims(const WindowAttnArgs& a, hipStream_t st) {
-    const int widest = a.D > a.Dv ? a.D : a.Dv;
-    return widest <= 64 ? window_prefill_one<T, 64>(a, st) : widest <= 128 ? window_prefill_one<T, 128>(a, st) : window_prefill_one<T, 256>(a, st);
+static int window_prefill_dims(const WindowAttnArgs& w, hipStream_t st) {
+    PromptAttnArgs a{};
+    a.q = w.q; a.q_b = static_cast<int64_t>(w.L) * w.H * w.D; a.q_t = static_cast<int64_t>(w.H) * w.D; a.q_h = w.D;
+    a.k = w.k_new; a.k_b = w.L * w.k_row; a.k_t = w.k_row; a.k_h = w.D;
+    a.v = w.v_new; a.v_b = w.L * w.v_row; a.v_t = w.v_row; a.v_h = w.Dv;
+    a.k_ring = w.k_ring; a.v_ring = w.v_ring; a.cap = w.cap; a.window = w.window; a.slopes = w.slopes;
+    a.start = w.start; a.out = w.out; a.out_row = w.out_row; a.out_scale = w.out_scale; a.scale = w.scale;
+    a.B = w.B; a.L = w.L; a.Lk = w.pos + w.L; a.H = w.H; a.G = w.G; a.D = w.D; a.Dv = w.Dv;
+    const int widest = w.D > w.Dv ? w.D : w.Dv;
+    return widest <= 64 ? launch_prompt_attn<T, 64, 64, true, true>(a, st) : widest <= 128 ? launch_prompt_attn<T, 128, 128, true, true>(a, st)
+                                                                                           : launch_prompt_attn<T, 256, 256, true, true>(a, st);
 }
 int launch_window_prefill(const WindowAttnArgs& a, int dtype, hipStream_t st) {
     return dtype == 0 ? window_prefill_dims<F16>(a, st) : window_prefill_dims<BF16>(a, st);

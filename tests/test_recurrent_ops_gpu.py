@@ -132,6 +132,35 @@ def test_one_key_at_the_windows_edge(gpu):
                 assert err(run_window(gpu, p, wq, wk, *args, cuts), want[None]) < 1.5e-2, (window, at, cuts[:3])
 
 
+@pytest.mark.parametrize("D,Dv", [(64, 64), (8, 64), (128, 120), (72, 128), (256, 136), (192, 256)])
+@pytest.mark.parametrize("past", [0, 1, 63, 64, 200])
+def test_prompt_tiles_from_ring_and_call(gpu, D, Dv, past):
+    """A prompt whose keys come from the ring, from the call, or from both inside one tile, padded at the front of one sequence,
+    with scales of either sign and none; windows that begin at the edges of tiles."""
+    B, H, G, L = 2, 4, 2, 131
+    g = torch.Generator().manual_seed(D + past)
+    for dt in ("bf16", "f16"):
+        q, k, v = rand(g, B, L, H, D, dt=dt), rand(g, B, past + L, G, D, dt=dt), rand(g, B, past + L, G, Dv, dt=dt)
+        for window, scale in ((64, D ** -0.5), (65, -1.5 * D ** -0.5), (past + L, 0.0), (1, 1.0)):
+            ring = ops.WindowRing(B, G, D, Dv, window, DT[dt], gpu)
+            slots = torch.arange(max(0, past - ring.cap), past)
+            ring.k[:, :, slots % ring.cap] = k[:, slots].transpose(1, 2).to(gpu)
+            ring.v[:, :, slots % ring.cap] = v[:, slots].transpose(1, 2).to(gpu)
+            slopes, start = torch.tensor([0.3, 0.0, 0.01, 0.05]), torch.tensor([0, 70], dtype=torch.int32)
+            out = torch.empty(B * L, H * Dv, dtype=DT[dt], device=gpu)
+            ops.window_attention(q.view(B * L, -1).to(gpu), ring, slopes.to(gpu), scale, Step(B, L, past, start=start.to(gpu)), out, 1.0,
+                                 k[:, past:].reshape(B * L, -1).to(gpu), v[:, past:].reshape(B * L, -1).to(gpu))
+            got = out.view(B, L, H * Dv)
+            for b in range(B):
+                s0 = int(start[b])
+                full = torch.zeros(past + L, H, D).double()
+                full[past:] = q[b].double()
+                want = ko.window_attention_fast(full[s0:], k[b, s0:].double(), v[b, s0:].double(), scale, slopes.double(), window)
+                rows = slice(max(past, s0) - s0, None)              # (a query before its sequence's start sees nothing)
+                # weights and results are rounded to the dtype; scores up to ~10 carry its rounding nowhere else
+                assert err(got[b, max(past, s0) - past:], want[rows]) < TOL[dt], (dt, window, scale, b)
+
+
 # ---------------------------------------------------------------- gated delta rule
 def delta_case(g, B, T, G, H, dim, vdim, taps, dt):
     kd, vd = G * dim, H * vdim
