@@ -79,10 +79,8 @@ class Fp16KVGraphDecoder(PolarGraphDecoder):
             h = rmsnorm(x, nn_.weight, nn_.variance_epsilon, residual=y, sum_out=x)
         logits = model.lm_head(h[:, -1:, :])
         self.B, self.kv_len, self.n_resid = B, L, L
-        self.pos = torch.full((1,), L, dtype=torch.int64, device=dev)
-        self.resid_idx = self.pos.clone()                      # the key's row is the position as well
+        self._set_counters(B, L, L, dev)                       # the key's row is the position as well
         self.n_groups_dev = torch.zeros((B,), dtype=torch.int32, device=dev)
-        self.n_resid_dev = torch.full((B,), L + 1, dtype=torch.int32, device=dev)     # keys INCLUDING the new one
         self.ids = torch.zeros((B, 1), dtype=torch.long, device=dev)
         self.mask8 = None
         inv_freq = m.rotary_emb.inv_freq.float().to(dev)
