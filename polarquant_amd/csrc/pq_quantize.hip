@@ -12,11 +12,21 @@
 //
 // Arithmetic follows eager torch on half tensors op by op: every reference op
 // is evaluated in fp32 and rounded to the key dtype before the next.
+//
+// What bounds it: the vector unit, about 65 instructions a pair of which two at a quarter of the rate (111 of the 125 to 131 us that
+// 131072 tokens of 8 heads take; their bytes need 68).  With the codes' quotients by three operations and rounded by conversions,
+// the angle's sign put on and taken off again and a test of each pair's range it was 143 to 155 us.  Gathering a workgroup's entries
+// for the exact routines so that one wavefront does them all: 128 instead of 131 us at best, short calls slower; not kept.
 #include "pq_device.h"
 #include "pq_internal.h"
 #include "pq_math.h"
 
 namespace pq {
+
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef __bf16 bfloat2v __attribute__((ext_vector_type(2)));
+typedef float float2v __attribute__((ext_vector_type(2)));
+typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
 
 template <typename T>
 __device__ __forceinline__ float rnd(float f) { return lo2f<T>(f2lo<T>(f)); }
@@ -36,8 +46,8 @@ __device__ __forceinline__ float rnd(float f) { return lo2f<T>(f2lo<T>(f)); }
 template <typename T> struct IsHalf { static constexpr bool value = false; };
 template <> struct IsHalf<F16> { static constexpr bool value = true; };
 template <typename T> struct DT;
-template <> struct DT<F16> { static constexpr uint32_t kLowMask = 0x1fffu, kMid = 0x1000u; static constexpr float kMinNormal = 6.103515625e-05f; };
-template <> struct DT<BF16> { static constexpr uint32_t kLowMask = 0xffffu, kMid = 0x8000u; static constexpr float kMinNormal = 1.17549435e-38f; };
+template <> struct DT<F16> { static constexpr uint32_t kMid = 0x1000u; static constexpr int kHighBits = 19; static constexpr float kMinNormal = 6.103515625e-05f; };
+template <> struct DT<BF16> { static constexpr uint32_t kMid = 0x8000u; static constexpr int kHighBits = 16; static constexpr float kMinNormal = 1.17549435e-38f; };
 
 constexpr uint32_t kAtanGuardUlps = 5;   // the fast arctangent stays within 4 ulp of the exact routine (exhaustive self-test)
 constexpr uint32_t kSqrtGuardUlps = 2;   // v_sqrt_f32 is within 1 ulp
@@ -58,14 +68,15 @@ __device__ __forceinline__ float atan2_exact(float y, float x) {
 
 template <typename T>
 __device__ __forceinline__ bool near_rounding_boundary(float a, uint32_t guard) {
-    // |low mantissa bits - midpoint pattern| <= guard, computed without a branch
-    const uint32_t low = (__float_as_uint(a) + (guard - DT<T>::kMid)) & DT<T>::kLowMask;
-    return low <= 2u * guard;
+    // |low mantissa bits - midpoint pattern| <= guard: the sum's low bits at the top of the word, one shifted addition and one comparison
+    const uint32_t low = (__float_as_uint(a) + (guard - DT<T>::kMid)) << DT<T>::kHighBits;
+    return low < (2u * guard + 1u) << DT<T>::kHighBits;
 }
 
-__device__ __forceinline__ float atan2_fast(float y, float x) {
+// the angle's magnitude
+__device__ __forceinline__ float atan2_fast_abs(float y, float x) {
     const float ax = fabsf(x), ay = fabsf(y);
-    const float mx = fmaxf(ax, ay), mn = fminf(ax, ay);
+    const float mx = ay > ax ? ay : ax, mn = ay > ax ? ax : ay;
     const float r = mn * __builtin_amdgcn_rcpf(mx);
     const float s = r * r;
     float u = 0.00282363896258175373077393f;
@@ -78,31 +89,33 @@ __device__ __forceinline__ float atan2_fast(float y, float x) {
     u = __builtin_fmaf(u, s, -0.333331018686294555664062f);
     float a = __builtin_fmaf(u * s, r, r);
     a = ay > ax ? 1.57079637050628662109f - a : a;
-    a = x < 0.0f ? 3.14159274101257324219f - a : a;
-    return __builtin_copysignf(a, y);
+    return x < 0.0f ? 3.14159274101257324219f - a : a;
 }
 
-// Cheap estimates of the angle (in [-pi, pi]) and radius, NOT yet rounded; returns true when
-// the exact routines must be used instead (see above).
+// Cheap estimates of the angle's magnitude (its sign is y's) and of the radius, NOT yet rounded; returns true when
+// the exact routines must be used instead (see above), or when *ss_out says so (squares_out_of_range).
 template <typename T, bool LIBM = false>
-__device__ __forceinline__ bool angle_radius_fast(float x, float y, float* a_out, float* r_out) {
+__device__ __forceinline__ bool angle_radius_fast(float x, float y, float* a_out, float* r_out, float* ss_out) {
     const float ss = __builtin_fmaf(x, x, y * y);          // x*x, y*y are exact for half/bf16 operands
-    const float a = atan2_fast(y, x);
+    const float a = atan2_fast_abs(y, x);
     const float r = __builtin_amdgcn_sqrtf(ss);
-    // Infinities, NaNs, and (bfloat16 only) magnitudes at which the reciprocal or the hardware
-    // square root leave their accurate range: one comparison for half, whose finite squares all lie
-    // inside (2^-80, 2^80).  Zeros need no test of their own: with one zero operand the estimate is
+    // (bfloat16 only) magnitudes at which the reciprocal or the hardware square root leave their accurate range; half's
+    // finite squares all lie inside (2^-80, 2^80).  Zeros need no test of their own: with one zero operand the estimate is
     // exactly 0, pi/2 or pi like the exact routine's (0 then fails the kMinNormal test below), and
     // x == y == 0 gives a NaN angle with radius 0, which fails that test as well.
     // (bitwise | on purpose: one straight-line predicate instead of a chain of exec-mask branches)
-    int special = static_cast<int>(!(ss < 0x1p80f));
+    int special = 0;
     if constexpr (!IsHalf<T>::value) special |= static_cast<int>(!(ss > 0x1p-80f));
     *a_out = a;
     *r_out = r;
-    return (special | static_cast<int>(fminf(fabsf(a), r) < DT<T>::kMinNormal) |
+    *ss_out = ss;
+    return (special | static_cast<int>(fminf(a, r) < DT<T>::kMinNormal) |
             static_cast<int>(near_rounding_boundary<T>(a, Atan<LIBM>::kGuardUlps)) |
             static_cast<int>(near_rounding_boundary<T>(r, kSqrtGuardUlps))) != 0;
 }
+// Infinities, NaNs and large bfloat16 magnitudes, of one pair's squares or, as patterns order like the numbers and NaNs lie above
+// them all, of the largest pattern of many.
+__device__ __forceinline__ bool squares_out_of_range(uint32_t ss_bits) { return ss_bits >= 0x67800000u; }      // 2^80
 
 // Correctly rounded fp32 square root.  NOT __fsqrt_rn: HIP defines that as the native (1 ulp)
 // instruction unless OCML_BASIC_ROUNDED_OPERATIONS is set; sqrtf() is expanded by the compiler to
@@ -113,8 +126,10 @@ __device__ __forceinline__ float sqrt_rn(float s) { return __builtin_sqrtf(s); }
 // -> (angle in [-pi, pi], radius), both rounded to the key dtype
 template <typename T, bool LIBM = false>
 __device__ __forceinline__ void angle_radius(float x, float y, float* phi, float* rad) {
-    float a, r;
-    if (__builtin_expect(angle_radius_fast<T, LIBM>(x, y, &a, &r), 0)) {
+    float a, r, ss;
+    const bool risky = angle_radius_fast<T, LIBM>(x, y, &a, &r, &ss);
+    a = __builtin_copysignf(a, y);
+    if (__builtin_expect(risky || squares_out_of_range(__float_as_uint(ss)), 0)) {
         a = atan2_exact<LIBM>(y, x);
         r = sqrt_rn(__builtin_fmaf(x, x, y * y));
     }
@@ -138,12 +153,38 @@ __device__ __forceinline__ uint32_t code_of(float v, float mn, float scale, floa
     const float qf = floorf(rnd<T>(d / scale));
     return static_cast<uint32_t>(__builtin_amdgcn_fmed3f(qf, 0.0f, topf));
 }
-// The same with div_faithful in place of the division; `inv` = v_rcp_f32(scale), scale accepted by fast_div_ok.
+// The same of the rounded distance d >= 0 for scales that fast_div_ok accepts and top <= 127, without a division.
+//
+// Rounding to the dtype carries a quotient to the integer k or over it exactly if half a unit in the last place of its own binade
+// does (an integer up to 128 is even in both dtypes: a tie goes to it), and adding kMid to the fp32 pattern adds that half: no
+// conversion there and back, no floor.  So only the side of B = k - half a unit on which d / scale lies has to be right.  d is a
+// number of 11 bits (bfloat16: 8) and B * scale one of 23 (17), so a quotient below B is below it by 2^-23 (2^-17) of it at least.
+// Half: the inverse in two parts; the product's one rounding then neither reaches B from there nor leaves it.  Bfloat16: an inverse
+// too large by 2^-22 to 2^-20 is enough.  Every pair of operands is checked on the device.  A NaN stays one and converts to 0.
+struct Inverse { float hi, lo; };
 template <typename T>
-__device__ __forceinline__ uint32_t code_of_fast(float v, float mn, float scale, float inv, float topf) {
-    const float d = rnd<T>(v - mn);
-    const float qf = floorf(rnd<T>(div_faithful(d, scale, inv)));
-    return static_cast<uint32_t>(__builtin_amdgcn_fmed3f(qf, 0.0f, topf));
+__device__ __forceinline__ Inverse inverse_of(float scale) {
+    const float inv = __builtin_amdgcn_rcpf(scale);                  // within 1 ulp
+    if constexpr (IsHalf<T>::value) return {inv, __builtin_fmaf(-scale, inv, 1.0f) * inv};
+    else return {__builtin_fmaf(inv, 0x1p-21f, inv), 0.0f};
+}
+template <typename T>
+__device__ __forceinline__ uint32_t code_of_fast(float d, Inverse inv, uint32_t top) {
+    const float q = IsHalf<T>::value ? __builtin_fmaf(d, inv.hi, d * inv.lo) : d * inv.hi;
+    const uint32_t k = static_cast<uint32_t>(__uint_as_float(__float_as_uint(q) + DT<T>::kMid));
+    return k < top ? k : top;
+}
+// (angle - its minimum | radius - its minimum << 16), each rounded to the dtype.  Half: one packed subtraction (a sum or difference of
+// two halves that is rounded to fp32 first is the same half).
+template <typename T> __device__ __forceinline__ void pair_distance(uint32_t v, uint32_t mn, float* da, float* dr);
+template <> __device__ __forceinline__ void pair_distance<F16>(uint32_t v, uint32_t mn, float* da, float* dr) {
+    const half2v d = __builtin_bit_cast(half2v, v) - __builtin_bit_cast(half2v, mn);
+    *da = static_cast<float>(d.x);
+    *dr = static_cast<float>(d.y);
+}
+template <> __device__ __forceinline__ void pair_distance<BF16>(uint32_t v, uint32_t mn, float* da, float* dr) {
+    *da = rnd<BF16>(__uint_as_float(v << 16) - __uint_as_float(mn << 16));
+    *dr = rnd<BF16>(__uint_as_float(v & 0xffff0000u) - __uint_as_float(mn & 0xffff0000u));
 }
 __device__ __forceinline__ float clamp_bound(float scale, int top) { return scale > 0.0f ? static_cast<float>(top) : 0.0f; }
 
@@ -151,19 +192,20 @@ constexpr int kQThreads = 256;
 constexpr int kTokPerThread = kGroup / 16;   // 8
 constexpr int kEntries = kTokPerThread * 4;  // (token, pair) entries per thread
 
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
-
 // Packed min / max of two (angle word | radius word << 16) registers.  Both values are
 // non-negative (the angle after the 2*pi wrap, the radius always) and their sign bits are
 // cleared, so bfloat16 words order like unsigned integers; half words use v_pk_max/min_f16.
 template <typename T> __device__ __forceinline__ uint32_t pk_max(uint32_t a, uint32_t b);
 template <typename T> __device__ __forceinline__ uint32_t pk_min(uint32_t a, uint32_t b);
 template <> __device__ __forceinline__ uint32_t pk_max<F16>(uint32_t a, uint32_t b) {
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(half2v, a), __builtin_bit_cast(half2v, b)));
+    uint32_t r;                                 // (the builtin first passes what comes from memory through a maximum of its own)
+    asm("v_pk_max_f16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
 }
 template <> __device__ __forceinline__ uint32_t pk_min<F16>(uint32_t a, uint32_t b) {
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(half2v, a), __builtin_bit_cast(half2v, b)));
+    uint32_t r;
+    asm("v_pk_min_f16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
 }
 template <> __device__ __forceinline__ uint32_t pk_max<BF16>(uint32_t a, uint32_t b) {
     return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(ushort2v, a), __builtin_bit_cast(ushort2v, b)));
@@ -183,20 +225,29 @@ struct AngleMode {
     float two_pi;      // reference mode: the constant added to negative angles
     float tmn, tscale; // uniform mode
     int ttop;
+    float minus_one;
 };
 
-// (angle word | radius word << 16) of one pair: wrap applied, sign bits cleared
-template <typename T, bool UNIFORM>
-__device__ __forceinline__ uint32_t pack_angle_radius(float a, float r, const AngleMode& am) {
-    float phi = rnd<T>(a);
-    uint32_t aw;
+// (angle word | radius word << 16) of one pair: wrap applied, sign bits cleared.  ESTIMATE: of angle_radius_fast's values where it
+// does not ask for the exact routines; no zero is among them, so neither is a sign that the wrap leaves.
+// (its magnitude; the angle is negative where y's sign bit is set)
+template <typename T, bool UNIFORM, bool ESTIMATE>
+__device__ __forceinline__ uint32_t pack_angle_radius(float a, float r, float y, const AngleMode& am) {
+    uint32_t w;
+    const bool below = static_cast<int>(__float_as_uint(y)) < 0;
     if constexpr (UNIFORM) {
-        aw = code_of_fast<T>(phi, am.tmn, am.tscale, __builtin_amdgcn_rcpf(am.tscale), static_cast<float>(am.ttop));
+        const uint32_t aw = code_of_fast<T>(rnd<T>(rnd<T>(__builtin_copysignf(a, y)) - am.tmn), inverse_of<T>(am.tscale), am.ttop);
+        w = aw | (static_cast<uint32_t>(f2lo<T>(r)) << 16);
+    } else if constexpr (IsHalf<T>::value) {
+        // (times minus one: a subtraction with the conversions of its operand and of its result built in)
+        const _Float16 phi = static_cast<_Float16>(a);
+        const _Float16 turned = static_cast<_Float16>(__builtin_fmaf(static_cast<float>(phi), am.minus_one, am.two_pi));       // :144
+        w = __builtin_bit_cast(uint32_t, half2v{below && (ESTIMATE || phi > static_cast<_Float16>(0.0f)) ? turned : phi, static_cast<_Float16>(r)});
     } else {
-        if (phi < 0.0f) phi = rnd<T>(phi + am.two_pi);             // :144
-        aw = f2lo<T>(phi);
+        const float phi = rnd<T>(a);
+        w = __builtin_bit_cast(uint32_t, __builtin_convertvector((float2v{below && (ESTIMATE || phi > 0.0f) ? am.two_pi - phi : phi, r}), bfloat2v));       // :144
     }
-    return (aw | (static_cast<uint32_t>(f2lo<T>(r)) << 16)) & 0x7fff7fffu;
+    return ESTIMATE ? w : w & 0x7fff7fffu;
 }
 
 template <typename T, bool UNIFORM, bool PK6, bool LIBM>
@@ -216,7 +267,7 @@ __global__ __launch_bounds__(kQThreads) void quantize_kernel(
     const uint16_t* kb = k + b * sb + h * sh + static_cast<int64_t>(grp) * kGroup * st;
 
     // ---- pass 1: cheap estimates for every entry; remember which entries need the exact routines
-    uint32_t risky_mask = 0;
+    uint32_t risky_mask = 0, ss_most = 0;
 #pragma unroll
     for (int it = 0; it < kTokPerThread; it++) {
         const uint16_t* row = kb + (it * 16 + tl) * st;
@@ -228,22 +279,25 @@ __global__ __launch_bounds__(kQThreads) void quantize_kernel(
                                 static_cast<uint16_t>(yw.y), static_cast<uint16_t>(yw.y >> 16)};
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            float a, r;
-            const bool risky = angle_radius_fast<T, LIBM>(lo2f<T>(xs[i]), lo2f<T>(ys[i]), &a, &r);   // :143, :150
-            risky_mask |= static_cast<uint32_t>(risky) << (it * 4 + i);
-            pr[it * 4 + i][tid] = pack_angle_radius<T, UNIFORM>(a, rnd<T>(r), am);
+            float a, r, ss;
+            const float y = lo2f<T>(ys[i]);
+            const bool risky = angle_radius_fast<T, LIBM>(lo2f<T>(xs[i]), y, &a, &r, &ss);   // :143, :150
+            risky_mask = risky_mask + risky_mask + (risky ? 1u : 0u);                         // (entry e in bit 31 - e)
+            ss_most = ss_most > __float_as_uint(ss) ? ss_most : __float_as_uint(ss);
+            pr[it * 4 + i][tid] = pack_angle_radius<T, UNIFORM, true>(a, r, y, am);
         }
     }
+    if (squares_out_of_range(ss_most)) risky_mask = 0xffffffffu;
     // ---- fix-up: each lane redoes ITS risky entries with the exact routines (a lane has ~0.1 of
     // them, so the wavefront makes one or two trips instead of branching at all 32 entries)
     while (risky_mask) {
-        const int e = __builtin_ctz(risky_mask);
-        risky_mask &= risky_mask - 1;
+        const int e = __builtin_clz(risky_mask);
+        risky_mask &= ~(0x80000000u >> e);
         const uint16_t* row = kb + ((e >> 2) * 16 + tl) * st;
         const float x = lo2f<T>(row[4 * pq4 + (e & 3)]), y = lo2f<T>(row[kPairs + 4 * pq4 + (e & 3)]);
         float a, r;
         angle_radius_exact<T, LIBM>(x, y, &a, &r);
-        pr[e][tid] = pack_angle_radius<T, UNIFORM>(a, r, am);
+        pr[e][tid] = pack_angle_radius<T, UNIFORM, false>(fabsf(a), r, a, am);
     }
     // ---- per-pair max / min of angle and radius over the 128 tokens (packed: both at once)
     uint32_t vmax[4], vmin[4];
@@ -311,12 +365,12 @@ __global__ __launch_bounds__(kQThreads) void quantize_kernel(
     uint8_t* cb = codes + plane * (kGroup * (PK6 ? kPackedRowBytes : kPairs));
     // scales of 0 (degenerate pairs), infinities and the far ends of the bfloat16 range take the division
     bool fast = true;
-    float tinv[4], rinv[4];
+    Inverse tinv[4], rinv[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         fast = fast && fast_div_ok(ts[i]) && fast_div_ok(rs[i]);
-        tinv[i] = __builtin_amdgcn_rcpf(ts[i]);
-        rinv[i] = __builtin_amdgcn_rcpf(rs[i]);
+        tinv[i] = inverse_of<T>(ts[i]);
+        rinv[i] = inverse_of<T>(rs[i]);
     }
     auto store_codes = [&](int it, uint32_t w) {
         if constexpr (PK6) {
@@ -334,17 +388,21 @@ __global__ __launch_bounds__(kQThreads) void quantize_kernel(
     };
     // PK6 exchanges words between lanes, so the whole wavefront takes one side together
     if (__builtin_expect(PK6 ? __all(fast) : fast, 1)) {
+        const uint32_t tlast = (1u << tbits) - 1u, rlast = (1u << rbits) - 1u;
+        uint32_t least[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) least[i] = fin[1][4 * pq4 + i];
 #pragma unroll
         for (int it = 0; it < kTokPerThread; it++) {
             uint32_t w = 0;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const uint32_t v = pr[it * 4 + i][tid];
-                const float phi = lo2f<T>(static_cast<uint16_t>(v & 0xffffu));
-                const float r = lo2f<T>(static_cast<uint16_t>(v >> 16));
-                const uint32_t th = UNIFORM ? (v & 0xffffu) : code_of_fast<T>(phi, tm[i], ts[i], tinv[i], ttop[i]);    // :148
-                const uint32_t rh = code_of_fast<T>(r, rm[i], rs[i], rinv[i], rtop[i]);      // :153
-                w |= (((rh << tbits) + th) & 0xffu) << (8 * i);             // :155
+                float da, dr;
+                pair_distance<T>(v, least[i], &da, &dr);
+                const uint32_t th = UNIFORM ? (v & 0xffffu) : code_of_fast<T>(da, tinv[i], tlast);    // :148
+                const uint32_t rh = code_of_fast<T>(dr, rinv[i], rlast);                             // :153
+                w |= ((rh << tbits) + th) << (8 * i);                       // :155 (below 256)
             }
             store_codes(it, w);
         }
@@ -392,14 +450,14 @@ __global__ __launch_bounds__(256) void selftest_kernel(unsigned long long* misma
             const double hi = 0.5 * (static_cast<double>(rr) + static_cast<double>(__uint_as_float(__float_as_uint(rr) + 1u)));
             bad += !(lo * lo <= static_cast<double>(s) && static_cast<double>(s) <= hi * hi);
         }
-        const float a = atan2_fast(y, x), r = __builtin_amdgcn_sqrtf(__builtin_fmaf(x, x, y * y));
+        const float a = atan2_fast_abs(y, x), r = __builtin_amdgcn_sqrtf(__builtin_fmaf(x, x, y * y));
         slow += near_rounding_boundary<T>(a, Atan<LIBM>::kGuardUlps) || near_rounding_boundary<T>(r, kSqrtGuardUlps);
     }
     if (bad) atomicAdd(mismatches, static_cast<unsigned long long>(bad));
     if (slow) atomicAdd(slow_lanes, static_cast<unsigned long long>(slow));
 }
 
-// Exhaustive check of div_faithful: block == bit pattern of the dividend d, thread t covers the
+// Exhaustive check of div_faithful and of the codes taken from it: block == bit pattern of the dividend d, thread t covers the
 // divisor patterns t, t+256, ...  Pairs the quantizers can meet: divisor accepted by fast_div_ok,
 // 0 <= d <= 1024 * sc (d is a distance from the group minimum and sc the group's range over at
 // most 2^8 bins).  Quotients below 1/4 may differ in denormal digits; floor() and rint() of both
@@ -415,6 +473,7 @@ __global__ __launch_bounds__(256) void selftest_div_kernel(unsigned long long* m
             const float exact = rnd<T>(d / sc);
             const float fast = rnd<T>(div_faithful(d, sc, __builtin_amdgcn_rcpf(sc)));
             bad += (exact != fast) && !(exact < 0.25f && fast < 0.25f);
+            bad += code_of_fast<T>(d, inverse_of<T>(sc), 127u) != static_cast<uint32_t>(__builtin_amdgcn_fmed3f(floorf(exact), 0.0f, 127.0f));
         }
     }
     if (bad) atomicAdd(mismatches, static_cast<unsigned long long>(bad));
@@ -445,6 +504,7 @@ int launch_quantize(const void* k, const int64_t* strides, int dtype, int B, int
     const bool uniform = (flags & 2u) != 0;
     am.two_pi = (flags & 1u) ? two_pi_f : 6.28125f;
     am.ttop = (1 << tbits) - 1;
+    am.minus_one = -1.0f;
     const bool bf = dtype != 0;
     auto round_dt = [bf](float f) {
         return bf ? math::bf16_bits_to_float(math::float_to_bf16_bits(f)) : math::half_bits_to_float(math::float_to_half_bits(f));

@@ -200,6 +200,25 @@ def test_quantizer_math_selftest_exhaustive(gpu, dtype_code, name):
     assert bad_div == 0     # reciprocal + two fused multiply-adds against the fp32 division, every (dividend, scale) pair
 
 
+@pytest.mark.parametrize("dtype,exponents", [(torch.float16, (-15, -9, 0, 7, 14)), (torch.bfloat16, (-90, -45, -39, 0, 38, 41, 60))])
+@pytest.mark.parametrize("rbits,tbits", [(4, 4), (7, 1), (1, 7)])
+def test_magnitudes_zeros_and_equal_keys(gpu, dtype, exponents, rbits, tbits):
+    """Keys at both ends of the dtype's range and on either side of where squares leave the estimates' range, with zeros of both
+    signs, keys of few distinct values (distances and scales whose quotients are whole numbers) and groups of one value."""
+    for e in exponents:
+        g = torch.Generator().manual_seed(1000 + e)
+        k = (torch.randn(1, 2, 384, 128, generator=g) * 2.0 ** e).to(dtype)
+        k[0, 0, 5::9, ::2] = 0.0
+        k[0, 0, 7::11, 1::3] = -0.0
+        k[0, 0, :128, 90:] = k[0, 0, :1, 90:]
+        k[0, 1, 128:256] = (torch.randint(-3, 4, (128, 128), generator=g) * 2.0 ** e).to(dtype)
+        k[0, 1, 256:, :64] = (torch.randint(1, 130, (128, 64), generator=g) * 2.0 ** (e - 6)).to(dtype)    # radii on a grid
+        k[0, 1, 256:, 64:] = 0.0
+        flips = count_flips(quantize_and_pack_nbit(k.to(gpu), rbits, tbits), po.quantize_and_pack_nbit(k, rbits, tbits))
+        scales = po.quantize_and_pack_nbit(k, rbits, tbits)
+        assert all(v == 0 for v in flips.values()), (e, flips, scales[1].float().min())
+
+
 def test_radius_on_a_double_rounding_tie(gpu):
     """x = 0xa2cd, y = 0x15b1 (half words): the correctly rounded fp32 square root of x^2 + y^2 lies one ulp above
     a midpoint between two half values, a 1-ulp-low square root lies exactly on it and rounds (to even) the other
