@@ -48,8 +48,8 @@ template <> __device__ __forceinline__ uint16_t f2lo<BF16>(float f) {
 
 // ---- division of two key-dtype values, rounded to the key dtype ----------------
 // Eager torch evaluates a / b on half / bfloat16 tensors as round_dtype(fp32 quotient).  The
-// IEEE fp32 division is ~10 instructions; the quantizers divide every element by a scale that
-// is shared by many elements, so they use instead
+// IEEE fp32 division is ~10 instructions; the value quantizer divides every element by a scale that
+// is shared by many elements, so it uses instead
 //     q0 = d * inv,  r = fma(-q0, sc, d),  q1 = fma(r, inv, q0),      inv = v_rcp_f32(sc) (1 ulp)
 // q1 is a faithful fp32 quotient (the residual r is exact, so q1 is the rounding of a value
 // within 2^-46 of d / sc).  It may differ from the correctly rounded fp32 quotient in the last
