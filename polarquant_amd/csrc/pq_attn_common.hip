@@ -104,7 +104,10 @@ constexpr long long kGroupSlices = 320;
 static bool runs_groups(const AttnArgs& a) {
     if (a.tbits > 4 || a.single_wave || a.silent_scorer || static_cast<long long>(a.n_splits) * a.B * a.Nk > kGroupSlices) return false;
     const int groups = a.n_groups_per_seq ? a.group_capacity : a.n_groups < a.group_capacity ? a.n_groups : a.group_capacity;
-    return groups <= 2 * a.n_splits && a.min_groups_per_split <= 2;
+    // the window of residual keys is one slice's here; slices cut on the device spread a long one (8 KV heads, us, pairs / groups: 500
+    // keys 9.3 / 8.8, 2000 keys 9.9 / 22.2; evenly cut slices keep it in one either way: 100.7 / 22.3)
+    const int resid = a.n_resid_per_seq ? a.resid_capacity : a.n_resid;
+    return groups <= 2 * a.n_splits && a.min_groups_per_split <= 2 && !(a.balanced && resid > 4 * kGroup);
 }
 
 int launch_attn_partials(const AttnArgs& a, hipStream_t st) {

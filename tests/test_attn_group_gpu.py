@@ -75,6 +75,17 @@ def test_ragged_counts_and_a_long_window(gpu, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("resid", [511, 512, 513, 1100])
+def test_slices_cut_on_the_device_of_a_long_window(gpu, dtype, resid):
+    """Either side of the longest window that one slice keeps when the device cuts the slices."""
+    q, codes, kres, v = inputs(1, 8, 2, 1, resid, 4, 4, dtype, 8, cap=resid)
+    got = polar_decode_attention(q.to(gpu), *[t.to(gpu) for t in codes], kres.to(gpu), v.to(gpu), 1, resid, balanced=True, n_splits=20,
+                                 n_groups_per_seq=torch.tensor([1], dtype=torch.int32, device=gpu),
+                                 n_resid_per_seq=torch.tensor([resid], dtype=torch.int32, device=gpu))
+    assert close(got, po.decode_attention_exact(q, kres, *codes, v), dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("B,N,Nk,groups,resid,packed", [(1, 8, 2, 1, 128, False), (2, 28, 4, 3, 17, True), (1, 8, 8, 2, 1, False), (1, 8, 1, 5, 0, True)])
 def test_four_bit_values(gpu, dtype, B, N, Nk, groups, resid, packed):
     bits = 3 if packed else 4
