@@ -116,7 +116,7 @@ def kernels(s, B, ctx, emit):
     fl = L * L * H * (D + Dv)
     q4, k4, v4 = r(1, H, L, D), r(1, s["kv_heads"], L, D), r(1, s["kv_heads"], L, D)
     us2 = _graph_time_us(lambda i: F.scaled_dot_product_attention(q4, k4, v4, is_causal=True, enable_gqa=True), 4)
-    emit(_line("latent_prefill_kernel, %d tokens" % L, us, 4 * L * H * D * 2, fl, _line("scaled_dot_product_attention, causal", us2, 0, fl)))
+    emit(_line("prompt attention, %d tokens" % L, us, 4 * L * H * D * 2, fl, _line("scaled_dot_product_attention, causal", us2, 0, fl)))
     del q, k, gate, vt, q4, k4, v4
     x, y = torch.randn(1, L, W, device=dev), r(1, L, W)
     state = ops.ConvState(1, 4, W, dev)

@@ -134,7 +134,7 @@ def kernels(s, B, ctx, emit):
     sdpa = _line("scaled_dot_product_attention, causal", _graph_time_us(lambda i: F.scaled_dot_product_attention(q4, k4, v4, is_causal=True, enable_gqa=True), 4), 0,
                  2 * L * L * H * D)
     ql, vt, sink = r(1, L, H, D), r(1, H, D, L), torch.zeros(H, device=dev)
-    like = _line("latent_prefill_kernel, causal", _graph_time_us(lambda i: latent_ops.latent_prefill_attention(ql, ql, vt, sink, 0.08), 4), 4 * L * H * D * 2, 2 * L * L * H * D)
+    like = _line("latent prompt attention, causal", _graph_time_us(lambda i: latent_ops.latent_prefill_attention(ql, ql, vt, sink, 0.08), 4), 4 * L * H * D * 2, 2 * L * L * H * D)
     emit(dict(sdpa))
     del q4, k4, v4, vt
     q, kn, vn, out = ql.view(L, H * D), r(L, G * D), r(L, G * D), torch.empty(L, H * D, dtype=dt, device=dev)

@@ -74,7 +74,8 @@ class PolarGraphDecoder(GraphDecoder):
         rotation is bit-identical to the eager ops; the norms and SiLU agree to the dtype's last bit.
         small_m_gemm (with fused_ops, batch <= 16): o_proj, gate/up (with the SiLU product in its epilogue) and
         down_proj through the weight-streaming kernel `decode_ops.linear_small_m` instead of the BLAS library;
-        fp32 accumulation in a different order, so logits agree to rounding.
+        fp32 accumulation in a different order, so logits agree to rounding.  (The logits' product is the model's own
+        module, which takes that kernel for up to 16 rows either way.)
         fused_qkv_rope (with small_m_gemm, batch <= 8): the q|k|v projection, the rotation and the two cache
         appends as one launch, `decode_ops.qkv_rope_append`, bit-identical to the projection followed by the rotation.
         fused_prefill: the prompt pass runs the norms and the MLP activation through the same fused kernels
