@@ -26,10 +26,16 @@ struct PromptAttnArgs {
 constexpr int kPromptTileRows = 128, kPromptTileKeys = 64;
 
 // 16 bytes per lane from global memory into 1 KiB of LDS at `lds` (uniform), lane after lane.  Not known to the compiler's count
-// of loads in flight: wait_lds_loads() before the barrier behind which the data is read.
+// of loads in flight: wait_lds_loads() before the barrier behind which the data is read.  (The builtin is known to it, and makes every
+// read of LDS wait for the next tile's loads.)  The load reads M0 one wait state after a scalar write at the earliest; the compiler
+// leaves that to us inside an asm statement.  (M0 is named as written, so that nothing else relies on it; it is never allocated, which is
+// what the warning would say.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void load_to_lds(const void* p, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "s"(lds) : "memory");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "s"(lds) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 __device__ __forceinline__ void wait_lds_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 typedef float floatx2_a __attribute__((ext_vector_type(2)));
