@@ -70,6 +70,36 @@ def test_values_by_token(B, L, N, Nk, layout, dtype):
     assert got.shape == (B, L, N, 128) and off(got, reference(*[t.transpose(1, 2) for t in (q, k, v)], 128 ** -0.5)) < UNIT[dtype]
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("form", ["channel", "token", "window"])
+def test_the_largest_weight_is_exact(form, dtype):
+    """A key of the first tile, then one of the second that exceeds it by 0.2 to 5 and is the only one with values.  Its weight is 1 in any
+    dtype, so that what is left is the rounding of the result: the nearest number, but for the float32 sums' 1e-6 of a unit that is
+    2^-8 or 2^-11.  A weight that is itself rounded moves about a quarter of the results to a neighbour."""
+    from polarquant_amd import recurrent_ops
+    from polarquant_amd.attention import prompt_attention
+    from polarquant_amd.latent_ops import latent_prefill_attention
+    g = torch.Generator(device="cuda").manual_seed(3)
+    L, H = 130, 24
+    q, k, v = [torch.zeros(1, L, H, 128, device="cuda", dtype=dtype) for _ in range(3)]
+    q[..., 0] = 1.0
+    k[..., 0] = -40.0
+    k[:, 3, :, 0] = 0.0
+    k[:, 100, :, 0] = torch.linspace(0.2, 5.0, H, device="cuda").to(dtype)
+    v[:, 100] = torch.randn(1, H, 128, generator=g, device="cuda").to(dtype)
+    if form == "channel":
+        sink, vt = torch.full((H,), -60.0, device="cuda"), torch.zeros(1, H, 128, 192, device="cuda", dtype=dtype)
+        vt[..., :L] = v.permute(0, 2, 3, 1)
+        got = latent_prefill_attention(q, k, vt, sink, 1.0).view(1, L, H, 128)
+    elif form == "token":
+        got = prompt_attention(*[t.transpose(1, 2) for t in (q, k, v)], 1.0)
+    else:
+        ring, out = recurrent_ops.WindowRing(1, H, 128, 128, L, dtype, "cuda"), torch.empty(L, H * 128, device="cuda", dtype=dtype)
+        got = recurrent_ops.window_attention(q.view(L, -1), ring, None, 1.0, recurrent_ops.Step(1, L, 0), out, 1.0, k.view(L, -1), v.view(L, -1)).view(1, L, H, 128)
+    want = reference(q, k, v, 1.0)[:, 100:].to(dtype)
+    assert float((got[:, 100:] != want).float().mean()) < 0.005
+
+
 def test_what_prompt_attention_refuses():
     from polarquant_amd.attention import prompt_attention_takes
     x = torch.randn(2, 4, 70, 128, device="cuda").bfloat16()
