@@ -163,15 +163,19 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
     float m = kNone, l = 0.0f;
 
     // LDS addresses of this lane's reads: row `col` of K, chunk 2 i + hi
-    uint32_t ka[KS], va[VT];
+    // A row per channel: 8 chunks at VT distances.  Up to 128 channels the compiler may keep all 32 sums (with the chunks' addresses kept
+    // and the distances as offsets 190 registers instead of 246, but 668 against 637 us); 64 sums do not fit beside 256 channels' tile
+    // (86 registers spilled, 16 heads, 8192 tokens: 1652 us, with kept chunks 847, with tiles passed through registers 999).
+    constexpr bool kChunks = !TOKEN_ROWS && DVP > 128;
+    uint32_t ka[KS], va[kChunks ? 8 : VT];
     static_for<KS>([&](auto I) { ka[I] = lds0 + col * (DKP * 2) + ((2 * I + hi) ^ k_swz(col)) * 16; });
-    static_for<VT>([&](auto I) {
+    static_for<kChunks ? 8 : VT>([&](auto I) {
         constexpr int i = decltype(I)::value;
         if (TOKEN_ROWS) {           // 16 lanes read 4 tokens x 16 channels and get them transposed
             const int row = 4 * hi + ((lane & 15) >> 2), chunk = 4 * i + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
             va[i] = lds0 + 2 * KBYTES + row * (DVP * 2) + (chunk ^ v_swz(row)) * 16 + (lane & 1) * 8;
-        } else {
-            va[i] = lds0 + 2 * KBYTES + (32 * i + col) * 128 + hi * 8;
+        } else {                    // chunk i of row `col`, or row 32 i + col: rows 32 apart have the same swizzle
+            va[i] = lds0 + 2 * KBYTES + hi * 8 + (kChunks ? col * 128 + (i ^ v_swz(col)) * 16 : (32 * i + col) * 128);
         }
     });
     auto step = [&](int it, auto BUF) {
@@ -237,9 +241,9 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
                         w0 = __builtin_bit_cast(u32x2_a, __builtin_amdgcn_ds_read_tr16_b64_v4i16(lds_ptr<lds_short4>(at)));
                         w1 = __builtin_bit_cast(u32x2_a, __builtin_amdgcn_ds_read_tr16_b64_v4i16(lds_ptr<lds_short4>(at + 8 * DVP * 2)));
                     } else {
-                        const uint32_t at = va[i] + buf * VBYTES;
-                        w0 = *lds_ptr<lds_u32x2>(at + ((2 * j) ^ v_swz(col)) * 16);
-                        w1 = *lds_ptr<lds_u32x2>(at + ((2 * j + 1) ^ v_swz(col)) * 16);
+                        auto at = [&](int chunk) { return (kChunks ? va[chunk] + 32 * i * 128 : va[i] + (chunk ^ v_swz(col)) * 16) + buf * VBYTES; };
+                        w0 = *lds_ptr<lds_u32x2>(at(2 * j));
+                        w1 = *lds_ptr<lds_u32x2>(at(2 * j + 1));
                     }
                     o[i] = mma32<T>(u32x4_a{w0.x, w0.y, w1.x, w1.y}, p[j], o[i]);
                 });
