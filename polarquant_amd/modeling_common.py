@@ -178,13 +178,29 @@ def _on_gpu_in_half(*ts) -> bool:
                     and t.numel() > 0 for t in ts))
 
 
+def _streams_faster(rows: int, n: int, k: int) -> bool:
+    """Where the weight-streaming kernel beats the BLAS library, weights not in a cache (us, kernel / library, bfloat16):
+    rows of up to 4096 elements, 1 and 8 rows: 4096 x 4096 8.3 / 15.9, 8.9 / 15.7; 32768 x 4096 47 / 64, 48 / 64; 5120 x 4096, a last
+    wave of workgroups that is a quarter full, 11.0 / 14.2, 13.8 / 14.2.  9 to 16 rows, another kernel: 4096 x 4096 10.4 / 15.8, but
+    6144 x 4096 17.8 / 14.8 and 128256 x 4096 252 / 188.
+    Longer rows: 4096 x 14336 22 / 27, 24 / 27; 3584 x 18944 25 / 47, 30 / 48.  The library splits the sum, the kernel at most eight ways: few
+    outputs are slower (1024 x 8192, 8 rows, 13.1 / 11.9; 16 x 7168 10.1 / 7.6), so is a device half filled (5120 x 13824 38 / 31), and so are
+    rows 32 KiB apart, which meet in the same memory channels (6144 x 16384 47 / 42)."""
+    if rows > 8:
+        return n <= 4096 and k <= 4096
+    if k <= 4096:
+        return True
+    groups = n // 16                                     # workgroups, on 256 compute units
+    return n >= 3072 and 4 * groups >= 3 * 256 * -(-groups // 256) and k % 16384 != 0
+
+
 class Linear(nn.Linear):
-    """`nn.Linear`; up to 16 rows, a stream of the weights, through the weight-streaming kernel, which does the step's products in 60 to
-    80 % of the BLAS library's time (one row, us: 4096 x 4096 12.6 against 19.5, 14336 x 4096 22 against 28, 32768 x 4096 41 against 59)."""
+    """`nn.Linear`; up to 16 rows, a stream of the weights, through the weight-streaming kernel where that is faster."""
 
     def forward(self, x):
         if (0 < x.numel() <= 16 * self.in_features and x.shape[-1] == self.in_features and x.is_cuda and x.dtype == self.weight.dtype
                 and x.stride(-1) == 1 and self.out_features % 16 == 0 and self.in_features % 32 == 0 and self.weight.device == x.device
+                and _streams_faster(x.numel() // self.in_features, self.out_features, self.in_features)
                 and _on_gpu_in_half(*((self.weight,) if self.bias is None else (self.weight, self.bias)))):
             from .decode_ops import linear_small_m
             rows = x.reshape(-1, self.in_features)
