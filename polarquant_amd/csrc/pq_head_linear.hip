@@ -10,7 +10,7 @@ int launch_head_linear_mfma(const HeadLinearArgs& a, int dtype, hipStream_t st) 
     const int kstep = m8 ? 64 : 32;
     int ks = (m8 && a.K >= 8192) ? 8 : 4;
     while (ks > 1 && ((a.K % (kstep * ks)) != 0 || a.K / (kstep * ks) < 2)) ks >>= 1;
-    const int nt = m8 && a.heads == 1 ? small_m8_row_tiles(a.N, ks, 1) : 2;      // (several heads: their K is short, nothing is gained)
+    const int nt = m8 && a.heads == 1 ? small_m8_row_tiles(a.M, a.N, ks, 1) : 2;      // (several heads: their K is short, nothing is gained)
     dim3 grid(a.N / (8 * nt), a.heads), block(kWave * ks);
     const HeadEpi he{a.x_head, static_cast<int64_t>(a.N) * a.K, a.y_head, static_cast<const uint16_t*>(a.gate), a.gate_row};
 #define PQ_H(KERNEL)                                                                                                 \

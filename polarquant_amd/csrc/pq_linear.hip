@@ -179,7 +179,7 @@ int launch_small_m_linear(const void* x, int64_t x_stride, const void* w, const 
     const int kstep = m8 ? 64 : 32;
     int ks = (m8 && K >= 8192) ? 8 : 4;
     while (ks > 1 && (K % (kstep * ks)) != 0) ks >>= 1;
-    const int nt = m8 ? small_m8_row_tiles(N, ks, gated ? 2 : 1) : 2;
+    const int nt = m8 ? small_m8_row_tiles(M, N, ks, gated ? 2 : 1) : 2;
     dim3 grid(N / (8 * nt)), block(kWave * ks);
 #define PQ_LAUNCH_L(KERNEL)                                                                                          \
     hipLaunchKernelGGL((KERNEL), grid, block, 0, st, (const uint16_t*)x, x_stride,                                   \

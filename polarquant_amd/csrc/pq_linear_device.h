@@ -23,6 +23,7 @@
 // pq_steps_internal.h: plain, square of relu, times sigmoid(gate), or unrounded float32 output.
 #pragma once
 #include "pq_device.h"
+#include "pq_linear_rules.h"
 #include "pq_steps_internal.h"
 
 namespace pq {
@@ -191,29 +192,7 @@ __global__ __launch_bounds__(kWave * KSPLIT) void small_m_linear_kernel(
 // duplicate row of x, a wavefront load of W covers 8 rows x 128 contiguous bytes (whole cache lines,
 // which is what lets the weight stream carry the non-temporal hint: with half lines the hint drops a
 // line before its second half is asked for), and the workgroup's 8 NT rows of W are NT such tiles that
-// share one x operand.
-//
-// NT: what a compute unit can have on its way from memory is about its share of the HBM rate, so the unit with the most rows sets
-// the time, and x, which every workgroup reads from L2, comes on top (without the x loads 28672 x 4096 takes 37.4 us, the plain
-// stream's time).  small_m8_row_tiles therefore takes the NT for which the fullest unit's W and x bytes are least.  Measured in a
-// chain of calls, 8 rows, NT 2 / 4 / 8 in us: 6144 x 4096 13.5 / 12.3 / 23.9; 10240 x 4096 20.7 / 22.6 / 24.9; 21504 x 4096
-// 37.6 / 34.9 / 38.6; 43136 x 4096 65.6 / 62.3 / 59.1; 32768 x 4096 50.3 / 45.8 / 44.8.  (x kept in registers by persistent
-// workgroups: 41 / 59 us at N 28672 / 43136, and 10.2 instead of 8.8 at 4096.)
-inline int small_m8_row_tiles(int N, int ksplit, int matrices) {
-    constexpr int kUnits = 256;
-    int best = 2;
-    double least = 0.0;
-    for (int nt = 2; nt * matrices <= 8; nt *= 2) {
-        if (N % (8 * nt)) break;
-        const int groups = N / (8 * nt);
-        // too few wavefronts to keep loads on the way: 3 per unit with four tiles' loads each, 7 with eight
-        if (nt > 2 && groups * ksplit < (nt * matrices == 8 ? 7 : 3) * kUnits) break;
-        const double cost = ((groups + kUnits - 1) / kUnits) * nt * (1.0 + 0.42 / (nt * matrices));
-        if (nt == 2 || cost < least) { best = nt; least = cost; }
-    }
-    return best;
-}
-
+// share one x operand.  (Which NT: pq_linear_rules.h.)
 template <bool GATED, int NT, int kStage>
 struct Stage8T {
     u32x4_l w[NT][kStage], x[kStage], u[GATED ? NT : 1][GATED ? kStage : 1];

@@ -1,5 +1,9 @@
-"""Which products of up to 16 rows leave the BLAS library for the weight-streaming kernel.  The sizes are those both were timed at, weights
-read from memory; a side is listed where it was faster by more than 5 %.  No GPU is needed."""
+"""Which products of up to 16 rows leave the BLAS library for the weight-streaming kernel, and how many rows of W its workgroups take.
+The sizes are those both sides were timed at, weights read from memory.  No GPU is needed."""
+import ctypes
+import os
+import subprocess
+
 import pytest
 
 from polarquant_amd.modeling_common import _streams_faster
@@ -20,3 +24,26 @@ def test_the_kernel_takes(rows, n, k):
 @pytest.mark.parametrize("rows,n,k", LIBRARY)
 def test_the_library_keeps(rows, n, k):
     assert not _streams_faster(rows, n, k)
+
+
+@pytest.fixture(scope="module")
+def row_tiles():
+    here = os.path.dirname(os.path.abspath(__file__))
+    os.makedirs(os.path.join(here, "_build"), exist_ok=True)
+    so = os.path.join(here, "_build", "liblinear_rules.so")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-x", "c++", "-", "-o", so, "-I", os.path.join(os.path.dirname(here), "polarquant_amd", "csrc")],
+                   input=b'#include "pq_linear_rules.h"\nextern "C" int tiles(int m, int n, int ks, int mats) { return pq::small_m8_row_tiles(m, n, ks, mats); }', check=True)
+    return ctypes.CDLL(so).tiles
+
+
+@pytest.mark.parametrize("n,k,tiles", [(6144, 4096, [4] * 8), (10240, 4096, [2] * 8), (21504, 4096, [4] * 8), (4096, 4096, [2] * 8), (14336, 4096, [4] * 8),
+                                       (28672, 4096, [2, 2, 2, 2]), (28672, 8192, [2, 2, 2, 2]), (43136, 4096, [2, 2, 2]), (8192, 8192, [2, 2, 2]), (5120, 13824, [2, 2])])
+def test_tiles_of_the_faster_side(row_tiles, n, k, tiles):
+    for rows, want in enumerate(tiles, 1):
+        assert row_tiles(rows, n, 8 if k >= 8192 else 4, 1) == want, rows
+
+
+def test_eight_tiles_only_where_x_is_what_costs(row_tiles):
+    """32768 and 43136 outputs: 8 tiles gain 7 to 10 % with 8 rows and lose 4 to 5 % with one."""
+    for n in (32768, 43136):
+        assert row_tiles(8, n, 4, 1) == 8 and all(row_tiles(m, n, 4, 1) < 8 for m in (1, 2, 3, 4))
