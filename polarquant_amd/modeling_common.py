@@ -204,7 +204,8 @@ class Linear(nn.Linear):
                 and _on_gpu_in_half(*((self.weight,) if self.bias is None else (self.weight, self.bias)))):
             from .decode_ops import linear_small_m
             rows = x.reshape(-1, self.in_features)
-            if rows.data_ptr() % 16 == 0 and rows.stride(0) % 8 == 0:
+            # (the kernel takes rows that lie apart: not one row expanded to many, nor rows that overlap)
+            if rows.data_ptr() % 16 == 0 and rows.stride(0) % 8 == 0 and (rows.shape[0] == 1 or rows.stride(0) >= self.in_features):
                 return linear_small_m(rows, self.weight, self.bias).view(*x.shape[:-1], self.out_features)
         return super().forward(x)
 

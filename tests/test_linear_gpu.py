@@ -182,3 +182,17 @@ def test_linear_module_takes_the_kernel_only_where_it_may(gpu, dtype):
         assert lin(wide[:0, :, :160]).shape == (0, 9, 64)
     assert lin(wide[:1, :, :160].clone().requires_grad_()).requires_grad
     assert Linear(160, 64)(torch.randn(3, 160)).shape == (3, 64)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_linear_module_takes_rows_that_share_storage(gpu, dtype):
+    """One row expanded to several, rows that overlap, a sequence expanded over the batch: the kernel refuses such strides, the module
+    does not."""
+    from polarquant_amd.modeling_common import Linear
+    g = torch.Generator(device=gpu).manual_seed(4)
+    lin = Linear(160, 64, bias=True).to(gpu, dtype)
+    x = torch.randn(3, 1, 320, generator=g, device=gpu).to(dtype)
+    with torch.no_grad():
+        for t in (x[:1, :, :160].expand(4, 1, 160), x[0, :, :160].expand(5, 160), x.as_strided((3, 160), (8, 1)), x.as_strided((3, 160), (152, 1)),
+                  x[:1, :, :160].expand(2, 3, 160), x[:, :, :160].expand(3, 4, 160), x.as_strided((2, 1, 160), (160, 0, 1)), x[:1, :, :160].expand(1, 1, 160)):
+            _check(lin(t), F.linear(t.double(), lin.weight.double(), lin.bias.double()), dtype)
