@@ -29,6 +29,7 @@ from typing import List, Optional, Tuple
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.utils._device import DeviceContext
 
 from .attention import polar_decode_attention, polar_decode_attention_v4, prompt_attention, prompt_attention_takes
 from .quantize import quantize_and_pack_nbit
@@ -170,10 +171,24 @@ class RotaryEmbedding(nn.Module):
         return emb.cos().to(x.dtype), emb.sin().to(x.dtype)
 
 
+def _nobody_looks_on(*ts) -> bool:
+    """Whether these are plain tensors in plain eager execution.  A launch through the C ABI is invisible to whatever follows torch's
+    operations: gradients of either direction (no_grad leaves forward-mode differentiation on: the tangent would be lost), vmap and the
+    other function transforms, traces (which would record an empty result), compilation, autocast, dispatch and function modes, tensor
+    subclasses."""
+    if torch.is_grad_enabled() or torch.compiler.is_compiling():
+        return False
+    functions = torch._C._len_torch_function_stack()
+    return (torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
+            and torch._C._get_tracing_state() is None and not torch.is_autocast_enabled("cuda") and torch._C._len_torch_dispatch_stack() == 0
+            and all(type(torch._C._get_function_stack_at(i)) is DeviceContext for i in range(functions))        # (a default device)
+            and all(type(t) is torch.Tensor or type(t) is nn.Parameter for t in ts))
+
+
 def _on_gpu_in_half(*ts) -> bool:
     """Whether the fused launches can take these tensors as they lie: one half-precision dtype, one GPU, contiguous, 16-byte aligned,
-    not empty, no gradients wanted."""
-    return (not torch.is_grad_enabled() and ts[0].dtype in (torch.float16, torch.bfloat16)
+    not empty, and nobody who follows torch's operations."""
+    return (ts[0].dtype in (torch.float16, torch.bfloat16) and _nobody_looks_on(*ts)
             and all(t.is_cuda and t.dtype == ts[0].dtype and t.device == ts[0].device and t.is_contiguous() and t.data_ptr() % 16 == 0
                     and t.numel() > 0 for t in ts))
 
@@ -201,7 +216,7 @@ class Linear(nn.Linear):
         if (0 < x.numel() <= 16 * self.in_features and x.shape[-1] == self.in_features and x.is_cuda and x.dtype == self.weight.dtype
                 and x.stride(-1) == 1 and self.out_features % 16 == 0 and self.in_features % 32 == 0 and self.weight.device == x.device
                 and _streams_faster(x.numel() // self.in_features, self.out_features, self.in_features)
-                and _on_gpu_in_half(*((self.weight,) if self.bias is None else (self.weight, self.bias)))):
+                and type(x) is torch.Tensor and _on_gpu_in_half(*((self.weight,) if self.bias is None else (self.weight, self.bias)))):
             from .decode_ops import linear_small_m
             rows = x.reshape(-1, self.in_features)
             # (the kernel takes rows that lie apart: not one row expanded to many, nor rows that overlap)
@@ -642,7 +657,7 @@ def _prefill_attention(q, k, v, attention_mask, n_rep, is_causal):
     if attention_mask is None or bool((attention_mask != 0).all()):
         # the library's flash attention takes twice the time from 512 tokens on (32 heads, 512 / 8192 / 16384 tokens: 34, 1270, 4484
         # against 18, 564, 2121 us) and the same below; it stays for what the kernel does not take: float32, tensors on the host, gradients
-        if is_causal and not torch.is_grad_enabled() and prompt_attention_takes(q, k, v):
+        if is_causal and _nobody_looks_on(q, k, v) and prompt_attention_takes(q, k, v):
             return prompt_attention(q, k, v)
         out = F.scaled_dot_product_attention(q, k, v, is_causal=is_causal and L > 1, enable_gqa=n_rep > 1)
     else:
