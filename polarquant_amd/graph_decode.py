@@ -24,7 +24,7 @@ import torch
 
 from . import _ffi
 from .attention import _num_cus, new_workspace, plan_splits, polar_decode_attention, polar_decode_attention_v4
-from .modeling_common import GROUP, apply_rotary_pos_emb
+from .modeling_common import GROUP, Linear, apply_rotary_pos_emb
 
 
 class GraphDecoder:
@@ -69,18 +69,19 @@ class GraphDecoder:
 class PolarGraphDecoder(GraphDecoder):
     def __init__(self, model, max_len: int, use_graph: bool = True, fused_ops: bool = True, small_m_gemm: bool = True,
                  fused_prefill: bool = False, fused_qkv_rope: bool = True):
-        """fused_ops: run RoPE + cache append, the norms and the MLP activation as one HIP launch each
-        (polarquant_amd.decode_ops) instead of the eager modules' chains of elementwise launches.  The
-        rotation is bit-identical to the eager ops; the norms and SiLU agree to the dtype's last bit.
+        """fused_ops: run RoPE + cache append, the norms with the residual additions before them and the MLP activation
+        as one HIP launch each (polarquant_amd.decode_ops).  Off: the step is the eager modules' own, launch for launch
+        (their norms and activations are one launch each as well, the rotation and the appends are not).  The rotation is
+        bit-identical to the eager ops; the norms and SiLU agree to the dtype's last bit.
         small_m_gemm (with fused_ops, batch <= 16): o_proj, gate/up (with the SiLU product in its epilogue) and
-        down_proj through the weight-streaming kernel `decode_ops.linear_small_m` instead of the BLAS library;
-        fp32 accumulation in a different order, so logits agree to rounding.  (The logits' product is the model's own
-        module, which takes that kernel for up to 16 rows either way.)
+        down_proj through the weight-streaming kernel `decode_ops.linear_small_m` instead of the BLAS library, and the
+        logits' product as the eager module has it (that kernel where it is faster); fp32 accumulation in a different
+        order, so logits agree to rounding.  Off: the BLAS library for every product of the fused step.
         fused_qkv_rope (with small_m_gemm, batch <= 8): the q|k|v projection, the rotation and the two cache
         appends as one launch, `decode_ops.qkv_rope_append`, bit-identical to the projection followed by the rotation.
-        fused_prefill: the prompt pass runs the norms and the MLP activation through the same fused kernels
-        instead of the eager modules' elementwise chains (about a sixth of the prompt time); the cache it
-        builds and the logits then agree with the eager model to rounding instead of bit for bit."""
+        fused_prefill: in the prompt pass the residual additions become part of the norms behind them (the eager modules'
+        norms and activations are one launch each by themselves); the cache it builds and the logits then agree with the
+        eager model to rounding instead of bit for bit."""
         self.fused_ops = fused_ops
         self.small_m_gemm = small_m_gemm
         self.fused_prefill = fused_prefill
@@ -222,6 +223,7 @@ class PolarGraphDecoder(GraphDecoder):
         folded in), RoPE + append, SiLU * up, plus the GEMMs and the attention, per layer."""
         from .decode_ops import linear_small_m, qkv_rope_append, rmsnorm, rope_append, silu_mul
         model, B = self.model, self.B
+        product = lambda module, t: module(t, library=True) if isinstance(module, Linear) and not self.small_m_gemm else module(t)
         layers = model.model.layers
         x = model.model.embed_tokens(self.ids).contiguous()                 # residual stream [B,1,H], updated in place
         h = rmsnorm(x, layers[0].input_layernorm.weight, layers[0].input_layernorm.variance_epsilon)
@@ -252,18 +254,18 @@ class PolarGraphDecoder(GraphDecoder):
                 act = linear_small_m(h, mlp.gate_proj.weight, up_weight=mlp.up_proj.weight)
                 m = linear_small_m(act, mlp.down_proj.weight, mlp.down_proj.bias)
             else:
-                a = att.o_proj(o.reshape(B, 1, -1))
+                a = product(att.o_proj, o.reshape(B, 1, -1))
                 h = rmsnorm(x, pn.weight, pn.variance_epsilon, residual=a, sum_out=x)
                 # (gate | up as one library GEMM was measured too: no faster than the two, so they stay separate)
-                m = mlp.down_proj(silu_mul(mlp.gate_proj(h), mlp.up_proj(h)))
+                m = product(mlp.down_proj, silu_mul(product(mlp.gate_proj, h), product(mlp.up_proj, h)))
             nn_ = layers[li + 1].input_layernorm if li + 1 < len(layers) else model.model.norm
             h = rmsnorm(x, nn_.weight, nn_.variance_epsilon, residual=m, sum_out=x)
-        logits = model.lm_head(h)
+        logits = product(model.lm_head, h)
         self._counters.add_(self._advance)
         return logits
 
     def _step_body(self):
-        """The decode step on the static state; identical arithmetic to the eager modules."""
+        """The decode step on the static state; unfused with the arithmetic of the eager modules, which it calls."""
         if self.fused_ops:
             return self._step_body_fused()
         model = self.model

@@ -210,10 +210,11 @@ def _streams_faster(rows: int, n: int, k: int) -> bool:
 
 
 class Linear(nn.Linear):
-    """`nn.Linear`; up to 16 rows, a stream of the weights, through the weight-streaming kernel where that is faster."""
+    """`nn.Linear`; up to 16 rows, a stream of the weights, through the weight-streaming kernel where that is faster.  library: the BLAS
+    library in any case."""
 
-    def forward(self, x):
-        if (0 < x.numel() <= 16 * self.in_features and x.shape[-1] == self.in_features and x.is_cuda and x.dtype == self.weight.dtype
+    def forward(self, x, library=False):
+        if (not library and 0 < x.numel() <= 16 * self.in_features and x.shape[-1] == self.in_features and x.is_cuda and x.dtype == self.weight.dtype
                 and x.stride(-1) == 1 and self.out_features % 16 == 0 and self.in_features % 32 == 0 and self.weight.device == x.device
                 and _streams_faster(x.numel() // self.in_features, self.out_features, self.in_features)
                 and type(x) is torch.Tensor and _on_gpu_in_half(*((self.weight,) if self.bias is None else (self.weight, self.bias)))):

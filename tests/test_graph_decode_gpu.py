@@ -237,3 +237,22 @@ def test_graph_decoder_rejects_overflow(gpu):
     dec.step(tok)
     with pytest.raises(AssertionError):
         dec.step(tok)
+
+
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("options,launches", [(dict(), {"linear_small_m", "qkv_rope_append", "rmsnorm"}), (dict(fused_qkv_rope=False), {"linear_small_m", "rope_append", "rmsnorm"}),
+                                              (dict(small_m_gemm=False), {"rope_append", "rmsnorm", "silu_mul"})])
+def test_options_say_which_launches_a_step_makes(gpu, monkeypatch, options, launches, bias):
+    """Without `small_m_gemm` no product of a fused step leaves the BLAS library, the logits' neither."""
+    from polarquant_amd import decode_ops
+    torch.manual_seed(3)
+    model = LlamaPolarForCausalLM(_tiny(mlp_bias=bias)).half().to(gpu).eval()
+    dec = PolarGraphDecoder(model, max_len=200, use_graph=False, **options)
+    ids = torch.randint(0, 1000, (2, 130), device=gpu)
+    dec.prefill(ids)
+    made = set()
+    for name in ("linear_small_m", "qkv_rope_append", "rope_append", "rmsnorm", "silu_mul"):
+        f = getattr(decode_ops, name)
+        monkeypatch.setattr(decode_ops, name, lambda *a, _f=f, _n=name, **k: (made.add(_n), _f(*a, **k))[1])
+    dec.step(ids[:, :1])
+    assert made == launches | ({"silu_mul"} if bias else set())
