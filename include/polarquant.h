@@ -458,6 +458,11 @@ int pq_validate_decode_attn_v4(const void *q,
                                int n_splits, int min_groups_per_split, const void *workspace, size_t workspace_bytes,
                                const void *out, unsigned flags);
 
+/* Up to this many slices (n_splits * B * Nk) of at most two groups, angles of at most 4 bits, run a kernel in which eight
+ * wavefronts share a slice.  There n_splits = groups + 1 gives the keys not yet quantized a slice of their own; beyond it, and
+ * in the other kernels, such a slot stays empty. */
+#define PQ_FEW_SLICES 320
+
 /* Suggested n_splits for a shape (host-only; `max_groups` = largest group count
  * of any sequence, `n_cus` = compute units of the device or 0 for 256). */
 int pq_decode_attn_plan(int B, int Nk, int max_groups, int n_cus);

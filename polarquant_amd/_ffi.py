@@ -20,6 +20,7 @@ PQ_ANGLE_UNIFORM = 2
 PQ_CODES_PACKED6 = 4
 PQ_DEVICE_ATAN2 = 8
 PQ_BALANCED_SLICES = 16
+PQ_FEW_SLICES = 320
 PQ_SINGLE_WAVEFRONT = 32
 PQ_TEST_SILENT_SCORER = 0x40000000      # honoured by the test build of the library only; the one loaded here refuses it
 PQ_STATUS_HANDOVER_TIMEOUT = 1

@@ -75,6 +75,16 @@ def _pick_workspace(workspace: Optional[torch.Tensor], B: int, N: int, n_splits:
     return workspace
 
 
+def _window_slot(n_splits: int, groups: int, resid: int, B: int, N: int, Nk: int, tbits: int, workspace: Optional[torch.Tensor]) -> int:
+    """`n_splits` as planned, plus one where every group has a slice of its own and the keys not yet quantized can have one too: only the
+    kernel of few slices puts them there, and a caller's workspace has to hold it."""
+    more = n_splits + 1
+    if (1 < n_splits == groups and resid > 0 and tbits <= 4 and more * B * Nk <= _ffi.PQ_FEW_SLICES
+            and (workspace is None or workspace.numel() * workspace.element_size() >= workspace_bytes(B, N, more))):
+        return more
+    return n_splits
+
+
 def polar_decode_attention(
     query_states: torch.Tensor,               # [B,N,1,128] or [B,N,128]
     indices: Optional[torch.Tensor],          # [B,Nk,cap,128,64] u8 (cap >= used groups; last dim 48: packed 6-bit codes) or None
@@ -161,8 +171,8 @@ def polar_decode_attention(
         min_gps = min_groups_per_split
     if n_splits is None:
         n_splits = plan_splits(B, Nk, max_groups, dev)
-        if 1 < n_splits == max_groups:
-            n_splits += 1                  # one group per slice: the residual keys get a slice of their own too
+        if not single_wavefront and min_gps <= 1:
+            n_splits = _window_slot(n_splits, max_groups, n_resid if n_resid_per_seq is None else r_cap, B, N, Nk, tbits, workspace)
     ws = _pick_workspace(workspace, B, N, n_splits, dev)
     if out is None:
         out = torch.empty((B, N, 1, hd), dtype=query_states.dtype, device=dev)
@@ -241,8 +251,8 @@ def polar_decode_attention_v4(
             n_splits = balanced_slots(B, Nk, max_groups, total_groups, (8 if N // Nk <= 4 else 4) * _num_cus(dev), r_cap)
     if n_splits is None:
         n_splits = _ffi.lib().pq_decode_attn_v4_plan(B, N, Nk, max(max_groups, 1), _num_cus(dev))
-        if 1 < n_splits == max_groups:
-            n_splits += 1
+        if not single_wavefront and min_groups_per_split <= 1:
+            n_splits = _window_slot(n_splits, max_groups, n_resid if n_resid_per_seq is None else r_cap, B, N, Nk, tbits, workspace)
     sptr = None
     if status is not None:
         if status.dtype != torch.int32 or status.device != dev or status.numel() != 1:

@@ -6,6 +6,7 @@
 // groups that share the partials when there are 32 / 128 or more: combines the n_splits
 // partials (m, l, acc[128]) of a query head and writes half words.
 #include "pq_attn_device.h"
+#include "../../include/polarquant.h"
 #include <mutex>
 
 namespace pq {
@@ -100,7 +101,7 @@ static int device_compute_units() {
 // Calls of few, short slices run eight wavefronts per slice.  Both sides, attention kernel alone, us (pairs / groups): 120 slices of one
 // group 11.3 / 8.6, 248 slices 11.4 / 8.8, with 7 heads per KV head 64 slices 13.4 / 10.4, 252 slices 13.6 / 11.3; 504 slices 11.7 /
 // 11.9, 744 slices 12.2 / 15.8 (a unit then has more workgroups than it holds); a slice of three groups 12 / 12.
-constexpr long long kGroupSlices = 320;
+constexpr long long kGroupSlices = PQ_FEW_SLICES;
 static bool runs_groups(const AttnArgs& a) {
     if (a.tbits > 4 || a.single_wave || a.silent_scorer || static_cast<long long>(a.n_splits) * a.B * a.Nk > kGroupSlices) return false;
     const int groups = a.n_groups_per_seq ? a.group_capacity : a.n_groups < a.group_capacity ? a.n_groups : a.group_capacity;

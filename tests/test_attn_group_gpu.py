@@ -4,8 +4,8 @@ import pytest
 import torch
 
 from oracle import polar_oracle as po
-from polarquant_amd import workloads as wl
-from polarquant_amd.attention import polar_decode_attention, polar_decode_attention_v4
+from polarquant_amd import _ffi, attention, workloads as wl
+from polarquant_amd.attention import new_workspace, plan_splits, polar_decode_attention, polar_decode_attention_v4
 from polarquant_amd.quantize import convert_codes6
 
 pytestmark = pytest.mark.gpu
@@ -110,3 +110,32 @@ def test_nan_scores_stay_visible(gpu):
     got = run(q, n_splits=1).cpu()
     assert torch.isnan(got[0, 3]).all() and not torch.isnan(got[0, [0, 1, 2, 4, 5, 6, 7]]).any()
     assert not run(torch.zeros_like(q), torch.zeros(1, 261, dtype=torch.uint8, device=gpu)).any()
+
+
+@pytest.mark.parametrize("B,N,Nk,groups,resid,tbits,more,kw", [
+    (1, 8, 8, 39, 5, 4, True, {}), (1, 8, 8, 40, 5, 4, False, {}),         # 312 and 320 slices: 320 with the window's, 328
+    (16, 8, 8, 8, 5, 4, False, {}), (1, 8, 8, 5, 0, 4, False, {}), (1, 8, 8, 5, 1, 4, True, {}), (1, 8, 8, 5, 1, 5, False, {}), (1, 8, 8, 1, 5, 4, False, {}),
+    (1, 8, 8, 5, 5, 4, False, dict(single_wavefront=True)), (1, 8, 8, 5, 5, 4, False, dict(min_groups_per_split=2))])
+def test_when_the_window_has_a_slot_of_its_own(gpu, monkeypatch, B, N, Nk, groups, resid, tbits, more, kw):
+    """One more slot than planned only where the kernel of few slices runs and there are keys for it; a workspace of the planned size is
+    enough in any case."""
+    q, codes, kres, v = inputs(B, N, Nk, groups, resid, 3, tbits, torch.float16, groups)
+    want = po.decode_attention_exact(q, kres[:, :, :resid], *codes, v, rbits=3, tbits=tbits)
+    args = [q.to(gpu), *[t.to(gpu) for t in codes], kres.to(gpu), v.to(gpu), groups, resid]
+    plan = plan_splits(B, Nk, groups, gpu)
+    assert plan == groups
+    taken = []
+    pick = attention._pick_workspace
+    monkeypatch.setattr(attention, "_pick_workspace", lambda ws, b, n, splits, dev: (taken.append(splits), pick(ws, b, n, splits, dev))[1])
+    for ws, splits in ((None, plan + more), (new_workspace(B, N, plan, gpu), plan), (new_workspace(B, N, plan + 1, gpu), plan + more)):
+        assert close(polar_decode_attention(*args, rbits=3, tbits=tbits, workspace=ws, **kw), want, torch.float16)
+        assert taken.pop() == splits, (ws is None, splits)
+    if tbits == 4:
+        plan4 = _ffi.lib().pq_decode_attn_v4_plan(B, N, Nk, groups, attention._num_cus(gpu))
+        vq = po.quantize_values_along_last_dim(v[:, :, :groups * 128].contiguous())
+        vres = torch.zeros_like(kres)
+        vres[:, :, :resid] = v[:, :, groups * 128:]
+        want = po.decode_attention_mixed_exact(q, kres[:, :, :resid], *codes, vres[:, :, :resid], *vq, rbits=3, tbits=tbits)
+        got = polar_decode_attention_v4(*args[:7], vres.to(gpu), *[t.to(gpu) for t in vq], groups, resid, rbits=3, tbits=tbits,
+                                        workspace=new_workspace(B, N, plan4, gpu), **kw)
+        assert close(got, want, torch.float16) and taken.pop() == plan4
