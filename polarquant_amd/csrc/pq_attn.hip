@@ -282,7 +282,7 @@ __device__ __forceinline__ void attn_piece(const AttnParams& p, const V4Args& v4
 #pragma unroll
         for (int j = 1; j < REPP; j++) { mm = (n == j) ? st.m[j] : mm; ll = (n == j) ? lsum[j] : ll; }
         float* pw = ws + ((static_cast<size_t>(b) * N + static_cast<size_t>(kvh) * p.rep_stride + n) * n_splits + slot) * kPartialFloats;
-        if (g == 0) { pw[0] = mm; pw[1] = ll; }
+        if (g == 0) { pw[0] = ll == ll ? mm : ll; pw[1] = ll; }              // (the merge passes over a slice without a maximum)
         float* pa = pw + 4 + 32 * g;
 #pragma unroll
         for (int i = 0; i < 4; i++) {

@@ -318,7 +318,7 @@ __global__ __launch_bounds__(kWave * kGroupWaves, 4) void attn_group_kernel(PQ_A
             direct_out[row * kHeadDim + dim] = f2lo<T>(den > 0.0f ? num / den : (den == den ? 0.0f : den));
         } else {
             float* pw = ws + (row * n_splits + split) * kPartialFloats;
-            if (dim == 0) { pw[0] = mx; pw[1] = den; }
+            if (dim == 0) { pw[0] = den == den ? mx : den; pw[1] = den; }       // (the merge passes over a slice without a maximum)
             pw[4 + dim] = num;
         }
     }

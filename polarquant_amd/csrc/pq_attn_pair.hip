@@ -324,7 +324,8 @@ __device__ __forceinline__ bool pair_accumulator(const AttnParams& p, const Pair
         float mm = st.m[0], ll = lsum[0];
 #pragma unroll
         for (int j = 1; j < REPP; j++) { mm = (n == j) ? st.m[j] : mm; ll = (n == j) ? lsum[j] : ll; }
-        if (!ok) mm = __builtin_nanf("");            // the scorer stopped answering: poison the result
+        // the scorer stopped answering: poison the result; nor may the merge take NaN scores, which leave no maximum, for no scores
+        if (!ok || ll != ll) mm = __builtin_nanf("");
         if (direct_out) {
             // the only slice of its plane: what the merge kernel would make of this one partial, written directly
             // (weight exp2(m - m) = 1, so out = acc / l; no token to attend to -> zeros; a poisoned slice -> NaN)

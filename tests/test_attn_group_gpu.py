@@ -139,3 +139,23 @@ def test_when_the_window_has_a_slot_of_its_own(gpu, monkeypatch, B, N, Nk, group
         got = polar_decode_attention_v4(*args[:7], vres.to(gpu), *[t.to(gpu) for t in vq], groups, resid, rbits=3, tbits=tbits,
                                         workspace=new_workspace(B, N, plan4, gpu), **kw)
         assert close(got, want, torch.float16) and taken.pop() == plan4
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_nan_scores_stay_visible_in_several_slices(gpu, dtype):
+    """A head whose scores are all NaN has no maximum in any slice; its sums are NaN and have to reach the output through the merge, in
+    every kernel, and no other head's."""
+    B, N, Nk, groups, resid = 1, 8, 2, 6, 5
+    q, codes, kres, v = inputs(B, N, Nk, groups, resid, 4, 4, dtype, 1)
+    q[0, 3, 0, 7] = float("nan")
+    q, cache, kres, v = q.to(gpu), [t.to(gpu) for t in codes], kres.to(gpu), v.to(gpu)
+    vq, vres = [t.to(gpu) for t in po.quantize_values_along_last_dim(v[:, :, :groups * 128].contiguous().cpu())], torch.zeros_like(kres)
+    counts = dict(n_groups_per_seq=torch.full((1,), groups, dtype=torch.int32, device=gpu), n_resid_per_seq=torch.full((1,), resid, dtype=torch.int32, device=gpu))
+    for name, kw in (("default", {}), ("three", dict(n_splits=3)), ("one", dict(n_splits=1)), ("few", dict(n_splits=FEW // 2)), ("pairs", dict(n_splits=FEW // 2 + 1)),
+                     ("single", dict(single_wavefront=True)), ("balanced", dict(counts, balanced=True)), ("balanced pairs", dict(counts, balanced=True, n_splits=FEW // 2 + 1))):
+        for bits in (16, 4):
+            if bits == 16:
+                got = polar_decode_attention(q, *cache, kres, v, groups, resid, **kw)
+            else:
+                got = polar_decode_attention_v4(q, *cache, kres, vres, *vq, groups, resid, **kw)
+            assert torch.isnan(got[0, 3]).all() and not torch.isnan(got[0, [0, 1, 2, 4, 5, 6, 7]]).any(), (name, bits)
