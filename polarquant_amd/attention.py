@@ -126,6 +126,8 @@ def polar_decode_attention(
     Nk = value_states.shape[1]
     assert hd == 128
     dt = _dtype_code(query_states)
+    if query_states.numel() != B * N * hd:
+        raise RuntimeError("polarquant_amd: decode attention takes one query token per sequence, not %s" % (tuple(query_states.shape),))
     q = query_states
     if not q.is_contiguous() or q.data_ptr() % 16:
         q = q.reshape(B, N, hd).clone(memory_format=torch.contiguous_format)
@@ -219,6 +221,8 @@ def polar_decode_attention_v4(
     Nk = key_resid.shape[1]
     assert hd == 128
     dt = _dtype_code(query_states)
+    if query_states.numel() != B * N * hd:
+        raise RuntimeError("polarquant_amd: decode attention takes one query token per sequence, not %s" % (tuple(query_states.shape),))
     q = query_states
     if not q.is_contiguous() or q.data_ptr() % 16:
         q = q.reshape(B, N, hd).clone(memory_format=torch.contiguous_format)

@@ -159,3 +159,17 @@ def test_nan_scores_stay_visible_in_several_slices(gpu, dtype):
             else:
                 got = polar_decode_attention_v4(q, *cache, kres, vres, *vq, groups, resid, **kw)
             assert torch.isnan(got[0, 3]).all() and not torch.isnan(got[0, [0, 1, 2, 4, 5, 6, 7]]).any(), (name, bits)
+
+
+@pytest.mark.parametrize("shape", [(1, 8, 2, 128), (1, 8, 0, 128), (1, 8, 3, 1, 128)])
+def test_only_one_query_token_is_taken(gpu, shape):
+    """Several tokens of a contiguous tensor would be read as other heads' queries."""
+    q, codes, kres, v = inputs(1, 8, 2, 2, 5, 4, 4, torch.float16, 1)
+    args = [*[t.to(gpu) for t in codes], kres.to(gpu)]
+    vq = [t.to(gpu) for t in po.quantize_values_along_last_dim(v[:, :, :256].contiguous())]
+    bad = torch.zeros(shape, dtype=torch.float16, device=gpu)
+    for call in (lambda t: polar_decode_attention(t, *args, v.to(gpu), 2, 5), lambda t: polar_decode_attention_v4(t, *args, torch.zeros_like(args[-1]), *vq, 2, 5)):
+        want = call(q.to(gpu))
+        assert torch.equal(call(q.to(gpu).view(1, 8, 128)), want) and torch.equal(call(q.to(gpu).view(1, 8, 1, 1, 128)), want)
+        with pytest.raises(RuntimeError):
+            call(bad)
