@@ -66,9 +66,10 @@ template <> __device__ __forceinline__ uint32_t pack_pair<F16>(float a, float b)
 // 64 bits grows: by 3 % with normal scores, by 15 % where a few keys have most of the weight.
 // WINDOW: a query sees the last `window` positions, with a bias per position of distance; tiles that a workgroup's windows do not touch
 // are not visited, those before the call come from a ring, or from both where the call begins inside a tile.  8192 tokens, window
-// 2048, 32 query and 8 KV heads of 128: 440 -> 370 us against tiles passed through registers (16 heads of 256: 640 -> 580).  The
-// bias is where a score's accumulator starts, in units of an unscaled score (with a second multiply-add per score: 385 us); rows
-// come from ring or call by selection (with branches: 436 -> 448 us at 5000 tokens before the call).
+// 2048, 32 query and 8 KV heads of 128: 394 -> 341 us against tiles passed through registers (16 heads of 256: 649 -> 506).  The bias is
+// added to a finished score in one multiply-add.  (As the start of the score's accumulator it takes 327 us, but every partial sum
+// then rounds at the bias's size: where a bias of 2^17 cancels against the product, 1.7 times the error.)  Rows come from ring or call
+// by selection (with branches: 3 % more at 5000 tokens before the call).
 template <typename T, int DKP, int DVP, bool TOKEN_ROWS, bool WINDOW = false>
 __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(PromptAttnArgs a) {
     constexpr int KS = DKP / 16, VT = DVP / 32, KC = DKP / 8, VC = TOKEN_ROWS ? DVP / 8 : 8;        // 16-byte chunks of a row of K, of V
@@ -96,7 +97,7 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
     const int it0 = key_lo / kPromptTileKeys, it1 = (past + q_last) / kPromptTileKeys + 1;
     // a scale of zero: the scores of zero queries, times one (a masked score, -inf, stays one)
     const float scale2 = a.scale != 0.0f ? fabsf(a.scale) * kLog2e : 1.0f;
-    const float slope = WINDOW && a.slopes ? a.slopes[h] * kLog2e / scale2 : 0.0f;      // (of a score before it is scaled)
+    const float slope2 = WINDOW && a.slopes ? a.slopes[h] * kLog2e : 0.0f;
 
     u32x4_a q[KS];
     {
@@ -185,16 +186,23 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
         if (key0 <= wave_last && (!WINDOW || key0 + kPromptTileKeys - 1 > wave_first - a.window)) {        // uniform over the wavefront
             floatx16_a s[2];
             // (this lane: query qi, keys key0 + 32 u + 8 (j / 4) + 4 hi + j % 4)
-            const float base = WINDOW ? -slope * static_cast<float>(limit - key0 - 4 * hi) : 0.0f;
 #pragma unroll
             for (int u = 0; u < 2; u++)
 #pragma unroll
-                for (int j = 0; j < 16; j++) s[u][j] = WINDOW ? __builtin_fmaf(slope, static_cast<float>(32 * u + 8 * (j >> 2) + (j & 3)), base) : 0.0f;
+                for (int j = 0; j < 16; j++) s[u][j] = 0.0f;
             static_for<KS>([&](auto I) {
                 constexpr int i = decltype(I)::value;
                 s[0] = mma32<T>(*lds_ptr<lds_u32x4>(ka[i] + buf * KBYTES), q[i], s[0]);
                 s[1] = mma32<T>(*lds_ptr<lds_u32x4>(ka[i] + buf * KBYTES + 32 * DKP * 2), q[i], s[1]);
             });
+            if (WINDOW) {                                           // from here on in units of the exponent, the bias taken off
+                const float base = -slope2 * static_cast<float>(limit - key0 - 4 * hi);
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+#pragma unroll
+                    for (int j = 0; j < 16; j++)
+                        s[u][j] = __builtin_fmaf(s[u][j], scale2, __builtin_fmaf(slope2, static_cast<float>(32 * u + 8 * (j >> 2) + (j & 3)), base));
+            }
             if (key0 + kPromptTileKeys - 1 > past + qw || key0 < lo || (WINDOW && key0 <= wave_last - a.window)) {
                 const int oldest = WINDOW && limit - a.window + 1 > lo ? limit - a.window + 1 : lo;
                 const int last = limit - key0 - 4 * hi, first = oldest - key0 - 4 * hi;
@@ -209,7 +217,7 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
             float mx = fmaxf(s[0][0], s[1][0]);
 #pragma unroll
             for (int j = 1; j < 16; j++) mx = fmaxf(fmaxf(mx, s[0][j]), s[1][j]);
-            mx = fmaxf(mx, __shfl_xor(mx, 32)) * scale2;
+            mx = fmaxf(mx, __shfl_xor(mx, 32)) * (WINDOW ? 1.0f : scale2);
             if (__any(mx > m)) {
                 const float mn = fmaxf(m, mx), al = exp2_hw(m - mn);
                 l *= al;
@@ -225,7 +233,8 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
             for (int u = 0; u < 2; u++)
 #pragma unroll
                 for (int j = 0; j < 16; j += 2) {
-                    const float e0 = exp2_hw(__builtin_fmaf(s[u][j], scale2, -m)), e1 = exp2_hw(__builtin_fmaf(s[u][j + 1], scale2, -m));
+                    auto weight = [&](float x) { return exp2_hw(WINDOW ? x - m : __builtin_fmaf(x, scale2, -m)); };
+                    const float e0 = weight(s[u][j]), e1 = weight(s[u][j + 1]);
                     sum[0] += e0;
                     sum[1] += e1;
                     p[2 * u + (j >> 3)][(j & 7) >> 1] = pack_pair<T>(e0, e1);

@@ -111,6 +111,31 @@ def test_window_attention(gpu, H, G, D, Dv, window):
             assert err(run_window(gpu, p, wq, wk, H, G, D, Dv, window, scale, slopes, cut(T, [9]), n_splits=n), want) < tol, (dt, n)
 
 
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_a_large_bias_is_rounded_once(gpu, dt):
+    """A bias of up to 2^17 that the product cancels but for 7 steps of 16 channels, each below the last place of the bias.  In units of the
+    exponent two float32 roundings of less than 2^18 are left, half a unit of 2^-6 each: evenly spread, sqrt(2 / 3) 2^-7 ln 2 = 0.0045 of
+    a weight; beside it the roundings of weight and result, u / sqrt(3) each.  Partial sums that start at the bias lose all seven steps."""
+    L, D, H, slope, n = 2048, 128, 4, 64.0, 112
+    g = torch.Generator(device=gpu).manual_seed(1)
+    before = torch.arange(L, device=gpu, dtype=torch.float32) - L                      # exact in fp16; in bf16 as two numbers of 8 bits
+    q, k = torch.zeros(L, H, D, device=gpu), torch.zeros(L, H, D, device=gpu)
+    q[..., 126:], k[..., 127] = -slope, 16 * (before / 16).floor()[:, None]
+    k[..., 126] = before[:, None] - k[..., 127]
+    q[..., :n] = 2.0 ** -5
+    signs = 2.0 * torch.randint(0, 2, (L, H, 1), generator=g, device=gpu) - 1
+    k[..., :n] = signs * 2.0 ** -8 * torch.rand(L, H, n // 16, generator=g, device=gpu).repeat_interleave(16, 2)
+    q, k, v = [t.to(dt) for t in (q, k, torch.randn(L, H, D, generator=g, device=gpu))]
+    ring, out = ops.WindowRing(1, H, D, D, L, dt, gpu), torch.empty(L, H * D, device=gpu, dtype=dt)
+    ops.window_attention(q.view(L, -1), ring, torch.full((H,), slope, device=gpu), 1.0, Step(1, L, 0), out, 1.0, k.view(L, -1), v.view(L, -1))
+    i = torch.arange(L, device=gpu)
+    distance = (i[1024:, None] - i).double()
+    want = torch.stack([(q[1024:, h].double() @ k[:, h].double().T - slope * distance).masked_fill(distance < 0, -float("inf")).softmax(-1) @ v[:, h].double()
+                        for h in range(H)], 1)
+    u = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8
+    assert float((out.view(L, H, D)[1024:].double() - want).norm() / want.norm()) < (2 / 3 * (2.0 ** -7 * 0.6931) ** 2 + 2 / 3 * u * u) ** 0.5
+
+
 def test_one_key_at_the_windows_edge(gpu):
     """One key stands out; queries just inside and just outside its reach, in prompts and in decoding, at every offset of the
     ring's and the tiles' borders."""
