@@ -12,6 +12,7 @@
 // All of this is fp32 arithmetic on whatever the operands' dtype is; results are rounded to it once.
 #include "pq_elem.h"
 #include "pq_steps_internal.h"
+#include "pq_steps_rules.h"
 
 namespace pq {
 
@@ -257,13 +258,7 @@ int launch_norm_conv(const NormConvArgs& args, int dtype, hipStream_t st) {
     const int per = (pieces + nthr - 1) / nthr;
     const int NC = per <= 1 ? 1 : per <= 2 ? 2 : per <= 4 ? 4 : 8;
     if (per > 8) return static_cast<int>(hipErrorInvalidValue);
-    // Strips as long as the device stays full with them: every strip recomputes taps - 1 norms, and its tokens follow each other
-    // (2.2 us a token).  Full is one workgroup per unit, two where a thread has one piece.  8192 tokens of 4096, taps 4, strips
-    // of 32 / 16 / 8: 103 / 108 / 126 us; 2048 tokens 77 / 46 / 31; 512 tokens, down to strips of 4: 71 / 41 / 26 / 18.
-    constexpr int64_t kUnits = 256;
-    const int64_t full = NC == 1 ? 2 * kUnits : kUnits, tokens = static_cast<int64_t>(a.B) * a.L;
-    a.strip = 32;
-    while (a.strip > 4 && a.strip / 2 >= a.taps && tokens / (a.strip / 2) <= full) a.strip /= 2;
+    a.strip = norm_conv_strip(static_cast<int64_t>(a.B) * a.L, a.taps, NC);
     if (a.L <= kConvInPlaceTokens) a.strip = a.L;
     const size_t shared = (static_cast<size_t>(NC) * nthr + a.groups) * sizeof(float);
     if (shared > 64 * 1024) return static_cast<int>(hipErrorInvalidValue);

@@ -1,5 +1,5 @@
-"""Which products of up to 16 rows leave the BLAS library for the weight-streaming kernel, and how many rows of W its workgroups take.
-The sizes are those both sides were timed at, weights read from memory.  No GPU is needed."""
+"""Which products of up to 16 rows leave the BLAS library for the weight-streaming kernel, how many rows of W its workgroups take, how many
+tokens a strip of the norm with convolution.  The sizes are those both sides were timed at, weights read from memory.  No GPU is needed."""
 import ctypes
 import os
 import subprocess
@@ -27,13 +27,26 @@ def test_the_library_keeps(rows, n, k):
 
 
 @pytest.fixture(scope="module")
-def row_tiles():
+def rules():
     here = os.path.dirname(os.path.abspath(__file__))
     os.makedirs(os.path.join(here, "_build"), exist_ok=True)
-    so = os.path.join(here, "_build", "liblinear_rules.so")
+    so = os.path.join(here, "_build", "liblaunch_rules.so")
     subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-x", "c++", "-", "-o", so, "-I", os.path.join(os.path.dirname(here), "polarquant_amd", "csrc")],
-                   input=b'#include "pq_linear_rules.h"\nextern "C" int tiles(int m, int n, int ks, int mats) { return pq::small_m8_row_tiles(m, n, ks, mats); }', check=True)
-    return ctypes.CDLL(so).tiles
+                   input=b'#include "pq_linear_rules.h"\n#include "pq_steps_rules.h"\nextern "C" {\n'
+                         b'int tiles(int m, int n, int ks, int mats) { return pq::small_m8_row_tiles(m, n, ks, mats); }\n'
+                         b'int strip(int tokens, int taps, int pieces) { return pq::norm_conv_strip(tokens, taps, pieces); }\n}', check=True)
+    return ctypes.CDLL(so)
+
+
+@pytest.fixture
+def row_tiles(rules):
+    return rules.tiles
+
+
+@pytest.mark.parametrize("tokens,taps,pieces,want", [(8192, 4, 2, 32), (2048, 4, 2, 8), (512, 4, 2, 4), (6000, 4, 1, 16), (33, 4, 1, 4), (6000, 5, 1, 32), (6000, 8, 1, 32),
+                                                     (6000, 12, 1, 32), (3000, 8, 1, 16), (700, 9, 2, 16), (300, 16, 2, 16), (300, 17, 2, 32)])
+def test_strips_are_shortened_only_where_the_recomputed_norms_pay(rules, tokens, taps, pieces, want):
+    assert rules.strip(tokens, taps, pieces) == want
 
 
 @pytest.mark.parametrize("n,k,tiles", [(6144, 4096, [4] * 8), (10240, 4096, [2] * 8), (21504, 4096, [4] * 8), (4096, 4096, [2] * 8), (14336, 4096, [4] * 8),
