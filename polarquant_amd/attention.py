@@ -278,8 +278,11 @@ def polar_decode_attention_v4(
 
 def prompt_attention_takes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
     """Whether `prompt_attention` can read these [B, heads, L, 128] tensors as they lie."""
-    return (q.is_cuda and q.dtype in (torch.float16, torch.bfloat16) and q.dtype == k.dtype == v.dtype and q.shape[-1] == 128 and q.shape[2] > 0
-            and k.shape == v.shape == (q.shape[0], k.shape[1], q.shape[2], 128) and 0 < q.shape[0] <= 65535 and q.shape[1] % k.shape[1] == 0
+    if not (q.is_cuda and q.dtype in (torch.float16, torch.bfloat16) and q.dtype == k.dtype == v.dtype and q.dim() == k.dim() == 4 and q.shape[-1] == 128):
+        return False
+    (B, N, L, _), Nk = q.shape, k.shape[1]
+    # (a grid holds 65535 query tiles, sequences and, as the C ABI has it, heads)
+    return (0 < B <= 65535 and 0 < L <= 65535 * 128 and 0 < N <= 65535 and Nk > 0 and N % Nk == 0 and k.shape == v.shape == (B, Nk, L, 128)
             and all(t.device == q.device and t.stride(3) == 1 and all(s % 8 == 0 for s in t.stride()[:3]) and t.data_ptr() % 16 == 0 for t in (q, k, v)))
 
 

@@ -111,3 +111,9 @@ def test_what_prompt_attention_refuses():
     assert not prompt_attention_takes(y[..., :128], x, x)                          # rows 132 apart
     z = torch.randn(2 * 4 * 70 * 128 + 4, device="cuda").bfloat16()[4:].view(2, 4, 70, 128)
     assert not prompt_attention_takes(z, x, x)                                     # 8-byte aligned
+    # what the grid or the C ABI do not hold: the caller falls back instead of meeting an error
+    w = x[:1, :1, :1]
+    for B, N, L in ((65536, 1, 1), (1, 65536, 1), (1, 1, 65535 * 128 + 1), (1, 0, 1), (0, 1, 1)):
+        wide = w.expand(B, N, L, 128) if B and N else x.new_empty(B, N, L, 128)
+        assert not prompt_attention_takes(wide, wide, wide)
+    assert prompt_attention_takes(*[w.expand(1, 1, 65535 * 128, 128)] * 3) and not prompt_attention_takes(x, x[:, :0], x[:, :0]) and not prompt_attention_takes(x[0], x[0], x[0])
