@@ -44,7 +44,8 @@ def row_tiles(rules):
 
 
 @pytest.mark.parametrize("tokens,taps,pieces,want", [(8192, 4, 2, 32), (2048, 4, 2, 8), (512, 4, 2, 4), (6000, 4, 1, 16), (33, 4, 1, 4), (6000, 5, 1, 32), (6000, 8, 1, 32),
-                                                     (6000, 12, 1, 32), (3000, 8, 1, 16), (700, 9, 2, 16), (300, 16, 2, 16), (300, 17, 2, 32)])
+                                                     (6000, 12, 1, 32), (3000, 8, 1, 16), (700, 9, 2, 16), (300, 16, 2, 16), (300, 17, 2, 32), (3000, 9, 2, 32), (1500, 9, 2, 16),
+                                                     (700, 9, 4, 32), (1500, 9, 4, 16), (700, 8, 4, 8)])
 def test_strips_are_shortened_only_where_the_recomputed_norms_pay(rules, tokens, taps, pieces, want):
     assert rules.strip(tokens, taps, pieces) == want
 
