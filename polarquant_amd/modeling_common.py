@@ -186,9 +186,14 @@ def _nobody_looks_on(*ts) -> bool:
 
 
 def _on_gpu_in_half(*ts) -> bool:
-    """Whether the fused launches can take these tensors as they lie: one half-precision dtype, one GPU, contiguous, 16-byte aligned,
-    not empty, and nobody who follows torch's operations."""
-    return (ts[0].dtype in (torch.float16, torch.bfloat16) and _nobody_looks_on(*ts)
+    """Whether the fused launches can take these tensors as they lie: nobody who follows torch's operations (asked before anything else:
+    a symbolic trace has no dtype to compare, a dynamic size no value), one half-precision dtype, one GPU, contiguous, 16-byte
+    aligned, not empty."""
+    return _nobody_looks_on(*ts) and _lie_in_half(*ts)
+
+
+def _lie_in_half(*ts) -> bool:
+    return (ts[0].dtype in (torch.float16, torch.bfloat16)
             and all(t.is_cuda and t.dtype == ts[0].dtype and t.device == ts[0].device and t.is_contiguous() and t.data_ptr() % 16 == 0
                     and t.numel() > 0 for t in ts))
 
@@ -214,10 +219,11 @@ class Linear(nn.Linear):
     library in any case."""
 
     def forward(self, x, library=False):
-        if (not library and 0 < x.numel() <= 16 * self.in_features and x.shape[-1] == self.in_features and x.is_cuda and x.dtype == self.weight.dtype
+        own = (self.weight,) if self.bias is None else (self.weight, self.bias)
+        if (_nobody_looks_on(x, *own) and not library and 0 < x.numel() <= 16 * self.in_features and x.shape[-1] == self.in_features and x.is_cuda and x.dtype == self.weight.dtype
                 and x.stride(-1) == 1 and self.out_features % 16 == 0 and self.in_features % 32 == 0 and self.weight.device == x.device
                 and _streams_faster(x.numel() // self.in_features, self.out_features, self.in_features)
-                and type(x) is torch.Tensor and _on_gpu_in_half(*((self.weight,) if self.bias is None else (self.weight, self.bias)))):
+                and _lie_in_half(*own)):
             from .decode_ops import linear_small_m
             rows = x.reshape(-1, self.in_features)
             # (the kernel takes rows that lie apart: not one row expanded to many, nor rows that overlap)
