@@ -220,15 +220,16 @@ class Linear(nn.Linear):
 
     def forward(self, x, library=False):
         own = (self.weight,) if self.bias is None else (self.weight, self.bias)
-        if (_nobody_looks_on(x, *own) and not library and 0 < x.numel() <= 16 * self.in_features and x.shape[-1] == self.in_features and x.is_cuda and x.dtype == self.weight.dtype
-                and x.stride(-1) == 1 and self.out_features % 16 == 0 and self.in_features % 32 == 0 and self.weight.device == x.device
-                and _streams_faster(x.numel() // self.in_features, self.out_features, self.in_features)
-                and _lie_in_half(*own)):
-            from .decode_ops import linear_small_m
-            rows = x.reshape(-1, self.in_features)
-            # (the kernel takes rows that lie apart: not one row expanded to many, nor rows that overlap)
-            if rows.data_ptr() % 16 == 0 and rows.stride(0) % 8 == 0 and (rows.shape[0] == 1 or rows.stride(0) >= self.in_features):
-                return linear_small_m(rows, self.weight, self.bias).view(*x.shape[:-1], self.out_features)
+        if _nobody_looks_on(x, *own) and not library and self.weight.dim() == 2 and x.dim() > 0:
+            n, k = self.weight.shape                     # (the weight counts, not the sizes the module was made with)
+            if (0 < x.numel() <= 16 * k and x.shape[-1] == k and x.is_cuda and x.dtype == self.weight.dtype and x.stride(-1) == 1
+                    and n % 16 == 0 and k % 32 == 0 and self.weight.device == x.device and (self.bias is None or self.bias.shape == (n,))
+                    and _streams_faster(x.numel() // k, n, k) and _lie_in_half(*own)):
+                from .decode_ops import linear_small_m
+                rows = x.reshape(-1, k)
+                # (the kernel takes rows that lie apart: not one row expanded to many, nor rows that overlap)
+                if rows.data_ptr() % 16 == 0 and rows.stride(0) % 8 == 0 and (rows.shape[0] == 1 or rows.stride(0) >= k):
+                    return linear_small_m(rows, self.weight, self.bias).view(*x.shape[:-1], n)
         return super().forward(x)
 
 

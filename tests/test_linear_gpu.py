@@ -196,3 +196,18 @@ def test_linear_module_takes_rows_that_share_storage(gpu, dtype):
         for t in (x[:1, :, :160].expand(4, 1, 160), x[0, :, :160].expand(5, 160), x.as_strided((3, 160), (8, 1)), x.as_strided((3, 160), (152, 1)),
                   x[:1, :, :160].expand(2, 3, 160), x[:, :, :160].expand(3, 4, 160), x.as_strided((2, 1, 160), (160, 0, 1)), x[:1, :, :160].expand(1, 1, 160)):
             _check(lin(t), F.linear(t.double(), lin.weight.double(), lin.bias.double()), dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_linear_module_goes_by_its_weight(gpu, dtype):
+    """A weight set afterwards, as tied or resized embeddings are, need not have the sizes the module was made with."""
+    from polarquant_amd.modeling_common import Linear
+    g = torch.Generator(device=gpu).manual_seed(5)
+    for (n, k), bias in (((96, 160), None), ((64, 192), None), ((40, 160), None), ((64, 160), 1)):
+        lin = Linear(160, 64, bias=bias is not None).to(gpu, dtype)
+        lin.weight = torch.nn.Parameter(torch.randn(n, k, generator=g, device=gpu).to(dtype))
+        if bias:
+            lin.bias = torch.nn.Parameter(torch.randn(bias, generator=g, device=gpu).to(dtype))          # (one for all outputs)
+        x = torch.randn(2, k, generator=g, device=gpu).to(dtype)
+        with torch.no_grad():
+            _check(lin(x), F.linear(x.double(), lin.weight.double(), lin.bias if bias is None else lin.bias.double()), dtype)
