@@ -214,23 +214,49 @@ def _streams_faster(rows: int, n: int, k: int) -> bool:
     return n >= 3072 and 4 * groups >= 3 * 256 * -(-groups // 256) and k % 16384 != 0
 
 
+# What the modules below launch by themselves, or None.  (Functions of their own: a script compiles the modules' forward, and passes over what
+# it does not run.)
+def _streamed_linear(x, weight, bias, library):
+    own = (weight,) if bias is None else (weight, bias)
+    if not _nobody_looks_on(x, *own) or library or weight.dim() != 2 or x.dim() == 0:
+        return None
+    n, k = weight.shape                                  # (the weight counts, not the sizes the module was made with)
+    if not (0 < x.numel() <= 16 * k and x.shape[-1] == k and x.is_cuda and x.dtype == weight.dtype and x.stride(-1) == 1
+            and n % 16 == 0 and k % 32 == 0 and weight.device == x.device and (bias is None or bias.shape == (n,))
+            and _streams_faster(x.numel() // k, n, k) and _lie_in_half(*own)):
+        return None
+    from .decode_ops import linear_small_m
+    rows = x.reshape(-1, k)
+    # (the kernel takes rows that lie apart: not one row expanded to many, nor rows that overlap)
+    if rows.data_ptr() % 16 or rows.stride(0) % 8 or not (rows.shape[0] == 1 or rows.stride(0) >= k):
+        return None
+    return linear_small_m(rows, weight, bias).view(*x.shape[:-1], n)
+
+
+def _fused_rmsnorm(x, weight, eps):
+    if not _on_gpu_in_half(x, weight) or x.shape[-1] % 8:
+        return None
+    from .decode_ops import rmsnorm                      # one pass over memory for the eight below (8192 x 4096: 23 against 125 us)
+    return rmsnorm(x, weight, eps)
+
+
+def _fused_silu_mul(gate, up):
+    if not _on_gpu_in_half(gate, up) or gate.shape[-1] % 8:
+        return None
+    from .decode_ops import silu_mul                     # (8192 x 14336: 120 against 220 us)
+    return silu_mul(gate, up)
+
+
 class Linear(nn.Linear):
     """`nn.Linear`; up to 16 rows, a stream of the weights, through the weight-streaming kernel where that is faster.  library: the BLAS
     library in any case."""
 
-    def forward(self, x, library=False):
-        own = (self.weight,) if self.bias is None else (self.weight, self.bias)
-        if _nobody_looks_on(x, *own) and not library and self.weight.dim() == 2 and x.dim() > 0:
-            n, k = self.weight.shape                     # (the weight counts, not the sizes the module was made with)
-            if (0 < x.numel() <= 16 * k and x.shape[-1] == k and x.is_cuda and x.dtype == self.weight.dtype and x.stride(-1) == 1
-                    and n % 16 == 0 and k % 32 == 0 and self.weight.device == x.device and (self.bias is None or self.bias.shape == (n,))
-                    and _streams_faster(x.numel() // k, n, k) and _lie_in_half(*own)):
-                from .decode_ops import linear_small_m
-                rows = x.reshape(-1, k)
-                # (the kernel takes rows that lie apart: not one row expanded to many, nor rows that overlap)
-                if rows.data_ptr() % 16 == 0 and rows.stride(0) % 8 == 0 and (rows.shape[0] == 1 or rows.stride(0) >= k):
-                    return linear_small_m(rows, self.weight, self.bias).view(*x.shape[:-1], n)
-        return super().forward(x)
+    def forward(self, x, library: bool = False):
+        if not torch.jit.is_scripting():
+            y = _streamed_linear(x, self.weight, self.bias, library)
+            if y is not None:
+                return y
+        return F.linear(x, self.weight, self.bias)
 
 
 class RMSNorm(nn.Module):
@@ -240,9 +266,10 @@ class RMSNorm(nn.Module):
         self.variance_epsilon = eps
 
     def forward(self, x):
-        if _on_gpu_in_half(x, self.weight) and x.shape[-1] % 8 == 0:
-            from .decode_ops import rmsnorm            # one pass over memory for the eight below (8192 x 4096: 23 against 125 us)
-            return rmsnorm(x, self.weight, self.variance_epsilon)
+        if not torch.jit.is_scripting():
+            y = _fused_rmsnorm(x, self.weight, self.variance_epsilon)
+            if y is not None:
+                return y
         dt = x.dtype
         x = x.float()
         x = x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + self.variance_epsilon)
@@ -259,9 +286,10 @@ class MLP(nn.Module):
 
     def forward(self, x):
         gate, up = self.gate_proj(x), self.up_proj(x)
-        if _on_gpu_in_half(gate, up) and gate.shape[-1] % 8 == 0:
-            from .decode_ops import silu_mul           # (8192 x 14336: 120 against 220 us)
-            return self.down_proj(silu_mul(gate, up))
+        if not torch.jit.is_scripting():
+            y = _fused_silu_mul(gate, up)
+            if y is not None:
+                return self.down_proj(y)
         return self.down_proj(F.silu(gate) * up)
 
 

@@ -52,12 +52,13 @@ def test_what_counts_as_plain():
 
 @pytest.mark.parametrize("grad", [False, True])
 @pytest.mark.parametrize("make", [lambda: mc.RMSNorm(64, 1e-5), lambda: mc.MLP(mc.PolarConfig(hidden_size=64, intermediate_size=32)), lambda: mc.Linear(64, 32)])
-def test_symbolic_traces_and_dynamic_sizes(make, grad):
-    """Neither values nor sizes are known there, so that nothing may be asked of them."""
+def test_symbolic_traces_scripts_and_dynamic_sizes(make, grad):
+    """Neither values nor sizes are known there, so that nothing may be asked of them; a script compiles what it can see."""
     m, x = make(), torch.randn(40, 64)
     with torch.set_grad_enabled(grad):
         want = m(x)
         assert torch.equal(torch.fx.symbolic_trace(m)(x), want)
+        assert torch.equal(torch.jit.script(m)(x), want)
         rows = torch.export.Dim("rows", min=2, max=4096)
         exported = torch.export.export(m, (torch.randn(3, 64),), dynamic_shapes=({0: rows},)).module()
         assert torch.equal(exported(x), want)
