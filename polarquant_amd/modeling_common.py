@@ -234,14 +234,15 @@ def _streamed_linear(x, weight, bias, library):
 
 
 def _fused_rmsnorm(x, weight, eps):
-    if not _on_gpu_in_half(x, weight) or x.shape[-1] % 8:
+    # (the launch has one workgroup a row, of 2^32 threads together at most, and does not broadcast)
+    if not _on_gpu_in_half(x, weight) or x.dim() == 0 or x.shape[-1] % 8 or weight.shape != x.shape[-1:] or x.numel() // x.shape[-1] >= 1 << 24:
         return None
     from .decode_ops import rmsnorm                      # one pass over memory for the eight below (8192 x 4096: 23 against 125 us)
     return rmsnorm(x, weight, eps)
 
 
 def _fused_silu_mul(gate, up):
-    if not _on_gpu_in_half(gate, up) or gate.shape[-1] % 8:
+    if not _on_gpu_in_half(gate, up) or gate.dim() == 0 or gate.shape[-1] % 8 or gate.shape != up.shape:
         return None
     from .decode_ops import silu_mul                     # (8192 x 14336: 120 against 220 us)
     return silu_mul(gate, up)

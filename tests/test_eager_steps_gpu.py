@@ -42,3 +42,15 @@ def test_gated_activation(ff, bias, dtype):
     want = mlp(x).detach() if torch.is_grad_enabled() else None
     # the products' sums run over `ff` activations, each within two roundings
     assert float((got.double() - want.double()).norm() / want.double().norm()) < 2 * UNIT[dtype]
+
+
+def test_norm_beyond_the_launch():
+    """2^24 rows are more than one launch takes, a weight of one element is broadcast: the torch operations run."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    norm = RMSNorm(8, 1e-5).to("cuda", torch.bfloat16)
+    few = torch.randn(1 << 10, 8, generator=g, device="cuda").to(torch.bfloat16)
+    with torch.no_grad():
+        many = norm(few.repeat(1 << 14, 1))
+        assert bool((many.view(1 << 14, 1 << 10, 8) == many[:1 << 10]).all()) and close(many[:1 << 10], norm(few), torch.bfloat16)
+        norm.weight = torch.nn.Parameter(norm.weight[:1] * 3)
+        assert close(norm(few), 3 * many[:1 << 10], torch.bfloat16)
