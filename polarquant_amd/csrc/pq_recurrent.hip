@@ -257,8 +257,8 @@ __global__ __launch_bounds__(256) void scan_kernel(ScanArgs a) {
         static_for<RPL / 4>([&](auto C) {
             constexpr int c = decltype(C)::value;
             const int r = row_of(4 * c);
-            const float4 w = *reinterpret_cast<const float4*>(sp + (r < dim ? r : 0));       // (rows past the last: a copy that meets zeros)
-            S[4 * c] = w.x; S[4 * c + 1] = w.y; S[4 * c + 2] = w.z; S[4 * c + 3] = w.w;
+            const float4 w = *reinterpret_cast<const float4*>(sp + (r < dim ? r : 0));       // (rows past the last are zero)
+            S[4 * c] = r < dim ? w.x : 0.0f; S[4 * c + 1] = r < dim ? w.y : 0.0f; S[4 * c + 2] = r < dim ? w.z : 0.0f; S[4 * c + 3] = r < dim ? w.w : 0.0f;
         });
     } else {
 #pragma unroll

@@ -69,3 +69,17 @@ def test_memory(dim, vdim, H, L, pad, dtype):
         wden.append(torch.maximum(e[..., -1].abs(), (-mx).exp()) + 1e-6)
     assert off(state, S) < 1e-5 and off(m[:, :, 0], mx) < 1e-5
     assert off(o, torch.stack(want, 1).reshape(B * L, H * vdim)) < 1e-5 and off(den, torch.stack(wden, 1).reshape(B * L, H)) < 1e-5
+
+
+@pytest.mark.parametrize("dim", [100, 30])                                  # (quads with rows to spare; row by row)
+def test_infinite_state(dim):
+    """An infinite entry of the state makes its column's result infinite where q does not vanish, and nothing NaN: no other row repeats it."""
+    B, H, vdim = 1, 1, 20
+    g = torch.Generator(device="cuda").manual_seed(dim)
+    q, k, v = torch.randn(B, 2 * dim + vdim, generator=g, device="cuda").split((dim, dim, vdim), 1)
+    log_i, log_f = torch.full((B, H), -1.0, device="cuda"), torch.full((B, H), -0.5, device="cuda")
+    state, m = ops.memory_state(B, H, dim, vdim, "cuda")
+    state[:, :, 7, 1], q[:, 1] = float("inf"), -2.0
+    o, _ = ops.memory_scan(q, k, v, log_i, log_f, state, m, 0.3, Step(B, 1, 7))
+    assert float(o[0, 7]) == float("-inf") and int(torch.isinf(state).sum()) == 1 and not torch.isnan(state).any()
+    assert bool(torch.isfinite(o).sum() == vdim - 1)
