@@ -171,7 +171,8 @@ int launch_qkv_rope_append(const void* x, int64_t x_stride, const void* w, const
 // Launch shapes measured at the decode shapes of Llama-3-8B (K-split 4 / 8 / 16 and stages of 1 / 2 / 4 / 8
 // loads were swept): the 16-row kernel runs four wavefronts per workgroup with stages of 4 (2 when gated); the
 // M <= 8 kernel four wavefronts, or eight when K >= 8192 (down_proj), with stages of 1 (2 with eight wavefronts on two row tiles).
-// K / KSPLIT must stay a whole number of k-steps.  The split of K, and with it every sum's order, depends on K alone.
+// K / KSPLIT must stay a whole number of k-steps.  Within a kernel the split of K, and with it every sum's order, depends on K alone: not on N
+// or the rows per workgroup.  The two kernels (up to 8 rows, 9 to 16) add in different orders.
 int launch_small_m_linear(const void* x, int64_t x_stride, const void* w, const void* w_up, const void* bias, void* y,
                           int64_t y_stride, int M, int N, int K, int dtype, hipStream_t st) {
     const bool gated = w_up != nullptr;

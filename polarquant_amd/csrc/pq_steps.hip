@@ -374,7 +374,7 @@ int launch_stream_add(const StreamAddArgs& a, int dtype, hipStream_t st) {
     return static_cast<int>(hipGetLastError());
 }
 
-// V channels a thread; a workgroup takes 1024 / V neighbouring pieces of one row after another (8192 rows of 4096 in bfloat16: 101 us
+// V channels a thread; a workgroup takes 256 neighbouring pieces of one row after another (8192 rows of 4096 in bfloat16: 101 us
 // channel by channel, 44 with four).
 template <typename T, int V>
 __global__ __launch_bounds__(256) void embed_rows_kernel(const void* table, const int64_t* ids, float scale, float* out, int64_t rows, int width, int64_t vocab) {
