@@ -692,8 +692,8 @@ def _prefill_attention(q, k, v, attention_mask, n_rep, is_causal):
     `attention_mask` [B, L] of {0,1} marks left padding."""
     B, N, L, hd = q.shape
     if attention_mask is None or bool((attention_mask != 0).all()):
-        # the library's flash attention takes twice the time from 512 tokens on (32 heads, 512 / 8192 / 16384 tokens: 34, 1270, 4484
-        # against 18, 564, 2121 us) and the same below; it stays for what the kernel does not take: float32, tensors on the host, gradients
+        # the library's flash attention takes twice the time from 512 tokens on (32 heads, 8 KV heads, 512 / 8192 / 16384 tokens: 33, 1266,
+        # 4464 against 17, 577, 2242 us) and the same below; it stays for what the kernel does not take: float32, tensors on the host, gradients
         if is_causal and _nobody_looks_on(q, k, v) and prompt_attention_takes(q, k, v):
             return prompt_attention(q, k, v)
         out = F.scaled_dot_product_attention(q, k, v, is_causal=is_causal and L > 1, enable_gqa=n_rep > 1)
