@@ -117,3 +117,16 @@ def test_what_prompt_attention_refuses():
         wide = w.expand(B, N, L, 128) if B and N else x.new_empty(B, N, L, 128)
         assert not prompt_attention_takes(wide, wide, wide)
     assert prompt_attention_takes(*[w.expand(1, 1, 65535 * 128, 128)] * 3) and not prompt_attention_takes(x, x[:, :0], x[:, :0]) and not prompt_attention_takes(x[0], x[0], x[0])
+
+
+def test_a_prompt_of_one_token_is_the_librarys(monkeypatch):
+    """Its attention is a copy of the values; the library needs 6 us for it, whatever the batch, a tile of the kernel 7 to 14."""
+    from polarquant_amd import modeling_common as mc
+    taken, own = [], mc.prompt_attention
+    monkeypatch.setattr(mc, "prompt_attention", lambda q, k, v: (taken.append(q.shape[2]), own(q, k, v))[1])
+    with torch.no_grad():
+        for L in (1, 2, 3):
+            q, k, v = [torch.randn(2, n, L, 128, device="cuda").bfloat16() for n in (8, 2, 2)]
+            got = mc._prefill_attention(q, k, v, None, 4, True)
+            assert got.shape == (2, L, 8, 128) and off(got, reference(*[t.transpose(1, 2) for t in (q, k, v)], 128 ** -0.5)) < UNIT[torch.bfloat16]
+    assert taken == [2, 3]
