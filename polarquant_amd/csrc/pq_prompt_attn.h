@@ -99,17 +99,24 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
     const float scale2 = a.scale != 0.0f ? fabsf(a.scale) * kLog2e : 1.0f;
     const float slope2 = WINDOW && a.slopes ? a.slopes[h] * kLog2e : 0.0f;
 
+    // the queries: requested here, and masked once the first tile is on its way.  (A selection of what is loaded becomes a branch around each
+    // load, and each is waited for by itself: 20 tokens, 32 heads of 128 9.0 us, 8.4 so; 16 heads of 192 10.4 and 9.5, 8 of 256 14.1 and
+    // 12.4; with tiles passed through registers 8.0, 9.0, 12.7.)
     u32x4_a q[KS];
     {
         const uint16_t* qp = static_cast<const uint16_t*>(a.q) + b * a.q_b + qc * a.q_t + h * a.q_h;
-        const uint32_t flip = a.scale < 0.0f ? 0x80008000u : 0u;
         static_for<KS>([&](auto I) {
-            constexpr int i = decltype(I)::value;
-            const int c = i * 16 + 8 * hi;
-            const u32x4_a t = *reinterpret_cast<const u32x4_a*>(qp + (c < D ? c : 0));
-            q[i] = c < D && a.scale != 0.0f ? u32x4_a{t.x ^ flip, t.y ^ flip, t.z ^ flip, t.w ^ flip} : u32x4_a{0, 0, 0, 0};
+            const int c = decltype(I)::value * 16 + 8 * hi;
+            q[I] = *reinterpret_cast<const u32x4_a*>(qp + (c < D ? c : 0));
         });
     }
+    auto mask_queries = [&]() {
+        const uint32_t flip = a.scale < 0.0f ? 0x80008000u : 0u, zero = a.scale != 0.0f ? 0xffffffffu : 0u;
+        static_for<KS>([&](auto I) {
+            const uint32_t keep = decltype(I)::value * 16 + 8 * hi < D ? zero : 0u;
+            q[I] = u32x4_a{(q[I].x ^ flip) & keep, (q[I].y ^ flip) & keep, (q[I].z ^ flip) & keep, (q[I].w ^ flip) & keep};
+        });
+    };
     // where this lane's 16 bytes of each load come from: load i of a wavefront fills chunks (wv KL + i) 64 .. + 63 of a tile
     const uint16_t* kb = static_cast<const uint16_t*>(a.k) + b * a.k_b + g * a.k_h;
     const uint16_t* vb = static_cast<const uint16_t*>(a.v) + b * a.v_b + g * a.v_h;
@@ -135,14 +142,15 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
     };
     const uint16_t *ks[KL], *vs[VL];
     if (!WINDOW) {
-        static_for<KL>([&](auto I) { ks[I] = k_src(I, it0 * kPromptTileKeys, 0, kPromptTileKeys - 1); });
-        static_for<VL>([&](auto I) { vs[I] = v_src(I, it0 * kPromptTileKeys, 0, kPromptTileKeys - 1); });
+        const int last = a.Lk - 1 - it0 * kPromptTileKeys > 0 ? a.Lk - 1 - it0 * kPromptTileKeys : 0;
+        static_for<KL>([&](auto I) { ks[I] = k_src(I, it0 * kPromptTileKeys, 0, last); });
+        static_for<VL>([&](auto I) { vs[I] = v_src(I, it0 * kPromptTileKeys, 0, last); });
     }
     auto fetch = [&](int it, auto BUF) {
         constexpr int buf = decltype(BUF)::value;
         const int last = a.Lk - 1 - it * kPromptTileKeys;          // rows past the end: copies of the last one, with weight zero
         // (the addresses of whole tiles of this call's tokens only advance)
-        if (last < kPromptTileKeys - 1 || (WINDOW && (it == it0 || (it - 1) * kPromptTileKeys < past))) {
+        if ((it > it0 && last < kPromptTileKeys - 1) || (WINDOW && (it == it0 || (it - 1) * kPromptTileKeys < past))) {
             const int first = it * kPromptTileKeys, slot = WINDOW ? first % a.cap : 0;
             static_for<KL>([&](auto I) { ks[I] = k_src(I, first, slot, last); });
             if (TOKEN_ROWS) static_for<VL>([&](auto I) { vs[I] = v_src(I, first, slot, last); });
@@ -262,6 +270,7 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
         __syncthreads();
     };
     if (it0 < it1) fetch(it0, IC<0>{});
+    mask_queries();
     wait_lds_loads();
     __syncthreads();
     for (int it = it0; it < it1; it += 2) {

@@ -64,3 +64,14 @@ def test_latent_prompts_of_any_width_stay_in_registers():
     in every tile (256 wide: 1.6 times the time)."""
     spilled = {name: int(n) for name, n in re.findall(r"\.name: +(\S*prompt_attn_kernel\S*)\n(?:.*\n)*? +\.vgpr_spill_count: (\d+)", _listing("pq_latent_attn.hip", ()))}
     assert len(spilled) == 8 and not any(spilled.values()), spilled
+
+
+@pytest.mark.parametrize("src,defines", [u[:2] for u in WITH_LOADS], ids=[u[0] + u[2] for u in WITH_LOADS])
+def test_the_first_tile_waits_for_no_load(src, defines):
+    """The queries are asked for first, but the first tile must not wait for them, nor one of them for another: a prompt of a tile or two
+    is little else than its start."""
+    kernels = re.findall(r"^(\S*prompt_attn_kernel\S*):.*\n((?:.*\n)*?).*\bglobal_load_lds", _listing(src, defines), re.M)
+    assert kernels
+    for name, start in kernels:
+        loads, waits = len(re.findall(r"^\s+global_load_dwordx4", start, re.M)), re.findall(r"s_waitcnt .*vmcnt", start)
+        assert loads >= 4 and not waits, (name, loads, len(waits))
