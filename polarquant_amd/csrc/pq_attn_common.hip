@@ -108,6 +108,10 @@ static bool runs_groups(const AttnArgs& a) {
     // the window of residual keys is one slice's here; slices cut on the device spread a long one (8 KV heads, us, pairs / groups: 500
     // keys 9.3 / 8.8, 2000 keys 9.9 / 22.2; evenly cut slices keep it in one either way: 100.7 / 22.3)
     const int resid = a.n_resid_per_seq ? a.resid_capacity : a.n_resid;
+    // With 4-bit values and one or two heads per KV head one wavefront a slice is as fast alone, and of more than 256 slices some unit has two
+    // workgroups here: 264 to 320 slices 3 to 8 % slower (288, one head: 11.1 / 11.9 us, two 12.6 / 13.0; 256 10.6 / 9.8), unless the
+    // window has a slice of its own (288, one key 12.6 / 12.2, 127 keys 14.4 / 12.4).  Three heads gain up to 320 (14.6 / 14.1).
+    if (a.v4_codes && a.N <= 2 * a.Nk && static_cast<long long>(a.n_splits) * a.B * a.Nk > 256 && groups <= a.n_splits && !(resid > 0 && groups < a.n_splits)) return false;
     return groups <= 2 * a.n_splits && a.min_groups_per_split <= 2 && !(a.balanced && resid > 4 * kGroup);
 }
 

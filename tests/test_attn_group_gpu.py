@@ -173,3 +173,20 @@ def test_only_one_query_token_is_taken(gpu, shape):
         assert torch.equal(call(q.to(gpu).view(1, 8, 128)), want) and torch.equal(call(q.to(gpu).view(1, 8, 1, 1, 128)), want)
         with pytest.raises(RuntimeError):
             call(bad)
+
+
+@pytest.mark.parametrize("N", [8, 16, 24])
+@pytest.mark.parametrize("groups,resid", [(32, 0), (33, 0), (33, 1), (40, 0), (40, 1)])
+def test_four_bit_values_around_a_workgroup_a_unit(gpu, N, groups, resid):
+    """256 slices of 8 KV heads and more, where one or two heads per KV head change the kernel."""
+    q, codes, kres, v = inputs(1, N, 8, groups, resid, 4, 4, torch.float16, groups + N)
+    vq = po.quantize_values_along_last_dim(v[:, :, :groups * 128].contiguous())
+    vres = torch.zeros_like(kres)
+    vres[:, :, :resid] = v[:, :, groups * 128:]
+    want = po.decode_attention_mixed_exact(q, kres[:, :, :resid], *codes, vres[:, :, :resid], *vq, rbits=4, tbits=4)
+    args = [q.to(gpu), *[t.to(gpu) for t in codes], kres.to(gpu), vres.to(gpu), *[t.to(gpu) for t in vq], groups, resid]
+    assert close(polar_decode_attention_v4(*args), want, torch.float16)
+    nan = args[0].clone()
+    nan[0, 1] = float("nan")
+    got = polar_decode_attention_v4(nan, *args[1:])
+    assert torch.isnan(got[0, 1]).all() and not torch.isnan(got[0, 2:]).any() and not torch.isnan(got[0, 0]).any()
