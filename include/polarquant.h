@@ -460,8 +460,8 @@ int pq_validate_decode_attn_v4(const void *q,
 
 /* Up to this many slices (n_splits * B * Nk) of at most two groups, angles of at most 4 bits, run a kernel in which eight
  * wavefronts share a slice.  There n_splits = groups + 1 gives the keys not yet quantized a slice of their own; beyond it, and
- * in the other kernels, such a slot stays empty.  (With 4-bit values and one or two heads per KV head: up to 256 slices, more only
- * with such a slot.) */
+ * in the other kernels, such a slot stays empty.  (Packed codes, more than 4 heads per KV head, or 4-bit values with one or two: up
+ * to 256 slices, more only with such a slot.) */
 #define PQ_FEW_SLICES 320
 
 /* Suggested n_splits for a shape (host-only; `max_groups` = largest group count

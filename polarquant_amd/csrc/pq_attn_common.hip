@@ -108,10 +108,12 @@ static bool runs_groups(const AttnArgs& a) {
     // the window of residual keys is one slice's here; slices cut on the device spread a long one (8 KV heads, us, pairs / groups: 500
     // keys 9.3 / 8.8, 2000 keys 9.9 / 22.2; evenly cut slices keep it in one either way: 100.7 / 22.3)
     const int resid = a.n_resid_per_seq ? a.resid_capacity : a.n_resid;
-    // With 4-bit values and one or two heads per KV head one wavefront a slice is as fast alone, and of more than 256 slices some unit has two
-    // workgroups here: 264 to 320 slices 3 to 8 % slower (288, one head: 11.1 / 11.9 us, two 12.6 / 13.0; 256 10.6 / 9.8), unless the
-    // window has a slice of its own (288, one key 12.6 / 12.2, 127 keys 14.4 / 12.4).  Three heads gain up to 320 (14.6 / 14.1).
-    if (a.v4_codes && a.N <= 2 * a.Nk && static_cast<long long>(a.n_splits) * a.B * a.Nk > 256 && groups <= a.n_splits && !(resid > 0 && groups < a.n_splits)) return false;
+    // Of more than 256 slices some unit has two workgroups here.  Unless the window has a slice of its own (of 288 slices with it 0.83 to 1.05
+    // of the other kernels' time) that pays only with one byte a code for up to 4 heads per KV head, or with 4-bit values for 3 and more.
+    // Others / here at 288 slices without a window, us: 4 heads 14.5 / 14.1, 5 heads 15.0 / 16.3, 8 heads 17.1 / 17.9, packed codes and 4
+    // heads 14.0 / 14.6; 4-bit values, 1 head 11.1 / 11.9, 2 heads 12.6 / 13.0, 3 heads 14.4 / 13.7.  256 slices, 5 heads 14.8 / 13.0.
+    const bool own_slice = resid > 0 && groups < a.n_splits, pays = a.v4_codes ? a.N > 2 * a.Nk : a.N <= 4 * a.Nk && !a.packed6;
+    if (static_cast<long long>(a.n_splits) * a.B * a.Nk > 256 && groups <= a.n_splits && !own_slice && !pays) return false;
     return groups <= 2 * a.n_splits && a.min_groups_per_split <= 2 && !(a.balanced && resid > 4 * kGroup);
 }
 

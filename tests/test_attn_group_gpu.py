@@ -190,3 +190,16 @@ def test_four_bit_values_around_a_workgroup_a_unit(gpu, N, groups, resid):
     nan[0, 1] = float("nan")
     got = polar_decode_attention_v4(nan, *args[1:])
     assert torch.isnan(got[0, 1]).all() and not torch.isnan(got[0, 2:]).any() and not torch.isnan(got[0, 0]).any()
+
+
+@pytest.mark.parametrize("N,packed", [(32, False), (40, False), (64, False), (8, True), (32, True)])
+@pytest.mark.parametrize("groups,resid", [(32, 0), (33, 0), (33, 1), (40, 0), (40, 1)])
+def test_half_precision_values_around_a_workgroup_a_unit(gpu, N, packed, groups, resid):
+    """The same, where packed codes or more than four heads per KV head change the kernel."""
+    bits = 3 if packed else 4
+    q, codes, kres, v = inputs(1, N, 8, groups, resid, bits, bits, torch.bfloat16, groups + N)
+    want = po.decode_attention_exact(q, kres[:, :, :resid], *codes, v, rbits=bits, tbits=bits)
+    codes = [t.to(gpu) for t in codes]
+    if packed:
+        codes[0] = convert_codes6(codes[0], True)
+    assert close(polar_decode_attention(q.to(gpu), *codes, kres.to(gpu), v.to(gpu), groups, resid, rbits=bits, tbits=bits), want, torch.bfloat16)
