@@ -1,4 +1,4 @@
-"""ctypes binding of libpolarquant_hip.so (the C ABI declared in include/polarquant.h).
+"""Binding of libpolarquant_hip.so (the C ABI declared in include/polarquant.h): ctypes, and builtins for what the wrappers call.
 
 The library is loaded from the package directory; it is never built implicitly
 on import of this module when a built library exists.  If it is missing the
@@ -7,8 +7,12 @@ loader raises: there is no CPU fallback for any op of this package.
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
+import types
 from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_uint, c_void_p
+
+import torch  # noqa: F401  (its libraries have to be there before _calls is loaded)
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libpolarquant_hip.so")
@@ -163,19 +167,43 @@ class PolarQuantError(RuntimeError):
 _LOADED = {}
 
 
+class _CallsOnceBuilt:
+    """Stands for `_calls` (csrc/pq_calls.cpp) where the package is imported before it is built."""
+
+    def __getattr__(self, name):
+        try:
+            return getattr(importlib.import_module(__package__ + "._calls"), name)
+        except ImportError as e:
+            raise RuntimeError("polarquant_amd: %s cannot be loaded (%s); build it with `python -m polarquant_amd.build`"
+                               % (os.path.join(HERE, "_calls.so"), e)) from e
+
+
+try:
+    from . import _calls as calls
+except ImportError:
+    calls = _CallsOnceBuilt()
+
+
+def declare(handle: ctypes.CDLL, signatures) -> ctypes.CDLL:
+    """`handle` with its symbols' types set, and as `handle.call` the functions that the wrappers call as builtins of `_calls`
+    (csrc/pq_calls.cpp): same arguments, tensors in the place of their pointers, tuples in the place of integer arrays."""
+    handle.call = types.SimpleNamespace()
+    for name, (res, args) in signatures.items():
+        fn = getattr(handle, name)
+        fn.restype = res
+        fn.argtypes = args
+        setattr(handle.call, name, calls.bind(name, ctypes.cast(fn, c_void_p).value) or fn)
+    return handle
+
+
 def _load(path: str, signatures) -> ctypes.CDLL:
-    """The library at `path` with its symbols' types set, loaded once.  Raises if it has not been built."""
+    """The library at `path` with its symbols declared, loaded once.  Raises if it has not been built."""
     handle = _LOADED.get(path)
     if handle is None:
         if not os.path.exists(path):
             raise RuntimeError("polarquant_amd: %s is missing; build it with `python -m polarquant_amd.build` "
                                "(there is no CPU fallback)" % path)
-        handle = ctypes.CDLL(path)
-        for name, (res, args) in signatures.items():
-            fn = getattr(handle, name)
-            fn.restype = res
-            fn.argtypes = args
-        _LOADED[path] = handle
+        handle = _LOADED[path] = declare(ctypes.CDLL(path), signatures)
     return handle
 
 

@@ -6,7 +6,6 @@ LlamaPolarGroupAttention.forward computes between RoPE and o_proj
 """
 from __future__ import annotations
 
-import ctypes
 import functools
 import math
 from typing import Optional
@@ -14,6 +13,7 @@ from typing import Optional
 import torch
 
 from . import _ffi
+from ._ffi import calls as _calls
 from .kernel4group import _dtype_code, _on_device, _stream_ptr
 
 GROUP = 128
@@ -26,11 +26,11 @@ def _num_cus(device: torch.device) -> int:
 
 
 def plan_splits(B: int, Nk: int, max_groups: int, device: torch.device) -> int:
-    return _ffi.lib().pq_decode_attn_plan(B, Nk, max(max_groups, 1), _num_cus(device))
+    return _ffi.lib().call.pq_decode_attn_plan(B, Nk, max(max_groups, 1), _num_cus(device))
 
 
 def workspace_bytes(B: int, N: int, n_splits: int) -> int:
-    return _ffi.lib().pq_decode_attn_workspace_bytes(B, N, n_splits)
+    return _ffi.lib().call.pq_decode_attn_workspace_bytes(B, N, n_splits)
 
 
 def new_workspace(B: int, N: int, n_splits: int, device: torch.device) -> torch.Tensor:
@@ -121,35 +121,41 @@ def polar_decode_attention(
     if not query_states.is_cuda:
         raise RuntimeError("polarquant_amd: decode attention needs tensors on the GPU (no CPU fallback)")
     dev = query_states.device
-    B, N = query_states.shape[:2]
-    hd = query_states.shape[-1]
-    Nk = value_states.shape[1]
-    assert hd == 128
-    dt = _dtype_code(query_states)
-    if query_states.numel() != B * N * hd:
-        raise RuntimeError("polarquant_amd: decode attention takes one query token per sequence, not %s" % (tuple(query_states.shape),))
-    q = query_states
-    if not q.is_contiguous() or q.data_ptr() % 16:
-        q = q.reshape(B, N, hd).clone(memory_format=torch.contiguous_format)
-    assert value_states.is_contiguous() and value_states.dtype == query_states.dtype
-    v_cap = value_states.shape[2]
-    if indices is not None:
-        assert indices.is_contiguous() and all(m.is_contiguous() for m in (rscale, rmn, tscale, tmn))
-        g_cap = indices.shape[2]
-        cptr = [indices.data_ptr(), rscale.data_ptr(), rmn.data_ptr(), tscale.data_ptr(), tmn.data_ptr()]
-        flags = _ffi.PQ_CODES_PACKED6 if indices.shape[-1] == 48 else 0      # [.., 128, 48]: packed 6-bit codes
+    plain = _calls.plain_cache(query_states, indices, rscale, rmn, tscale, tmn, key_resid, value_states, None, None, None, attention_mask)
+    if plain is not None:                    # nothing to check or to copy
+        B, N, Nk, g_cap, r_cap, v_cap, packed, dt, mstride = plain
+        q, cptr, m8, hd, flags = query_states, (indices, rscale, rmn, tscale, tmn), attention_mask, 128, _ffi.PQ_CODES_PACKED6 if packed else 0
+        if indices is None:
+            cptr = (None,) * 5
     else:
-        g_cap, cptr, flags = 0, [None] * 5, 0
-    if key_resid is not None:
-        assert key_resid.is_contiguous() and key_resid.dtype == query_states.dtype
-        r_cap, kptr = key_resid.shape[2], key_resid.data_ptr()
-    else:
-        r_cap, kptr = 0, None
-    mptr, mstride = None, 0
-    if attention_mask is not None:
-        m8 = attention_mask if attention_mask.dtype == torch.uint8 else (attention_mask != 0).to(torch.uint8)
-        m8 = m8.contiguous()
-        mptr, mstride = m8.data_ptr(), m8.stride(0)
+        B, N = query_states.shape[:2]
+        hd = query_states.shape[-1]
+        Nk = value_states.shape[1]
+        assert hd == 128
+        dt = _dtype_code(query_states)
+        if query_states.numel() != B * N * hd:
+            raise RuntimeError("polarquant_amd: decode attention takes one query token per sequence, not %s" % (tuple(query_states.shape),))
+        q = query_states
+        if not q.is_contiguous() or q.data_ptr() % 16:
+            q = q.reshape(B, N, hd).clone(memory_format=torch.contiguous_format)
+        assert value_states.is_contiguous() and value_states.dtype == query_states.dtype
+        v_cap = value_states.shape[2]
+        if indices is not None:
+            assert indices.is_contiguous() and all(m.is_contiguous() for m in (rscale, rmn, tscale, tmn))
+            g_cap = indices.shape[2]
+            cptr = (indices, rscale, rmn, tscale, tmn)
+            flags = _ffi.PQ_CODES_PACKED6 if indices.shape[-1] == 48 else 0      # [.., 128, 48]: packed 6-bit codes
+        else:
+            g_cap, cptr, flags = 0, (None,) * 5, 0
+        r_cap = 0
+        if key_resid is not None:
+            assert key_resid.is_contiguous() and key_resid.dtype == query_states.dtype
+            r_cap = key_resid.shape[2]
+        m8, mstride = None, 0
+        if attention_mask is not None:
+            m8 = attention_mask if attention_mask.dtype == torch.uint8 else (attention_mask != 0).to(torch.uint8)
+            m8 = m8.contiguous()
+            mstride = m8.stride(0)
     if sm_scale is None:
         sm_scale = 1.0 / math.sqrt(hd)
     max_groups = g_cap if n_groups_per_seq is not None else n_groups
@@ -177,19 +183,15 @@ def polar_decode_attention(
             n_splits = _window_slot(n_splits, max_groups, n_resid if n_resid_per_seq is None else r_cap, B, N, Nk, tbits, workspace)
     ws = _pick_workspace(workspace, B, N, n_splits, dev)
     if out is None:
-        out = torch.empty((B, N, 1, hd), dtype=query_states.dtype, device=dev)
-    gps = n_groups_per_seq.data_ptr() if n_groups_per_seq is not None else None
-    rps = n_resid_per_seq.data_ptr() if n_resid_per_seq is not None else None
-    sptr = None
+        out = _calls.empty(query_states, 0, B, N, 1, hd)
     if status is not None:
         if status.dtype != torch.int32 or status.device != dev or status.numel() != 1:
             raise ValueError("polarquant_amd: status must be one int32 on %s" % dev)
-        sptr = status.data_ptr()
     with _on_device(dev):
-        rc = _ffi.lib().pq_decode_attn(
-            q.data_ptr(), *cptr, g_cap, n_groups, gps, kptr, r_cap, n_resid, rps,
-            value_states.data_ptr(), v_cap, mptr, mstride, float(sm_scale), B, N, Nk, rbits, tbits, dt,
-            n_splits, min_gps, ws.data_ptr(), ws.numel() * 4, out.data_ptr(), flags, sptr, _stream_ptr(dev))
+        rc = _ffi.lib().call.pq_decode_attn(
+            q, *cptr, g_cap, n_groups, n_groups_per_seq, key_resid, r_cap, n_resid, n_resid_per_seq, value_states, v_cap, m8, mstride,
+            float(sm_scale), B, N, Nk, rbits, tbits, dt,
+            n_splits, min_gps, ws, ws.numel() * 4, out, flags, status, _stream_ptr(dev))
     _ffi.check(rc, "pq_decode_attn")
     return out
 
@@ -216,34 +218,40 @@ def polar_decode_attention_v4(
     if not query_states.is_cuda:
         raise RuntimeError("polarquant_amd: decode attention needs tensors on the GPU (no CPU fallback)")
     dev = query_states.device
-    B, N = query_states.shape[:2]
-    hd = query_states.shape[-1]
-    Nk = key_resid.shape[1]
-    assert hd == 128
-    dt = _dtype_code(query_states)
-    if query_states.numel() != B * N * hd:
-        raise RuntimeError("polarquant_amd: decode attention takes one query token per sequence, not %s" % (tuple(query_states.shape),))
-    q = query_states
-    if not q.is_contiguous() or q.data_ptr() % 16:
-        q = q.reshape(B, N, hd).clone(memory_format=torch.contiguous_format)
-    assert key_resid.is_contiguous() and value_resid.is_contiguous() and key_resid.shape == value_resid.shape
-    assert key_resid.dtype == query_states.dtype == value_resid.dtype
-    r_cap = key_resid.shape[2]
-    if indices is not None:
-        assert indices.is_contiguous() and all(m.is_contiguous() for m in (rscale, rmn, tscale, tmn))
-        assert value_codes is not None and value_codes.is_contiguous() and value_codes.dtype == torch.int32
-        assert value_scale.is_contiguous() and value_mn.is_contiguous() and value_scale.dtype == query_states.dtype
-        g_cap, v4_cap = indices.shape[2], value_codes.shape[2]
-        cptr = [indices.data_ptr(), rscale.data_ptr(), rmn.data_ptr(), tscale.data_ptr(), tmn.data_ptr()]
-        vptr = [value_codes.data_ptr(), value_scale.data_ptr(), value_mn.data_ptr()]
-        flags = _ffi.PQ_CODES_PACKED6 if indices.shape[-1] == 48 else 0
+    plain = _calls.plain_cache(query_states, indices, rscale, rmn, tscale, tmn, key_resid, value_resid, value_codes, value_scale, value_mn,
+                               attention_mask)
+    if plain is not None and indices is not None and value_codes is not None:         # nothing to check or to copy
+        B, N, Nk, g_cap, r_cap, v4_cap, packed, dt, mstride = plain
+        q, cptr, vptr, m8, hd = query_states, (indices, rscale, rmn, tscale, tmn), (value_codes, value_scale, value_mn), attention_mask, 128
+        flags = _ffi.PQ_CODES_PACKED6 if packed else 0
     else:
-        g_cap, v4_cap, cptr, vptr, flags = 0, 0, [None] * 5, [None] * 3, 0
-    mptr, mstride = None, 0
-    if attention_mask is not None:
-        m8 = attention_mask if attention_mask.dtype == torch.uint8 else (attention_mask != 0).to(torch.uint8)
-        m8 = m8.contiguous()
-        mptr, mstride = m8.data_ptr(), m8.stride(0)
+        B, N = query_states.shape[:2]
+        hd = query_states.shape[-1]
+        Nk = key_resid.shape[1]
+        assert hd == 128
+        dt = _dtype_code(query_states)
+        if query_states.numel() != B * N * hd:
+            raise RuntimeError("polarquant_amd: decode attention takes one query token per sequence, not %s" % (tuple(query_states.shape),))
+        q = query_states
+        if not q.is_contiguous() or q.data_ptr() % 16:
+            q = q.reshape(B, N, hd).clone(memory_format=torch.contiguous_format)
+        assert key_resid.is_contiguous() and value_resid.is_contiguous() and key_resid.shape == value_resid.shape
+        assert key_resid.dtype == query_states.dtype == value_resid.dtype
+        r_cap = key_resid.shape[2]
+        if indices is not None:
+            assert indices.is_contiguous() and all(m.is_contiguous() for m in (rscale, rmn, tscale, tmn))
+            assert value_codes is not None and value_codes.is_contiguous() and value_codes.dtype == torch.int32
+            assert value_scale.is_contiguous() and value_mn.is_contiguous() and value_scale.dtype == query_states.dtype
+            g_cap, v4_cap = indices.shape[2], value_codes.shape[2]
+            cptr, vptr = (indices, rscale, rmn, tscale, tmn), (value_codes, value_scale, value_mn)
+            flags = _ffi.PQ_CODES_PACKED6 if indices.shape[-1] == 48 else 0
+        else:
+            g_cap, v4_cap, cptr, vptr, flags = 0, 0, (None,) * 5, (None,) * 3, 0
+        m8, mstride = None, 0
+        if attention_mask is not None:
+            m8 = attention_mask if attention_mask.dtype == torch.uint8 else (attention_mask != 0).to(torch.uint8)
+            m8 = m8.contiguous()
+            mstride = m8.stride(0)
     if sm_scale is None:
         sm_scale = 1.0 / math.sqrt(hd)
     max_groups = g_cap if n_groups_per_seq is not None else n_groups
@@ -254,24 +262,20 @@ def polar_decode_attention_v4(
         if n_splits is None:
             n_splits = balanced_slots(B, Nk, max_groups, total_groups, (8 if N // Nk <= 4 else 4) * _num_cus(dev), r_cap)
     if n_splits is None:
-        n_splits = _ffi.lib().pq_decode_attn_v4_plan(B, N, Nk, max(max_groups, 1), _num_cus(dev))
+        n_splits = _ffi.lib().call.pq_decode_attn_v4_plan(B, N, Nk, max(max_groups, 1), _num_cus(dev))
         if not single_wavefront and min_groups_per_split <= 1:
             n_splits = _window_slot(n_splits, max_groups, n_resid if n_resid_per_seq is None else r_cap, B, N, Nk, tbits, workspace)
-    sptr = None
     if status is not None:
         if status.dtype != torch.int32 or status.device != dev or status.numel() != 1:
             raise ValueError("polarquant_amd: status must be one int32 on %s" % dev)
-        sptr = status.data_ptr()
     ws = _pick_workspace(workspace, B, N, n_splits, dev)
     if out is None:
-        out = torch.empty((B, N, 1, hd), dtype=query_states.dtype, device=dev)
-    gps = n_groups_per_seq.data_ptr() if n_groups_per_seq is not None else None
-    rps = n_resid_per_seq.data_ptr() if n_resid_per_seq is not None else None
+        out = _calls.empty(query_states, 0, B, N, 1, hd)
     with _on_device(dev):
-        rc = _ffi.lib().pq_decode_attn_v4(
-            q.data_ptr(), *cptr, g_cap, n_groups, gps, key_resid.data_ptr(), r_cap, n_resid, rps,
-            value_resid.data_ptr(), *vptr, v4_cap, mptr, mstride, float(sm_scale), B, N, Nk, rbits, tbits, dt,
-            n_splits, min_groups_per_split, ws.data_ptr(), ws.numel() * 4, out.data_ptr(), flags, sptr, _stream_ptr(dev))
+        rc = _ffi.lib().call.pq_decode_attn_v4(
+            q, *cptr, g_cap, n_groups, n_groups_per_seq, key_resid, r_cap, n_resid, n_resid_per_seq, value_resid, *vptr, v4_cap, m8, mstride,
+            float(sm_scale), B, N, Nk, rbits, tbits, dt,
+            n_splits, min_groups_per_split, ws, ws.numel() * 4, out, flags, status, _stream_ptr(dev))
     _ffi.check(rc, "pq_decode_attn_v4")
     return out
 
@@ -293,10 +297,9 @@ def prompt_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sm_scale
         raise ValueError("polarquant_amd: prompt attention takes half-precision [B, heads, L, 128] tensors on one GPU, strides multiples of 8")
     B, N, L, _ = q.shape
     out = torch.empty((B, L, N, 128), dtype=q.dtype, device=q.device)
-    strides = (ctypes.c_int64 * 9)(*q.stride()[:3], *k.stride()[:3], *v.stride()[:3])
     with _on_device(q.device):
-        rc = _ffi.lib().pq_prompt_attn(q.data_ptr(), k.data_ptr(), v.data_ptr(), ctypes.cast(strides, ctypes.c_void_p), out.data_ptr(),
-                                       float(sm_scale if sm_scale is not None else 1.0 / math.sqrt(128)), B, L, N, k.shape[1], _dtype_code(q),
-                                       _stream_ptr(q.device))
+        rc = _ffi.lib().call.pq_prompt_attn(q, k, v, q.stride()[:3] + k.stride()[:3] + v.stride()[:3], out,
+                                            float(sm_scale if sm_scale is not None else 1.0 / math.sqrt(128)), B, L, N, k.shape[1], _dtype_code(q),
+                                            _stream_ptr(q.device))
     _ffi.check(rc, "pq_prompt_attn")
     return out

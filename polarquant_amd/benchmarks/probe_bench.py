@@ -51,11 +51,7 @@ def _direct_bins(args):
     # the same keys through the shipping library, loaded beside whichever one is being timed
     import ctypes
     timed = _ffi.lib()
-    ship = ctypes.CDLL(SHIPPING_LIB)
-    for name, (res, argtypes) in _ffi.SIGNATURES.items():
-        fn = getattr(ship, name)
-        fn.restype, fn.argtypes = res, argtypes
-    _ffi._LOADED[_ffi.LIB_PATH] = ship
+    _ffi._LOADED[_ffi.LIB_PATH] = _ffi.declare(ctypes.CDLL(SHIPPING_LIB), _ffi.SIGNATURES)
     same = quantize_and_pack_nbit(keys[0], sh.rbits, sh.tbits)[0]
     _ffi._LOADED[_ffi.LIB_PATH] = timed
     torch.cuda.synchronize()

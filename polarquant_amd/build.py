@@ -2,6 +2,7 @@
 
     python -m polarquant_amd.build                    # (re)build polarquant_amd/libpolarquant_hip.so, its test build and libpolarquant_bench.so
     python -m polarquant_amd.build --layers [steps] [latent] [recurrent]   # those libraries alone
+    python -m polarquant_amd.build --calls            # the builtins through which the wrappers call them (_calls.so) alone
     python -m polarquant_amd.build --phase-timers     # the measuring build (benchmarks/phase_timing.py)
     python -m polarquant_amd.build --probe no_values  # a probe build (benchmarks/probe_bench.py)
 
@@ -42,6 +43,9 @@ LAYER_LIBS = {name: os.path.join(HERE, "libpolarquant_%s.so" % name) for name in
 # their own, loaded by bench.py and its tests only
 BENCH_LIB = os.path.join(HERE, "libpolarquant_bench.so")
 BENCH_SOURCES = ["pq_stream.hip"]
+# the C ABI's functions as CPython builtins: host code against torch's headers, no GPU code
+CALLS_LIB = os.path.join(HERE, "_calls.so")
+CALLS_SOURCE = "pq_calls.cpp"
 ARCH = "gfx950"
 FLAGS = ["--offload-arch=" + ARCH, "-O3", "-fPIC", "-std=c++17", "-ffp-contract=off",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wall", "-Wno-unused-function"]
@@ -74,6 +78,24 @@ def _compile(src: str, defines=(), tag: str = "") -> str:
     if err.strip():
         sys.stderr.write(err + "\n")
     return obj
+
+
+def build_calls() -> str:
+    import sysconfig
+    import torch
+    root = os.path.dirname(torch.__file__)
+    include = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"), sysconfig.get_paths()["include"]]
+    tmp = CALLS_LIB + ".tmp"
+    cmd = ([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+            "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI] + ["-isystem" + d for d in include]
+           + [os.path.join(CSRC, CALLS_SOURCE), "-o", tmp, "-L" + os.path.join(root, "lib"), "-lc10", "-ltorch_cpu", "-ltorch_python"])
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("%s failed for %s:\n%s" % (cmd[0], CALLS_SOURCE, r.stderr))
+    if r.stderr.strip():
+        sys.stderr.write(r.stderr)
+    os.replace(tmp, CALLS_LIB)
+    return CALLS_LIB
 
 
 def _link(objs, lib: str) -> None:
@@ -126,6 +148,8 @@ def ensure(libraries, verbose: bool = True) -> None:
     """Build those of the named LIBRARIES that are not there, and nothing else."""
     if "hip" in libraries and not os.path.exists(LIB):
         build(verbose)
+    if not os.path.exists(CALLS_LIB):
+        build_calls()
     missing = [n for n in libraries if n in LAYER_LIBS and not os.path.exists(LAYER_LIBS[n])]
     if missing:
         build_layers(missing, verbose)
@@ -146,7 +170,9 @@ def build(verbose: bool = True, phase_timers: bool = False) -> str:
         jobs = main + [u for u in hooks if u not in main] + [u for us in LAYER_UNITS.values() for u in us] + bench
     # the units are listed longest compilation first
     with ThreadPoolExecutor(max_workers=min(8, len(jobs))) as ex:
+        calls = ex.submit(build_calls)
         built = dict(zip(jobs, ex.map(lambda j: _compile(*j), jobs)))
+        calls.result()
     lib = TIMERS_LIB if phase_timers else LIB
     _link([built[u] for u in main], lib)
     if not phase_timers:
@@ -157,6 +183,7 @@ def build(verbose: bool = True, phase_timers: bool = False) -> str:
         if verbose:
             for path in LAYER_LIBS.values():
                 print("built", path)
+            print("built", CALLS_LIB)
             print("built", HOOKS_LIB)
             print("built", BENCH_LIB)
     if verbose:
@@ -167,6 +194,8 @@ def build(verbose: bool = True, phase_timers: bool = False) -> str:
 if __name__ == "__main__":
     if "--probe" in sys.argv[1:]:
         build_probe(sys.argv[sys.argv.index("--probe") + 1])
+    elif "--calls" in sys.argv[1:]:
+        print("built", build_calls())
     elif "--layers" in sys.argv[1:]:
         build_layers(sys.argv[sys.argv.index("--layers") + 1:] or tuple(LAYER_UNITS))
     else:

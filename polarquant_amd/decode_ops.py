@@ -34,11 +34,9 @@ def rope_append(q_lin: torch.Tensor, k_lin: torch.Tensor, v_lin: torch.Tensor, c
     assert k_dst.shape[:2] == (B, n_kv_heads) == v_dst.shape[:2] and k_dst.shape[3] == 128 == v_dst.shape[3]
     q_out = torch.empty((B, n_heads, 1, 128), dtype=q_lin.dtype, device=q_lin.device)
     with _on_device(q_lin.device):
-        rc = _ffi.lib().pq_rope_append(q_lin.data_ptr(), k_lin.data_ptr(), v_lin.data_ptr(), cos_table.data_ptr(),
-                                       sin_table.data_ptr(), cos_table.shape[0], pos.data_ptr(), q_out.data_ptr(),
-                                       k_dst.data_ptr(), k_dst.shape[2], k_row.data_ptr(), v_dst.data_ptr(), v_dst.shape[2],
-                                       v_row.data_ptr(), B, n_heads, n_kv_heads, _dtype_code(q_lin),
-                                       q_lin.stride(0), k_lin.stride(0), _stream_ptr(q_lin.device))
+        rc = _ffi.lib().call.pq_rope_append(q_lin, k_lin, v_lin, cos_table, sin_table, cos_table.shape[0], pos, q_out, k_dst, k_dst.shape[2], k_row,
+                                            v_dst, v_dst.shape[2], v_row, B, n_heads, n_kv_heads, _dtype_code(q_lin),
+                                            q_lin.stride(0), k_lin.stride(0), _stream_ptr(q_lin.device))
     _ffi.check(rc, "pq_rope_append")
     return q_out
 
@@ -56,9 +54,8 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, residual: Optiona
         assert sum_out.is_contiguous() and sum_out.shape == x.shape and sum_out.dtype == x.dtype
     y = torch.empty_like(x)
     with _on_device(x.device):
-        rc = _ffi.lib().pq_rmsnorm(x.data_ptr(), None if residual is None else residual.data_ptr(), weight.data_ptr(),
-                                   y.data_ptr(), None if sum_out is None else sum_out.data_ptr(), x.numel() // hidden, hidden,
-                                   float(eps), _dtype_code(x), _stream_ptr(x.device))
+        rc = _ffi.lib().call.pq_rmsnorm(x, residual, weight, y, sum_out, x.numel() // hidden, hidden, float(eps), _dtype_code(x),
+                                        _stream_ptr(x.device))
     _ffi.check(rc, "pq_rmsnorm")
     return y
 
@@ -79,7 +76,7 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     with _on_device(gate.device):
         for r0 in range(0, rows, 65535):          # one launch covers at most 65535 rows (a prompt has more)
             n = min(65535, rows - r0)
-            rc = _ffi.lib().pq_silu_mul(gate.data_ptr() + r0 * stride * esz, up.data_ptr() + r0 * stride * esz,
+            rc = _ffi.lib().call.pq_silu_mul(gate.data_ptr() + r0 * stride * esz, up.data_ptr() + r0 * stride * esz,
                                         y.data_ptr() + r0 * cols * esz, n, cols, stride, _dtype_code(gate),
                                         _stream_ptr(gate.device))
             _ffi.check(rc, "pq_silu_mul")
@@ -103,10 +100,8 @@ def linear_small_m(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
         assert bias.is_contiguous() and bias.numel() == N and bias.dtype == x.dtype
     y = torch.empty(x.shape[:-1] + (N,), dtype=x.dtype, device=x.device)
     with _on_device(x.device):
-        rc = _ffi.lib().pq_linear_small_m(x2.data_ptr(), x2.stride(0) if M > 1 else K, weight.data_ptr(),
-                                          None if up_weight is None else up_weight.data_ptr(),
-                                          None if bias is None else bias.data_ptr(), y.data_ptr(), N, M, N, K,
-                                          _dtype_code(x), _stream_ptr(x.device))
+        rc = _ffi.lib().call.pq_linear_small_m(x2, x2.stride(0) if M > 1 else K, weight, up_weight, bias, y, N, M, N, K, _dtype_code(x),
+                                               _stream_ptr(x.device))
     _ffi.check(rc, "pq_linear_small_m")
     return y
 
@@ -128,12 +123,9 @@ def qkv_rope_append(x: torch.Tensor, w_qkv: torch.Tensor, b_qkv: Optional[torch.
     assert k_dst.shape[:2] == (B, n_kv_heads) == v_dst.shape[:2] and k_dst.shape[3] == 128 == v_dst.shape[3]
     q_out = torch.empty((B, n_heads, 1, 128), dtype=x.dtype, device=x.device)
     with _on_device(x.device):
-        rc = _ffi.lib().pq_qkv_rope_append(x2.data_ptr(), x2.stride(0) if B > 1 else K, w_qkv.data_ptr(),
-                                           None if b_qkv is None else b_qkv.data_ptr(), B, K, _dtype_code(x),
-                                           cos_table.data_ptr(), sin_table.data_ptr(), cos_table.shape[0], pos.data_ptr(),
-                                           q_out.data_ptr(), k_dst.data_ptr(), k_dst.shape[2], k_row.data_ptr(),
-                                           v_dst.data_ptr(), v_dst.shape[2], v_row.data_ptr(), n_heads, n_kv_heads,
-                                           _stream_ptr(x.device))
+        rc = _ffi.lib().call.pq_qkv_rope_append(x2, x2.stride(0) if B > 1 else K, w_qkv, b_qkv, B, K, _dtype_code(x), cos_table, sin_table,
+                                                cos_table.shape[0], pos, q_out, k_dst, k_dst.shape[2], k_row, v_dst, v_dst.shape[2], v_row,
+                                                n_heads, n_kv_heads, _stream_ptr(x.device))
     _ffi.check(rc, "pq_qkv_rope_append")
     return q_out
 
@@ -161,8 +153,7 @@ def rope_qk(q_lin: torch.Tensor, k_lin: torch.Tensor, cos: torch.Tensor, sin: to
     q_out = torch.empty((B, L, n_heads, 128), dtype=q_lin.dtype, device=q_lin.device)
     k_out = torch.empty((B, L, n_kv_heads, 128), dtype=q_lin.dtype, device=q_lin.device)
     with _on_device(q_lin.device):
-        rc = _ffi.lib().pq_rope_qk(q_lin.data_ptr(), qs, k_lin.data_ptr(), ks, cos.data_ptr(), sin.data_ptr(),
-                                   0 if cos.shape[0] == 1 else L * 128, q_out.data_ptr(), k_out.data_ptr(), B, L, n_heads,
-                                   n_kv_heads, _dtype_code(q_lin), _stream_ptr(q_lin.device))
+        rc = _ffi.lib().call.pq_rope_qk(q_lin, qs, k_lin, ks, cos, sin, 0 if cos.shape[0] == 1 else L * 128, q_out, k_out, B, L, n_heads,
+                                        n_kv_heads, _dtype_code(q_lin), _stream_ptr(q_lin.device))
     _ffi.check(rc, "pq_rope_qk")
     return q_out.transpose(1, 2), k_out.transpose(1, 2)

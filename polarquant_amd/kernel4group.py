@@ -12,6 +12,7 @@ import contextlib
 import torch
 
 from . import _ffi
+from ._ffi import calls as _calls
 
 
 def _dtype_code(t: torch.Tensor) -> int:
@@ -47,6 +48,15 @@ def attention_decode_forward_hip_impl(
 ) -> torch.Tensor:
     if not query_states.is_cuda:
         raise RuntimeError("polarquant_amd: decode scores need tensors on the GPU (no CPU fallback)")
+    plain = _calls.plain_scores(query_states, indices, rscale, rmn, tscale, tmn)
+    if plain is not None:               # nothing to check or to copy: the common call, whose host side this is
+        B, N, Nk, Nb, packed, dt = plain
+        out = _calls.empty(query_states, 3, B, N, 1, Nb * 128)
+        with _on_device(query_states.device):
+            rc = _ffi.lib().call.pq_decode_scores(query_states, indices, rscale, rmn, tscale, tmn, out, B, N, Nk, Nb, rbits, tbits, dt,
+                                                  _ffi.PQ_CODES_PACKED6 if packed else 0, _stream_ptr(query_states.device))
+        _ffi.check(rc, "pq_decode_scores")
+        return out
     B, Nk, Nb, G, D = indices.shape
     N = query_states.shape[1]
     # last dim 64: one byte per pair code (the reference's layout); 48: packed 6-bit codes
@@ -65,8 +75,7 @@ def attention_decode_forward_hip_impl(
     meta = [m.contiguous() for m in meta]
     out = torch.empty((B, N, 1, Nb * G), device=q.device, dtype=torch.float32)
     with _on_device(q.device):
-        rc = _ffi.lib().pq_decode_scores(q.data_ptr(), indices.data_ptr(), *[m.data_ptr() for m in meta],
-                                         out.data_ptr(), B, N, Nk, Nb, rbits, tbits, dt, flags, _stream_ptr(q.device))
+        rc = _ffi.lib().call.pq_decode_scores(q, indices, *meta, out, B, N, Nk, Nb, rbits, tbits, dt, flags, _stream_ptr(q.device))
     _ffi.check(rc, "pq_decode_scores")
     return out
 

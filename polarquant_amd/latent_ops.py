@@ -10,7 +10,7 @@ from . import _ffi
 from .attention import _num_cus
 from .kernel4group import _on_device, _stream_ptr
 
-from .layer_ops import (_DTYPES, _code, _ptr, ConvState, IN_PLACE_TOKENS, SMALL_M, head_linear, linear, linear_f32,  # noqa: F401
+from .layer_ops import (_DTYPES, _code, ConvState, IN_PLACE_TOKENS, SMALL_M, head_linear, linear, linear_f32,  # noqa: F401
                         norm_conv, relu_sq, streams)
 
 
@@ -25,15 +25,15 @@ def latent_norm(p: torch.Tensor, w_q: torch.Tensor, w_kv: Optional[torch.Tensor]
     qr = w_q.numel()
     out = torch.empty(B, L, qr, dtype=p.dtype, device=p.device)
     with _on_device(p.device):
-        rc = _ffi.latent_lib().pq_latent_norm(_ptr(p), ld, _ptr(w_q), _ptr(w_kv), _ptr(out), _ptr(cache) if w_kv is not None else None,
-                                              cache.shape[1] if w_kv is not None else 0, _ptr(pos_dev), pos, B, L, qr,
+        rc = _ffi.latent_lib().call.pq_latent_norm(p, ld, w_q, w_kv, out, cache if w_kv is not None else None,
+                                              cache.shape[1] if w_kv is not None else 0, pos_dev, pos, B, L, qr,
                                               w_kv.numel() if w_kv is not None else 1, float(eps), dt, _stream_ptr(p.device))
     _ffi.check(rc, "pq_latent_norm")
     return out
 
 
 def decode_splits(B: int, L: int, H: int, max_keys: int, device) -> int:
-    return _ffi.latent_lib().pq_latent_decode_plan(B, L, H, max_keys, _num_cus(device))
+    return _ffi.latent_lib().call.pq_latent_decode_plan(B, L, H, max_keys, _num_cus(device))
 
 
 def latent_decode_attention(q: torch.Tensor, cache: torch.Tensor, sink: torch.Tensor, scale: float, pos: int,
@@ -49,19 +49,19 @@ def latent_decode_attention(q: torch.Tensor, cache: torch.Tensor, sink: torch.Te
     if n_splits is None:
         assert pos_dev is None
         n_splits = decode_splits(B, L, H, pos + L, q.device)
-    lib = _ffi.latent_lib()
+    lib = _ffi.latent_lib().call
     nbytes = lib.pq_latent_decode_workspace_bytes(B, L, H, R, n_splits)
     ws = torch.empty(nbytes // 4, dtype=torch.float32, device=q.device) if dt != _ffi.PQ_F32 else None
     out = torch.empty_like(q)
     with _on_device(q.device):
-        rc = lib.pq_latent_decode(_ptr(q), _ptr(cache), cache.shape[1], _ptr(sink), _ptr(start), _ptr(pos_dev), pos, _ptr(out), B, L, H,
-                                  R, float(scale), n_splits, _ptr(ws), nbytes if ws is not None else 0, dt, _stream_ptr(q.device))
+        rc = lib.pq_latent_decode(q, cache, cache.shape[1], sink, start, pos_dev, pos, out, B, L, H,
+                                  R, float(scale), n_splits, ws, nbytes if ws is not None else 0, dt, _stream_ptr(q.device))
     _ffi.check(rc, "pq_latent_decode")
     return out
 
 
 def prefill_takes(dim: int, vdim: int, dtype: torch.dtype) -> bool:
-    return bool(_ffi.latent_lib().pq_latent_prefill_takes(dim, vdim, _DTYPES[dtype]))
+    return bool(_ffi.latent_lib().call.pq_latent_prefill_takes(dim, vdim, _DTYPES[dtype]))
 
 
 def latent_prefill_attention(q: torch.Tensor, k: torch.Tensor, vt: torch.Tensor, sink: torch.Tensor, scale: float,
@@ -79,7 +79,7 @@ def latent_prefill_attention(q: torch.Tensor, k: torch.Tensor, vt: torch.Tensor,
             gate = gate.contiguous()
     out = torch.empty(B, L, H * Dv, dtype=q.dtype, device=q.device)
     with _on_device(q.device):
-        rc = _ffi.latent_lib().pq_latent_prefill(_ptr(q), _ptr(k), _ptr(vt), ld, _ptr(sink), _ptr(gate), 0 if gate is None else gate.stride(0),
-                                                 _ptr(start), _ptr(out), B, L, Lk, H, D, Dv, float(scale), dt, _stream_ptr(q.device))
+        rc = _ffi.latent_lib().call.pq_latent_prefill(q, k, vt, ld, sink, gate, 0 if gate is None else gate.stride(0),
+                                                 start, out, B, L, Lk, H, D, Dv, float(scale), dt, _stream_ptr(q.device))
     _ffi.check(rc, "pq_latent_prefill")
     return out

@@ -21,10 +21,6 @@ def _code(t: torch.Tensor) -> int:
     return _DTYPES[t.dtype]
 
 
-def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else t.data_ptr()
-
-
 class ConvState:
     """Inputs of a causal convolution that later tokens still need: float32 [B, taps - 1, width], oldest first.  A call of
     many tokens writes the other of two buffers (its first workgroup reads what its last one writes)."""
@@ -70,9 +66,9 @@ def norm_conv(x: torch.Tensor, w_pre: torch.Tensor, groups: int, eps: float, y: 
         assert s_in.shape == (B, taps - 1, W)
     h = torch.empty(B, L, W, dtype=w_pre.dtype, device=x.device)
     with _on_device(x.device):
-        rc = _ffi.steps_lib().pq_norm_conv(
-            _ptr(x), _ptr(y), _ptr(w_post) if y is not None else None, _ptr(x_out), _ptr(w_pre), _ptr(conv_w),
-            _ptr(s_in) if taps > 1 else None, _ptr(s_out) if taps > 1 else None, _ptr(h), _ptr(start), _ptr(pos_dev), pos, B, L, W,
+        rc = _ffi.steps_lib().call.pq_norm_conv(
+            x, y, w_post if y is not None else None, x_out, w_pre, conv_w,
+            s_in if taps > 1 else None, s_out if taps > 1 else None, h, start, pos_dev, pos, B, L, W,
             groups, taps, float(eps), dt, _stream_ptr(x.device))
     _ffi.check(rc, "pq_norm_conv")
     return (x if y is None else x_out), h
@@ -83,7 +79,7 @@ def relu_sq(x: torch.Tensor) -> torch.Tensor:
     dt = _code(x)
     assert x.is_contiguous()
     with _on_device(x.device):
-        rc = _ffi.steps_lib().pq_relu_sq(_ptr(x), _ptr(x), x.numel(), dt, _stream_ptr(x.device))
+        rc = _ffi.steps_lib().call.pq_relu_sq(x, x, x.numel(), dt, _stream_ptr(x.device))
     _ffi.check(rc, "pq_relu_sq")
     return x
 
@@ -96,7 +92,7 @@ def gelu_mul(gate: torch.Tensor, up: torch.Tensor, out: Optional[torch.Tensor] =
     assert up.shape == out.shape == (M, N) and gate.stride() == up.stride() and gate.stride(1) == out.stride(1) == 1
     assert up.dtype == out.dtype == gate.dtype
     with _on_device(gate.device):
-        rc = _ffi.steps_lib().pq_gelu_mul(_ptr(gate), _ptr(up), gate.stride(0), _ptr(out), out.stride(0), M, N, dt, _stream_ptr(gate.device))
+        rc = _ffi.steps_lib().call.pq_gelu_mul(gate, up, gate.stride(0), out, out.stride(0), M, N, dt, _stream_ptr(gate.device))
     _ffi.check(rc, "pq_gelu_mul")
     return out
 
@@ -114,7 +110,7 @@ def stream_add(x: torch.Tensor, y: Optional[torch.Tensor] = None, e: Optional[to
     _code(x)
     out = torch.empty_like(x)
     with _on_device(x.device):
-        rc = _ffi.steps_lib().pq_stream_add(_ptr(x), _ptr(y), _ptr(e), _ptr(v), _ptr(out), x.numel() // W, W, _DTYPES[dtype], _stream_ptr(x.device))
+        rc = _ffi.steps_lib().call.pq_stream_add(x, y, e, v, out, x.numel() // W, W, _DTYPES[dtype], _stream_ptr(x.device))
     _ffi.check(rc, "pq_stream_add")
     return out
 
@@ -126,7 +122,7 @@ def embed_rows(table: torch.Tensor, ids: torch.Tensor, scale: float = 1.0) -> to
     assert table.is_contiguous() and ids.dtype == torch.int64 and ids.is_cuda
     out = torch.empty(tuple(ids.shape) + (table.shape[1],), dtype=torch.float32, device=table.device)
     with _on_device(table.device):
-        rc = _ffi.steps_lib().pq_embed_rows(_ptr(table), _ptr(ids), float(scale), _ptr(out), ids.numel(), table.shape[1], table.shape[0], dt,
+        rc = _ffi.steps_lib().call.pq_embed_rows(table, ids, float(scale), out, ids.numel(), table.shape[1], table.shape[0], dt,
                                             _stream_ptr(table.device))
     _ffi.check(rc, "pq_embed_rows")
     return out
@@ -137,7 +133,7 @@ def softcap(x: torch.Tensor, scale: float, cap: Optional[float]) -> torch.Tensor
     _code(x)
     assert x.is_contiguous() and x.dtype == torch.float32
     with _on_device(x.device):
-        rc = _ffi.steps_lib().pq_softcap(_ptr(x), x.numel(), float(scale), float(cap or 0.0), _stream_ptr(x.device))
+        rc = _ffi.steps_lib().call.pq_softcap(x, x.numel(), float(scale), float(cap or 0.0), _stream_ptr(x.device))
     _ffi.check(rc, "pq_softcap")
     return x
 
@@ -156,9 +152,9 @@ def head_linear(x: torch.Tensor, w: torch.Tensor, gate: Optional[torch.Tensor] =
     rows = SMALL_M if (dt != _ffi.PQ_F32 and N % 16 == 0 and K % 32 == 0) else 65535
     with _on_device(x.device):
         for m in range(0, M, rows):
-            xs, ys, gs = x[m:m + rows], y[m:m + rows], None if gate is None else gate[m:m + rows]
-            rc = _ffi.steps_lib().pq_head_linear(_ptr(xs), x.stride(0), x.stride(1), _ptr(w), _ptr(gs), 0 if gate is None else gate.stride(0),
-                                                  _ptr(ys), H * N, N, xs.shape[0], H, N, K, epilogue, dt, _stream_ptr(x.device))
+            xs, ys, gs = (x, y, gate) if M <= rows else (x[m:m + rows], y[m:m + rows], None if gate is None else gate[m:m + rows])
+            rc = _ffi.steps_lib().call.pq_head_linear(xs, x.stride(0), x.stride(1), w, gs, 0 if gate is None else gate.stride(0),
+                                                  ys, H * N, N, xs.shape[0], H, N, K, epilogue, dt, _stream_ptr(x.device))
             _ffi.check(rc, "pq_head_linear")
     return y
 

@@ -31,6 +31,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 from torch.utils._device import DeviceContext
 
+from ._ffi import calls as _calls
 from .attention import polar_decode_attention, polar_decode_attention_v4, prompt_attention, prompt_attention_takes
 from .quantize import quantize_and_pack_nbit
 from .values import quantize_values
@@ -178,6 +179,10 @@ def _nobody_looks_on(*ts) -> bool:
     subclasses."""
     if torch.is_grad_enabled() or torch.compiler.is_compiling():
         return False
+    return bool(_calls.plain_eager(*ts)) or _looked_at_closely(*ts)
+
+
+def _looked_at_closely(*ts) -> bool:
     functions = torch._C._len_torch_function_stack()
     return (torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
             and torch._C._get_tracing_state() is None and not torch.is_autocast_enabled("cuda") and torch._C._len_torch_dispatch_stack() == 0
@@ -189,7 +194,10 @@ def _on_gpu_in_half(*ts) -> bool:
     """Whether the fused launches can take these tensors as they lie: nobody who follows torch's operations (asked before anything else:
     a symbolic trace has no dtype to compare, a dynamic size no value), one half-precision dtype, one GPU, contiguous, 16-byte
     aligned, not empty."""
-    return _nobody_looks_on(*ts) and _lie_in_half(*ts)
+    if torch.is_grad_enabled() or torch.compiler.is_compiling():
+        return False
+    plain = _calls.plain_half(*ts)
+    return plain if plain is not None else _looked_at_closely(*ts) and _lie_in_half(*ts)
 
 
 def _lie_in_half(*ts) -> bool:

@@ -2,12 +2,12 @@
 (reference: models/modeling_llama_polar.py:135-157)."""
 from __future__ import annotations
 
-import ctypes
 from typing import Optional, Tuple
 
 import torch
 
 from . import _ffi
+from ._ffi import calls as _calls
 from .kernel4group import _dtype_code, _on_device, _stream_ptr
 
 GROUP = 128
@@ -43,30 +43,36 @@ def quantize_and_pack_nbit(key_states: torch.Tensor, rbits: int = 4, tbits: int 
     row = 48 if packed else PAIRS
     if not key_states.is_cuda:
         raise RuntimeError("polarquant_amd: the quantizer needs tensors on the GPU (no CPU fallback)")
-    B, Nk, L, D2 = key_states.shape
-    assert D2 == 2 * PAIRS and group_size == GROUP, "head_dim 128 and group size 128 only"
+    plain = _calls.plain_rows(key_states, 4, 8)
+    if plain is not None:
+        B, Nk, L, strides, dt = plain
+        assert group_size == GROUP, "head_dim 128 and group size 128 only"
+    else:
+        B, Nk, L, D2 = key_states.shape
+        assert D2 == 2 * PAIRS and group_size == GROUP, "head_dim 128 and group size 128 only"
     assert L % GROUP == 0 and rbits + tbits <= 8
     Nb = L // GROUP
-    dt = _dtype_code(key_states)
-    if key_states.stride(3) != 1 or any(s % 4 for s in key_states.stride()[:3]) or key_states.data_ptr() % 8:
-        key_states = key_states.contiguous()
+    if plain is None:
+        dt = _dtype_code(key_states)
+        if key_states.stride(3) != 1 or any(s % 4 for s in key_states.stride()[:3]) or key_states.data_ptr() % 8:
+            key_states = key_states.contiguous()
+        strides = key_states.stride()
     dev = key_states.device
     if out is None:
-        codes = torch.empty((B, Nk, Nb, GROUP, row), dtype=torch.uint8, device=dev)
-        meta = [torch.empty((B, Nk, Nb, 1, PAIRS), dtype=key_states.dtype, device=dev) for _ in range(4)]
+        codes = _calls.empty(key_states, 1, B, Nk, Nb, GROUP, row)
+        meta = [_calls.empty(key_states, 0, B, Nk, Nb, 1, PAIRS) for _ in range(4)]
         cap, off = Nb, 0
     else:
         codes, meta = out[0], list(out[1:])
         cap, off = codes.shape[2], group_offset
         assert codes.is_contiguous() and all(m.is_contiguous() for m in meta) and codes.shape[-1] == row
-    strides = (ctypes.c_int64 * 4)(*key_states.stride())
     with _on_device(dev):
-        rc = _ffi.lib().pq_quantize_groups(key_states.data_ptr(), ctypes.cast(strides, ctypes.c_void_p), dt, B, Nk, Nb,
+        rc = _ffi.lib().call.pq_quantize_groups(key_states, strides, dt, B, Nk, Nb,
                                            rbits, tbits, (_ffi.PQ_WRAP_FP32 if wrap_fp32 or eager_gpu else 0)
                                            | (_ffi.PQ_DEVICE_ATAN2 if device_atan2 or eager_gpu else 0)
                                            | (_ffi.PQ_ANGLE_UNIFORM if angle_mode == "uniform" else 0)
                                            | (_ffi.PQ_CODES_PACKED6 if packed else 0),
-                                           codes.data_ptr(), *[m.data_ptr() for m in meta], cap, off,
+                                           codes, *meta, cap, off,
                                            _stream_ptr(dev))
     _ffi.check(rc, "pq_quantize_groups")
     if out is None:
@@ -84,6 +90,6 @@ def convert_codes6(indices: torch.Tensor, pack: bool) -> torch.Tensor:
     src = indices.contiguous()
     dst = torch.empty(src.shape[:-1] + (dst_row,), dtype=torch.uint8, device=src.device)
     with _on_device(src.device):
-        rc = _ffi.lib().pq_convert_codes6(src.data_ptr(), dst.data_ptr(), src.numel() // src_row, int(pack), _stream_ptr(src.device))
+        rc = _ffi.lib().call.pq_convert_codes6(src.data_ptr(), dst.data_ptr(), src.numel() // src_row, int(pack), _stream_ptr(src.device))
     _ffi.check(rc, "pq_convert_codes6")
     return dst

@@ -11,7 +11,7 @@ import torch
 from . import _ffi
 from .attention import _num_cus
 from .kernel4group import _on_device, _stream_ptr
-from .layer_ops import _DTYPES, ConvState, _code, _ptr
+from .layer_ops import _DTYPES, ConvState, _code
 
 WINDOW_SMALL = 16          # new tokens per sequence up to which keys go to the ring before they are read
 MAX_DIM = 256              # of a recurrent head
@@ -61,8 +61,8 @@ def qk_norm(q, k, v, w_q, w_k, heads: int, eps: float, ring: WindowRing, step: S
     assert w_q.numel() == heads * D and w_k.numel() == G * D and w_q.dtype == w_k.dtype == q.dtype and w_q.is_contiguous() and w_k.is_contiguous()
     q_out = torch.empty(M, heads * D, dtype=q.dtype, device=q.device)
     k_out = None if step.L <= WINDOW_SMALL else torch.empty(M, G * D, dtype=q.dtype, device=q.device)
-    _run(_ffi.recurrent_lib().pq_qk_norm, "pq_qk_norm", q.device, _ptr(q), _ptr(k), _ptr(v), q.stride(0), _ptr(w_q), _ptr(w_k), _ptr(q_out),
-         _ptr(k_out), _ptr(ring.k), _ptr(ring.v), _ptr(step.pos_dev), step.pos, B, step.L, heads, G, D, Dv, cap, float(eps), dt)
+    _run(_ffi.recurrent_lib().call.pq_qk_norm, "pq_qk_norm", q.device, q, k, v, q.stride(0), w_q, w_k, q_out,
+         k_out, ring.k, ring.v, step.pos_dev, step.pos, B, step.L, heads, G, D, Dv, cap, float(eps), dt)
     return q_out, k_out
 
 
@@ -83,7 +83,7 @@ def window_attention(q, ring: WindowRing, slopes: Optional[torch.Tensor], scale:
         _rows(v_new, M, G * Dv, q.dtype)
     else:
         assert step.L <= WINDOW_SMALL
-    lib = _ffi.recurrent_lib()
+    lib = _ffi.recurrent_lib().call
     if k_new is not None:
         n_splits = 1
     elif n_splits is None:
@@ -91,11 +91,11 @@ def window_attention(q, ring: WindowRing, slopes: Optional[torch.Tensor], scale:
     nbytes = lib.pq_window_workspace_bytes(B, step.L, H, Dv, n_splits)
     ws = torch.empty(nbytes // 4, dtype=torch.float32, device=q.device) if nbytes else None
     kr, vr = (0, 0) if k_new is None else (k_new.stride(0), v_new.stride(0))
-    _run(lib.pq_window_attn, "pq_window_attn", q.device, _ptr(q), _ptr(ring.k), _ptr(ring.v), _ptr(k_new), kr, _ptr(v_new), vr, _ptr(slopes),
-         _ptr(step.start), _ptr(step.pos_dev), step.pos, _ptr(out), out.stride(0), B, step.L, H, G, D, Dv, cap, ring.window, float(scale),
-         float(out_scale), n_splits, _ptr(ws), nbytes, dt)
+    _run(lib.pq_window_attn, "pq_window_attn", q.device, q, ring.k, ring.v, k_new, kr, v_new, vr, slopes,
+         step.start, step.pos_dev, step.pos, out, out.stride(0), B, step.L, H, G, D, Dv, cap, ring.window, float(scale),
+         float(out_scale), n_splits, ws, nbytes, dt)
     if k_new is not None:
-        _run(lib.pq_ring_append, "pq_ring_append", q.device, _ptr(k_new), kr, _ptr(v_new), vr, _ptr(ring.k), _ptr(ring.v), step.pos, B, step.L,
+        _run(lib.pq_ring_append, "pq_ring_append", q.device, k_new, kr, v_new, vr, ring.k, ring.v, step.pos, B, step.L,
              G, D, Dv, cap, dt)
     return out
 
@@ -104,7 +104,7 @@ def window_attention(q, ring: WindowRing, slopes: Optional[torch.Tensor], scale:
 def _scan_workspace(delta: bool, dtype: torch.dtype, step: Step, heads: int, dim: int, device) -> Optional[torch.Tensor]:
     if dtype == torch.float32 or step.L < CHUNKED_TOKENS or step.pos_dev is not None:
         return None
-    need = lambda tokens: _ffi.recurrent_lib().pq_scan_workspace_bytes(int(delta), step.B, heads, dim, tokens, _DTYPES[dtype])
+    need = lambda tokens: _ffi.recurrent_lib().call.pq_scan_workspace_bytes(int(delta), step.B, heads, dim, tokens, _DTYPES[dtype])
     return torch.empty(min(need(step.L), max(WORKSPACE_BYTES, need(1))), dtype=torch.uint8, device=device)
 
 
@@ -137,9 +137,9 @@ def delta_prep(q, k, v, b, a, w_q, w_k, w_v, A_log, dt_bias, conv: ConvState, di
     r = DeltaInputs(e(G * dim, q.dtype), e(G * dim, q.dtype), e(H * vdim, q.dtype), e(G, torch.float32), e(G, torch.float32),
                     e(H * dim, torch.float32), e(H, torch.float32))
     has = taps > 1
-    _run(_ffi.recurrent_lib().pq_delta_prep, "pq_delta_prep", dev, _ptr(q), _ptr(k), _ptr(v), _ptr(b), q.stride(0), _ptr(a), a.stride(0), _ptr(w_q),
-         _ptr(w_k), _ptr(w_v), _ptr(A_log), _ptr(dt_bias), _ptr(s_in) if has else None, _ptr(s_out) if has else None, _ptr(r.q), _ptr(r.k),
-         _ptr(r.v), _ptr(r.q_inv), _ptr(r.k_inv), _ptr(r.log_g), _ptr(r.beta), _ptr(step.start), _ptr(step.pos_dev), step.pos, step.B, step.L, G, H,
+    _run(_ffi.recurrent_lib().call.pq_delta_prep, "pq_delta_prep", dev, q, k, v, b, q.stride(0), a, a.stride(0), w_q,
+         w_k, w_v, A_log, dt_bias, s_in if has else None, s_out if has else None, r.q, r.k,
+         r.v, r.q_inv, r.k_inv, r.log_g, r.beta, step.start, step.pos_dev, step.pos, step.B, step.L, G, H,
          dim, vdim, taps, dt)
     return r
 
@@ -152,9 +152,9 @@ def delta_scan(x: DeltaInputs, state: torch.Tensor, step: Step) -> torch.Tensor:
     assert all(t.is_contiguous() for t in x) and x.log_g.shape == (M, H * dim) and x.beta.shape == (M, H)
     o = torch.empty(M, H * vdim, dtype=torch.float32, device=state.device)
     ws = _scan_workspace(True, x.q.dtype, step, H, dim, state.device)
-    _run(_ffi.recurrent_lib().pq_delta_scan, "pq_delta_scan", state.device, _ptr(x.q), _ptr(x.k), _ptr(x.v), _ptr(x.q_inv), _ptr(x.k_inv),
-         _ptr(x.log_g), _ptr(x.beta), _ptr(state), _ptr(o), _ptr(step.start), _ptr(step.pos_dev), step.pos, B, step.L, G, H, dim, vdim,
-         _ptr(ws), 0 if ws is None else ws.numel(), dt)
+    _run(_ffi.recurrent_lib().call.pq_delta_scan, "pq_delta_scan", state.device, x.q, x.k, x.v, x.q_inv, x.k_inv,
+         x.log_g, x.beta, state, o, step.start, step.pos_dev, step.pos, B, step.L, G, H, dim, vdim,
+         ws, 0 if ws is None else ws.numel(), dt)
     return o
 
 
@@ -167,7 +167,7 @@ def memory_gates(i, f, b_i, b_f, cap: float):
     _rows(f, M, H, i.dtype)
     assert i.stride(0) == f.stride(0) and b_i.numel() == b_f.numel() == H and b_i.dtype == b_f.dtype == i.dtype
     li, lf = [torch.empty(M, H, dtype=torch.float32, device=i.device) for _ in range(2)]
-    _run(_ffi.recurrent_lib().pq_memory_gates, "pq_memory_gates", i.device, _ptr(i), _ptr(f), i.stride(0), _ptr(b_i), _ptr(b_f), _ptr(li), _ptr(lf),
+    _run(_ffi.recurrent_lib().call.pq_memory_gates, "pq_memory_gates", i.device, i, f, i.stride(0), b_i, b_f, li, lf,
          M, H, float(cap), dt)
     return li, lf
 
@@ -192,9 +192,9 @@ def memory_scan(q, k, v, log_i, log_f, state: torch.Tensor, m: torch.Tensor, q_s
     o = torch.empty(M, H * vdim, dtype=torch.float32, device=q.device)
     den = torch.empty(M, H, dtype=torch.float32, device=q.device)
     ws = _scan_workspace(False, q.dtype, step, H, dim, q.device)
-    _run(_ffi.recurrent_lib().pq_memory_scan, "pq_memory_scan", q.device, _ptr(q), _ptr(k), _ptr(v), q.stride(0), _ptr(log_i), _ptr(log_f),
-         _ptr(state), _ptr(m), _ptr(o), _ptr(den), float(q_scale), _ptr(step.start), _ptr(step.pos_dev), step.pos, B, step.L, H, dim, vdim,
-         _ptr(ws), 0 if ws is None else ws.numel(), dt)
+    _run(_ffi.recurrent_lib().call.pq_memory_scan, "pq_memory_scan", q.device, q, k, v, q.stride(0), log_i, log_f,
+         state, m, o, den, float(q_scale), step.start, step.pos_dev, step.pos, B, step.L, H, dim, vdim,
+         ws, 0 if ws is None else ws.numel(), dt)
     return o, den
 
 
@@ -208,6 +208,6 @@ def head_norm_gate(o: torch.Tensor, w: torch.Tensor, gate: torch.Tensor, heads: 
     _rows(out, M, n, gate.dtype)
     assert o.is_contiguous() and o.dtype == torch.float32 and w.numel() in (vdim, n) and w.is_contiguous() and w.dtype == gate.dtype
     assert den is None or (den.is_contiguous() and den.dtype == torch.float32 and den.shape == (M, heads))
-    _run(_ffi.recurrent_lib().pq_head_norm_gate, "pq_head_norm_gate", o.device, _ptr(o), _ptr(den), _ptr(w), 0 if w.numel() == vdim else vdim,
-         _ptr(gate), gate.stride(0), _ptr(out), out.stride(0), M, heads, vdim, float(eps), float(out_scale), dt)
+    _run(_ffi.recurrent_lib().call.pq_head_norm_gate, "pq_head_norm_gate", o.device, o, den, w, 0 if w.numel() == vdim else vdim,
+         gate, gate.stride(0), out, out.stride(0), M, heads, vdim, float(eps), float(out_scale), dt)
     return out

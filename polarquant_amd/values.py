@@ -3,12 +3,12 @@
 LlamaPolarMixedGroupAttention (reference: models/modeling_llama_polar.py:236,275)."""
 from __future__ import annotations
 
-import ctypes
 from typing import Optional, Tuple
 
 import torch
 
 from . import _ffi
+from ._ffi import calls as _calls
 from .kernel4group import _dtype_code, _on_device, _stream_ptr
 
 HEAD_DIM = 128
@@ -24,25 +24,28 @@ def quantize_values(value_states: torch.Tensor, group_size: int = HEAD_DIM, bits
     cache tensors that receive the T rows at token index `token_offset`."""
     if not value_states.is_cuda:
         raise RuntimeError("polarquant_amd: the value quantizer needs tensors on the GPU (no CPU fallback)")
-    B, Nk, T, D = value_states.shape
-    assert D == HEAD_DIM and group_size == HEAD_DIM and bits == 4, "head_dim 128, one group per row, 4 bits only"
-    dt = _dtype_code(value_states)
-    if value_states.stride(3) != 1 or any(s % 8 for s in value_states.stride()[:3]) or value_states.data_ptr() % 16:
-        value_states = value_states.contiguous()
+    plain = _calls.plain_rows(value_states, 8, 16)
+    if plain is not None and group_size == HEAD_DIM and bits == 4:
+        B, Nk, T, strides, dt = plain
+    else:
+        B, Nk, T, D = value_states.shape
+        assert D == HEAD_DIM and group_size == HEAD_DIM and bits == 4, "head_dim 128, one group per row, 4 bits only"
+        dt = _dtype_code(value_states)
+        if value_states.stride(3) != 1 or any(s % 8 for s in value_states.stride()[:3]) or value_states.data_ptr() % 16:
+            value_states = value_states.contiguous()
+        strides = value_states.stride()
     dev = value_states.device
     if out is None:
-        code = torch.empty((B, Nk, T, WORDS), dtype=torch.int32, device=dev)
-        scale = torch.empty((B, Nk, T, 1), dtype=value_states.dtype, device=dev)
-        mn = torch.empty((B, Nk, T, 1), dtype=value_states.dtype, device=dev)
+        code = _calls.empty(value_states, 2, B, Nk, T, WORDS)
+        scale, mn = [_calls.empty(value_states, 0, B, Nk, T, 1) for _ in range(2)]
         cap, off = T, 0
     else:
         code, scale, mn = out
         cap, off = code.shape[2], token_offset
         assert code.is_contiguous() and scale.is_contiguous() and mn.is_contiguous() and code.dtype == torch.int32
-    strides = (ctypes.c_int64 * 4)(*value_states.stride())
     with _on_device(dev):
-        rc = _ffi.lib().pq_quantize_values(value_states.data_ptr(), ctypes.cast(strides, ctypes.c_void_p), dt, B, Nk, T,
-                                           code.data_ptr(), scale.data_ptr(), mn.data_ptr(), cap, off, _stream_ptr(dev))
+        rc = _ffi.lib().call.pq_quantize_values(value_states, strides, dt, B, Nk, T, code, scale, mn, cap, off,
+                                                _stream_ptr(dev))
     _ffi.check(rc, "pq_quantize_values")
     if out is None:
         return code, scale, mn

@@ -1,0 +1,64 @@
+"""The C ABI's functions as builtins (csrc/pq_calls.cpp): the same answers as through ctypes, and questions that are answered only for
+tensors as they should lie."""
+import ctypes
+
+import pytest
+import torch
+
+from polarquant_amd import _ffi
+from polarquant_amd._ffi import calls
+
+
+@pytest.mark.parametrize("args", [(1, 8, 100, 256), (16, 8, 1, 256), (0, 0, 0, 0), (-1, 8, 100, 256), ((1 << 32) + 1, 8, 100, 256), (True, 8, 2 ** 40, 256)])
+def test_the_same_integers_as_through_ctypes(args):
+    lib = _ffi.lib()
+    assert lib.call.pq_decode_attn_plan(*args) == lib.pq_decode_attn_plan(*args)
+    assert lib.call.pq_decode_attn_workspace_bytes(*args[:3]) == lib.pq_decode_attn_workspace_bytes(*args[:3])
+
+
+@pytest.mark.parametrize("pointer", [None, 0, 16, 17])
+def test_the_same_refusals_as_through_ctypes(pointer):
+    lib = _ffi.lib()
+    args = [pointer] + [None] * 6 + [1, 8, 8, 4, 4, 4, 0, 0, None]                  # (a null pointer among them: never launched)
+    assert lib.call.pq_decode_scores(*args) == lib.pq_decode_scores(*args) != 0
+    strides = (128, 128, 128, 2)                                                    # no unit stride
+    args = [16, strides, 0, 1, 1, 1, 4, 4, 0] + [16] * 5 + [1, 0, None]
+    assert lib.call.pq_quantize_groups(*args) == lib.pq_quantize_groups(args[0], ctypes.cast((ctypes.c_int64 * 4)(*strides), ctypes.c_void_p), *args[2:])
+
+
+def test_wrong_arguments_raise():
+    call = _ffi.lib().call
+    with pytest.raises(TypeError):
+        call.pq_decode_attn_plan(1, 2, 3)
+    for wrong in ("8", 1.5, None):
+        with pytest.raises(ctypes.ArgumentError):
+            call.pq_decode_attn_plan(1, wrong, 3, 4)
+    with pytest.raises(ctypes.ArgumentError):
+        call.pq_decode_scores("q", *[None] * 6, 1, 8, 8, 4, 4, 4, 0, 0, None)
+
+
+def test_tensors_that_are_not_plain_are_left_to_the_general_path():
+    q, codes, meta = torch.zeros(1, 8, 1, 128, dtype=torch.float16), torch.zeros(1, 8, 2, 128, 64, dtype=torch.uint8), torch.zeros(1, 8, 2, 1, 64, dtype=torch.float16)
+    assert calls.plain_scores(q, codes, meta, meta, meta, meta) is None             # (not on a GPU)
+    assert calls.plain_cache(q, codes, meta, meta, meta, meta, None, q, None, None, None, None) is None
+    assert calls.plain_rows(q, 4, 8) is None and calls.plain_rows(None, 4, 8) is None
+    with torch.no_grad():
+        assert calls.plain_half(q) is False and calls.plain_eager(q) is True
+        assert calls.plain_eager(torch.nn.Parameter(q)) is True and calls.plain_eager(q.as_subclass(type("Sub", (torch.Tensor,), {}))) is None
+        with torch.device("cpu"):
+            assert calls.plain_eager(q) is None                                     # (a mode: looked at more closely)
+        with torch.autograd.forward_ad.dual_level():
+            assert calls.plain_eager(q) is None
+        seen = []
+        torch.func.vmap(lambda t: (t, seen.append(calls.plain_half(t)))[0])(q)
+        assert seen == [None]
+    assert calls.plain_eager(q) is None                                             # (gradients are on)
+
+
+def test_empty():
+    like = torch.zeros(1, dtype=torch.bfloat16)
+    for code, dtype in ((0, torch.bfloat16), (1, torch.uint8), (2, torch.int32), (3, torch.float32)):
+        t = calls.empty(like, code, 2, 0, 3)
+        assert t.shape == (2, 0, 3) and t.dtype == dtype and t.device == like.device and t.is_contiguous()
+    with pytest.raises(RuntimeError):
+        calls.empty(like, 0, -1)
