@@ -210,13 +210,14 @@ __global__ __launch_bounds__(kWave * kGroupWaves, 4) void attn_group_kernel(PQ_A
             static_for<16>([&](auto D) {
                 constexpr int d = decltype(D)::value, c = d >> 2, i = d & 3;
                 const uint32_t theta = ((cw[c] & tmask) >> (8 * i)) & 0xFFu, rho = (((cw[c] >> tbits) & rmask) >> (8 * i)) & 0xFFu;
-                float e[REPP];
+                float e[L::WORDS];
                 const uint32_t at = base + d * L::PB + ((theta ^ d) << L::SH);
                 lds_load_w<L::W0>(at, e);
                 if constexpr (L::W1 > 0) lds_load_w<L::W1>(at + L::HB, e + 4);
                 const float r = static_cast<float>(rho) + cds[d];
 #pragma unroll
                 for (int j = 0; j < REPP; j++) s[j] = __builtin_fmaf(e[j], r, s[j]);
+                keep_spare_word<REPP>(e);
                 if constexpr ((d & 3) == 3) __builtin_amdgcn_sched_barrier(0);     // (four codes' entries in registers at a time)
             });
 #pragma unroll

@@ -101,6 +101,7 @@ struct Lut {
     static constexpr int NB = 1 << TB;
     static constexpr int W0 = REPP < 4 ? REPP : 4;        // heads in the first half's entries
     static constexpr int W1 = REPP - W0;                  // heads in the second half's entries (0: no second half)
+    static constexpr int WORDS = REPP % 4 == 3 ? REPP + 1 : REPP;     // registers of a lookup: three heads come as four words
     static constexpr int HALVES = W1 > 0 ? 2 : 1;
     static constexpr int EB = REPP == 1 ? 4 : (REPP == 2 ? 8 : 16);   // entry stride in bytes
     static constexpr int SH = REPP == 1 ? 2 : (REPP == 2 ? 3 : 4);
@@ -137,7 +138,8 @@ __device__ __forceinline__ uint32_t lds_addr(void* p) {
 // W (1..4) consecutive floats of a table entry at LDS byte address `addr`, as one ds_read / ds_write of that width.
 // Three floats move as four (entries are 16 bytes apart, the fourth word belongs to nobody): a 96-bit LDS access
 // keeps the LDS busy longer than a 128-bit one (measured at 7 heads per KV head, 3-bit angles, ragged batch of 64:
-// SQ_LDS_IDX_ACTIVE 22.1 M with ds_read_b96 against 18.7 M with two ds_read_b128 for the same lookups).
+// SQ_LDS_IDX_ACTIVE 22.1 M with ds_read_b96 against 18.7 M with two ds_read_b128 for the same lookups).  `e` has room
+// for the fourth word.
 template <int W>
 __device__ __forceinline__ void lds_load_w(uint32_t addr, float* e) {
     if constexpr (W == 1) {
@@ -146,8 +148,8 @@ __device__ __forceinline__ void lds_load_w(uint32_t addr, float* e) {
         const lds_e2* p = lds_ptr<lds_e2>(addr);
         e[0] = p->x; e[1] = p->y;
     } else if constexpr (W == 3) {
-        const float4_v v = *lds_ptr<const lds_f4>(addr);           // one 128-bit access; the fourth word is not used
-        e[0] = v.x; e[1] = v.y; e[2] = v.z;
+        const float4_v v = *lds_ptr<const lds_f4>(addr);           // one 128-bit access; the fourth word belongs to no head
+        e[0] = v.x; e[1] = v.y; e[2] = v.z; e[3] = v.w;
     } else {
         const lds_e4* p = lds_ptr<lds_e4>(addr);
         e[0] = p->x; e[1] = p->y; e[2] = p->z; e[3] = p->w;
@@ -167,6 +169,15 @@ __device__ __forceinline__ void lds_store_w(uint32_t addr, const float* e) {
         lds_e4* p = lds_ptr<lds_e4>(addr);
         p->x = e[0]; p->y = e[1]; p->z = e[2]; p->w = e[3];
     }
+}
+
+// The word of no head (three heads move as four words) stays live until its lookup has been consumed.  If it is dead at birth
+// the compiler gives its register to the address or radius arithmetic of the same batch while the read is still under way,
+// which costs a wait for every read in flight per code word.  A tile of 64 tokens, four scorers on a unit: 7 heads, 3-bit
+// angles 2.19 -> 1.83 us, 4-bit 2.03 -> 1.71 (8 heads: 1.72); 3 heads 1.25 -> 1.09.
+template <int REPP, int WORDS>
+__device__ __forceinline__ void keep_spare_word(const float (&e)[WORDS]) {
+    if constexpr (WORDS > REPP) asm volatile("" :: "v"(e[REPP]));
 }
 
 // sin and cos of a bin-centre angle.  Three-constant Cody-Waite reduction by
@@ -245,7 +256,7 @@ __device__ __forceinline__ void score_token(uint32_t lut, const uint32_t (&codes
     constexpr int nbm = L::NB - 1;
     constexpr int BW = REPP >= 4 ? 1 : 2;      // code words per batch
     constexpr int NBATCH = 16 / BW;
-    float e[2][BW * 4][REPP];
+    float e[2][BW * 4][L::WORDS];
     uint32_t r4s[2][BW];
 
     auto load = [&](auto BI) {
@@ -289,6 +300,7 @@ __device__ __forceinline__ void score_token(uint32_t lut, const uint32_t (&codes
                     constexpr int j = decltype(JJ)::value;
                     acc[j] = __builtin_fmaf(e[buf][cc * 4 + i][j], t, acc[j]);
                 });
+                keep_spare_word<REPP>(e[buf][cc * 4 + i]);
             });
         });
     };
