@@ -13,10 +13,13 @@
 // Arithmetic follows eager torch on half tensors op by op: every reference op
 // is evaluated in fp32 and rounded to the key dtype before the next.
 //
-// What bounds it: the vector unit, about 65 instructions a pair of which two at a quarter of the rate (111 of the 125 to 131 us that
-// 131072 tokens of 8 heads take; their bytes need 68).  With the codes' quotients by three operations and rounded by conversions,
-// the angle's sign put on and taken off again and a test of each pair's range it was 143 to 155 us.  Gathering a workgroup's entries
-// for the exact routines so that one wavefront does them all: 128 instead of 131 us at best, short calls slower; not kept.
+// What bounds it: the vector unit, about 50 instructions a pair of which two at a quarter of the rate (96 of the 98 us that 131072
+// tokens of 8 heads take with the device library's arctangent as the exact routine, 106 with SLEEF's, whose double-float sequence a
+// wavefront runs once or twice; their bytes need 68).  It was 65 instructions and 119 us with the angle from the smaller over the
+// larger operand (a comparison, two selections and a second turn more), each code converted and bounded by itself, and scales by IEEE
+// divisions; keys requested two rows at a time and words read from LDS for each pass cost 8 us of it.
+// Gathering a workgroup's entries for the exact routines so that one wavefront does them all: 128 instead of 131 us at best, short
+// calls slower; not kept.
 #include "pq_device.h"
 #include "pq_internal.h"
 #include "pq_math.h"
@@ -34,8 +37,8 @@ __device__ __forceinline__ float rnd(float f) { return lo2f<T>(f2lo<T>(f)); }
 // ---- angle and radius of one pair, rounded to the key dtype -------------------
 // Eager torch gives round_dtype(atan2f_sleef(y, x)) and round_dtype(sqrt_rn(x*x + y*y)).
 // The exact routines cost ~100 instructions per pair, so a cheap estimate is tried
-// first: a 3.5-ulp arctangent (reciprocal, degree-8 polynomial in r^2, quadrant
-// fix-up; it stays within 4 ulp of the exact routine) and the hardware square
+// first: an arctangent of the half angle (reciprocal, polynomial of degree 7 or 6 in
+// its square; half stays within 5 ulp of the exact routine, bfloat16 within 12) and the hardware square
 // root (1 ulp).  Rounding the estimate to the key dtype gives the same word as
 // rounding the exact value unless the estimate lies within its error bound of a
 // rounding boundary of the dtype (a midpoint between two neighbouring dtype
@@ -49,17 +52,17 @@ template <typename T> struct DT;
 template <> struct DT<F16> { static constexpr uint32_t kMid = 0x1000u; static constexpr int kHighBits = 19; static constexpr float kMinNormal = 6.103515625e-05f; };
 template <> struct DT<BF16> { static constexpr uint32_t kMid = 0x8000u; static constexpr int kHighBits = 16; static constexpr float kMinNormal = 1.17549435e-38f; };
 
-constexpr uint32_t kAtanGuardUlps = 5;   // the fast arctangent stays within 4 ulp of the exact routine (exhaustive self-test)
-constexpr uint32_t kSqrtGuardUlps = 2;   // v_sqrt_f32 is within 1 ulp
+// An estimate further than its largest error from a midpoint rounds like the exact value.
+constexpr uint32_t kSqrtGuardUlps = 1;   // v_sqrt_f32
 
 // Which arctangent the angle must reproduce.  Eager torch evaluates atan2 on half tensors in fp32 and
 // rounds once: on the CPU with SLEEF's Sleef_atan2f_u10 (restated in pq_math.h), on the GPU with the
 // device math library's atan2f, which is what `atan2f` in device code here resolves to as well.  The
 // two differ in the last fp32 bits on about a third of all operands, and after rounding to half on a
-// few dozen per million.  LIBM = true selects the device library's routine as the exact one; it lies
-// within 3 ulp of SLEEF's on every operand pair seen, so the estimate's guard band is widened by that
-// (the exhaustive self-test checks the wider band against the library routine itself).
-template <bool LIBM> struct Atan { static constexpr uint32_t kGuardUlps = LIBM ? kAtanGuardUlps + 4 : kAtanGuardUlps; };
+// few dozen per million.  LIBM = true selects the device library's routine as the exact one (the
+// exhaustive self-test checks each guard band against its routine).  The bands are the estimate's largest
+// distance from the routine over every pair of operands.
+template <typename T, bool LIBM> struct Atan { static constexpr uint32_t kGuardUlps = (IsHalf<T>::value ? 5 : 12) + (LIBM ? 1 : 0); };
 template <bool LIBM>
 __device__ __forceinline__ float atan2_exact(float y, float x) {
     if constexpr (LIBM) return atan2f(y, x);
@@ -73,22 +76,32 @@ __device__ __forceinline__ bool near_rounding_boundary(float a, uint32_t guard) 
     return low < (2u * guard + 1u) << DT<T>::kHighBits;
 }
 
-// the angle's magnitude
-__device__ __forceinline__ float atan2_fast_abs(float y, float x) {
-    const float ax = fabsf(x), ay = fabsf(y);
-    const float mx = ay > ax ? ay : ax, mn = ay > ax ? ax : ay;
-    const float r = mn * __builtin_amdgcn_rcpf(mx);
-    const float s = r * r;
-    float u = 0.00282363896258175373077393f;
-    u = __builtin_fmaf(u, s, -0.0159569028764963150024414f);
-    u = __builtin_fmaf(u, s, 0.0425049886107444763183594f);
-    u = __builtin_fmaf(u, s, -0.0748900920152664184570312f);
-    u = __builtin_fmaf(u, s, 0.106347933411598205566406f);
-    u = __builtin_fmaf(u, s, -0.142027363181114196777344f);
-    u = __builtin_fmaf(u, s, 0.199926957488059997558594f);
-    u = __builtin_fmaf(u, s, -0.333331018686294555664062f);
-    float a = __builtin_fmaf(u * s, r, r);
-    a = ay > ax ? 1.57079637050628662109f - a : a;
+// the angle's magnitude, r being the pair's radius: twice the arctangent of |y| / (r + |x|), which is the half angle's tangent and never
+// above 1, so that no larger of the two operands has to be found and only the side of x to be put right.  Polynomials in the tangent's
+// square with the least largest relative error: 1.1e-7 for half, 7.3e-7 for bfloat16.  A coefficient more or less moves it by a factor
+// of 6.6; a wider guard band sends more entries to the exact routines.
+template <typename T>
+__device__ __forceinline__ float atan2_fast_abs(float y, float x, float r) {
+    const float t = fabsf(y) * __builtin_amdgcn_rcpf(fabsf(x) + r);
+    const float s = t * t;
+    float u;
+    if constexpr (IsHalf<T>::value) {
+        u = 2.0f * -0.00482253451f;
+        u = __builtin_fmaf(u, s, 2.0f * 0.0247340649f);
+        u = __builtin_fmaf(u, s, 2.0f * -0.0602031313f);
+        u = __builtin_fmaf(u, s, 2.0f * 0.0996847302f);
+        u = __builtin_fmaf(u, s, 2.0f * -0.140413284f);
+        u = __builtin_fmaf(u, s, 2.0f * 0.199742138f);
+        u = __builtin_fmaf(u, s, 2.0f * -0.333323926f);
+    } else {
+        u = 2.0f * 0.00810636859f;
+        u = __builtin_fmaf(u, s, 2.0f * -0.0377967246f);
+        u = __builtin_fmaf(u, s, 2.0f * 0.0848410428f);
+        u = __builtin_fmaf(u, s, 2.0f * -0.135445759f);
+        u = __builtin_fmaf(u, s, 2.0f * 0.198978737f);
+        u = __builtin_fmaf(u, s, 2.0f * -0.333284914f);
+    }
+    const float a = t * __builtin_fmaf(u, s, 2.0f);
     return x < 0.0f ? 3.14159274101257324219f - a : a;
 }
 
@@ -97,8 +110,8 @@ __device__ __forceinline__ float atan2_fast_abs(float y, float x) {
 template <typename T, bool LIBM = false>
 __device__ __forceinline__ bool angle_radius_fast(float x, float y, float* a_out, float* r_out, float* ss_out) {
     const float ss = __builtin_fmaf(x, x, y * y);          // x*x, y*y are exact for half/bf16 operands
-    const float a = atan2_fast_abs(y, x);
     const float r = __builtin_amdgcn_sqrtf(ss);
+    const float a = atan2_fast_abs<T>(y, x, r);
     // (bfloat16 only) magnitudes at which the reciprocal or the hardware square root leave their accurate range; half's
     // finite squares all lie inside (2^-80, 2^80).  Zeros need no test of their own: with one zero operand the estimate is
     // exactly 0, pi/2 or pi like the exact routine's (0 then fails the kMinNormal test below), and
@@ -110,7 +123,7 @@ __device__ __forceinline__ bool angle_radius_fast(float x, float y, float* a_out
     *r_out = r;
     *ss_out = ss;
     return (special | static_cast<int>(fminf(a, r) < DT<T>::kMinNormal) |
-            static_cast<int>(near_rounding_boundary<T>(a, Atan<LIBM>::kGuardUlps)) |
+            static_cast<int>(near_rounding_boundary<T>(a, Atan<T, LIBM>::kGuardUlps)) |
             static_cast<int>(near_rounding_boundary<T>(r, kSqrtGuardUlps))) != 0;
 }
 // Infinities, NaNs and large bfloat16 magnitudes, of one pair's squares or, as patterns order like the numbers and NaNs lie above
@@ -156,11 +169,10 @@ __device__ __forceinline__ uint32_t code_of(float v, float mn, float scale, floa
 // The same of the rounded distance d >= 0 for scales that fast_div_ok accepts and top <= 127, without a division.
 //
 // Rounding to the dtype carries a quotient to the integer k or over it exactly if half a unit in the last place of its own binade
-// does (an integer up to 128 is even in both dtypes: a tie goes to it), and adding kMid to the fp32 pattern adds that half: no
-// conversion there and back, no floor.  So only the side of B = k - half a unit on which d / scale lies has to be right.  d is a
-// number of 11 bits (bfloat16: 8) and B * scale one of 23 (17), so a quotient below B is below it by 2^-23 (2^-17) of it at least.
-// Half: the inverse in two parts; the product's one rounding then neither reaches B from there nor leaves it.  Bfloat16: an inverse
-// too large by 2^-22 to 2^-20 is enough.  Every pair of operands is checked on the device.  A NaN stays one and converts to 0.
+// does (an integer up to 128 is even in both dtypes: a tie goes to it).  So only the side of B = k - half a unit on which d / scale
+// lies has to be right.  d is a number of 11 bits (bfloat16: 8) and B * scale one of 23 (17), so a quotient below B is below it by
+// 2^-23 (2^-17) of it at least.  Half: the inverse in two parts; the product's one rounding then neither reaches B from there nor
+// leaves it.  Bfloat16: an inverse too large by 2^-22 to 2^-20 is enough.  Every pair of operands is checked on the device.
 struct Inverse { float hi, lo; };
 template <typename T>
 __device__ __forceinline__ Inverse inverse_of(float scale) {
@@ -168,11 +180,48 @@ __device__ __forceinline__ Inverse inverse_of(float scale) {
     if constexpr (IsHalf<T>::value) return {inv, __builtin_fmaf(-scale, inv, 1.0f) * inv};
     else return {__builtin_fmaf(inv, 0x1p-21f, inv), 0.0f};
 }
+// The codes of four pairs: angles in bits tbits - 1 .. 0 of each byte, radii above them.  `add` takes a pair's distances.
+// Half: both quotients are rounded by one conversion, the dtype's own (a multiply-add, half a unit and a conversion to a whole number
+// for each: 3 instructions a pair more).  A NaN converts to 0.
+struct CodeTops { uint32_t both; int tbits; };
+template <typename T> struct CodeWord {
+    uint32_t c[4];                                                                          // angle code | radius code << 16
+    template <int I> __device__ __forceinline__ void add(float da, Inverse ia, float dr, Inverse ir, const CodeTops& top) {
+        // (plus zero: a product whose operand is converted on the way in)
+        const float qa = __builtin_fmaf(da, ia.hi, __builtin_fmaf(da, ia.lo, 0.0f)), qr = __builtin_fmaf(dr, ir.hi, __builtin_fmaf(dr, ir.lo, 0.0f));
+        const ushort2v k = __builtin_convertvector(__builtin_convertvector((float2v{qa, qr}), half2v), ushort2v);
+        c[I] = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(k, __builtin_bit_cast(ushort2v, top.both)));
+    }
+    __device__ __forceinline__ uint32_t word(const CodeTops& top) const {
+        const uint32_t c01 = __builtin_amdgcn_perm(c[1], c[0], 0x06020400u), c23 = __builtin_amdgcn_perm(c[3], c[2], 0x06020400u);
+        return (__builtin_amdgcn_perm(c23, c01, 0x07060302u) << top.tbits) | __builtin_amdgcn_perm(c23, c01, 0x05040100u);
+    }
+    static __device__ __forceinline__ CodeTops tops(int tbits, int rbits) { return {((1u << tbits) - 1u) | (((1u << rbits) - 1u) << 16), tbits}; }
+};
+// Bfloat16: adding kMid to the fp32 pattern adds the half unit; the sum is then scaled to 2^8 and converted to a byte, which saturates,
+// so that the code is its upper bits and needs no bound.  The conversion rounds to nearest: half is taken off first, without error (below
+// 2^8 the difference has the sum's unit), and a tie at a multiple of the code's step goes to it, being even.  A NaN converts to 0.
+struct CodeScales { float t, r; int tshift, rshift; uint32_t tmask, rmask; };
+template <> struct CodeWord<BF16> {
+    uint32_t t, r;                                                                          // bytes: code and fraction
+    template <int I> __device__ __forceinline__ void add(float da, Inverse ia, float dr, Inverse ir, const CodeScales& top) {
+        auto up = [](float q, float scale) { return __builtin_fmaf(__uint_as_float(__float_as_uint(q) + DT<BF16>::kMid), scale, -0.5f); };
+        t = __builtin_amdgcn_cvt_pk_u8_f32(up(da * ia.hi, top.t), I, I == 0 ? 0u : t);
+        r = __builtin_amdgcn_cvt_pk_u8_f32(up(dr * ir.hi, top.r), I, I == 0 ? 0u : r);
+    }
+    __device__ __forceinline__ uint32_t word(const CodeScales& top) const { return ((t >> top.tshift) & top.tmask) | ((r >> top.rshift) & top.rmask); }
+    static __device__ __forceinline__ CodeScales tops(int tbits, int rbits) {
+        return {static_cast<float>(256 >> tbits), static_cast<float>(256 >> rbits), 8 - tbits, 8 - rbits - tbits,
+                0x01010101u * ((1u << tbits) - 1u), 0x01010101u * (((1u << rbits) - 1u) << tbits)};
+    }
+};
+// one code of 2^bits
 template <typename T>
-__device__ __forceinline__ uint32_t code_of_fast(float d, Inverse inv, uint32_t top) {
-    const float q = IsHalf<T>::value ? __builtin_fmaf(d, inv.hi, d * inv.lo) : d * inv.hi;
-    const uint32_t k = static_cast<uint32_t>(__uint_as_float(__float_as_uint(q) + DT<T>::kMid));
-    return k < top ? k : top;
+__device__ __forceinline__ uint32_t code_of_fast(float d, Inverse inv, int bits) {
+    const auto top = CodeWord<T>::tops(bits, 0);
+    CodeWord<T> w{};
+    w.template add<0>(d, inv, 0.0f, inv, top);
+    return w.word(top) & 0xffu;
 }
 // (angle - its minimum | radius - its minimum << 16), each rounded to the dtype.  Half: one packed subtraction (a sum or difference of
 // two halves that is rounded to fp32 first is the same half).
@@ -183,8 +232,10 @@ template <> __device__ __forceinline__ void pair_distance<F16>(uint32_t v, uint3
     *dr = static_cast<float>(d.y);
 }
 template <> __device__ __forceinline__ void pair_distance<BF16>(uint32_t v, uint32_t mn, float* da, float* dr) {
-    *da = rnd<BF16>(__uint_as_float(v << 16) - __uint_as_float(mn << 16));
-    *dr = rnd<BF16>(__uint_as_float(v & 0xffff0000u) - __uint_as_float(mn & 0xffff0000u));
+    const float2v d = {__uint_as_float(v << 16) - __uint_as_float(mn << 16), __uint_as_float(v & 0xffff0000u) - __uint_as_float(mn & 0xffff0000u)};
+    const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(d, bfloat2v));
+    *da = __uint_as_float(w << 16);
+    *dr = __uint_as_float(w & 0xffff0000u);
 }
 __device__ __forceinline__ float clamp_bound(float scale, int top) { return scale > 0.0f ? static_cast<float>(top) : 0.0f; }
 
@@ -224,7 +275,7 @@ template <> struct PkInit<BF16> { static constexpr uint32_t kMax = 0x00000000u, 
 struct AngleMode {
     float two_pi;      // reference mode: the constant added to negative angles
     float tmn, tscale; // uniform mode
-    int ttop;
+    int tbits;
     float minus_one;
 };
 
@@ -236,13 +287,13 @@ __device__ __forceinline__ uint32_t pack_angle_radius(float a, float r, float y,
     uint32_t w;
     const bool below = static_cast<int>(__float_as_uint(y)) < 0;
     if constexpr (UNIFORM) {
-        const uint32_t aw = code_of_fast<T>(rnd<T>(rnd<T>(__builtin_copysignf(a, y)) - am.tmn), inverse_of<T>(am.tscale), am.ttop);
+        const uint32_t aw = code_of_fast<T>(rnd<T>(rnd<T>(__builtin_copysignf(a, y)) - am.tmn), inverse_of<T>(am.tscale), am.tbits);
         w = aw | (static_cast<uint32_t>(f2lo<T>(r)) << 16);
     } else if constexpr (IsHalf<T>::value) {
-        // (times minus one: a subtraction with the conversions of its operand and of its result built in)
+        // (times minus one: a subtraction with its operand's conversion built in; angle and radius are rounded by one conversion)
         const _Float16 phi = static_cast<_Float16>(a);
-        const _Float16 turned = static_cast<_Float16>(__builtin_fmaf(static_cast<float>(phi), am.minus_one, am.two_pi));       // :144
-        w = __builtin_bit_cast(uint32_t, half2v{below && (ESTIMATE || phi > static_cast<_Float16>(0.0f)) ? turned : phi, static_cast<_Float16>(r)});
+        const float turned = __builtin_fmaf(static_cast<float>(phi), am.minus_one, am.two_pi);       // :144
+        w = __builtin_bit_cast(uint32_t, __builtin_convertvector((float2v{below && (ESTIMATE || phi > static_cast<_Float16>(0.0f)) ? turned : a, r}), half2v));
     } else {
         const float phi = rnd<T>(a);
         w = __builtin_bit_cast(uint32_t, __builtin_convertvector((float2v{below && (ESTIMATE || phi > 0.0f) ? am.two_pi - phi : phi, r}), bfloat2v));       // :144
@@ -267,12 +318,19 @@ __global__ __launch_bounds__(kQThreads) void quantize_kernel(
     const uint16_t* kb = k + b * sb + h * sh + static_cast<int64_t>(grp) * kGroup * st;
 
     // ---- pass 1: cheap estimates for every entry; remember which entries need the exact routines
+    // (all of a thread's keys are requested at once: two rows at a time, as the compiler has it, do not cover the way to memory)
     uint32_t risky_mask = 0, ss_most = 0;
+    uint2 xr[kTokPerThread], yr[kTokPerThread];
 #pragma unroll
     for (int it = 0; it < kTokPerThread; it++) {
         const uint16_t* row = kb + (it * 16 + tl) * st;
-        const uint2 xw = *reinterpret_cast<const uint2*>(row + 4 * pq4);
-        const uint2 yw = *reinterpret_cast<const uint2*>(row + kPairs + 4 * pq4);
+        xr[it] = *reinterpret_cast<const uint2*>(row + 4 * pq4);
+        yr[it] = *reinterpret_cast<const uint2*>(row + kPairs + 4 * pq4);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int it = 0; it < kTokPerThread; it++) {
+        const uint2 xw = xr[it], yw = yr[it];
         const uint16_t xs[4] = {static_cast<uint16_t>(xw.x), static_cast<uint16_t>(xw.x >> 16),
                                 static_cast<uint16_t>(xw.y), static_cast<uint16_t>(xw.y >> 16)};
         const uint16_t ys[4] = {static_cast<uint16_t>(yw.x), static_cast<uint16_t>(yw.x >> 16),
@@ -300,14 +358,16 @@ __global__ __launch_bounds__(kQThreads) void quantize_kernel(
         pr[e][tid] = pack_angle_radius<T, UNIFORM, false>(fabsf(a), r, a, am);
     }
     // ---- per-pair max / min of angle and radius over the 128 tokens (packed: both at once)
-    uint32_t vmax[4], vmin[4];
+    // (each word is read back once and stays in a register for the codes)
+    uint32_t vmax[4], vmin[4], word[kEntries];
 #pragma unroll
     for (int i = 0; i < 4; i++) { vmax[i] = PkInit<T>::kMax; vmin[i] = PkInit<T>::kMin; }
 #pragma unroll
+    for (int e = 0; e < kEntries; e++) word[e] = pr[e][tid];
+#pragma unroll
     for (int e = 0; e < kEntries; e++) {
-        const uint32_t w = pr[e][tid];
-        vmax[e & 3] = pk_max<T>(vmax[e & 3], w);
-        vmin[e & 3] = pk_min<T>(vmin[e & 3], w);
+        vmax[e & 3] = pk_max<T>(vmax[e & 3], word[e]);
+        vmin[e & 3] = pk_min<T>(vmin[e & 3], word[e]);
     }
     // the 16 token lanes of a pair: 4 inside the wavefront (lane bits 4,5), 4 wavefronts
 #pragma unroll
@@ -332,16 +392,17 @@ __global__ __launch_bounds__(kQThreads) void quantize_kernel(
     }
     __syncthreads();
 
-    const float inv_t = static_cast<float>(1 << tbits), inv_r = static_cast<float>(1 << rbits);
+    // (a product with the inverse of a power of two is the quotient's one rounding)
+    const float inv_t = 1.0f / static_cast<float>(1 << tbits), inv_r = 1.0f / static_cast<float>(1 << rbits);
     float ts[4], tm[4], rs[4], rm[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const uint32_t wmax = fin[0][4 * pq4 + i], wmin = fin[1][4 * pq4 + i];
         tm[i] = lo2f<T>(static_cast<uint16_t>(wmin & 0xffffu));
         rm[i] = lo2f<T>(static_cast<uint16_t>(wmin >> 16));
-        ts[i] = rnd<T>(rnd<T>(lo2f<T>(static_cast<uint16_t>(wmax & 0xffffu)) - tm[i]) / inv_t);   // :147
+        ts[i] = rnd<T>(rnd<T>(lo2f<T>(static_cast<uint16_t>(wmax & 0xffffu)) - tm[i]) * inv_t);   // :147
         if constexpr (UNIFORM) { tm[i] = am.tmn; ts[i] = am.tscale; }
-        rs[i] = rnd<T>(rnd<T>(lo2f<T>(static_cast<uint16_t>(wmax >> 16)) - rm[i]) / inv_r);       // :152
+        rs[i] = rnd<T>(rnd<T>(lo2f<T>(static_cast<uint16_t>(wmax >> 16)) - rm[i]) * inv_r);       // :152
     }
     const size_t plane = static_cast<size_t>(bh) * cap + off + grp;
     if (tl == 0) {
@@ -388,22 +449,23 @@ __global__ __launch_bounds__(kQThreads) void quantize_kernel(
     };
     // PK6 exchanges words between lanes, so the whole wavefront takes one side together
     if (__builtin_expect(PK6 ? __all(fast) : fast, 1)) {
-        const uint32_t tlast = (1u << tbits) - 1u, rlast = (1u << rbits) - 1u;
         uint32_t least[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) least[i] = fin[1][4 * pq4 + i];
+        const auto top = CodeWord<T>::tops(tbits, rbits);
 #pragma unroll
         for (int it = 0; it < kTokPerThread; it++) {
-            uint32_t w = 0;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const uint32_t v = pr[it * 4 + i][tid];
+            CodeWord<T> cw;
+            uint32_t known = 0;
+            static_for<4>([&](auto II) {
+                constexpr int i = decltype(II)::value;
+                const uint32_t v = word[it * 4 + i];
                 float da, dr;
                 pair_distance<T>(v, least[i], &da, &dr);
-                const uint32_t th = UNIFORM ? (v & 0xffffu) : code_of_fast<T>(da, tinv[i], tlast);    // :148
-                const uint32_t rh = code_of_fast<T>(dr, rinv[i], rlast);                             // :153
-                w |= ((rh << tbits) + th) << (8 * i);                       // :155 (below 256)
-            }
+                if constexpr (UNIFORM) { da = 0.0f; known |= (v & 0xffffu) << (8 * i); }
+                cw.template add<i>(da, tinv[i], dr, rinv[i], top);               // :148, :153
+            });
+            const uint32_t w = cw.word(top) | known;                        // :155 (each below 256)
             store_codes(it, w);
         }
     } else {
@@ -412,7 +474,7 @@ __global__ __launch_bounds__(kQThreads) void quantize_kernel(
             uint32_t w = 0;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const uint32_t v = pr[it * 4 + i][tid];
+                const uint32_t v = word[it * 4 + i];
                 const float phi = lo2f<T>(static_cast<uint16_t>(v & 0xffffu));
                 const float r = lo2f<T>(static_cast<uint16_t>(v >> 16));
                 const uint32_t th = UNIFORM ? (v & 0xffffu) : code_of<T>(phi, tm[i], ts[i], ttop[i]);    // :148
@@ -450,8 +512,8 @@ __global__ __launch_bounds__(256) void selftest_kernel(unsigned long long* misma
             const double hi = 0.5 * (static_cast<double>(rr) + static_cast<double>(__uint_as_float(__float_as_uint(rr) + 1u)));
             bad += !(lo * lo <= static_cast<double>(s) && static_cast<double>(s) <= hi * hi);
         }
-        const float a = atan2_fast_abs(y, x), r = __builtin_amdgcn_sqrtf(__builtin_fmaf(x, x, y * y));
-        slow += near_rounding_boundary<T>(a, Atan<LIBM>::kGuardUlps) || near_rounding_boundary<T>(r, kSqrtGuardUlps);
+        const float r = __builtin_amdgcn_sqrtf(__builtin_fmaf(x, x, y * y)), a = atan2_fast_abs<T>(y, x, r);
+        slow += near_rounding_boundary<T>(a, Atan<T, LIBM>::kGuardUlps) || near_rounding_boundary<T>(r, kSqrtGuardUlps);
     }
     if (bad) atomicAdd(mismatches, static_cast<unsigned long long>(bad));
     if (slow) atomicAdd(slow_lanes, static_cast<unsigned long long>(slow));
@@ -473,7 +535,8 @@ __global__ __launch_bounds__(256) void selftest_div_kernel(unsigned long long* m
             const float exact = rnd<T>(d / sc);
             const float fast = rnd<T>(div_faithful(d, sc, __builtin_amdgcn_rcpf(sc)));
             bad += (exact != fast) && !(exact < 0.25f && fast < 0.25f);
-            bad += code_of_fast<T>(d, inverse_of<T>(sc), 127u) != static_cast<uint32_t>(__builtin_amdgcn_fmed3f(floorf(exact), 0.0f, 127.0f));
+            for (int bits : {7, 4, 3})
+                bad += code_of_fast<T>(d, inverse_of<T>(sc), bits) != static_cast<uint32_t>(__builtin_amdgcn_fmed3f(floorf(exact), 0.0f, static_cast<float>((1 << bits) - 1)));
         }
     }
     if (bad) atomicAdd(mismatches, static_cast<unsigned long long>(bad));
@@ -503,7 +566,7 @@ int launch_quantize(const void* k, const int64_t* strides, int dtype, int B, int
     AngleMode am;
     const bool uniform = (flags & 2u) != 0;
     am.two_pi = (flags & 1u) ? two_pi_f : 6.28125f;
-    am.ttop = (1 << tbits) - 1;
+    am.tbits = tbits;
     am.minus_one = -1.0f;
     const bool bf = dtype != 0;
     auto round_dt = [bf](float f) {
