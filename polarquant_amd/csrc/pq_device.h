@@ -48,24 +48,25 @@ template <> __device__ __forceinline__ uint16_t f2lo<BF16>(float f) {
 
 // ---- division of two key-dtype values, rounded to the key dtype ----------------
 // Eager torch evaluates a / b on half / bfloat16 tensors as round_dtype(fp32 quotient).  The
-// IEEE fp32 division is ~10 instructions; the value quantizer divides every element by a scale that
-// is shared by many elements, so it uses instead
-//     q0 = d * inv,  r = fma(-q0, sc, d),  q1 = fma(r, inv, q0),      inv = v_rcp_f32(sc) (1 ulp)
-// q1 is a faithful fp32 quotient (the residual r is exact, so q1 is the rounding of a value
-// within 2^-46 of d / sc).  It may differ from the correctly rounded fp32 quotient in the last
+// IEEE fp32 division is ~10 instructions; the quantizers divide many elements by one scale and
+// multiply by its inverse in two parts instead, hi = v_rcp_f32(sc) (1 ulp) and lo = (1 - sc hi) hi:
+// hi + lo is 1 / sc to 2^-46, so fma(d, hi, d lo) is within 1 ulp of d / sc and is d / sc itself where that is an fp32 number.
+// It may differ from the correctly rounded fp32 quotient in the last
 // bit, but never across a rounding boundary of the dtype: such a boundary t has at most 12
 // significant bits and sc 11 (9 and 8 for bfloat16), so t * sc is exact in fp32 arithmetic and
-// d / sc is either exactly t (then q1 == t as well) or more than 2 fp32 ulps away from it.
-// Hence round_dtype(q1) == round_dtype(RN32(d / sc)).  Conditions: sc finite, positive and far
+// d / sc is either exactly t (then the product is t as well) or more than 2 fp32 ulps away from it.
+// Conditions: sc finite, positive and far
 // from the ends of the fp32 range (fast_div_ok), d finite with d / sc far below overflow; callers
 // take the plain division otherwise.  pq_selftest_quantizer_math checks the identity on the
 // device for every operand pair of the dtype that meets them.
 __device__ __forceinline__ bool fast_div_ok(float sc) { return sc >= 0x1p-100f && sc <= 0x1p100f; }
-__device__ __forceinline__ float div_faithful(float d, float sc, float inv) {
-    const float q0 = d * inv;
-    const float r = __builtin_fmaf(-q0, sc, d);
-    return __builtin_fmaf(r, inv, q0);
+struct Inverse { float hi, lo; };
+__device__ __forceinline__ Inverse two_part_inverse(float sc) {
+    const float inv = __builtin_amdgcn_rcpf(sc);
+    return {inv, __builtin_fmaf(-sc, inv, 1.0f) * inv};
 }
+// (plus zero: a product whose half-precision operand is converted on the way in)
+__device__ __forceinline__ float quotient(float d, Inverse inv) { return __builtin_fmaf(d, inv.hi, __builtin_fmaf(d, inv.lo, 0.0f)); }
 
 // v of lane (l & ~15) | ((l + N) & 15): a rotation inside each row of 16 lanes, as a DPP
 // modifier of a move instead of a trip through the LDS crossbar

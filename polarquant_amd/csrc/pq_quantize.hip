@@ -173,12 +173,11 @@ __device__ __forceinline__ uint32_t code_of(float v, float mn, float scale, floa
 // lies has to be right.  d is a number of 11 bits (bfloat16: 8) and B * scale one of 23 (17), so a quotient below B is below it by
 // 2^-23 (2^-17) of it at least.  Half: the inverse in two parts; the product's one rounding then neither reaches B from there nor
 // leaves it.  Bfloat16: an inverse too large by 2^-22 to 2^-20 is enough.  Every pair of operands is checked on the device.
-struct Inverse { float hi, lo; };
 template <typename T>
 __device__ __forceinline__ Inverse inverse_of(float scale) {
+    if constexpr (IsHalf<T>::value) return two_part_inverse(scale);
     const float inv = __builtin_amdgcn_rcpf(scale);                  // within 1 ulp
-    if constexpr (IsHalf<T>::value) return {inv, __builtin_fmaf(-scale, inv, 1.0f) * inv};
-    else return {__builtin_fmaf(inv, 0x1p-21f, inv), 0.0f};
+    return {__builtin_fmaf(inv, 0x1p-21f, inv), 0.0f};
 }
 // The codes of four pairs: angles in bits tbits - 1 .. 0 of each byte, radii above them.  `add` takes a pair's distances.
 // Half: both quotients are rounded by one conversion, the dtype's own (a multiply-add, half a unit and a conversion to a whole number
@@ -187,9 +186,7 @@ struct CodeTops { uint32_t both; int tbits; };
 template <typename T> struct CodeWord {
     uint32_t c[4];                                                                          // angle code | radius code << 16
     template <int I> __device__ __forceinline__ void add(float da, Inverse ia, float dr, Inverse ir, const CodeTops& top) {
-        // (plus zero: a product whose operand is converted on the way in)
-        const float qa = __builtin_fmaf(da, ia.hi, __builtin_fmaf(da, ia.lo, 0.0f)), qr = __builtin_fmaf(dr, ir.hi, __builtin_fmaf(dr, ir.lo, 0.0f));
-        const ushort2v k = __builtin_convertvector(__builtin_convertvector((float2v{qa, qr}), half2v), ushort2v);
+        const ushort2v k = __builtin_convertvector(__builtin_convertvector((float2v{quotient(da, ia), quotient(dr, ir)}), half2v), ushort2v);
         c[I] = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(k, __builtin_bit_cast(ushort2v, top.both)));
     }
     __device__ __forceinline__ uint32_t word(const CodeTops& top) const {
@@ -519,7 +516,7 @@ __global__ __launch_bounds__(256) void selftest_kernel(unsigned long long* misma
     if (slow) atomicAdd(slow_lanes, static_cast<unsigned long long>(slow));
 }
 
-// Exhaustive check of div_faithful and of the codes taken from it: block == bit pattern of the dividend d, thread t covers the
+// Exhaustive check of the two-part quotient and of the codes taken from it: block == bit pattern of the dividend d, thread t covers the
 // divisor patterns t, t+256, ...  Pairs the quantizers can meet: divisor accepted by fast_div_ok,
 // 0 <= d <= 1024 * sc (d is a distance from the group minimum and sc the group's range over at
 // most 2^8 bins).  Quotients below 1/4 may differ in denormal digits; floor() and rint() of both
@@ -533,7 +530,7 @@ __global__ __launch_bounds__(256) void selftest_div_kernel(unsigned long long* m
             const float sc = lo2f<T>(static_cast<uint16_t>(sb));
             if (!fast_div_ok(sc) || !(d <= 1024.0f * sc)) continue;
             const float exact = rnd<T>(d / sc);
-            const float fast = rnd<T>(div_faithful(d, sc, __builtin_amdgcn_rcpf(sc)));
+            const float fast = rnd<T>(quotient(d, two_part_inverse(sc)));
             bad += (exact != fast) && !(exact < 0.25f && fast < 0.25f);
             for (int bits : {7, 4, 3})
                 bad += code_of_fast<T>(d, inverse_of<T>(sc), bits) != static_cast<uint32_t>(__builtin_amdgcn_fmed3f(floorf(exact), 0.0f, static_cast<float>((1 << bits) - 1)));

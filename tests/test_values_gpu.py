@@ -274,3 +274,20 @@ def test_attention_long_flat_tail_under_a_peak_is_not_dropped(gpu, values4):
         nbad, emax = _close(out, ref64)
         print("flat tail, values4", values4, "n_splits", ns, "max abs err %.2e" % emax, flush=True)
         assert nbad == 0, (ns, nbad, emax)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_scale_of_every_range(gpu, dtype):
+    """A row's range runs through every finite number of the dtype: its scale, a fifteenth of it, is rounded as a division is, and the
+    codes of the range's own fractions (midpoints of codes among them) are the reference's."""
+    top = torch.arange(1, 32768, dtype=torch.int32).to(torch.int16).view(dtype)
+    top = top[torch.isfinite(top)]
+    parts = torch.arange(128, dtype=torch.float32) / 120.0
+    v = (top.float()[:, None] * parts.clamp(max=1.0)).to(dtype)
+    v[:, 0], v[:, 127] = 0.0, top
+    v = v[None, None]
+    got = [t.cpu() for t in quantize_values(v.to(gpu))]
+    ref = po.quantize_values_along_last_dim(v)
+    assert torch.equal(got[0], ref[0])
+    for a, b in zip(got[1:], ref[1:]):
+        assert torch.equal(a.float(), b.float())
