@@ -24,6 +24,7 @@ struct PromptAttnArgs {
 };
 
 constexpr int kPromptTileRows = 128, kPromptTileKeys = 64;
+constexpr int kAhead = 4;                     // steps of the score product whose keys are on their way from LDS
 
 // 16 bytes per lane from global memory into 1 KiB of LDS at `lds` (uniform), lane after lane.  Not known to the compiler's count
 // of loads in flight: wait_lds_loads() before the barrier behind which the data is read.  (The builtin is known to it, and makes every
@@ -37,6 +38,19 @@ __device__ __forceinline__ void load_to_lds(const void* p, uint32_t lds) {
 }
 #pragma clang diagnostic pop
 __device__ __forceinline__ void wait_lds_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// the larger of lanes l and l ^ 32, by an exchange of half wavefronts that stays in the vector unit
+__device__ __forceinline__ float both_halves_max(float v) {
+    typedef unsigned int uint2_x __attribute__((ext_vector_type(2)));
+    const uint2_x r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r.x), __uint_as_float(r.y));
+}
+
+// The order of a basic block's instructions by kind (a rule for the compiler's scheduler, which takes the calls in their order): so many
+// of one kind next.
+constexpr int kMatrix = 0x8, kDsRead = 0x100;
+template <int KIND, int N>
+__device__ __forceinline__ void order() { __builtin_amdgcn_sched_group_barrier(KIND, N, 0); }
 
 typedef float floatx2_a __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2_a __attribute__((ext_vector_type(2)));
@@ -54,13 +68,19 @@ template <> __device__ __forceinline__ uint32_t pack_pair<F16>(float a, float b)
 // register, and P^T the right operand of O^T = V^T P^T as it stands.  TOKEN_ROWS: V has a row per token and is transposed on the
 // way out of LDS; otherwise a row per channel, as a product with the weights on the left leaves it.
 //
-// What bounds it: the vector unit and the matrix cores need about the same time per tile (32 exponentials at a quarter of the rate and
-// 112 other vector instructions a lane; 32 products of 32 cycles), the LDS half of it, so the two wavefronts of a SIMD have to
-// overlap.  Tiles therefore go to LDS directly (no registers, no store instructions, the swizzle that keeps reads free of
-// conflicts is in the addresses that the lanes load from) and the scale is part of the exponential's multiply-add.  Measured at 8192
-// tokens, 32 heads of 128, bf16: 637 us (863 TFLOP/s) with a row per channel, 611 us with a row per token; 704 us with tiles passed
-// through registers.  A step that makes the next tile's scores beside this tile's weights needs more registers than two wavefronts
-// have; raised wavefront priority around the products changes nothing.
+// What bounds it: matrix cores and vector unit are both busy for half of the time (32 products of 32 cycles a tile; 32 exponentials and
+// some 150 other vector instructions a lane), and the two wavefronts of a SIMD overlap little of it beyond what each has side by
+// side itself.  So the order of a tile's instructions is laid down: keys for four steps of the score product are on their way from
+// LDS, and each product with V stands beside two of the next step's weights and the reads of its operand (left alone, the compiler waits
+// for LDS every second product and makes all weights before the first).  Tiles go to LDS directly (no registers, no store instructions);
+// the addresses that the lanes load from swizzle them so that 16 lanes' reads of 16 bytes, or 32 lanes' of 8, meet every bank once (by
+// 8 rows instead of 16 half of the LDS cycles were conflicts).  The scale is part of the exponential's multiply-add.
+// In turn with the kernel before (compiler's order, 8-row swizzle), bf16, us: 8192 tokens, 32 heads of 128, a row per token 586 -> 567,
+// per channel 585 -> 584 (its reads of V meet a bank twice whatever the swizzle); 2048 tokens 58.5 -> 54.7, 59.2 -> 56.0; 4096 tokens,
+// 16 heads of 192 / 256 143.6 -> 133.1, 238.7 -> 202.1.  No gain: three or four buffers; eight wavefronts that take turns at scores and
+// products; eight wavefronts over one tile of keys without turns 545 for 560.
+// A step that makes the next tile's scores beside this tile's weights needs more registers than two wavefronts have; raised wavefront
+// priority around the products changes nothing.
 // The maximum is raised whenever it is exceeded: the largest weight of a row is then 1, which its 16 bits hold exactly.  Raised at an
 // excess of 2^8 only, which saves most of the rescaling (615 and 592 us), that weight is rounded like the others and the error against
 // 64 bits grows: by 3 % with normal scores, by 15 % where a few keys have most of the weight.
@@ -120,8 +140,8 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
     // where this lane's 16 bytes of each load come from: load i of a wavefront fills chunks (wv KL + i) 64 .. + 63 of a tile
     const uint16_t* kb = static_cast<const uint16_t*>(a.k) + b * a.k_b + g * a.k_h;
     const uint16_t* vb = static_cast<const uint16_t*>(a.v) + b * a.v_b + g * a.v_h;
-    auto k_swz = [](int row) { return DKP == 64 ? (row >> 1) & 7 : row & 7; };
-    auto v_swz = [](int row) { return TOKEN_ROWS ? (DVP == 64 ? ((row >> 1) & 3) << 1 : (row & 7) << 1) : (row >> 1) & 7; };
+    auto k_swz = [](int row) { return DKP % 128 ? (row >> 1) & 7 : row & 15; };
+    auto v_swz = [](int row) { return TOKEN_ROWS ? (DVP == 64 ? ((row >> 1) & 1) << 2 : (row & 3) << 2) : (row >> 1) & 7; };
     // with WINDOW, row (first + row) of the sequence: the ring's before this call's own
     auto either = [&](const uint16_t* own, int64_t own_t, const void* ring, int width, int first, int slot, int row, int last) {
         const int key = first + (row < last ? row : last);
@@ -172,19 +192,17 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
     float m = kNone, l = 0.0f;
 
     // LDS addresses of this lane's reads: row `col` of K, chunk 2 i + hi
-    // A row per channel: 8 chunks at VT distances.  Up to 128 channels the compiler may keep all 32 sums (with the chunks' addresses kept
-    // and the distances as offsets 190 registers instead of 246, but 668 against 637 us); 64 sums do not fit beside 256 channels' tile
-    // (86 registers spilled, 16 heads, 8192 tokens: 1652 us, with kept chunks 847, with tiles passed through registers 999).
-    constexpr bool kChunks = !TOKEN_ROWS && DVP > 128;
-    uint32_t ka[KS], va[kChunks ? 8 : VT];
+    // A row per channel: 8 chunks at VT distances; the chunks' addresses are kept and the distances are offsets (32 or 64 sums do not fit, or
+    // are formed again beside every product: 8192 tokens 635 us).
+        uint32_t ka[KS], va[TOKEN_ROWS ? VT : 8];
     static_for<KS>([&](auto I) { ka[I] = lds0 + col * (DKP * 2) + ((2 * I + hi) ^ k_swz(col)) * 16; });
-    static_for<kChunks ? 8 : VT>([&](auto I) {
+    static_for<TOKEN_ROWS ? VT : 8>([&](auto I) {
         constexpr int i = decltype(I)::value;
         if (TOKEN_ROWS) {           // 16 lanes read 4 tokens x 16 channels and get them transposed
             const int row = 4 * hi + ((lane & 15) >> 2), chunk = 4 * i + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
             va[i] = lds0 + 2 * KBYTES + row * (DVP * 2) + (chunk ^ v_swz(row)) * 16 + (lane & 1) * 8;
-        } else {                    // chunk i of row `col`, or row 32 i + col: rows 32 apart have the same swizzle
-            va[i] = lds0 + 2 * KBYTES + hi * 8 + (kChunks ? col * 128 + (i ^ v_swz(col)) * 16 : (32 * i + col) * 128);
+        } else {                    // chunk i of row `col`: rows 32 apart have the same swizzle
+            va[i] = lds0 + 2 * KBYTES + hi * 8 + col * 128 + (i ^ v_swz(col)) * 16;
         }
     });
     auto step = [&](int it, auto BUF) {
@@ -198,11 +216,26 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
             for (int u = 0; u < 2; u++)
 #pragma unroll
                 for (int j = 0; j < 16; j++) s[u][j] = 0.0f;
+            constexpr int KD = KS < kAhead ? KS : kAhead;
+            u32x4_a kf[KD][2];
+            auto k_load = [&](auto I) {
+                constexpr int i = decltype(I)::value;
+                kf[i % KD][0] = *lds_ptr<lds_u32x4>(ka[i] + buf * KBYTES);
+                kf[i % KD][1] = *lds_ptr<lds_u32x4>(ka[i] + buf * KBYTES + 32 * DKP * 2);
+            };
+            static_for<KD>(k_load);
             static_for<KS>([&](auto I) {
                 constexpr int i = decltype(I)::value;
-                s[0] = mma32<T>(*lds_ptr<lds_u32x4>(ka[i] + buf * KBYTES), q[i], s[0]);
-                s[1] = mma32<T>(*lds_ptr<lds_u32x4>(ka[i] + buf * KBYTES + 32 * DKP * 2), q[i], s[1]);
+                s[0] = mma32<T>(kf[i % KD][0], q[i], s[0]);
+                s[1] = mma32<T>(kf[i % KD][1], q[i], s[1]);
+                if constexpr (i + KD < KS) k_load(IC<i + KD>{});
             });
+            order<kDsRead, 2 * KD>();
+            static_for<KS - KD>([&](auto) {
+                order<kMatrix, 2>();
+                order<kDsRead, 2>();
+            });
+            order<kMatrix, 2 * KD>();
             if (WINDOW) {                                           // from here on in units of the exponent, the bias taken off
                 const float base = -slope2 * static_cast<float>(limit - key0 - 4 * hi);
 #pragma unroll
@@ -225,7 +258,7 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
             float mx = fmaxf(s[0][0], s[1][0]);
 #pragma unroll
             for (int j = 1; j < 16; j++) mx = fmaxf(fmaxf(mx, s[0][j]), s[1][j]);
-            mx = fmaxf(mx, __shfl_xor(mx, 32)) * (WINDOW ? 1.0f : scale2);
+            mx = both_halves_max(mx) * (WINDOW ? 1.0f : scale2);
             if (__any(mx > m)) {
                 const float mn = fmaxf(m, mx), al = exp2_hw(m - mn);
                 l *= al;
@@ -235,36 +268,47 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
                 });
                 m = mn;
             }
-            u32x4_a p[4];                                           // right operands of the four 16-token steps
+            // right operands of the four 16-token steps, each made beside the products of the one before it
+            u32x4_a p[2], vf[2][VT];
             float sum[2] = {0.0f, 0.0f};
-#pragma unroll
-            for (int u = 0; u < 2; u++)
-#pragma unroll
-                for (int j = 0; j < 16; j += 2) {
-                    auto weight = [&](float x) { return exp2_hw(WINDOW ? x - m : __builtin_fmaf(x, scale2, -m)); };
-                    const float e0 = weight(s[u][j]), e1 = weight(s[u][j + 1]);
-                    sum[0] += e0;
-                    sum[1] += e1;
-                    p[2 * u + (j >> 3)][(j & 7) >> 1] = pack_pair<T>(e0, e1);
+            auto v_load = [&](auto J, auto I) {
+                constexpr int j = decltype(J)::value, i = decltype(I)::value;
+                u32x2_a w0, w1;
+                if constexpr (TOKEN_ROWS) {
+                    const uint32_t at = va[i] + buf * VBYTES + j * 16 * DVP * 2;
+                    w0 = __builtin_bit_cast(u32x2_a, __builtin_amdgcn_ds_read_tr16_b64_v4i16(lds_ptr<lds_short4>(at)));
+                    w1 = __builtin_bit_cast(u32x2_a, __builtin_amdgcn_ds_read_tr16_b64_v4i16(lds_ptr<lds_short4>(at + 8 * DVP * 2)));
+                } else {
+                    w0 = *lds_ptr<lds_u32x2>(va[2 * j] + 32 * i * 128 + buf * VBYTES);
+                    w1 = *lds_ptr<lds_u32x2>(va[2 * j + 1] + 32 * i * 128 + buf * VBYTES);
                 }
-            l += sum[0] + sum[1];
+                vf[j & 1][i] = u32x4_a{w0.x, w0.y, w1.x, w1.y};
+            };
+            auto weights = [&](auto J, auto N) {                    // the Nth two of step J
+                constexpr int u = decltype(J)::value >> 1, n = decltype(N)::value, j = 8 * (decltype(J)::value & 1) + 2 * n;
+                auto weight = [&](float x) { return exp2_hw(WINDOW ? x - m : __builtin_fmaf(x, scale2, -m)); };
+                const float e0 = weight(s[u][j]), e1 = weight(s[u][j + 1]);
+                sum[0] += e0;
+                sum[1] += e1;
+                p[decltype(J)::value & 1][n] = pack_pair<T>(e0, e1);
+            };
+            static_for<VT>([&](auto I) { v_load(IC<0>{}, I); });
+            static_for<4>([&](auto N) { weights(IC<0>{}, N); });
+            __builtin_amdgcn_sched_barrier(0);
             static_for<4>([&](auto J) {
                 constexpr int j = decltype(J)::value;
                 static_for<VT>([&](auto I) {
                     constexpr int i = decltype(I)::value;
-                    u32x2_a w0, w1;
-                    if constexpr (TOKEN_ROWS) {
-                        const uint32_t at = va[i] + buf * VBYTES + j * 16 * DVP * 2;
-                        w0 = __builtin_bit_cast(u32x2_a, __builtin_amdgcn_ds_read_tr16_b64_v4i16(lds_ptr<lds_short4>(at)));
-                        w1 = __builtin_bit_cast(u32x2_a, __builtin_amdgcn_ds_read_tr16_b64_v4i16(lds_ptr<lds_short4>(at + 8 * DVP * 2)));
-                    } else {
-                        auto at = [&](int chunk) { return (kChunks ? va[chunk] + 32 * i * 128 : va[i] + (chunk ^ v_swz(col)) * 16) + buf * VBYTES; };
-                        w0 = *lds_ptr<lds_u32x2>(at(2 * j));
-                        w1 = *lds_ptr<lds_u32x2>(at(2 * j + 1));
+                    o[i] = mma32<T>(vf[j & 1][i], p[j & 1], o[i]);
+                    if constexpr (j < 3) {
+                        v_load(IC<j + 1>{}, I);
+                        if constexpr (VT < 4) { weights(IC<j + 1>{}, IC<2 * i>{}); weights(IC<j + 1>{}, IC<2 * i + 1>{}); }
+                        else if constexpr (i % (VT / 4) == 0) weights(IC<j + 1>{}, IC<i / (VT / 4)>{});
                     }
-                    o[i] = mma32<T>(u32x4_a{w0.x, w0.y, w1.x, w1.y}, p[j], o[i]);
+                    __builtin_amdgcn_sched_barrier(0);              // (left alone, the compiler makes all weights first)
                 });
             });
+            l += sum[0] + sum[1];
         }
         wait_lds_loads();
         __syncthreads();
