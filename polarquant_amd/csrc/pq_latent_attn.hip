@@ -24,6 +24,10 @@ namespace pq {
 // only barrier), every wavefront runs the softmax of all rows, and multiplies its channels of V^T, the same LDS tile
 // transposed on the way out, with P^T.  So each key is read from HBM once, and from LDS once per product, for all rows.
 // 16-byte pieces of a key's row are XOR-swizzled by the key so that neither access meets in few banks.
+// Up to 32 rows (their state takes half of a SIMD's registers) a workgroup is two teams of such wavefronts, each with half of the
+// slice's tiles, whose states are joined in LDS: a unit holds two sets of wavefronts either way, and one partial of R floats a row
+// goes through memory instead of two (8 sequences of 4096 keys, 32 heads, rank 512, planned for 12288: 33 MB of them written and read
+// beside 34 MB of latents).  Both launches 25.1 -> 21.5 us; of 12000 keys 37.6 -> 32.8; 32 sequences of 8000 74.0 -> 67.1.
 // Workspace: [B, slices, L * H] pairs (maximum in log2 units, sum), then as many rows of R floats.
 constexpr int kDecodeTile = 32;
 __device__ __forceinline__ size_t pairs_floats(const LatentDecodeArgs& a) {     // up to the accumulators' 16-byte boundary
@@ -34,13 +38,27 @@ template <int RP> struct DecodeShape {
     static constexpr int NW = RP / CW;                         // wavefronts
 };
 
+template <int RP, int RT> struct DecodeTeams {
+    static constexpr int N = RT <= 2 ? 2 : 1, NW = DecodeShape<RP>::NW;
+    static constexpr int THREADS = kWave * NW * N;
+    static constexpr size_t TILES = static_cast<size_t>(N) * NW * kDecodeTile * DecodeShape<RP>::CW * 2;            // bytes of LDS
+    static constexpr size_t EXCH = static_cast<size_t>(N) * 2 * NW * 2 * RT * kWave * 16;
+    static constexpr size_t BYTES = TILES + EXCH;
+    // the second team's state, in the tiles' and the exchange's place
+    static_assert(N == 1 || static_cast<size_t>(NW) * kWave * RT * (DecodeShape<RP>::CW / 16 * 16 + 8) <= BYTES, "LDS");
+};
+
 template <typename T, int RP, int RT>
-__global__ __launch_bounds__(kWave * DecodeShape<RP>::NW, RT <= 2 ? 2 : 1) void latent_decode_kernel(LatentDecodeArgs a) {
+__global__ __launch_bounds__((DecodeTeams<RP, RT>::THREADS), RT <= 2 ? 2 : 1) void latent_decode_kernel(LatentDecodeArgs a) {
     constexpr int CW = DecodeShape<RP>::CW, NW = DecodeShape<RP>::NW, CH = CW / 8, KS = CW / 32, CT = CW / 16;
     constexpr int LPT = kDecodeTile * CH / kWave, RPW = 16 / CH;           // loads per lane; rows per 256 bytes of LDS
-    __shared__ __attribute__((aligned(16))) uint16_t tiles[NW][kDecodeTile * CW];
-    __shared__ floatx4_a exch[2][NW][2 * RT][kWave];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid / kWave, r16 = lane & 15, g = lane >> 4;
+    constexpr int TEAMS = DecodeTeams<RP, RT>::N;
+    extern __shared__ __attribute__((aligned(16))) uint8_t sm[];
+    auto tiles = reinterpret_cast<uint16_t(*)[kDecodeTile * CW]>(sm);
+    auto exchs = reinterpret_cast<floatx4_a(*)[2][NW][2 * RT][kWave]>(sm + DecodeTeams<RP, RT>::TILES);
+    const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), team = wave / NW, wv = wave % NW;
+    auto& exch = exchs[team];
     const int b = blockIdx.z, split = blockIdx.x, R = a.R, rows = a.L * a.H, n0 = blockIdx.y * 16 * RT;
     const int pos = a.pos_dev ? *a.pos_dev : a.pos;
     const int total = static_cast<int>(static_cast<int64_t>(pos) + a.L < a.capacity ? pos + a.L : a.capacity);   // (below 2^30)
@@ -59,7 +77,7 @@ __global__ __launch_bounds__(kWave * DecodeShape<RP>::NW, RT <= 2 ? 2 : 1) void 
     const int c0 = wv * CW;                          // this wavefront's first channel
 
     const uint16_t* cb = static_cast<const uint16_t*>(a.c) + static_cast<size_t>(b) * a.capacity * R;
-    uint16_t* tile = tiles[wv];
+    uint16_t* tile = tiles[wave];
 
     u32x4_a stage[LPT];
     uint32_t off[LPT], col[LPT];                     // elements from the tile's first key
@@ -69,7 +87,8 @@ __global__ __launch_bounds__(kWave * DecodeShape<RP>::NW, RT <= 2 ? 2 : 1) void 
         col[i] = c < R ? c : 0;
         off[i] = static_cast<uint32_t>(u / CH) * R + col[i];
     });
-    auto fetch = [&](int key0) {
+    auto fetch = [&](int key) {
+        const int key0 = TEAMS == 1 || key < s1 ? key : s0;
         const uint16_t* base = cb + static_cast<int64_t>(key0) * R;
         const int last = s1 - 1 - key0;              // uniform
         static_for<LPT>([&](auto I) {
@@ -80,7 +99,13 @@ __global__ __launch_bounds__(kWave * DecodeShape<RP>::NW, RT <= 2 ? 2 : 1) void 
             stage[i] = *reinterpret_cast<const u32x4_a*>(base + (tok <= last ? off[i] : static_cast<uint32_t>(last) * R + col[i]));
         });
     };
-    fetch(s0);
+    // A slice of one or two tiles is the first team's alone: joining costs what a tile does.  Otherwise both make the same number of
+    // steps; a tile past the slice is a copy of its first one, every key of it masked.
+    const int all = (s1 - s0 + kDecodeTile - 1) / kDecodeTile;
+    const bool alone = TEAMS == 1 || all <= 2;
+    if (alone && team == 1) return;
+    const int ntiles = alone ? all : (all + 1) / 2, t0 = s0 + team * ntiles * kDecodeTile;
+    fetch(t0);
     __builtin_amdgcn_sched_barrier(0);
     u32x4_a q[RT][KS];
     int limit[RT];                                   // keys a row may see: positions below it
@@ -120,10 +145,9 @@ __global__ __launch_bounds__(kWave * DecodeShape<RP>::NW, RT <= 2 ? 2 : 1) void 
     }
     static_assert((16 / RPW) % CH == 0, "rows 16 apart are swizzled alike");
 
-    const int ntiles = (s1 - s0 + kDecodeTile - 1) / kDecodeTile;
     put();
     for (int it = 0; it < ntiles; it++) {
-        if (it + 1 < ntiles) fetch(s0 + (it + 1) * kDecodeTile);
+        if (it + 1 < ntiles) fetch(t0 + (it + 1) * kDecodeTile);
         __builtin_amdgcn_sched_barrier(0);
         u32x4_a k[2][KS];
         static_for<KS>([&](auto I) {
@@ -156,7 +180,7 @@ __global__ __launch_bounds__(kWave * DecodeShape<RP>::NW, RT <= 2 ? 2 : 1) void 
             ex[wv][2 * j + 1][lane] = s[j][1];
         });
         __syncthreads();     // (the other buffer's readers are done before they arrive here)
-        const int tile0 = s0 + it * kDecodeTile, key0 = tile0 + 4 * g;
+        const int tile0 = t0 + it * kDecodeTile, key0 = tile0 + 4 * g;
         const bool whole = tile0 + kDecodeTile <= first_limit && tile0 + kDecodeTile <= s1;
         static_for<RT>([&](auto J) {
             constexpr int j = decltype(J)::value;
@@ -199,6 +223,30 @@ __global__ __launch_bounds__(kWave * DecodeShape<RP>::NW, RT <= 2 ? 2 : 1) void 
             });
         });
         if (it + 1 < ntiles) put();
+    }
+    if (!alone) {
+        // lane by lane: both teams hold the same rows and channels in it
+        auto sums = reinterpret_cast<floatx4_a(*)[RT * CT][kWave]>(sm);
+        auto pairs = reinterpret_cast<float(*)[2 * RT][kWave]>(sm + sizeof(floatx4_a) * NW * RT * CT * kWave);
+        __syncthreads();
+        if (team == 1) {
+            static_for<RT>([&](auto J) {
+                constexpr int j = decltype(J)::value;
+                static_for<CT>([&](auto I) { sums[wv][j * CT + I][lane] = o[j][I]; });
+                pairs[wv][2 * j][lane] = m[j];
+                pairs[wv][2 * j + 1][lane] = l[j];
+            });
+        }
+        __syncthreads();
+        if (team == 1) return;
+        static_for<RT>([&](auto J) {
+            constexpr int j = decltype(J)::value;
+            const float m1 = pairs[wv][2 * j][lane], l1 = pairs[wv][2 * j + 1][lane], mn = fmaxf(m[j], m1);
+            const float a0 = exp2_hw(m[j] - mn), a1 = exp2_hw(m1 - mn);
+            l[j] = l[j] * a0 + l1 * a1;
+            m[j] = mn;
+            static_for<CT>([&](auto I) { o[j][I] = o[j][I] * a0 + sums[wv][j * CT + I][lane] * a1; });
+        });
     }
     static_for<RT>([&](auto J) {
         constexpr int j = decltype(J)::value;
@@ -271,7 +319,15 @@ int launch_latent_decode(const LatentDecodeArgs& a, int dtype, hipStream_t st) {
     const int rows = a.L * a.H;
     const int rt = rows <= 16 ? 1 : rows <= 32 ? 2 : 4;
     dim3 grid(a.n_splits, (rows + 16 * rt - 1) / (16 * rt), a.B);
-#define PQ_LD1(T, RP, RT) hipLaunchKernelGGL((latent_decode_kernel<T, RP, RT>), grid, dim3(kWave * DecodeShape<RP>::NW), 0, st, a)
+    int err = 0;
+#define PQ_LD1(T, RP, RT)                                                                                            \
+    do {                                                                                                             \
+        using D = DecodeTeams<RP, RT>;                                                                               \
+        auto* kernel = &latent_decode_kernel<T, RP, RT>;                                                             \
+        if (D::BYTES > 64 * 1024)                                                                                    \
+            err = static_cast<int>(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(D::BYTES))); \
+        if (!err) hipLaunchKernelGGL(kernel, grid, dim3(D::THREADS), D::BYTES, st, a);                               \
+    } while (0)
 #define PQ_LD(T, RP) do { if (rt == 1) PQ_LD1(T, RP, 1); else if (rt == 2) PQ_LD1(T, RP, 2); else PQ_LD1(T, RP, 4); } while (0)
 #define PQ_LDT(T)                                                                                                    \
     do {                                                                                                             \
@@ -282,7 +338,7 @@ int launch_latent_decode(const LatentDecodeArgs& a, int dtype, hipStream_t st) {
 #undef PQ_LDT
 #undef PQ_LD
 #undef PQ_LD1
-    int err = static_cast<int>(hipGetLastError());
+    if (!err) err = static_cast<int>(hipGetLastError());
     if (err) return err;
     dim3 mgrid(rows, (a.R + 63) / 64, a.B), mblock(256);
     if (dtype == 0) hipLaunchKernelGGL(latent_merge_kernel<F16>, mgrid, mblock, 0, st, a);

@@ -159,6 +159,21 @@ def test_latent_decode(gpu, R, L, H):
                 assert err(got, want) < {"f32": 5e-6, "bf16": 1.2e-2, "f16": 2e-3}[dt], (dt, pos, S)
 
 
+@pytest.mark.parametrize("keys", [1, 33, 64, 65, 96, 97, 128, 129, 160, 161, 289])
+def test_latent_decode_halves_of_a_slice(gpu, keys):
+    """A workgroup's two halves of one slice: one to ten tiles of 32 keys, odd counts and broken last tiles; a key that stands out lies in
+    the first half, in the second and on the last row in turn."""
+    g = torch.Generator().manual_seed(keys)
+    for dt, H, R in (("bf16", 32, 512), ("f16", 16, 256), ("bf16", 5, 64)):
+        q, sink = rand(g, 2, 1, H, R, dt=dt, s=2.0), rand(g, H)
+        for at in {0, keys // 2, keys - 1}:
+            c = rand(g, 2, keys + 7, R, dt=dt)
+            c[:, at] = q[:, 0, 1] * 0.7
+            c[:, keys:] = 3e4
+            got = ops.latent_decode_attention(q.to(gpu), c.to(gpu), sink.to(gpu), R ** -0.5, keys - 1, n_splits=1)
+            assert err(got, decode_want(q, c, sink, R ** -0.5, keys - 1, None)) < {"bf16": 1.2e-2, "f16": 2e-3}[dt], (dt, at)
+
+
 def test_latent_decode_positions_in_device_memory_and_stale_rows(gpu):
     """Rows past the sequence hold large finite values from an earlier use; the position comes from the device."""
     g = torch.Generator().manual_seed(3)
