@@ -117,74 +117,119 @@ __global__ __launch_bounds__(256) void rope_qk_kernel(
     }
 }
 
-// One 256-thread block per row of `hidden` elements (hidden % 8 == 0).
+// s = x (+ r, rounded to the dtype), eight elements
+template <typename T>
+__device__ __forceinline__ uint4 sum8(const uint4& x, const uint4& r) {
+    const uint32_t xw[4] = {x.x, x.y, x.z, x.w}, rw[4] = {r.x, r.y, r.z, r.w};
+    uint32_t o[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const uint16_t lo = f2lo<T>(lo2f<T>(static_cast<uint16_t>(xw[j] & 0xffffu)) + lo2f<T>(static_cast<uint16_t>(rw[j] & 0xffffu)));
+        const uint16_t hi = f2lo<T>(lo2f<T>(static_cast<uint16_t>(xw[j] >> 16)) + lo2f<T>(static_cast<uint16_t>(rw[j] >> 16)));
+        o[j] = static_cast<uint32_t>(lo) | (static_cast<uint32_t>(hi) << 16);
+    }
+    return make_uint4(o[0], o[1], o[2], o[3]);
+}
+template <typename T>
+__device__ __forceinline__ float squares8(const uint4& x, float ss) {
+    const uint32_t xw[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const float a = lo2f<T>(static_cast<uint16_t>(xw[j] & 0xffffu)), c = lo2f<T>(static_cast<uint16_t>(xw[j] >> 16));
+        ss = __builtin_fmaf(a, a, ss);
+        ss = __builtin_fmaf(c, c, ss);
+    }
+    return ss;
+}
+// w * dtype(x * inv)
+template <typename T>
+__device__ __forceinline__ uint4 scaled8(const uint4& x, const uint4& w, float inv) {
+    const uint32_t xw[4] = {x.x, x.y, x.z, x.w}, ww[4] = {w.x, w.y, w.z, w.w};
+    uint32_t o[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const float a = rnd_a<T>(lo2f<T>(static_cast<uint16_t>(xw[j] & 0xffffu)) * inv);
+        const float c = rnd_a<T>(lo2f<T>(static_cast<uint16_t>(xw[j] >> 16)) * inv);
+        const uint16_t lo = f2lo<T>(lo2f<T>(static_cast<uint16_t>(ww[j] & 0xffffu)) * a);
+        const uint16_t hi = f2lo<T>(lo2f<T>(static_cast<uint16_t>(ww[j] >> 16)) * c);
+        o[j] = static_cast<uint32_t>(lo) | (static_cast<uint32_t>(hi) << 16);
+    }
+    return make_uint4(o[0], o[1], o[2], o[3]);
+}
+
+// One block per row of `hidden` elements (hidden % 8 == 0).
 //   s = x (+ res, rounded to the dtype; written to sum_out if given)
 //   y = w * dtype( float(s) * rsqrt(mean(float(s)^2) + eps) )
+// The row's NP pieces a thread stay in registers, and the weights are requested with them: one trip to memory before the sum and none
+// after it, which is all that a launch of a few rows consists of (8 rows of 4096 with a residual 2.4 us in a chain of launches; 3.3 with the
+// row read again and the weights after the sum; 4096 rows of 8192 50 -> 42, 8192 of 4096 43 -> 41).
+template <typename T, int NP>
+__global__ __launch_bounds__(512) void rmsnorm_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ res,
+                                                      const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
+                                                      uint16_t* __restrict__ sum_out, int hidden, float eps) {
+    __shared__ float part[8];
+    const size_t row = static_cast<size_t>(blockIdx.x) * hidden;
+    uint4 xv[NP], rv[NP], wv[NP];
+    auto at = [&](int p) { const int i = (p * static_cast<int>(blockDim.x) + static_cast<int>(threadIdx.x)) * 8; return i < hidden ? i : 0; };
+    auto own = [&](int p) { return (p * static_cast<int>(blockDim.x) + static_cast<int>(threadIdx.x)) * 8 < hidden; };
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+        xv[p] = *reinterpret_cast<const uint4*>(x + row + at(p));
+        rv[p] = *reinterpret_cast<const uint4*>((res ? res : x) + row + at(p));        // (no branch around a load: it would be waited for at the join)
+        wv[p] = *reinterpret_cast<const uint4*>(w + at(p));
+    }
+    float ss = 0.0f;
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+        if (res) {
+            xv[p] = sum8<T>(xv[p], rv[p]);
+            if (sum_out && own(p)) *reinterpret_cast<uint4*>(sum_out + row + at(p)) = xv[p];
+        }
+        if (own(p)) ss = squares8<T>(xv[p], ss);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    float total = part[0] + part[1] + part[2] + part[3];
+    if (blockDim.x == 512) total += part[4] + part[5] + part[6] + part[7];
+    const float inv = rsqrtf(total / static_cast<float>(hidden) + eps);
+#pragma unroll
+    for (int p = 0; p < NP; p++)
+        if (own(p)) *reinterpret_cast<uint4*>(y + row + at(p)) = scaled8<T>(xv[p], wv[p], inv);
+}
+
+// The same for rows of any length: read twice.
 template <typename T>
-__global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ res,
+__global__ __launch_bounds__(256) void rmsnorm_long_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ res,
                                                        const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
                                                        uint16_t* __restrict__ sum_out, int hidden, float eps) {
     __shared__ float part[4];
     const size_t row = static_cast<size_t>(blockIdx.x) * hidden;
+    auto load = [&](const uint16_t* p, int i) { return *reinterpret_cast<const uint4*>(p + i); };
     float ss = 0.0f;
     for (int i = threadIdx.x * 8; i < hidden; i += 256 * 8) {
-        const uint4 xv = *reinterpret_cast<const uint4*>(x + row + i);
-        uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w};
+        uint4 v = load(x + row, i);
         if (res) {
-            const uint4 rv = *reinterpret_cast<const uint4*>(res + row + i);
-            const uint32_t rw[4] = {rv.x, rv.y, rv.z, rv.w};
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const uint16_t lo = f2lo<T>(lo2f<T>(static_cast<uint16_t>(xw[j] & 0xffffu)) + lo2f<T>(static_cast<uint16_t>(rw[j] & 0xffffu)));
-                const uint16_t hi = f2lo<T>(lo2f<T>(static_cast<uint16_t>(xw[j] >> 16)) + lo2f<T>(static_cast<uint16_t>(rw[j] >> 16)));
-                xw[j] = static_cast<uint32_t>(lo) | (static_cast<uint32_t>(hi) << 16);
-            }
-            if (sum_out) *reinterpret_cast<uint4*>(sum_out + row + i) = make_uint4(xw[0], xw[1], xw[2], xw[3]);
+            v = sum8<T>(v, load(res + row, i));
+            if (sum_out) *reinterpret_cast<uint4*>(sum_out + row + i) = v;
         }
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const float a = lo2f<T>(static_cast<uint16_t>(xw[j] & 0xffffu)), c = lo2f<T>(static_cast<uint16_t>(xw[j] >> 16));
-            ss = __builtin_fmaf(a, a, ss);
-            ss = __builtin_fmaf(c, c, ss);
-        }
+        ss = squares8<T>(v, ss);
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
     __syncthreads();
     const float inv = rsqrtf((part[0] + part[1] + part[2] + part[3]) / static_cast<float>(hidden) + eps);
-    const uint16_t* src = (res && sum_out) ? sum_out : nullptr;
     for (int i = threadIdx.x * 8; i < hidden; i += 256 * 8) {
-        uint32_t xw[4];
-        if (src) {                                   // re-read the rounded sums this thread wrote
-            const uint4 sv = *reinterpret_cast<const uint4*>(src + row + i);
-            xw[0] = sv.x; xw[1] = sv.y; xw[2] = sv.z; xw[3] = sv.w;
+        uint4 v;
+        if (res && sum_out) {
+            v = load(sum_out + row, i);              // the rounded sums this thread wrote
         } else {
-            const uint4 xv = *reinterpret_cast<const uint4*>(x + row + i);
-            xw[0] = xv.x; xw[1] = xv.y; xw[2] = xv.z; xw[3] = xv.w;
-            if (res) {
-                const uint4 rv = *reinterpret_cast<const uint4*>(res + row + i);
-                const uint32_t rw[4] = {rv.x, rv.y, rv.z, rv.w};
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const uint16_t lo = f2lo<T>(lo2f<T>(static_cast<uint16_t>(xw[j] & 0xffffu)) + lo2f<T>(static_cast<uint16_t>(rw[j] & 0xffffu)));
-                    const uint16_t hi = f2lo<T>(lo2f<T>(static_cast<uint16_t>(xw[j] >> 16)) + lo2f<T>(static_cast<uint16_t>(rw[j] >> 16)));
-                    xw[j] = static_cast<uint32_t>(lo) | (static_cast<uint32_t>(hi) << 16);
-                }
-            }
+            v = load(x + row, i);
+            if (res) v = sum8<T>(v, load(res + row, i));
         }
-        const uint4 wv = *reinterpret_cast<const uint4*>(w + i);
-        const uint32_t ww[4] = {wv.x, wv.y, wv.z, wv.w};
-        uint32_t yo[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const float a = rnd_a<T>(lo2f<T>(static_cast<uint16_t>(xw[j] & 0xffffu)) * inv);
-            const float c = rnd_a<T>(lo2f<T>(static_cast<uint16_t>(xw[j] >> 16)) * inv);
-            const uint16_t lo = f2lo<T>(lo2f<T>(static_cast<uint16_t>(ww[j] & 0xffffu)) * a);
-            const uint16_t hi = f2lo<T>(lo2f<T>(static_cast<uint16_t>(ww[j] >> 16)) * c);
-            yo[j] = static_cast<uint32_t>(lo) | (static_cast<uint32_t>(hi) << 16);
-        }
-        *reinterpret_cast<uint4*>(y + row + i) = make_uint4(yo[0], yo[1], yo[2], yo[3]);
+        *reinterpret_cast<uint4*>(y + row + i) = scaled8<T>(v, load(w, i), inv);
     }
 }
 
@@ -277,12 +322,21 @@ int launch_rope_qk(const void* q_lin, int64_t q_stride, const void* k_lin, int64
 
 int launch_rmsnorm(const void* x, const void* res, const void* w, void* y, void* sum_out, int rows, int hidden, float eps,
                    int dtype, hipStream_t st) {
-    if (dtype == 0)
-        hipLaunchKernelGGL(rmsnorm_kernel<F16>, dim3(rows), dim3(256), 0, st, (const uint16_t*)x, (const uint16_t*)res,
-                           (const uint16_t*)w, (uint16_t*)y, (uint16_t*)sum_out, hidden, eps);
-    else
-        hipLaunchKernelGGL(rmsnorm_kernel<BF16>, dim3(rows), dim3(256), 0, st, (const uint16_t*)x, (const uint16_t*)res,
-                           (const uint16_t*)w, (uint16_t*)y, (uint16_t*)sum_out, hidden, eps);
+    // few rows: more threads, fewer pieces one after another; many: the units are full either way
+    const int nthr = rows < 1024 && hidden > 2048 ? 512 : 256, per = (hidden / 8 + nthr - 1) / nthr;
+#define PQ_RN(KERNEL, THREADS)                                                                                       \
+    hipLaunchKernelGGL((KERNEL), dim3(rows), dim3(THREADS), 0, st, (const uint16_t*)x, (const uint16_t*)res,         \
+                       (const uint16_t*)w, (uint16_t*)y, (uint16_t*)sum_out, hidden, eps)
+#define PQ_RNT(T)                                                                                                    \
+    do {                                                                                                             \
+        if (per <= 1) PQ_RN((rmsnorm_kernel<T, 1>), nthr);                                                           \
+        else if (per <= 2) PQ_RN((rmsnorm_kernel<T, 2>), nthr);                                                      \
+        else if (per <= 4) PQ_RN((rmsnorm_kernel<T, 4>), nthr);                                                      \
+        else PQ_RN(rmsnorm_long_kernel<T>, 256);                                                                     \
+    } while (0)
+    if (dtype == 0) PQ_RNT(F16); else PQ_RNT(BF16);
+#undef PQ_RNT
+#undef PQ_RN
     return static_cast<int>(hipGetLastError());
 }
 

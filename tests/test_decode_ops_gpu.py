@@ -82,6 +82,23 @@ def test_rmsnorm_matches_module(gpu, dtype, hidden):
         assert torch.equal(got4, got2)
 
 
+@pytest.mark.parametrize("rows,hidden", [(3, 8), (3, 2048), (3, 2056), (3, 4104), (3, 8200), (3, 16384), (3, 16392), (1030, 2048), (1030, 2056),
+                                         (1030, 4104), (1030, 8192), (1030, 8200)])
+def test_rmsnorm_pieces_in_registers(gpu, rows, hidden):
+    """One, two or four pieces a thread, 256 or 512 threads, the last piece broken, and rows that are read twice, against plain torch in
+    float32 (the inner rounding may move by one step, which the weight can turn into two)."""
+    g = torch.Generator().manual_seed(hidden + rows)
+    x, res = [(torch.randn(rows, hidden, generator=g) * 3).to(torch.bfloat16).to(gpu) for _ in range(2)]
+    w = (1 + 0.1 * torch.randn(hidden, generator=g)).to(torch.bfloat16).to(gpu)
+    for r in (None, res):
+        s = x if r is None else x + r
+        want = w * (s.float() * torch.rsqrt(s.float().pow(2).mean(-1, keepdim=True) + 1e-5)).to(torch.bfloat16)
+        out = torch.empty_like(x)
+        got = rmsnorm(x, w, 1e-5, residual=r, sum_out=None if r is None else out)
+        assert _ulps_off(got, want) <= 2 and (got != want).float().mean().item() < 0.05
+        assert r is None or torch.equal(out, s)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_silu_mul_matches_eager(gpu, dtype):
     torch.manual_seed(1)
