@@ -426,6 +426,10 @@ int pq_validate_prompt_attn(const void *q, const void *k, const void *v, const i
  * s = x, or s = dtype(x + residual) (also written to sum_out if given; sum_out may
  * alias x): the decoder layer's residual add + LlamaRMSNorm (:466-484).
  *
+ * pq_embed_rmsnorm: x_out[r] = table[ids[r]] (ids outside [0, vocab) are clamped), y = its norm: a
+ * decode step's first launch.  pq_rmsnorm_advance: pq_rmsnorm, and counters[i] += increments[i] for
+ * i < n_counters: its last one before the logits.  At most 1023 rows of at most 8192 elements.
+ *
  * pq_silu_mul: y = dtype(silu(gate)) * up for `rows` rows of `cols` elements (LlamaMLP, called at
  * :483); gate / up rows are in_row_stride elements apart (0 = dense; 2*cols when they are the two
  * halves of one fused gate|up projection output), y is dense.
@@ -438,6 +442,13 @@ int pq_rope_append(const void *q_lin, const void *k_lin, const void *v_lin,
 
 int pq_rmsnorm(const void *x, const void *residual, const void *weight, void *y, void *sum_out,
                int rows, int hidden, float eps, int dtype, void *stream);
+
+int pq_embed_rmsnorm(const void *table, const int64_t *ids, int64_t vocab, const void *weight, void *y, void *x_out,
+                     int rows, int hidden, float eps, int dtype, void *stream);
+
+int pq_rmsnorm_advance(const void *x, const void *residual, const void *weight, void *y, void *sum_out,
+                       int rows, int hidden, float eps, int32_t *counters, const int32_t *increments, int n_counters,
+                       int dtype, void *stream);
 
 int pq_silu_mul(const void *gate, const void *up, void *y, int rows, int cols, int64_t in_row_stride,
                 int dtype, void *stream);

@@ -26,12 +26,17 @@
  *
  * pq_stream_add: x_out = x + y + e + v; y in the dtype, e float32, v [width] in the
  *   dtype, each or null; x_out may be x.  pq_embed_rows: out[r] = table[ids[r]] * scale.
+ * pq_embed_norm_conv: pq_norm_conv of x' = table[ids] * scale, which goes to x_out, for what
+ *   pq_embed_norm_conv_takes says yes to (taps 1 without a convolution).
  * pq_softcap: x <- cap * tanh(x * scale / cap) in place (cap <= 0: x * scale).
  *
  * pq_head_linear: y[m, h, :] = epilogue(x[m, h, :] w[h]^T) with w [heads, N, K];
  *   PQ_EPI_SIGMOID_GATE multiplies by sigmoid(gate[m, h * N + n]), PQ_EPI_F32 stores
  *   float32.  M <= 16, N % 16 == 0, K % 32 == 0 in a 16-bit dtype stream the weights
  *   through the matrix-core kernels; other sizes and float32 run a plain kernel.
+ *
+ * pq_logits: y = cap * tanh(x w^T * scale / cap) in float32 (cap <= 0: x w^T * scale), sizes that stream
+ *   only; *advance (or null) is raised by one.
  */
 #ifndef POLARQUANT_STEPS_H
 #define POLARQUANT_STEPS_H
@@ -57,6 +62,12 @@ int pq_validate_norm_conv(const float *x_in, const void *y, const void *w_post, 
                           const int32_t *start, const int32_t *pos_dev, int pos, int B, int L, int width, int groups,
                           int taps, int dtype);
 
+int pq_embed_norm_conv_takes(int width, int groups, int taps, int dtype);
+int pq_embed_norm_conv(const void *table, const int64_t *ids, int64_t vocab, float scale, float *x_out, const void *w_pre,
+                       const void *conv_w, const float *state_in, float *state_out, void *h_out, const int32_t *start,
+                       const int32_t *pos_dev, int pos, int B, int L, int width, int groups, int taps, float eps, int dtype,
+                       void *stream);
+
 int pq_relu_sq(const void *x, void *y, size_t n, int dtype, void *stream);
 
 int pq_gelu_mul(const void *gate, const void *up, int64_t in_stride, void *y, int64_t out_stride, int64_t rows, int cols,
@@ -70,6 +81,8 @@ int pq_softcap(float *x, size_t n, float scale, float cap, void *stream);
 int pq_head_linear(const void *x, int64_t x_row_stride, int64_t x_head_stride, const void *w, const void *gate,
                    int64_t gate_row_stride, void *y, int64_t y_row_stride, int64_t y_head_stride, int M, int heads, int N,
                    int K, int epilogue, int dtype, void *stream);
+int pq_logits(const void *x, const void *w, float *y, int M, int N, int K, float scale, float cap, int32_t *advance, int dtype,
+              void *stream);
 int pq_validate_head_linear(const void *x, int64_t x_row_stride, int64_t x_head_stride, const void *w, const void *gate,
                             int64_t gate_row_stride, const void *y, int64_t y_row_stride, int64_t y_head_stride, int M,
                             int heads, int N, int K, int epilogue, int dtype);

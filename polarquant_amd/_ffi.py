@@ -75,6 +75,8 @@ SIGNATURES = {
     "pq_rope_append": (c_int, [c_void_p] * 5 + [c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int64,
                                                c_void_p, c_int, c_int, c_int, c_int, c_int64, c_int64, c_void_p]),
     "pq_rmsnorm": (c_int, [c_void_p] * 5 + [c_int, c_int, c_float, c_int, c_void_p]),
+    "pq_embed_rmsnorm": (c_int, [c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int, c_int, c_float, c_int, c_void_p]),
+    "pq_rmsnorm_advance": (c_int, [c_void_p] * 5 + [c_int, c_int, c_float, c_void_p, c_void_p, c_int, c_int, c_void_p]),
     "pq_silu_mul": (c_int, [c_void_p] * 3 + [c_int, c_int, c_int64, c_int, c_void_p]),
     "pq_linear_small_m": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_void_p]),
     "pq_validate_linear_small_m": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int]),
@@ -107,6 +109,9 @@ STEPS_LIB_PATH = os.path.join(HERE, "libpolarquant_steps.so")
 STEPS_SIGNATURES = {
     "pq_norm_conv": (c_int, [c_void_p] * 11 + [c_int] * 6 + [c_float] + [c_int] + [c_void_p]),
     "pq_validate_norm_conv": (c_int, [c_void_p] * 11 + [c_int] * 7),
+    "pq_embed_norm_conv_takes": (c_int, [c_int] * 4),
+    "pq_embed_norm_conv": (c_int, [c_void_p, c_void_p, c_int64, c_float] + [c_void_p] * 8 + [c_int] * 6 + [c_float, c_int, c_void_p]),
+    "pq_logits": (c_int, [c_void_p] * 3 + [c_int] * 3 + [c_float, c_float, c_void_p, c_int, c_void_p]),
     "pq_relu_sq": (c_int, [c_void_p] * 2 + [c_size_t] + [c_int] + [c_void_p]),
     "pq_gelu_mul": (c_int, [c_void_p] * 2 + [c_int64, c_void_p, c_int64, c_int64, c_int, c_int, c_void_p]),
     "pq_stream_add": (c_int, [c_void_p] * 5 + [c_int64, c_int, c_int, c_void_p]),

@@ -140,9 +140,10 @@ struct Call<R(A...)> {
 
 #define PQ_CALLS(X)                                                                                                                        \
     X(pq_decode_scores) X(pq_quantize_groups) X(pq_quantize_values) X(pq_decode_attn) X(pq_decode_attn_v4) X(pq_decode_attn_plan)          \
-    X(pq_decode_attn_v4_plan) X(pq_decode_attn_workspace_bytes) X(pq_rope_append) X(pq_rope_qk) X(pq_rmsnorm) X(pq_silu_mul)               \
+    X(pq_decode_attn_v4_plan) X(pq_decode_attn_workspace_bytes) X(pq_rope_append) X(pq_rope_qk) X(pq_rmsnorm) X(pq_embed_rmsnorm)          \
+    X(pq_rmsnorm_advance) X(pq_silu_mul)                                                                                                 \
     X(pq_linear_small_m) X(pq_qkv_rope_append) X(pq_prompt_attn) X(pq_norm_conv) X(pq_relu_sq) X(pq_gelu_mul) X(pq_stream_add)             \
-    X(pq_embed_rows) X(pq_softcap) X(pq_head_linear) X(pq_latent_norm) X(pq_latent_decode_plan) X(pq_latent_decode_workspace_bytes)        \
+    X(pq_embed_rows) X(pq_embed_norm_conv_takes) X(pq_embed_norm_conv) X(pq_logits) X(pq_softcap) X(pq_head_linear) X(pq_latent_norm) X(pq_latent_decode_plan) X(pq_latent_decode_workspace_bytes)        \
     X(pq_latent_decode) X(pq_latent_prefill_takes) X(pq_latent_prefill) X(pq_qk_norm) X(pq_ring_append) X(pq_window_plan)                  \
     X(pq_window_workspace_bytes) X(pq_window_attn) X(pq_delta_prep) X(pq_scan_workspace_bytes) X(pq_delta_scan) X(pq_memory_gates)         \
     X(pq_memory_scan) X(pq_head_norm_gate)

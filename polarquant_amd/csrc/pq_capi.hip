@@ -415,15 +415,41 @@ int pq_prompt_attn(const void* q, const void* k, const void* v, const int64_t* s
     return err == 0 ? PQ_OK : PQ_ERR_LAUNCH;
 }
 
-int pq_rmsnorm(const void* x, const void* residual, const void* weight, void* y, void* sum_out, int rows, int hidden,
-               float eps, int dtype, void* stream) {
+static int check_rmsnorm(const void* x, const void* residual, const void* weight, const void* y, const void* sum_out, int rows, int hidden, int dtype) {
     if (!x || !weight || !y) return PQ_ERR_NULL_POINTER;
     if (rows <= 0 || hidden <= 0 || hidden % 8) return PQ_ERR_BAD_SHAPE;
     if (dtype != PQ_F16 && dtype != PQ_BF16) return PQ_ERR_BAD_DTYPE;
     if (!aligned(x, 16) || !aligned(weight, 16) || !aligned(y, 16) || (residual && !aligned(residual, 16)) ||
         (sum_out && !aligned(sum_out, 16)))
         return PQ_ERR_MISALIGNED;
+    return PQ_OK;
+}
+
+int pq_rmsnorm(const void* x, const void* residual, const void* weight, void* y, void* sum_out, int rows, int hidden,
+               float eps, int dtype, void* stream) {
+    if (int rc = check_rmsnorm(x, residual, weight, y, sum_out, rows, hidden, dtype)) return rc;
     const int err = pq::launch_rmsnorm(x, residual, weight, y, sum_out, rows, hidden, eps, dtype, static_cast<hipStream_t>(stream));
+    return err == 0 ? PQ_OK : PQ_ERR_LAUNCH;
+}
+
+int pq_embed_rmsnorm(const void* table, const int64_t* ids, int64_t vocab, const void* weight, void* y, void* x_out, int rows, int hidden,
+                     float eps, int dtype, void* stream) {
+    if (!ids || !x_out) return PQ_ERR_NULL_POINTER;
+    if (int rc = check_rmsnorm(table, nullptr, weight, y, x_out, rows, hidden, dtype)) return rc;
+    if (vocab < 1 || rows > pq::kStepNormRows || hidden > pq::kStepNormMax) return PQ_ERR_BAD_SHAPE;
+    if (!aligned(ids, 8)) return PQ_ERR_MISALIGNED;
+    const int err = pq::launch_embed_rmsnorm(table, ids, vocab, weight, y, x_out, rows, hidden, eps, dtype, static_cast<hipStream_t>(stream));
+    return err == 0 ? PQ_OK : PQ_ERR_LAUNCH;
+}
+
+int pq_rmsnorm_advance(const void* x, const void* residual, const void* weight, void* y, void* sum_out, int rows, int hidden, float eps,
+                       int32_t* counters, const int32_t* increments, int n_counters, int dtype, void* stream) {
+    if (!counters || !increments) return PQ_ERR_NULL_POINTER;
+    if (int rc = check_rmsnorm(x, residual, weight, y, sum_out, rows, hidden, dtype)) return rc;
+    if (n_counters < 1 || rows > pq::kStepNormRows || hidden > pq::kStepNormMax) return PQ_ERR_BAD_SHAPE;
+    if (!aligned(counters, 4) || !aligned(increments, 4)) return PQ_ERR_MISALIGNED;
+    const int err = pq::launch_rmsnorm_advance(x, residual, weight, y, sum_out, rows, hidden, eps, counters, increments, n_counters, dtype,
+                                               static_cast<hipStream_t>(stream));
     return err == 0 ? PQ_OK : PQ_ERR_LAUNCH;
 }
 

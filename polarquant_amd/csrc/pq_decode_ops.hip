@@ -163,19 +163,39 @@ __device__ __forceinline__ uint4 scaled8(const uint4& x, const uint4& w, float i
 // The row's NP pieces a thread stay in registers, and the weights are requested with them: one trip to memory before the sum and none
 // after it, which is all that a launch of a few rows consists of (8 rows of 4096 with a residual 2.4 us in a chain of launches; 3.3 with the
 // row read again and the weights after the sum; 4096 rows of 8192 50 -> 42, 8192 of 4096 43 -> 41).
-template <typename T, int NP>
+// EDGES: of a decode step's ends, where a launch of its own would take 2 to 4 us.  `ids`: x is a table of `vocab` rows, block r's row of
+// it is ids[r], and s goes to sum_out all the same; `counters`: the first block raises them by `by` (nothing else in the step reads them
+// from here on).
+struct NormEdges {
+    const int64_t* ids;
+    int64_t vocab;
+    int32_t* counters;
+    const int32_t* by;
+    int n_counters;
+};
+template <typename T, int NP, bool EDGES>
 __global__ __launch_bounds__(512) void rmsnorm_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ res,
                                                       const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
-                                                      uint16_t* __restrict__ sum_out, int hidden, float eps) {
+                                                      uint16_t* __restrict__ sum_out, int hidden, float eps, NormEdges e) {
     __shared__ float part[8];
     const size_t row = static_cast<size_t>(blockIdx.x) * hidden;
+    const uint16_t* xr = x + row;
+    if constexpr (EDGES) {
+        if (blockIdx.x == 0)
+            for (int i = threadIdx.x; i < e.n_counters; i += blockDim.x) e.counters[i] += e.by[i];
+        if (e.ids) {
+            int64_t id = e.ids[blockIdx.x];
+            id = id < 0 ? 0 : (id >= e.vocab ? e.vocab - 1 : id);          // (never past the table)
+            xr = x + static_cast<size_t>(id) * hidden;
+        }
+    }
     uint4 xv[NP], rv[NP], wv[NP];
     auto at = [&](int p) { const int i = (p * static_cast<int>(blockDim.x) + static_cast<int>(threadIdx.x)) * 8; return i < hidden ? i : 0; };
     auto own = [&](int p) { return (p * static_cast<int>(blockDim.x) + static_cast<int>(threadIdx.x)) * 8 < hidden; };
 #pragma unroll
     for (int p = 0; p < NP; p++) {
-        xv[p] = *reinterpret_cast<const uint4*>(x + row + at(p));
-        rv[p] = *reinterpret_cast<const uint4*>((res ? res : x) + row + at(p));        // (no branch around a load: it would be waited for at the join)
+        xv[p] = *reinterpret_cast<const uint4*>(xr + at(p));
+        rv[p] = *reinterpret_cast<const uint4*>((res ? res + row : xr) + at(p));       // (no branch around a load: it would be waited for at the join)
         wv[p] = *reinterpret_cast<const uint4*>(w + at(p));
     }
     float ss = 0.0f;
@@ -185,6 +205,7 @@ __global__ __launch_bounds__(512) void rmsnorm_kernel(const uint16_t* __restrict
             xv[p] = sum8<T>(xv[p], rv[p]);
             if (sum_out && own(p)) *reinterpret_cast<uint4*>(sum_out + row + at(p)) = xv[p];
         }
+        if (EDGES && e.ids && own(p)) *reinterpret_cast<uint4*>(sum_out + row + at(p)) = xv[p];
         if (own(p)) ss = squares8<T>(xv[p], ss);
     }
 #pragma unroll
@@ -320,24 +341,44 @@ int launch_rope_qk(const void* q_lin, int64_t q_stride, const void* k_lin, int64
     return static_cast<int>(hipGetLastError());
 }
 
-int launch_rmsnorm(const void* x, const void* res, const void* w, void* y, void* sum_out, int rows, int hidden, float eps,
-                   int dtype, hipStream_t st) {
+static int launch_norm(const void* x, const void* res, const void* w, void* y, void* sum_out, int rows, int hidden, float eps, bool edges,
+                       const NormEdges& e, int dtype, hipStream_t st) {
     // few rows: more threads, fewer pieces one after another; many: the units are full either way
     const int nthr = rows < 1024 && hidden > 2048 ? 512 : 256, per = (hidden / 8 + nthr - 1) / nthr;
-#define PQ_RN(KERNEL, THREADS)                                                                                       \
+#define PQ_RN(KERNEL, THREADS, ...)                                                                                  \
     hipLaunchKernelGGL((KERNEL), dim3(rows), dim3(THREADS), 0, st, (const uint16_t*)x, (const uint16_t*)res,         \
-                       (const uint16_t*)w, (uint16_t*)y, (uint16_t*)sum_out, hidden, eps)
+                       (const uint16_t*)w, (uint16_t*)y, (uint16_t*)sum_out, hidden, eps __VA_OPT__(, ) __VA_ARGS__)
+#define PQ_RNE(T, E)                                                                                                 \
+    do {                                                                                                             \
+        if (per <= 1) PQ_RN((rmsnorm_kernel<T, 1, E>), nthr, e);                                                     \
+        else if (per <= 2) PQ_RN((rmsnorm_kernel<T, 2, E>), nthr, e);                                                \
+        else PQ_RN((rmsnorm_kernel<T, 4, E>), nthr, e);                                                              \
+    } while (0)
 #define PQ_RNT(T)                                                                                                    \
     do {                                                                                                             \
-        if (per <= 1) PQ_RN((rmsnorm_kernel<T, 1>), nthr);                                                           \
-        else if (per <= 2) PQ_RN((rmsnorm_kernel<T, 2>), nthr);                                                      \
-        else if (per <= 4) PQ_RN((rmsnorm_kernel<T, 4>), nthr);                                                      \
-        else PQ_RN(rmsnorm_long_kernel<T>, 256);                                                                     \
+        if (per > 4) PQ_RN(rmsnorm_long_kernel<T>, 256);                                                             \
+        else if (edges) PQ_RNE(T, true);                                                                             \
+        else PQ_RNE(T, false);                                                                                       \
     } while (0)
     if (dtype == 0) PQ_RNT(F16); else PQ_RNT(BF16);
 #undef PQ_RNT
+#undef PQ_RNE
 #undef PQ_RN
     return static_cast<int>(hipGetLastError());
+}
+
+int launch_rmsnorm(const void* x, const void* res, const void* w, void* y, void* sum_out, int rows, int hidden, float eps,
+                   int dtype, hipStream_t st) {
+    return launch_norm(x, res, w, y, sum_out, rows, hidden, eps, false, NormEdges{}, dtype, st);
+}
+// (hidden <= kStepNormMax: every row in registers)
+int launch_embed_rmsnorm(const void* table, const int64_t* ids, int64_t vocab, const void* w, void* y, void* x_out, int rows, int hidden,
+                         float eps, int dtype, hipStream_t st) {
+    return launch_norm(table, nullptr, w, y, x_out, rows, hidden, eps, true, NormEdges{ids, vocab, nullptr, nullptr, 0}, dtype, st);
+}
+int launch_rmsnorm_advance(const void* x, const void* res, const void* w, void* y, void* sum_out, int rows, int hidden, float eps,
+                           int32_t* counters, const int32_t* by, int n_counters, int dtype, hipStream_t st) {
+    return launch_norm(x, res, w, y, sum_out, rows, hidden, eps, true, NormEdges{nullptr, 0, counters, by, n_counters}, dtype, st);
 }
 
 int launch_silu_mul(const void* gate, const void* up, void* y, int rows, int cols, int64_t in_stride, int dtype, hipStream_t st) {

@@ -12,7 +12,7 @@ int launch_head_linear_mfma(const HeadLinearArgs& a, int dtype, hipStream_t st) 
     while (ks > 1 && ((a.K % (kstep * ks)) != 0 || a.K / (kstep * ks) < 2)) ks >>= 1;
     const int nt = m8 && a.heads == 1 ? small_m8_row_tiles(a.M, a.N, ks, 1) : 2;      // (several heads: their K is short, nothing is gained)
     dim3 grid(a.N / (8 * nt), a.heads), block(kWave * ks);
-    const HeadEpi he{a.x_head, static_cast<int64_t>(a.N) * a.K, a.y_head, static_cast<const uint16_t*>(a.gate), a.gate_row};
+    const HeadEpi he{a.x_head, static_cast<int64_t>(a.N) * a.K, a.y_head, static_cast<const uint16_t*>(a.gate), a.gate_row, a.scale, a.cap, a.advance};
 #define PQ_H(KERNEL)                                                                                                 \
     hipLaunchKernelGGL((KERNEL), grid, block, 0, st, (const uint16_t*)a.x, a.x_row,                                  \
                        (const uint16_t*)a.w, nullptr, nullptr, (uint16_t*)a.y, a.y_row, a.M, a.K, he)
@@ -41,6 +41,7 @@ int launch_head_linear_mfma(const HeadLinearArgs& a, int dtype, hipStream_t st) 
         if (a.epilogue == kEpiReluSq) PQ_HE(T, kEpiReluSq);                                                          \
         else if (a.epilogue == kEpiSigmoidGate) PQ_HE(T, kEpiSigmoidGate);                                           \
         else if (a.epilogue == kEpiF32) PQ_HE(T, kEpiF32);                                                           \
+        else if (a.epilogue == kEpiLogits) PQ_HE(T, kEpiLogits);                                                     \
         else PQ_HE(T, kEpiPlain);                                                                                    \
     } while (0)
     if (dtype == 0) PQ_HT(F16); else PQ_HT(BF16);

@@ -31,6 +31,11 @@ int launch_rope_append(const void* q_lin, const void* k_lin, const void* v_lin, 
                        int64_t q_stride, int64_t kv_stride, hipStream_t st);
 int launch_rmsnorm(const void* x, const void* res, const void* w, void* y, void* sum_out, int rows, int hidden, float eps,
                    int dtype, hipStream_t st);
+constexpr int kStepNormMax = 8192, kStepNormRows = 1023;        // what the two below keep in registers
+int launch_embed_rmsnorm(const void* table, const int64_t* ids, int64_t vocab, const void* w, void* y, void* x_out, int rows, int hidden,
+                         float eps, int dtype, hipStream_t st);
+int launch_rmsnorm_advance(const void* x, const void* res, const void* w, void* y, void* sum_out, int rows, int hidden, float eps,
+                           int32_t* counters, const int32_t* by, int n_counters, int dtype, hipStream_t st);
 int launch_silu_mul(const void* gate, const void* up, void* y, int rows, int cols, int64_t in_stride, int dtype, hipStream_t st);
 
 int launch_convert_codes6(const uint8_t* src, uint8_t* dst, size_t n_rows, bool pack, hipStream_t st);

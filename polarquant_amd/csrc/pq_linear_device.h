@@ -20,7 +20,7 @@
 //
 // EPI 0 is the kernel as described (bias, or the gated form); EPI 1 + e is the same stream for one of `heads` independent
 // products per launch (blockIdx.y == head, operands `x_head` / N * K / `y_head` elements apart) with epilogue e of
-// pq_steps_internal.h: plain, square of relu, times sigmoid(gate), or unrounded float32 output.
+// pq_steps_internal.h: plain, square of relu, times sigmoid(gate), unrounded float32 output, or that scaled and soft-capped.
 #pragma once
 #include "pq_device.h"
 #include "pq_linear_rules.h"
@@ -48,14 +48,32 @@ struct HeadEpi {
     int64_t x_head, w_head, y_head;
     const uint16_t* gate;
     int64_t gate_row;
+    float scale, cap;
+    int32_t* advance;
 };
+
+// of logits: a counter that nothing in this launch reads is raised by its first thread
+template <int EPI>
+__device__ __forceinline__ void advance_once(const HeadEpi& he) {
+    if constexpr (EPI == 1 + kEpiLogits)
+        if (he.advance && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *he.advance += 1;
+}
 
 // stores outputs y[r][n .. n + 3] (n: column inside the head) through epilogue EPI - 1
 template <typename T, int EPI>
 __device__ __forceinline__ void store_head(const float (&s)[4], uint16_t* y, int64_t y_stride, int r, int n, int N, const HeadEpi& he) {
     const size_t o = static_cast<size_t>(r) * y_stride + blockIdx.y * he.y_head + n;
-    if constexpr (EPI == 1 + kEpiF32) {
-        *reinterpret_cast<float4*>(reinterpret_cast<float*>(y) + o) = make_float4(s[0], s[1], s[2], s[3]);
+    if constexpr (EPI == 1 + kEpiF32 || EPI == 1 + kEpiLogits) {
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            v[i] = s[i];
+            if constexpr (EPI == 1 + kEpiLogits) {
+                v[i] *= he.scale;
+                if (he.cap > 0.0f) v[i] = he.cap * tanhf(v[i] / he.cap);
+            }
+        }
+        *reinterpret_cast<float4*>(reinterpret_cast<float*>(y) + o) = make_float4(v[0], v[1], v[2], v[3]);
     } else {
         uint16_t out[4];
 #pragma unroll
@@ -83,6 +101,7 @@ template <typename T, int KSPLIT, bool GATED, int kStage, int EPI = 0>
 __global__ __launch_bounds__(kWave * KSPLIT) void small_m_linear_kernel(
     const uint16_t* __restrict__ x, int64_t x_stride, const uint16_t* __restrict__ w, const uint16_t* __restrict__ w_up,
     const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, int64_t y_stride, int M, int K, HeadEpi he) {
+    advance_once<EPI>(he);
     if constexpr (EPI != 0) {
         x += blockIdx.y * he.x_head;
         w += blockIdx.y * he.w_head;
@@ -202,6 +221,7 @@ template <typename T, int KSPLIT, bool GATED, int kStage, int EPI = 0, int NT = 
 __global__ __launch_bounds__(kWave * KSPLIT) void small_m8_linear_kernel(
     const uint16_t* __restrict__ x, int64_t x_stride, const uint16_t* __restrict__ w, const uint16_t* __restrict__ w_up,
     const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, int64_t y_stride, int M, int K, HeadEpi he) {
+    advance_once<EPI>(he);
     if constexpr (EPI != 0) {
         x += blockIdx.y * he.x_head;
         w += blockIdx.y * he.w_head;

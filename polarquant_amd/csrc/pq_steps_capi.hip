@@ -37,7 +37,23 @@ int pq_norm_conv(const float* x_in, const void* y, const void* w_post, float* x_
                                        width, groups, taps, dtype))
         return rc;
     pq::NormConvArgs a{x_in, y, w_post, x_out, w_pre, conv_w, state_in, state_out, h_out, start, pos_dev,
-                       pos, B, L, width, groups, taps, 0, eps};
+                       pos, B, L, width, groups, taps, 0, eps, nullptr, nullptr, 0, 0.0f};
+    return status(pq::launch_norm_conv(a, dtype, static_cast<hipStream_t>(stream)));
+}
+
+int pq_embed_norm_conv_takes(int width, int groups, int taps, int dtype) { return pq::norm_conv_embeds(width, groups, taps, dtype); }
+
+int pq_embed_norm_conv(const void* table, const int64_t* ids, int64_t vocab, float scale, float* x_out, const void* w_pre, const void* conv_w,
+                       const float* state_in, float* state_out, void* h_out, const int32_t* start, const int32_t* pos_dev, int pos,
+                       int B, int L, int width, int groups, int taps, float eps, int dtype, void* stream) {
+    if (!table || !ids) return PQ_ERR_NULL_POINTER;
+    if (int rc = pq_validate_norm_conv(x_out, nullptr, nullptr, x_out, w_pre, conv_w, state_in, state_out, h_out, start, pos_dev, pos, B, L,
+                                       width, groups, taps, dtype))
+        return rc;
+    if (vocab < 1 || !pq::norm_conv_embeds(width, groups, conv_w ? taps : 1, dtype)) return PQ_ERR_BAD_SHAPE;
+    if (!aligned(table, 16) || !aligned(ids, 8)) return PQ_ERR_MISALIGNED;
+    pq::NormConvArgs a{x_out, nullptr, nullptr, x_out, w_pre, conv_w, state_in, state_out, h_out, start, pos_dev,
+                       pos, B, L, width, groups, taps, 0, eps, table, ids, vocab, scale};
     return status(pq::launch_norm_conv(a, dtype, static_cast<hipStream_t>(stream)));
 }
 
@@ -104,9 +120,17 @@ int pq_head_linear(const void* x, int64_t x_row_stride, int64_t x_head_stride, c
     if (int rc = pq_validate_head_linear(x, x_row_stride, x_head_stride, w, gate, gate_row_stride, y, y_row_stride, y_head_stride, M,
                                          heads, N, K, epilogue, dtype))
         return rc;
-    pq::HeadLinearArgs a{x, x_row_stride, x_head_stride, w, gate, gate_row_stride, y, y_row_stride, y_head_stride, M, heads, N, K, epilogue};
+    pq::HeadLinearArgs a{x, x_row_stride, x_head_stride, w, gate, gate_row_stride, y, y_row_stride, y_head_stride, M, heads, N, K, epilogue, 1.0f, 0.0f, nullptr};
     const hipStream_t st = static_cast<hipStream_t>(stream);
     return status(head_linear_fits_mfma(a, dtype) ? pq::launch_head_linear_mfma(a, dtype, st) : pq::launch_head_linear_any(a, dtype, st));
+}
+
+int pq_logits(const void* x, const void* w, float* y, int M, int N, int K, float scale, float cap, int32_t* advance, int dtype, void* stream) {
+    if (int rc = pq_validate_head_linear(x, K, 0, w, nullptr, 0, y, N, N, M, 1, N, K, PQ_EPI_F32, dtype)) return rc;
+    pq::HeadLinearArgs a{x, K, 0, w, nullptr, 0, y, N, N, M, 1, N, K, pq::kEpiLogits, scale, cap, advance};
+    if (dtype == PQ_F32 || M > 16 || N % 16 || K % 32) return PQ_ERR_BAD_SHAPE;
+    if (!aligned(x, 16) || !aligned(w, 16) || !aligned(y, 16) || (advance && !aligned(advance, 4))) return PQ_ERR_MISALIGNED;
+    return status(pq::launch_head_linear_mfma(a, dtype, static_cast<hipStream_t>(stream)));
 }
 
 }  // extern "C"

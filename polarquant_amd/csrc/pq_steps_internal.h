@@ -22,7 +22,13 @@ struct NormConvArgs {
     const int32_t* pos_dev;  // position of this call's first token on the device, or null (then `pos`)
     int pos, B, L, W, groups, taps, strip;
     float eps;
+    const void* table;       // [vocab, W] in the dtype: x_in is embed_scale times its rows `ids` [B, L] and goes to x_out; or null
+    const int64_t* ids;
+    int64_t vocab;
+    float embed_scale;
 };
+// what the launch that looks x up itself has forms for
+inline bool norm_conv_embeds(int W, int groups, int taps, int dtype) { return dtype != 2 && W > 0 && groups > 0 && (W / groups) % 4 == 0 && W <= 8192 && taps <= 4; }
 // A call of at most this many tokens per sequence is worked through by one workgroup per sequence, so that x_out may be
 // x_in and state_out may be state_in; longer calls are cut into strips, whose first workgroup reads what the last writes.
 constexpr int kConvInPlaceTokens = 32;
@@ -53,7 +59,7 @@ int launch_embed_rows(const void* table, const int64_t* ids, float scale, float*
 int launch_softcap(float* x, size_t n, float scale, float cap, hipStream_t st);
 
 // y[m, h, n] = epilogue(sum_k x[m, h, k] w[h, n, k])
-enum { kEpiPlain = 0, kEpiReluSq = 1, kEpiSigmoidGate = 2, kEpiF32 = 3 };
+enum { kEpiPlain = 0, kEpiReluSq = 1, kEpiSigmoidGate = 2, kEpiF32 = 3, kEpiLogits = 4 };      // (the last: float32, scaled and soft-capped)
 struct HeadLinearArgs {
     const void* x;
     int64_t x_row, x_head;
@@ -63,6 +69,8 @@ struct HeadLinearArgs {
     void* y;                 // in the dtype; float32 with kEpiF32
     int64_t y_row, y_head;
     int M, heads, N, K, epilogue;
+    float scale, cap;        // kEpiLogits: cap tanh(sum scale / cap), without a cap sum scale
+    int32_t* advance;        // kEpiLogits: raised by one, or null
 };
 int launch_head_linear_any(const HeadLinearArgs& a, int dtype, hipStream_t st);      // pq_steps.hip: any size, any dtype
 int launch_head_linear_mfma(const HeadLinearArgs& a, int dtype, hipStream_t st);     // pq_head_linear.hip: M <= 16, N % 16 == 0, K % 32 == 0

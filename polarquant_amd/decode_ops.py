@@ -41,10 +41,29 @@ def rope_append(q_lin: torch.Tensor, k_lin: torch.Tensor, v_lin: torch.Tensor, c
     return q_out
 
 
+STEP_NORM_ROWS, STEP_NORM_MAX = 1023, 8192      # rows and elements of them that `embed_rmsnorm` and a norm with counters take
+
+
+def embed_rmsnorm(table: torch.Tensor, ids: torch.Tensor, weight: torch.Tensor, eps: float):
+    """(table[ids], weight * rms_norm of it); ids int64, outside of the table they count as its nearest row."""
+    _gpu(table)
+    hidden = table.shape[1]
+    assert table.is_contiguous() and weight.is_contiguous() and weight.dtype == table.dtype and weight.numel() == hidden
+    assert ids.is_contiguous() and ids.dtype == torch.int64 and ids.device == table.device
+    x = torch.empty(tuple(ids.shape) + (hidden,), dtype=table.dtype, device=table.device)
+    y = torch.empty_like(x)
+    with _on_device(table.device):
+        rc = _ffi.lib().call.pq_embed_rmsnorm(table, ids, table.shape[0], weight, y, x, ids.numel(), hidden, float(eps), _dtype_code(table),
+                                              _stream_ptr(table.device))
+    _ffi.check(rc, "pq_embed_rmsnorm")
+    return x, y
+
+
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, residual: Optional[torch.Tensor] = None,
-            sum_out: Optional[torch.Tensor] = None) -> torch.Tensor:
+            sum_out: Optional[torch.Tensor] = None, counters: Optional[torch.Tensor] = None,
+            increments: Optional[torch.Tensor] = None) -> torch.Tensor:
     """weight * rms_norm(x), or of x + residual (the sum, rounded to the dtype, goes to sum_out,
-    which may be x itself)."""
+    which may be x itself).  counters += increments (int32) in the same launch, for up to STEP_NORM_ROWS rows of STEP_NORM_MAX."""
     _gpu(x)
     hidden = x.shape[-1]
     assert x.is_contiguous() and weight.is_contiguous() and weight.dtype == x.dtype and weight.numel() == hidden
@@ -53,6 +72,14 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, residual: Optiona
     if sum_out is not None:
         assert sum_out.is_contiguous() and sum_out.shape == x.shape and sum_out.dtype == x.dtype
     y = torch.empty_like(x)
+    if counters is not None:
+        assert counters.is_contiguous() and increments.is_contiguous() and counters.dtype == increments.dtype == torch.int32
+        assert counters.shape == increments.shape and counters.device == increments.device == x.device
+        with _on_device(x.device):
+            rc = _ffi.lib().call.pq_rmsnorm_advance(x, residual, weight, y, sum_out, x.numel() // hidden, hidden, float(eps), counters, increments,
+                                                    counters.numel(), _dtype_code(x), _stream_ptr(x.device))
+        _ffi.check(rc, "pq_rmsnorm_advance")
+        return y
     with _on_device(x.device):
         rc = _ffi.lib().call.pq_rmsnorm(x, residual, weight, y, sum_out, x.numel() // hidden, hidden, float(eps), _dtype_code(x),
                                         _stream_ptr(x.device))

@@ -24,6 +24,7 @@ import torch
 
 from . import _ffi
 from .attention import _num_cus, new_workspace, plan_splits, polar_decode_attention, polar_decode_attention_v4
+from .layer_ops import only_looks_up
 from .modeling_common import GROUP, Linear, apply_rotary_pos_emb
 
 
@@ -220,13 +221,20 @@ class PolarGraphDecoder(GraphDecoder):
 
     def _step_body_fused(self):
         """The decode step with one launch per elementwise stage: 2 norms (each with the residual add
-        folded in), RoPE + append, SiLU * up, plus the GEMMs and the attention, per layer."""
-        from .decode_ops import linear_small_m, qkv_rope_append, rmsnorm, rope_append, silu_mul
+        folded in), RoPE + append, SiLU * up, plus the GEMMs and the attention, per layer.  The first norm reads the embedding's
+        rows itself and the last one raises the counters."""
+        from .decode_ops import STEP_NORM_MAX, STEP_NORM_ROWS, embed_rmsnorm, linear_small_m, qkv_rope_append, rmsnorm, rope_append, silu_mul
         model, B = self.model, self.B
         product = lambda module, t: module(t, library=True) if isinstance(module, Linear) and not self.small_m_gemm else module(t)
         layers = model.model.layers
-        x = model.model.embed_tokens(self.ids).contiguous()                 # residual stream [B,1,H], updated in place
-        h = rmsnorm(x, layers[0].input_layernorm.weight, layers[0].input_layernorm.variance_epsilon)
+        embed, first = model.model.embed_tokens, layers[0].input_layernorm
+        edges = B <= STEP_NORM_ROWS and first.weight.numel() <= STEP_NORM_MAX
+        if edges and only_looks_up(embed, first.weight.dtype):
+            x, h = embed_rmsnorm(embed.weight, self.ids, first.weight, first.variance_epsilon)
+        else:
+            x = embed(self.ids).contiguous()
+            h = rmsnorm(x, first.weight, first.variance_epsilon)
+        # x: residual stream [B,1,H], updated in place
         for li, (layer, ar) in enumerate(zip(layers, self.arenas)):
             att, mlp = layer.self_attn, layer.mlp
             nq, nkv = att.num_heads * att.head_dim, att.num_key_value_heads * att.head_dim
@@ -258,10 +266,13 @@ class PolarGraphDecoder(GraphDecoder):
                 h = rmsnorm(x, pn.weight, pn.variance_epsilon, residual=a, sum_out=x)
                 # (gate | up as one library GEMM was measured too: no faster than the two, so they stay separate)
                 m = product(mlp.down_proj, silu_mul(product(mlp.gate_proj, h), product(mlp.up_proj, h)))
-            nn_ = layers[li + 1].input_layernorm if li + 1 < len(layers) else model.model.norm
-            h = rmsnorm(x, nn_.weight, nn_.variance_epsilon, residual=m, sum_out=x)
+            last = li + 1 == len(layers)
+            nn_ = model.model.norm if last else layers[li + 1].input_layernorm
+            more = dict(counters=self._counters, increments=self._advance) if last and edges else {}
+            h = rmsnorm(x, nn_.weight, nn_.variance_epsilon, residual=m, sum_out=x, **more)
         logits = product(model.lm_head, h)
-        self._counters.add_(self._advance)
+        if not edges:
+            self._counters.add_(self._advance)
         return logits
 
     def _step_body(self):
@@ -360,9 +371,7 @@ class LayeredGraphDecoder(GraphDecoder):
 
     def _step_body(self):
         h = self.model.model.run(self.ids, self.arenas, 0, self.pos, self.plan)
-        logits = self.model.logits(h)
-        self.pos.add_(1)
-        return logits
+        return self.model.logits(h, self.pos)
 
     @torch.no_grad()
     def step(self, ids: torch.Tensor) -> torch.Tensor:

@@ -10,7 +10,7 @@ from . import _ffi
 from .attention import _num_cus
 from .kernel4group import _on_device, _stream_ptr
 
-from .layer_ops import (_DTYPES, _code, ConvState, IN_PLACE_TOKENS, SMALL_M, head_linear, linear, linear_f32,  # noqa: F401
+from .layer_ops import (_DTYPES, _code, ConvState, IN_PLACE_TOKENS, SMALL_M, embed_norm_conv, embeds, head_linear, linear, linear_f32,  # noqa: F401
                         norm_conv, relu_sq, streams)
 
 

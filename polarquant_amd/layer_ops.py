@@ -74,6 +74,44 @@ def norm_conv(x: torch.Tensor, w_pre: torch.Tensor, groups: int, eps: float, y: 
     return (x if y is None else x_out), h
 
 
+def only_looks_up(embed, dtype: torch.dtype) -> bool:
+    """An embedding module without anything of its own or hung onto it, whose table a launch can read as it lies."""
+    w = getattr(embed, "weight", None)
+    return (type(embed) is torch.nn.Embedding and embed.max_norm is None and not embed._forward_hooks and not embed._forward_pre_hooks
+            and "forward" not in embed.__dict__ and w.dtype == dtype and w.is_contiguous() and w.data_ptr() % 16 == 0)
+
+
+def embeds(embed, ids: torch.Tensor, w_pre: torch.Tensor, groups: int, taps: int = 1) -> bool:
+    """Whether `embed_norm_conv` takes the place of embed(ids) and the norm behind it."""
+    return (ids.dtype == torch.int64 and ids.is_cuda and ids.device == w_pre.device and w_pre.dtype in _DTYPES and only_looks_up(embed, w_pre.dtype)
+            and bool(_ffi.steps_lib().call.pq_embed_norm_conv_takes(w_pre.numel(), groups, taps, _DTYPES[w_pre.dtype])))
+
+
+def embed_norm_conv(table: torch.Tensor, ids: torch.Tensor, scale: float, w_pre: torch.Tensor, groups: int, eps: float,
+                    conv_w: Optional[torch.Tensor] = None, state: Optional[ConvState] = None, start: Optional[torch.Tensor] = None, pos: int = 0,
+                    pos_dev: Optional[torch.Tensor] = None):
+    """x = scale * table[ids] as float32 [B, L, W] and `norm_conv` of it, in one launch."""
+    B, L = ids.shape
+    W = table.shape[1]
+    ids = ids.contiguous()
+    assert table.is_contiguous() and ids.dtype == torch.int64 and w_pre.numel() == W and w_pre.dtype == table.dtype
+    s_in = s_out = None
+    taps = 1
+    if conv_w is not None:
+        assert conv_w.is_contiguous() and conv_w.shape[0] == W and conv_w.dtype == w_pre.dtype and conv_w.shape[1] == state.taps
+        taps = conv_w.shape[1]
+        s_in, s_out = state.targets(L)
+        assert s_in.shape == (B, taps - 1, W)
+    x = torch.empty(B, L, W, dtype=torch.float32, device=table.device)
+    h = torch.empty(B, L, W, dtype=w_pre.dtype, device=table.device)
+    with _on_device(x.device):
+        rc = _ffi.steps_lib().call.pq_embed_norm_conv(
+            table, ids, table.shape[0], float(scale), x, w_pre, conv_w, s_in if taps > 1 else None, s_out if taps > 1 else None, h, start, pos_dev,
+            pos, B, L, W, groups, taps, float(eps), _code(w_pre), _stream_ptr(x.device))
+    _ffi.check(rc, "pq_embed_norm_conv")
+    return x, h
+
+
 def relu_sq(x: torch.Tensor) -> torch.Tensor:
     """max(x, 0)^2, in place."""
     dt = _code(x)
@@ -183,3 +221,23 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if M <= 4 * SMALL_M and streams(min(M, SMALL_M), w):
         return head_linear(x.reshape(M, 1, K), w.unsqueeze(0), epilogue=_ffi.PQ_EPI_F32).view(x.shape[:-1] + (w.shape[0],))
     return torch.nn.functional.linear(x, w).float()
+
+
+def logits(x: torch.Tensor, w: torch.Tensor, scale: float = 1.0, cap: Optional[float] = None, advance: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """cap * tanh(x w^T * scale / cap) as float32, without a cap x w^T * scale; x [..., K], w [N, K].  advance: an int32 on the device,
+    raised by one.  Up to SMALL_M rows all of it is the product's launch."""
+    K = w.shape[1]
+    M = x.numel() // K
+    if 0 < M <= SMALL_M and streams(M, w) and x.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0:
+        y = torch.empty(x.shape[:-1] + (w.shape[0],), dtype=torch.float32, device=x.device)
+        assert x.dtype == w.dtype and (advance is None or (advance.dtype == torch.int32 and advance.device == x.device))
+        with _on_device(x.device):
+            rc = _ffi.steps_lib().call.pq_logits(x, w, y, M, w.shape[0], K, float(scale), float(cap or 0.0), advance, _code(x), _stream_ptr(x.device))
+        _ffi.check(rc, "pq_logits")
+        return y
+    y = linear_f32(x, w)
+    if scale != 1.0 or cap:
+        y = softcap(y, scale, cap)
+    if advance is not None:
+        advance.add_(1)
+    return y

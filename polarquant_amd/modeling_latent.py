@@ -207,13 +207,17 @@ class LatentModel(LayeredModel):
     def run(self, input_ids: torch.Tensor, arenas: List[LatentArena], pos: int, pos_dev: Optional[torch.Tensor] = None,
             plan: Optional[List[int]] = None) -> torch.Tensor:
         """plan: each layer's number of slices."""
-        x = self.embed_tokens(input_ids).float()
-        y = w_post = None
+        x = y = w_post = None
         start = arenas[0].start
         for i, (layer, arena) in enumerate(zip(self.layers, arenas)):
             for state, (pre, conv, sublayer, post) in zip(arena.conv, layer.sublayers()):
                 first_of_layer = sublayer is layer.mix
-                x, h = ops.norm_conv(x, pre.weight, pre.groups, pre.eps, y, w_post, conv.weight, state, start, pos, pos_dev)
+                if x is None and ops.embeds(self.embed_tokens, input_ids, pre.weight, pre.groups, state.taps):
+                    x, h = ops.embed_norm_conv(self.embed_tokens.weight, input_ids, 1.0, pre.weight, pre.groups, pre.eps, conv.weight, state, start,
+                                               pos, pos_dev)
+                else:
+                    x = self.embed_tokens(input_ids).float() if x is None else x
+                    x, h = ops.norm_conv(x, pre.weight, pre.groups, pre.eps, y, w_post, conv.weight, state, start, pos, pos_dev)
                 if first_of_layer and i and self.capture is not None:
                     self.capture.append(x.clone())
                 if first_of_layer:

@@ -102,9 +102,14 @@ class LayeredForCausalLM(PolarForCausalLM):
         h = h[:, -num_logits_to_keep:] if logit_positions is None else h.index_select(1, logit_positions)
         return CausalLMOutputWithPast(logits=self.logits(h), past_key_values=past)
 
+    def logit_form(self):
+        """Scale and soft cap (or None) of the logits."""
+        return 1.0, None
+
     @torch.no_grad()
-    def logits(self, h: torch.Tensor) -> torch.Tensor:
-        return ops.linear_f32(h.contiguous(), self.lm_head.weight)
+    def logits(self, h: torch.Tensor, advance: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """advance: a counter on the device that is raised by one (a step's position)."""
+        return ops.logits(h.contiguous(), self.lm_head.weight, *self.logit_form(), advance)
 
     def new_cache(self, batch: int, capacity: int):
         """An empty cache of `capacity` tokens per sequence, to hand in as past_key_values."""

@@ -384,14 +384,21 @@ class RecurrentModel(LayeredModel):
         B, L = input_ids.shape
         step = Step(B, L, pos, pos_dev, arenas[0].start if arenas else None)
         norm = lambda x, n, y: layer_ops.norm_conv(x, n.weight, 1, n.eps, y, start=step.start, pos=pos, pos_dev=pos_dev)
-        e = layer_ops.embed_rows(self.embed_tokens.weight, input_ids, self.config.embedding_scale)
+        first = self.layers[self.runs[0][0]].norm1 if self.runs and self.runs[0][1] is None else None
         again = any(t for _, t in self.runs)            # the embedding is needed later, and short calls norm in place
-        x, y = (e.clone() if again and self.runs[0][1] is None else e), None
+        y = h = None
+        if first is not None and not again and layer_ops.embeds(self.embed_tokens, input_ids, first.weight, 1):
+            x, h = layer_ops.embed_norm_conv(self.embed_tokens.weight, input_ids, self.config.embedding_scale, first.weight, 1, first.eps,
+                                             start=step.start, pos=pos, pos_dev=pos_dev)
+        else:
+            e = layer_ops.embed_rows(self.embed_tokens.weight, input_ids, self.config.embedding_scale)
+            x = e.clone() if again and self.runs[0][1] is None else e
         for (i, t), arena in zip(self.runs, arenas):
             if t is not None:
                 x, y = layer_ops.stream_add(x, y, e if t > 0 else None, self.loop_step[t]), None
-            x, h = norm(x, self.layers[i].norm1, y)
-            y = self.layers[i](h, arena, step)
+            if h is None:
+                x, h = norm(x, self.layers[i].norm1, y)
+            y, h = self.layers[i](h, arena, step), None
             if self.capture is not None:
                 self.capture.append(x + y.float())
         return norm(x, self.norm, y)[1]
@@ -400,9 +407,8 @@ class RecurrentModel(LayeredModel):
 class RecurrentForCausalLM(LayeredForCausalLM):
     model_class = RecurrentModel
 
-    @torch.no_grad()
-    def logits(self, h):
-        return layer_ops.softcap(super().logits(h), self.config.logit_scale, self.config.logit_softcap)
+    def logit_form(self):
+        return self.config.logit_scale, self.config.logit_softcap
 
     def kv_cache_bytes_per_token(self) -> int:
         """Nothing grows with the sequence (state_bytes counts what a sequence holds)."""

@@ -4,7 +4,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from polarquant_amd.decode_ops import rmsnorm, rope_append, silu_mul
+from polarquant_amd.decode_ops import embed_rmsnorm, rmsnorm, rope_append, silu_mul
 from polarquant_amd.modeling_common import RMSNorm, apply_rotary_pos_emb
 
 pytestmark = pytest.mark.gpu
@@ -97,6 +97,29 @@ def test_rmsnorm_pieces_in_registers(gpu, rows, hidden):
         got = rmsnorm(x, w, 1e-5, residual=r, sum_out=None if r is None else out)
         assert _ulps_off(got, want) <= 2 and (got != want).float().mean().item() < 0.05
         assert r is None or torch.equal(out, s)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,hidden", [(1, 8), (8, 2056), (3, 4096), (2, 8192), (1023, 512)])
+def test_norms_at_a_steps_ends(gpu, dtype, rows, hidden):
+    """Rows of a table and their norm in one launch, ids outside of it among them; a norm that raises counters: the bits of the separate
+    launches, and counters raised once per call."""
+    g = torch.Generator().manual_seed(hidden)
+    table, w = [torch.randn(*s, generator=g).to(dtype).to(gpu) for s in ((50, hidden), (hidden,))]
+    ids = torch.randint(0, 50, (rows, 1), generator=g)
+    ids[0] = 49
+    if rows > 2:
+        ids[1], ids[2] = -3, 1000
+    x, y = embed_rmsnorm(table, ids.to(gpu), w, 1e-5)
+    want = table[ids.clamp(0, 49).to(gpu)]
+    assert torch.equal(x, want) and torch.equal(y, rmsnorm(want, w, 1e-5))
+    res = torch.randn(rows, 1, hidden, generator=g).to(dtype).to(gpu)
+    by = torch.tensor([1, 0, 5] + [2] * 600, dtype=torch.int32, device=gpu)
+    counters, s = torch.arange(603, dtype=torch.int32, device=gpu), torch.empty_like(x)
+    for call in (1, 2):
+        z = rmsnorm(x, w, 1e-5, residual=res, sum_out=s, counters=counters, increments=by)
+        assert torch.equal(counters, torch.arange(603, dtype=torch.int32, device=gpu) + call * by)
+        assert torch.equal(s, x + res) and torch.equal(z, rmsnorm(x, w, 1e-5, residual=res))
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])

@@ -247,3 +247,38 @@ def test_norm_conv_strips_give_the_bits_of_shorter_calls(W, groups, taps, B, L):
     got = [ops.norm_conv(x[:, i:i + 32].contiguous(), w, groups, 1e-5, y[:, i:i + 32].contiguous(), w, state=parts, **conv) for i in range(0, L, 32)]
     assert torch.equal(xs, torch.cat([a for a, _ in got], 1)) and torch.equal(hs, torch.cat([b for _, b in got], 1))
     assert not taps or torch.equal(whole.rows, parts.rows)
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,L,W,groups,taps", [(1, 1, 8, 1, 0), (8, 1, 4096, 4, 4), (3, 5, 96, 2, 3), (2, 40, 2056, 1, 4), (1, 300, 4096, 4, 2), (2, 33, 8192, 8, 1), (8, 1, 2048, 1, 0)])
+def test_embedding_rows_with_the_first_norm(gpu, dt, B, L, W, groups, taps):
+    """Rows of a table, their norm and convolution in one launch: the bits of the separate ones, ids outside of the table as its nearest row,
+    states and left padding like theirs."""
+    g = torch.Generator().manual_seed(W + L)
+    table, w = [torch.randn(*s, generator=g).to(dt).to(gpu) for s in ((40, W), (W,))]
+    conv_w = torch.randn(W, taps, generator=g).to(dt).to(gpu) if taps else None
+    ids = torch.randint(0, 40, (B, L), generator=g)
+    ids[-1, -1] = 77
+    start = torch.tensor([2] + [0] * (B - 1), dtype=torch.int32, device=gpu) if L > 3 else None
+    assert ops.embeds(torch.nn.Embedding.from_pretrained(table), ids.to(gpu), w, groups, max(taps, 1))
+    states = [ops.ConvState(B, taps, W, gpu) for _ in range(2)] if taps else [None, None]
+    for call in range(2):                                   # the second reads what the first left in the state
+        x, h = ops.embed_norm_conv(table, ids.to(gpu), 1.5, w, groups, 1e-5, conv_w, states[0], start, call * L)
+        rows = table[ids.clamp(0, 39).to(gpu)].float() * 1.5
+        _, want = ops.norm_conv(rows.clone(), w, groups, 1e-5, None, None, conv_w, states[1], start, call * L)
+        assert torch.equal(x, rows) and torch.equal(h, want)
+        assert taps < 2 or torch.equal(states[0].rows, states[1].rows)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 16, 32), (8, 4096, 2048), (5, 48, 96), (9, 1024, 512), (16, 272, 4096), (17, 64, 64), (8, 32768, 64)])
+@pytest.mark.parametrize("scale,cap", [(1.0, None), (0.25, 30.0), (2.0, None)])
+def test_logits_in_one_launch(gpu, M, N, K, scale, cap):
+    """Scale, soft cap and the raised counter beside the product: the bits of the separate launches."""
+    from polarquant_amd import layer_ops
+    g = torch.Generator().manual_seed(N + M)
+    x, w = [(torch.randn(*s, generator=g) * 3).to(torch.bfloat16).to(gpu) for s in ((M, K), (N, K))]
+    at = torch.tensor([41], dtype=torch.int32, device=gpu)
+    got = layer_ops.logits(x, w, scale, cap, at)
+    want = layer_ops.softcap(layer_ops.linear_f32(x, w).clone(), scale, cap)
+    assert torch.equal(got, want) and int(at) == 42
+    assert torch.equal(layer_ops.logits(x, w, scale, cap), want)
