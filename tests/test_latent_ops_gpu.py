@@ -103,6 +103,12 @@ def test_latent_norm(gpu, q_rank, kv_rank, extra):
         assert torch.equal(again[:, pos:pos + L], cache[:, pos:pos + L])
 
 
+@pytest.mark.parametrize("q_rank,kv_rank,extra", [(1020, 4, 0), (1024, 4, 4), (1500, 548, 12), (3072, 1024, 0), (3080, 1020, 4)])
+def test_latent_norm_pieces_in_registers(gpu, q_rank, kv_rank, extra):
+    """One, two or four pieces a thread, the last one broken, and rows of more."""
+    test_latent_norm(gpu, q_rank, kv_rank, extra)
+
+
 @pytest.mark.parametrize("n", [1, 8, 13, 4096, 100003])
 def test_relu_sq(gpu, n):
     g = torch.Generator().manual_seed(n)

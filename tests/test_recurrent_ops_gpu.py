@@ -88,6 +88,29 @@ def window_oracle(p, wq, wk, H, G, D, Dv, window, scale, slopes, eps=1e-3):
     return ko.window_attention_fast(q, k, p[:, (H + G) * D:].view(T, G, Dv), scale, s, window)
 
 
+@pytest.mark.parametrize("H,G,D,Dv", [(2, 1, 4, 8), (8, 8, 128, 128), (9, 9, 128, 64), (16, 8, 128, 256), (32, 16, 128, 128), (33, 1, 128, 128), (17, 17, 128, 128),
+                                       (1, 1, 1028, 4)])
+def test_qk_norm_pieces_in_registers(gpu, H, G, D, Dv):
+    """One to four pieces of a query and one or two of a key a thread, broken last ones, and wider rows: norms, the ring's row of a short call
+    and the key rows of a long one."""
+    g = torch.Generator().manual_seed(H * D)
+    for dt in ("bf16", "f16"):
+        for B, L, at in ((3, 1, 5), (2, 40, 0)):
+            p = rand(g, B * L, (H + G) * D + G * Dv, dt=dt, s=2.0)
+            wq, wk = (1 + rand(g, H * D, s=0.2)).to(DT[dt]), (1 + rand(g, G * D, s=0.2)).to(DT[dt])
+            ring = ops.WindowRing(B, G, D, Dv, 16, DT[dt], gpu)
+            rows = p.to(gpu)
+            q, k = ops.qk_norm(rows[:, :H * D], rows[:, H * D:(H + G) * D], rows[:, (H + G) * D:], wq.to(gpu), wk.to(gpu), H, 1e-3, ring, Step(B, L, at))
+            want_q, want_k = ko.rms_norm(p[:, :H * D].double(), wq.double(), 1e-3), ko.rms_norm(p[:, H * D:(H + G) * D].double(), wk.double(), 1e-3)
+            assert err(q, want_q) < TOL[dt]
+            if k is None:
+                slot = at % ring.k.shape[2]
+                assert err(ring.k[:, :, slot].reshape(B, G * D), want_k) < TOL[dt]
+                assert torch.equal(ring.v[:, :, slot].reshape(B, G * Dv).cpu(), p[:, (H + G) * D:])
+            else:
+                assert err(k, want_k) < TOL[dt]
+
+
 @pytest.mark.parametrize("H,G,D,Dv,window", [(4, 2, 32, 64, 40), (6, 1, 64, 32, 33), (2, 2, 128, 128, 150), (20, 1, 40, 24, 64), (1, 1, 136, 256, 17),
                                              (3, 3, 20, 12, 7), (4, 4, 5, 9, 1), (8, 2, 48, 96, 65), (2, 1, 256, 128, 300)])
 def test_window_attention(gpu, H, G, D, Dv, window):
