@@ -377,3 +377,26 @@ def test_header_compiles_as_c_and_library_links_without_python(tmp_path):
     run = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     assert run.returncode == 0, (run.returncode, run.stdout, run.stderr[-2000:])
     assert run.stdout.startswith("capi ok")
+
+
+def test_step_ends_refuse_what_they_do_not_take():
+    """The launches at a step's ends: null pointers, sizes beyond their registers, dtypes, alignment."""
+    lib, P = _ffi.lib(), 1 << 20
+    embed = lambda table=P, ids=P, vocab=9, w=P, y=P, x=P, rows=2, hidden=4096, dtype=0: lib.pq_embed_rmsnorm(table, ids, vocab, w, y, x, rows, hidden, 1e-5, dtype, None)
+    assert embed(table=None) == embed(ids=None) == embed(w=None) == embed(y=None) == embed(x=None) == -1
+    assert embed(vocab=0) == embed(rows=0) == embed(rows=1024) == embed(hidden=8200) == embed(hidden=4100) == -2
+    assert embed(dtype=2) == -4 and embed(table=P + 2) == embed(ids=P + 4) == embed(x=P + 8) == -5
+    advance = lambda x=P, c=P, by=P, n=4, rows=2, hidden=4096, dtype=0: lib.pq_rmsnorm_advance(x, None, P, P, None, rows, hidden, 1e-5, c, by, n, dtype, None)
+    assert advance(x=None) == advance(c=None) == advance(by=None) == -1
+    assert advance(n=0) == advance(rows=1024) == advance(hidden=8200) == -2
+    assert advance(dtype=5) == -4 and advance(c=P + 2) == advance(by=P + 1) == -5
+    steps = _ffi.steps_lib()
+    assert [steps.pq_embed_norm_conv_takes(*a) for a in ((4096, 4, 4, 1), (4096, 4, 5, 1), (4096, 4, 4, 2), (8208, 1, 1, 0), (6, 1, 1, 0))] == [1, 0, 0, 0, 0]
+    conv = lambda table=P, ids=P, vocab=9, x=P, L=1, width=4096, taps=4, dtype=1: steps.pq_embed_norm_conv(table, ids, vocab, 1.0, x, P, P, P, P, P, None, None, 0, 2, L, width, 4, taps, 1e-5, dtype, None)
+    assert conv(table=None) == conv(ids=None) == conv(x=None) == -1
+    assert conv(vocab=0) == conv(taps=5) == conv(width=8208) == conv(dtype=2) == -2
+    assert conv(table=P + 8) == conv(ids=P + 4) == -5
+    logits = lambda x=P, w=P, y=P, M=8, N=64, K=64, at=None, dtype=1: steps.pq_logits(x, w, y, M, N, K, 1.0, 0.0, at, dtype, None)
+    assert logits(x=None) == logits(w=None) == logits(y=None) == -1
+    assert logits(M=17) == logits(N=40) == logits(K=48) == logits(dtype=2) == -2
+    assert logits(x=P + 2) == logits(y=P + 4) == logits(at=P + 2) == -5
