@@ -371,7 +371,7 @@ class LayeredGraphDecoder(GraphDecoder):
 
     def _step_body(self):
         h = self.model.model.run(self.ids, self.arenas, 0, self.pos, self.plan)
-        return self.model.logits(h, self.pos)
+        return self.model.step_logits(h, self.pos)
 
     @torch.no_grad()
     def step(self, ids: torch.Tensor) -> torch.Tensor:

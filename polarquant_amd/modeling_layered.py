@@ -107,9 +107,17 @@ class LayeredForCausalLM(PolarForCausalLM):
         return 1.0, None
 
     @torch.no_grad()
-    def logits(self, h: torch.Tensor, advance: Optional[torch.Tensor] = None) -> torch.Tensor:
-        """advance: a counter on the device that is raised by one (a step's position)."""
-        return ops.logits(h.contiguous(), self.lm_head.weight, *self.logit_form(), advance)
+    def logits(self, h: torch.Tensor) -> torch.Tensor:
+        return ops.logits(h.contiguous(), self.lm_head.weight, *self.logit_form())
+
+    @torch.no_grad()
+    def step_logits(self, h: torch.Tensor, pos: torch.Tensor) -> torch.Tensor:
+        """The logits of a decode step, whose position on the device is raised by one."""
+        if type(self).logits is LayeredForCausalLM.logits and "logits" not in self.__dict__:
+            return ops.logits(h.contiguous(), self.lm_head.weight, *self.logit_form(), pos)
+        z = self.logits(h)                              # (a model's own)
+        pos.add_(1)
+        return z
 
     def new_cache(self, batch: int, capacity: int):
         """An empty cache of `capacity` tokens per sequence, to hand in as past_key_values."""

@@ -183,6 +183,23 @@ def test_graph_replays_equal_the_eager_step(gpu, tmp_path):
             assert dc.rel_rms(runs[0][b], want) < LIMIT[dtype], (name, b)
 
 
+def test_a_models_own_logits_in_a_captured_step(gpu, tmp_path):
+    """A model whose logits are its own keeps them in the captured step, replayed several times, and the position is raised once a step."""
+    model, _ = load(tmp_path, dc.ALL["even"], 11, torch.bfloat16, gpu)
+    plain = model.logits
+    ids = torch.arange(1, 8, device=gpu)[None]
+    steps = []
+    for own in (False, True):
+        if own:
+            model.logits = lambda h: plain(h) * 2.0
+        dec = LayeredGraphDecoder(model, 64)
+        dec.prefill(ids)
+        steps.append([dec.step(torch.tensor([[t]], device=gpu)).clone() for t in (3, 5, 9, 2)])
+        assert int(dec.pos) == 7 + 4
+    for a, b in zip(*steps):
+        assert torch.equal(2.0 * a, b)
+
+
 def _greedy(cfg, w, prompt, n):
     out = []
     for _ in range(n):
