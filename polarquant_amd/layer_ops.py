@@ -84,6 +84,7 @@ def only_looks_up(embed, dtype: torch.dtype) -> bool:
 def embeds(embed, ids: torch.Tensor, w_pre: torch.Tensor, groups: int, taps: int = 1) -> bool:
     """Whether `embed_norm_conv` takes the place of embed(ids) and the norm behind it."""
     return (ids.dtype == torch.int64 and ids.is_cuda and ids.device == w_pre.device and w_pre.dtype in _DTYPES and only_looks_up(embed, w_pre.dtype)
+            and embed.weight.device == ids.device               # (elsewhere: the module refuses the call, or the hooks that move its table run)
             and bool(_ffi.steps_lib().call.pq_embed_norm_conv_takes(w_pre.numel(), groups, taps, _DTYPES[w_pre.dtype])))
 
 
@@ -94,7 +95,9 @@ def embed_norm_conv(table: torch.Tensor, ids: torch.Tensor, scale: float, w_pre:
     B, L = ids.shape
     W = table.shape[1]
     ids = ids.contiguous()
+    dt = _code(table)
     assert table.is_contiguous() and ids.dtype == torch.int64 and w_pre.numel() == W and w_pre.dtype == table.dtype
+    assert all(t is None or t.device == table.device for t in (ids, w_pre, conv_w, state and state.rows, start, pos_dev))
     s_in = s_out = None
     taps = 1
     if conv_w is not None:
@@ -107,7 +110,7 @@ def embed_norm_conv(table: torch.Tensor, ids: torch.Tensor, scale: float, w_pre:
     with _on_device(x.device):
         rc = _ffi.steps_lib().call.pq_embed_norm_conv(
             table, ids, table.shape[0], float(scale), x, w_pre, conv_w, s_in if taps > 1 else None, s_out if taps > 1 else None, h, start, pos_dev,
-            pos, B, L, W, groups, taps, float(eps), _code(w_pre), _stream_ptr(x.device))
+            pos, B, L, W, groups, taps, float(eps), dt, _stream_ptr(x.device))
     _ffi.check(rc, "pq_embed_norm_conv")
     return x, h
 
