@@ -75,10 +75,13 @@ def norm_conv(x: torch.Tensor, w_pre: torch.Tensor, groups: int, eps: float, y: 
 
 
 def only_looks_up(embed, dtype: torch.dtype) -> bool:
-    """An embedding module without anything of its own or hung onto it, whose table a launch can read as it lies."""
+    """An embedding module without anything of its own or hung onto it (or onto all modules), whose table is a plain tensor that a launch
+    can read as it lies."""
     w = getattr(embed, "weight", None)
     return (type(embed) is torch.nn.Embedding and embed.max_norm is None and not embed._forward_hooks and not embed._forward_pre_hooks
-            and "forward" not in embed.__dict__ and w.dtype == dtype and w.is_contiguous() and w.data_ptr() % 16 == 0)
+            and "forward" not in embed.__dict__ and not torch.nn.modules.module._has_any_global_hook()
+            and (type(w) is torch.nn.Parameter or type(w) is torch.Tensor)              # (a subclass says for itself what its rows are)
+            and w.dtype == dtype and w.is_contiguous() and w.data_ptr() % 16 == 0)
 
 
 def embeds(embed, ids: torch.Tensor, w_pre: torch.Tensor, groups: int, taps: int = 1) -> bool:

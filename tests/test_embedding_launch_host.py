@@ -35,3 +35,26 @@ def test_the_launch_refuses_tensors_of_several_devices():
         layer_ops.embed_norm_conv(table, ids, 1.0, w, 4, 1e-5, conv, layer_ops.ConvState(2, 4, 4096, "cpu"))
     with pytest.raises(AssertionError):
         layer_ops.embed_norm_conv(table, ids, 1.0, w, 4, 1e-5, start=start)
+
+
+class Logged(torch.Tensor):
+    pass
+
+
+def test_only_a_plain_table_of_a_module_that_nobody_follows():
+    takes = lambda e: layer_ops.only_looks_up(e, torch.bfloat16)
+    e = module()
+    assert takes(e) and takes(torch.nn.Embedding.from_pretrained(e.weight.data))
+    assert not layer_ops.only_looks_up(e, torch.float16)
+    for register in (torch.nn.modules.module.register_module_forward_hook, torch.nn.modules.module.register_module_forward_pre_hook):
+        handle = register(lambda *a: None)
+        assert not takes(e)
+        handle.remove()
+        assert takes(e)
+    handle = e.register_forward_hook(lambda *a: None)
+    assert not takes(e)
+    handle.remove()
+    assert not takes(torch.nn.Embedding.from_pretrained(Logged(e.weight.data)))
+    own = module()
+    own.forward = lambda ids: None
+    assert not takes(own) and not takes(torch.nn.Embedding(40, 4096, max_norm=1.0, dtype=torch.bfloat16))
