@@ -241,7 +241,8 @@ PyObject* plain_scores(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (!p.ok) Py_RETURN_NONE;
     const int dt = half_code(*q);
     const int64_t row = codes->size(4);
-    p.ok = dt >= 0 && codes->scalar_type() == at::kByte && codes->size(3) == 128 && (row == 64 || row == 48) && q->size(2) == 1 && q->size(3) == 128;
+    p.ok = dt >= 0 && codes->scalar_type() == at::kByte && codes->size(3) == 128 && (row == 64 || row == 48) && q->size(2) == 1 && q->size(3) == 128 &&
+           q->size(0) == codes->size(0);          // (more queries than sequences: the general path answers the first ones)
     for (int i = 2; i < 6 && p.ok; i++)
         if (const at::Tensor* m = p.take(args[i], 5)) p.type(m, q->scalar_type());
     if (!p.ok) Py_RETURN_NONE;

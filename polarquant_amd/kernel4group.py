@@ -62,6 +62,8 @@ def attention_decode_forward_hip_impl(
     # last dim 64: one byte per pair code (the reference's layout); 48: packed 6-bit codes
     if G != 128 or D not in (64, 48) or query_states.shape[2] != 1 or query_states.shape[3] != 128:
         raise ValueError("polarquant_amd: expected group 128, head_dim 128 and one query token")
+    if query_states.shape[0] < B:
+        raise ValueError("polarquant_amd: %d sequences of codes and %d queries" % (B, query_states.shape[0]))
     flags = _ffi.PQ_CODES_PACKED6 if D == 48 else 0
     if indices.dtype != torch.uint8:
         raise TypeError("indices must be uint8")

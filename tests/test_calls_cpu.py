@@ -62,3 +62,12 @@ def test_empty():
         assert t.shape == (2, 0, 3) and t.dtype == dtype and t.device == like.device and t.is_contiguous()
     with pytest.raises(RuntimeError):
         calls.empty(like, 0, -1)
+
+
+def test_scores_want_a_query_for_every_sequence():
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from polarquant_amd.kernel4group import attention_decode_forward_triton_impl as scores
+    with FakeTensorMode():
+        q, codes, meta = [torch.zeros(*s, dtype=d, device="cuda") for s, d in (((1, 8, 1, 128), torch.float16), ((2, 8, 2, 128, 64), torch.uint8), ((2, 8, 2, 1, 64), torch.float16))]
+    with pytest.raises(ValueError, match="queries"):
+        scores(q, codes, meta, meta, meta, meta)

@@ -81,3 +81,13 @@ def test_scores_linearity_in_query(gpu):
     q2 = (torch.randint(-8, 9, (1, 32, 1, 128), generator=g).float() / 4).half()
     s1, s2, s12 = (_run(gpu, q, quant, 4, 4) for q in (q1, q2, q1 + q2))
     assert _rel_err(s1 + s2, s12) < 1e-5
+
+
+def test_scores_of_fewer_sequences_than_queries(gpu):
+    """The cache says how many sequences there are; queries beyond them are passed over."""
+    torch.manual_seed(3)
+    q = torch.randn(3, 16, 1, 128).half()
+    codes = torch.randint(0, 256, (2, 8, 2, 128, 64), dtype=torch.uint8)
+    meta = [torch.rand(2, 8, 2, 1, 64).half() for _ in range(4)]
+    got = _run(gpu, q, (codes, *meta), 4, 4)
+    assert got.shape == (2, 16, 1, 256) and torch.equal(got, _run(gpu, q[:2], (codes, *meta), 4, 4))
