@@ -57,12 +57,24 @@ bool integer(PyObject* o, uint64_t& v) {
     return true;
 }
 
-bool pointer(PyObject* o, Arg& a, void*& p) {
+// What a parameter takes besides None and a tensor: an untyped or byte pointer an address (handles, rows of a tensor); integers and floats (a
+// caller's own counts, positions, states) nothing, as a number or a tuple in their place is a mistake that the GPU would have to find; and
+// strides, of the functions that have them, a tuple.
+enum class Also { kNothing, kAddress, kStrides };
+
+bool pointer(PyObject* o, Arg& a, Also also, void*& p) {
     if (o == Py_None) {
         p = nullptr;
     } else if (plain_tensor(o)) {
         p = THPVariable_Unpack(o).data_ptr();
-    } else if (PyTuple_Check(o)) {                  // integers, for the length of the call
+    } else if (THPVariable_Check(o)) {              // a subclass says for itself what its pointer is
+        PyObject* at = PyObject_CallMethod(o, "data_ptr", nullptr);
+        uint64_t v = 0;
+        const bool ok = at && integer(at, v);
+        Py_XDECREF(at);
+        if (!ok) return refuse(o, "a pointer");
+        p = reinterpret_cast<void*>(v);
+    } else if (also == Also::kStrides && PyTuple_Check(o)) {      // for the length of the call
         const Py_ssize_t n = PyTuple_GET_SIZE(o);
         if (n > kListed) return refuse(o, "fewer integers");
         for (Py_ssize_t i = 0; i < n; i++) {
@@ -71,26 +83,25 @@ bool pointer(PyObject* o, Arg& a, void*& p) {
             a.list[i] = static_cast<int64_t>(v);
         }
         p = a.list;
-    } else if (THPVariable_Check(o)) {              // a subclass says for itself what its pointer is
-        PyObject* at = PyObject_CallMethod(o, "data_ptr", nullptr);
-        uint64_t v = 0;
-        const bool ok = at && integer(at, v);
-        Py_XDECREF(at);
-        if (!ok) return refuse(o, "a pointer");
-        p = reinterpret_cast<void*>(v);
-    } else {
+    } else if (also == Also::kAddress) {
         uint64_t v;
         if (!integer(o, v)) return false;
         p = reinterpret_cast<void*>(v);
+    } else {
+        return refuse(o, "a tensor");
     }
     return true;
 }
 
-template <typename T>
+template <typename T, bool STRIDES>
 bool convert(PyObject* o, Arg& a, T& out) {
     if constexpr (std::is_pointer_v<T>) {
+        using P = std::remove_cv_t<std::remove_pointer_t<T>>;
+        constexpr Also also = std::is_void_v<P> || std::is_same_v<P, uint8_t> ? Also::kAddress
+                              : STRIDES && std::is_same_v<P, int64_t>          ? Also::kStrides
+                                                                              : Also::kNothing;
         void* p;
-        if (!pointer(o, a, p)) return false;
+        if (!pointer(o, a, also, p)) return false;
         out = static_cast<T>(p);
         return true;
     } else if constexpr (std::is_floating_point_v<T>) {
@@ -109,15 +120,15 @@ bool convert(PyObject* o, Arg& a, T& out) {
     }
 }
 
-template <typename F> struct Call;
-template <typename R, typename... A>
-struct Call<R(A...)> {
+template <typename F, bool STRIDES> struct Call;
+template <bool STRIDES, typename R, typename... A>
+struct Call<R(A...), STRIDES> {
     static_assert(std::is_integral_v<R>, "a status, a count or a size");
     template <size_t... I>
     static PyObject* run(void* at, PyObject* const* args, std::index_sequence<I...>) {
         std::tuple<std::decay_t<A>...> v;
         Arg kept[sizeof...(A) + 1];
-        if (!(convert(args[I], kept[I], std::get<I>(v)) && ...)) return nullptr;
+        if (!(convert<std::decay_t<A>, STRIDES>(args[I], kept[I], std::get<I>(v)) && ...)) return nullptr;
         R r;
         Py_BEGIN_ALLOW_THREADS
         r = reinterpret_cast<R (*)(A...)>(at)(std::get<I>(v)...);
@@ -138,18 +149,22 @@ struct Call<R(A...)> {
     }
 };
 
-#define PQ_CALLS(X)                                                                                                                        \
-    X(pq_decode_scores) X(pq_quantize_groups) X(pq_quantize_values) X(pq_decode_attn) X(pq_decode_attn_v4) X(pq_decode_attn_plan)          \
+// The functions that the wrappers call: X without a parameter for strides, S with one.
+#define PQ_CALLS(X, S)                                                                                                                     \
+    X(pq_decode_scores) S(pq_quantize_groups) S(pq_quantize_values) X(pq_decode_attn) X(pq_decode_attn_v4) X(pq_decode_attn_plan)          \
     X(pq_decode_attn_v4_plan) X(pq_decode_attn_workspace_bytes) X(pq_rope_append) X(pq_rope_qk) X(pq_rmsnorm) X(pq_embed_rmsnorm)          \
-    X(pq_rmsnorm_advance) X(pq_silu_mul)                                                                                                 \
-    X(pq_linear_small_m) X(pq_qkv_rope_append) X(pq_prompt_attn) X(pq_norm_conv) X(pq_relu_sq) X(pq_gelu_mul) X(pq_stream_add)             \
-    X(pq_embed_rows) X(pq_embed_norm_conv_takes) X(pq_embed_norm_conv) X(pq_logits) X(pq_softcap) X(pq_head_linear) X(pq_latent_norm) X(pq_latent_decode_plan) X(pq_latent_decode_workspace_bytes)        \
-    X(pq_latent_decode) X(pq_latent_prefill_takes) X(pq_latent_prefill) X(pq_qk_norm) X(pq_ring_append) X(pq_window_plan)                  \
-    X(pq_window_workspace_bytes) X(pq_window_attn) X(pq_delta_prep) X(pq_scan_workspace_bytes) X(pq_delta_scan) X(pq_memory_gates)         \
-    X(pq_memory_scan) X(pq_head_norm_gate)
+    X(pq_rmsnorm_advance) X(pq_silu_mul) X(pq_linear_small_m) X(pq_qkv_rope_append) S(pq_prompt_attn) X(pq_norm_conv) X(pq_relu_sq)         \
+    X(pq_gelu_mul) X(pq_stream_add) X(pq_embed_rows) X(pq_embed_norm_conv_takes) X(pq_embed_norm_conv) X(pq_logits) X(pq_softcap)           \
+    X(pq_head_linear) X(pq_latent_norm) X(pq_latent_decode_plan) X(pq_latent_decode_workspace_bytes) X(pq_latent_decode)                   \
+    X(pq_latent_prefill_takes) X(pq_latent_prefill) X(pq_qk_norm) X(pq_ring_append) X(pq_window_plan) X(pq_window_workspace_bytes)         \
+    X(pq_window_attn) X(pq_delta_prep) X(pq_scan_workspace_bytes) X(pq_delta_scan) X(pq_memory_gates) X(pq_memory_scan)                    \
+    X(pq_head_norm_gate)
 
-#define PQ_METHOD(f) {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&Call<decltype(f)>::entry)), METH_FASTCALL, nullptr},
-PyMethodDef bound[] = {PQ_CALLS(PQ_METHOD)};
+#define PQ_BOUND(f, strides) \
+    {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&Call<decltype(f), strides>::entry)), METH_FASTCALL, nullptr},
+#define PQ_METHOD(f) PQ_BOUND(f, false)
+#define PQ_STRIDES(f) PQ_BOUND(f, true)
+PyMethodDef bound[] = {PQ_CALLS(PQ_METHOD, PQ_STRIDES)};
 
 // bind(name, address) -> the function at `address` of a loaded library as a builtin, None for a name that is not called from here
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {

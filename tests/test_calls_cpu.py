@@ -71,3 +71,17 @@ def test_scores_want_a_query_for_every_sequence():
         q, codes, meta = [torch.zeros(*s, dtype=d, device="cuda") for s, d in (((1, 8, 1, 128), torch.float16), ((2, 8, 2, 128, 64), torch.uint8), ((2, 8, 2, 1, 64), torch.float16))]
     with pytest.raises(ValueError, match="queries"):
         scores(q, codes, meta, meta, meta, meta)
+
+
+@pytest.mark.parametrize("wrong", [1 << 20, (1, 2), [1, 2], 0.5])
+def test_counts_and_positions_are_tensors(wrong):
+    """A number or a tuple where a count per sequence, a position or a state belongs is refused, not read as an address."""
+    call = _ffi.lib().call
+    nothing = [None] * 6
+    for groups, resid in ((wrong, None), (None, wrong)):
+        with pytest.raises(ctypes.ArgumentError):
+            call.pq_decode_attn(*nothing, 1, 1, groups, None, 0, 0, resid, None, 1, None, 0, 1.0, 1, 8, 8, 4, 4, 0, 1, 1, None, 0, None, 0, None, None)
+    with pytest.raises(ctypes.ArgumentError):
+        _ffi.latent_lib().call.pq_latent_decode(None, None, 1, None, None, wrong, 0, None, 1, 1, 1, 64, 1.0, 1, None, 0, 0, None)
+    with pytest.raises(ctypes.ArgumentError):
+        _ffi.steps_lib().call.pq_embed_rows(None, wrong, 1.0, None, 1, 8, 1, 0, None)
