@@ -197,7 +197,8 @@ def declare(handle: ctypes.CDLL, signatures) -> ctypes.CDLL:
         fn = getattr(handle, name)
         fn.restype = res
         fn.argtypes = args
-        setattr(handle.call, name, calls.bind(name, ctypes.cast(fn, c_void_p).value) or fn)
+        prototype = "".join(t._type_ for t in (res, *args))
+        setattr(handle.call, name, calls.bind(name, ctypes.cast(fn, c_void_p).value, prototype) or fn)
     return handle
 
 

@@ -7,6 +7,7 @@
 #include <torch/csrc/autograd/forward_grad.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
+#include <torch/version.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/autocast_mode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
@@ -160,28 +161,53 @@ struct Call<R(A...), STRIDES> {
     X(pq_window_attn) X(pq_delta_prep) X(pq_scan_workspace_bytes) X(pq_delta_scan) X(pq_memory_gates) X(pq_memory_scan)                    \
     X(pq_head_norm_gate)
 
-#define PQ_BOUND(f, strides) \
-    {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&Call<decltype(f), strides>::entry)), METH_FASTCALL, nullptr},
+// A prototype as ctypes writes types: the result's letter, then the parameters'.
+template <typename T>
+constexpr char letter() {
+    if constexpr (std::is_pointer_v<T>) return 'P';
+    else if constexpr (std::is_same_v<T, float>) return 'f';
+    else if constexpr (sizeof(T) == 4) return std::is_signed_v<T> ? 'i' : 'I';
+    else return std::is_signed_v<T> ? 'l' : 'L';
+}
+template <typename F> struct Prototype;
+template <typename R, typename... A>
+struct Prototype<R(A...)> {
+    static constexpr char text[] = {letter<R>(), letter<std::decay_t<A>>()..., 0};
+};
+
+struct Bound {
+    PyMethodDef method;
+    const char* prototype;
+};
+#define PQ_BOUND(f, strides)                                                                                                               \
+    {{#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&Call<decltype(f), strides>::entry)), METH_FASTCALL, nullptr},        \
+     Prototype<decltype(f)>::text},
 #define PQ_METHOD(f) PQ_BOUND(f, false)
 #define PQ_STRIDES(f) PQ_BOUND(f, true)
-PyMethodDef bound[] = {PQ_CALLS(PQ_METHOD, PQ_STRIDES)};
+Bound bound[] = {PQ_CALLS(PQ_METHOD, PQ_STRIDES)};
 
-// bind(name, address) -> the function at `address` of a loaded library as a builtin, None for a name that is not called from here
+// bind(name, address, prototype) -> the function at `address` of a loaded library as a builtin, None for a name that is not called from here.
+// The prototype is the caller's: another one than this file was compiled with raises, as the arguments would not be the library's.
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
-    if (n != 2 || !PyUnicode_Check(args[0])) {
-        PyErr_SetString(PyExc_TypeError, "bind(name, address)");
+    if (n != 3 || !PyUnicode_Check(args[0]) || !PyUnicode_Check(args[2])) {
+        PyErr_SetString(PyExc_TypeError, "bind(name, address, prototype)");
         return nullptr;
     }
-    const char* name = PyUnicode_AsUTF8(args[0]);
+    const char *name = PyUnicode_AsUTF8(args[0]), *prototype = PyUnicode_AsUTF8(args[2]);
     uint64_t at;
-    if (!name || !integer(args[1], at)) return nullptr;
-    for (PyMethodDef& m : bound) {
-        if (std::strcmp(m.ml_name, name) != 0) continue;
+    if (!name || !prototype || !integer(args[1], at)) return nullptr;
+    for (Bound& f : bound) {
+        if (std::strcmp(f.method.ml_name, name) != 0) continue;
+        if (std::strcmp(f.prototype, prototype) != 0) {
+            PyErr_Format(PyExc_RuntimeError, "polarquant_amd: _calls.so is of another version (%s is %s there, %s here); build it with "
+                         "`python -m polarquant_amd.build --calls`", name, f.prototype, prototype);
+            return nullptr;
+        }
         PyObject* self = PyCapsule_New(reinterpret_cast<void*>(at), nullptr, nullptr);
         if (!self) return nullptr;
-        PyObject* f = PyCFunction_New(&m, self);
+        PyObject* r = PyCFunction_New(&f.method, self);
         Py_DECREF(self);
-        return f;
+        return r;
     }
     Py_RETURN_NONE;
 }
@@ -391,11 +417,23 @@ PyObject* attribute(const char* from, const char* name) {
     return a;
 }
 
+// torch's C++ types are those of the version this was compiled against
+bool right_torch() {
+    PyObject* version = attribute("torch", "__version__");
+    PyObject* text = version ? PyObject_Str(version) : nullptr;
+    const char* has = text ? PyUnicode_AsUTF8(text) : nullptr;
+    const bool same = has && std::strncmp(has, TORCH_VERSION, std::strlen(TORCH_VERSION)) == 0;
+    if (has && !same) PyErr_Format(PyExc_ImportError, "compiled against torch %s, loaded beside %s", TORCH_VERSION, has);
+    Py_XDECREF(text);
+    Py_XDECREF(version);
+    return same;
+}
+
 }  // namespace
 
 extern "C" __attribute__((visibility("default"))) PyObject* PyInit__calls(void) {
     argument_error = attribute("ctypes", "ArgumentError");
     parameter_class = argument_error ? attribute("torch.nn", "Parameter") : nullptr;
     out_of_memory_error = parameter_class ? attribute("torch", "OutOfMemoryError") : nullptr;
-    return out_of_memory_error ? PyModule_Create(&module) : nullptr;
+    return out_of_memory_error && right_torch() ? PyModule_Create(&module) : nullptr;
 }

@@ -85,3 +85,14 @@ def test_counts_and_positions_are_tensors(wrong):
         _ffi.latent_lib().call.pq_latent_decode(None, None, 1, None, None, wrong, 0, None, 1, 1, 1, 64, 1.0, 1, None, 0, 0, None)
     with pytest.raises(ctypes.ArgumentError):
         _ffi.steps_lib().call.pq_embed_rows(None, wrong, 1.0, None, 1, 8, 1, 0, None)
+
+
+def test_another_prototype_is_not_bound():
+    """Builtins of other headers than the checkout's would hand a library arguments that are not its own."""
+    lib, name = _ffi.lib(), "pq_decode_attn_plan"
+    at = ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
+    assert calls.bind(name, at, "iiiii")(1, 8, 100, 256) == lib.pq_decode_attn_plan(1, 8, 100, 256)
+    for other in ("iiii", "iiiiii", "iiiil", "iiiif", "Iiiii", ""):
+        with pytest.raises(RuntimeError, match="another version"):
+            calls.bind(name, at, other)
+    assert calls.bind("pq_version", at, "i") is None
