@@ -121,6 +121,12 @@ bool convert(PyObject* o, Arg& a, T& out) {
     }
 }
 
+// The interpreter is other threads' for as long as this lives, also where what runs meanwhile throws.
+struct Released {
+    PyThreadState* thread = PyEval_SaveThread();
+    ~Released() { PyEval_RestoreThread(thread); }
+};
+
 template <typename F, bool STRIDES> struct Call;
 template <bool STRIDES, typename R, typename... A>
 struct Call<R(A...), STRIDES> {
@@ -130,10 +136,10 @@ struct Call<R(A...), STRIDES> {
         std::tuple<std::decay_t<A>...> v;
         Arg kept[sizeof...(A) + 1];
         if (!(convert<std::decay_t<A>, STRIDES>(args[I], kept[I], std::get<I>(v)) && ...)) return nullptr;
-        R r;
-        Py_BEGIN_ALLOW_THREADS
-        r = reinterpret_cast<R (*)(A...)>(at)(std::get<I>(v)...);
-        Py_END_ALLOW_THREADS
+        const R r = [&] {
+            Released others;
+            return reinterpret_cast<R (*)(A...)>(at)(std::get<I>(v)...);
+        }();
         return std::is_signed_v<R> ? PyLong_FromLongLong(static_cast<long long>(r)) : PyLong_FromUnsignedLongLong(static_cast<unsigned long long>(r));
     }
     static PyObject* entry(PyObject* self, PyObject* const* args, Py_ssize_t n) {
@@ -378,7 +384,11 @@ PyObject* empty(PyObject*, PyObject* const* args, Py_ssize_t n) {
     }
     try {
         const at::Tensor& like = THPVariable_Unpack(args[0]);
-        return THPVariable_Wrap(at::empty(sizes, at::TensorOptions().device(like.device()).dtype(type ? kTypes[type] : like.scalar_type())));
+        const auto options = at::TensorOptions().device(like.device()).dtype(type ? kTypes[type] : like.scalar_type());
+        return THPVariable_Wrap([&] {
+            Released others;                    // (a first allocation, or freeing and waiting on the way to one, takes milliseconds)
+            return at::empty(sizes, options);
+        }());
     } catch (const c10::OutOfMemoryError& e) {
         PyErr_SetString(out_of_memory_error, e.what_without_backtrace());
     } catch (const std::exception& e) {

@@ -1,6 +1,8 @@
 """The C ABI's functions as builtins (csrc/pq_calls.cpp): the same answers as through ctypes, and questions that are answered only for
 tensors as they should lie."""
 import ctypes
+import threading
+import time
 
 import pytest
 import torch
@@ -96,3 +98,28 @@ def test_another_prototype_is_not_bound():
         with pytest.raises(RuntimeError, match="another version"):
             calls.bind(name, at, other)
     assert calls.bind("pq_version", at, "i") is None
+
+
+def test_other_threads_run_while_memory_is_allocated():
+    """An allocation that takes long (1 GiB that the deterministic mode fills) does not hold the interpreter."""
+    seen, over = [], threading.Event()
+
+    def watch():
+        while not over.is_set():
+            seen.append(time.perf_counter())
+            time.sleep(0.001)
+    before = torch.are_deterministic_algorithms_enabled()
+    other = threading.Thread(target=watch)
+    torch.use_deterministic_algorithms(True)
+    try:
+        other.start()
+        first = time.perf_counter()
+        t = calls.empty(torch.zeros(1), 3, 1 << 28)
+        last = time.perf_counter()
+    finally:
+        torch.use_deterministic_algorithms(before)
+        over.set()
+        other.join()
+    assert torch.isnan(t[::1 << 20]).all()
+    spent = last - first
+    assert any(first + 0.1 * spent < s < last - 0.1 * spent for s in seen), spent
