@@ -341,6 +341,8 @@ int launch_rope_qk(const void* q_lin, int64_t q_stride, const void* k_lin, int64
     return static_cast<int>(hipGetLastError());
 }
 
+// Rows at a step's ends are never longer than two pieces a thread.
+static_assert(kStepNormRows < 1024 && kStepNormMax <= 2 * 8 * 512, "what launch_norm has for them");
 static int launch_norm(const void* x, const void* res, const void* w, void* y, void* sum_out, int rows, int hidden, float eps, bool edges,
                        const NormEdges& e, int dtype, hipStream_t st) {
     // few rows: more threads, fewer pieces one after another; many: the units are full either way
@@ -348,21 +350,18 @@ static int launch_norm(const void* x, const void* res, const void* w, void* y, v
 #define PQ_RN(KERNEL, THREADS, ...)                                                                                  \
     hipLaunchKernelGGL((KERNEL), dim3(rows), dim3(THREADS), 0, st, (const uint16_t*)x, (const uint16_t*)res,         \
                        (const uint16_t*)w, (uint16_t*)y, (uint16_t*)sum_out, hidden, eps __VA_OPT__(, ) __VA_ARGS__)
-#define PQ_RNE(T, E)                                                                                                 \
-    do {                                                                                                             \
-        if (per <= 1) PQ_RN((rmsnorm_kernel<T, 1, E>), nthr, e);                                                     \
-        else if (per <= 2) PQ_RN((rmsnorm_kernel<T, 2, E>), nthr, e);                                                \
-        else PQ_RN((rmsnorm_kernel<T, 4, E>), nthr, e);                                                              \
-    } while (0)
 #define PQ_RNT(T)                                                                                                    \
     do {                                                                                                             \
-        if (per > 4) PQ_RN(rmsnorm_long_kernel<T>, 256);                                                             \
-        else if (edges) PQ_RNE(T, true);                                                                             \
-        else PQ_RNE(T, false);                                                                                       \
+        if (edges) {                                                                                                 \
+            if (per <= 1) PQ_RN((rmsnorm_kernel<T, 1, true>), nthr, e);                                              \
+            else PQ_RN((rmsnorm_kernel<T, 2, true>), nthr, e);                                                       \
+        } else if (per <= 1) PQ_RN((rmsnorm_kernel<T, 1, false>), nthr, e);                                          \
+        else if (per <= 2) PQ_RN((rmsnorm_kernel<T, 2, false>), nthr, e);                                            \
+        else if (per <= 4) PQ_RN((rmsnorm_kernel<T, 4, false>), nthr, e);                                            \
+        else PQ_RN(rmsnorm_long_kernel<T>, 256);                                                                     \
     } while (0)
     if (dtype == 0) PQ_RNT(F16); else PQ_RNT(BF16);
 #undef PQ_RNT
-#undef PQ_RNE
 #undef PQ_RN
     return static_cast<int>(hipGetLastError());
 }
