@@ -73,8 +73,9 @@ __global__ __launch_bounds__(256) void qk_norm_kernel(QkNormArgs a) {
 
 // The same with every piece in registers (NQ of a query row, NK of a key and of a value row a thread): rows, weights and values are
 // requested at once and read once.  The sums' order is the general kernel's, and so are the bits.  8 tokens,
-// 32 query and 8 KV heads of 128 4.0 -> 3.0 us in a chain of launches, 8192 tokens 35 -> 29.
-template <typename T, int NQ, int NK>
+// 32 query and 8 KV heads of 128 4.0 -> 3.0 us in a chain of launches, 8192 tokens 35 -> 29 (30.6 with the values read all the same).  RING: keys and values go to the ring; a long
+// call's keys go to k_out and its values are not read.
+template <typename T, int NQ, int NK, bool RING>
 __global__ __launch_bounds__(256) void qk_norm_row_kernel(QkNormArgs a) {
     constexpr int V = 4, STEP = 256 * V;
     __shared__ float part[2][4];
@@ -93,7 +94,7 @@ __global__ __launch_bounds__(256) void qk_norm_row_kernel(QkNormArgs a) {
 #pragma unroll
     for (int p = 0; p < NK; p++) {
         ldv<T, V>(a.w_k, at(p, nk), wk[p]);
-        ldv<T, V>(static_cast<const elem_t<T>*>(a.v) + row, at(p, nv), v[p]);
+        if constexpr (RING) ldv<T, V>(static_cast<const elem_t<T>*>(a.v) + row, at(p, nv), v[p]);
     }
     const int pos = (a.pos_dev ? *a.pos_dev : a.pos) + t;
     float sq = 0.0f, sk = 0.0f;
@@ -128,13 +129,14 @@ __global__ __launch_bounds__(256) void qk_norm_row_kernel(QkNormArgs a) {
 #pragma unroll
         for (int j = 0; j < V; j++) k[p][j] = k[p][j] * rk * wk[p][j];
         if (!own(p, nk)) continue;
-        if (a.k_out) stv<T, V>(static_cast<elem_t<T>*>(a.k_out) + static_cast<size_t>(tok) * nk, at(p, nk), k[p]);
-        else stv<T, V>(ring(a.k_ring, at(p, nk), a.D), 0, k[p]);
+        if constexpr (RING) stv<T, V>(ring(a.k_ring, at(p, nk), a.D), 0, k[p]);
+        else stv<T, V>(static_cast<elem_t<T>*>(a.k_out) + static_cast<size_t>(tok) * nk, at(p, nk), k[p]);
     }
-    if (a.k_out) return;
+    if constexpr (RING) {
 #pragma unroll
-    for (int p = 0; p < NK; p++)
-        if (own(p, nv)) stv<T, V>(ring(a.v_ring, at(p, nv), a.Dv), 0, v[p]);
+        for (int p = 0; p < NK; p++)
+            if (own(p, nv)) stv<T, V>(ring(a.v_ring, at(p, nv), a.Dv), 0, v[p]);
+    }
 }
 
 int launch_qk_norm(const QkNormArgs& a, int dtype, hipStream_t st) {
@@ -145,7 +147,8 @@ int launch_qk_norm(const QkNormArgs& a, int dtype, hipStream_t st) {
     dim3 grid(static_cast<unsigned>(a.B * a.L)), block(256);
     const int widest = a.G * (a.D > a.Dv ? a.D : a.Dv), NQ = (a.H * a.D + 1023) / 1024, NK = (widest + 1023) / 1024;
     if (v4 && dtype != 2 && NQ <= 4 && NK <= 2) {
-#define PQ_QR(T, Q, K) hipLaunchKernelGGL((qk_norm_row_kernel<T, Q, K>), grid, block, 0, st, a)
+#define PQ_QR(T, Q, K) do { if (a.k_out) hipLaunchKernelGGL((qk_norm_row_kernel<T, Q, K, false>), grid, block, 0, st, a); \
+                            else hipLaunchKernelGGL((qk_norm_row_kernel<T, Q, K, true>), grid, block, 0, st, a); } while (0)
 #define PQ_QRK(T, Q) do { if (NK == 1) PQ_QR(T, Q, 1); else PQ_QR(T, Q, 2); } while (0)
 #define PQ_QRT(T) do { if (NQ == 1) PQ_QRK(T, 1); else if (NQ == 2) PQ_QRK(T, 2); else PQ_QRK(T, 4); } while (0)
         if (dtype == 0) PQ_QRT(F16); else PQ_QRT(BF16);
