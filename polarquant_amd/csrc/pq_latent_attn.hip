@@ -53,7 +53,7 @@ __global__ __launch_bounds__((DecodeTeams<RP, RT>::THREADS), RT <= 2 ? 2 : 1) vo
     constexpr int CW = DecodeShape<RP>::CW, NW = DecodeShape<RP>::NW, CH = CW / 8, KS = CW / 32, CT = CW / 16;
     constexpr int LPT = kDecodeTile * CH / kWave, RPW = 16 / CH;           // loads per lane; rows per 256 bytes of LDS
     constexpr int TEAMS = DecodeTeams<RP, RT>::N;
-    extern __shared__ __attribute__((aligned(16))) uint8_t sm[];
+    __shared__ __attribute__((aligned(16))) uint8_t sm[DecodeTeams<RP, RT>::BYTES];
     auto tiles = reinterpret_cast<uint16_t(*)[kDecodeTile * CW]>(sm);
     auto exchs = reinterpret_cast<floatx4_a(*)[2][NW][2 * RT][kWave]>(sm + DecodeTeams<RP, RT>::TILES);
     const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
@@ -319,15 +319,7 @@ int launch_latent_decode(const LatentDecodeArgs& a, int dtype, hipStream_t st) {
     const int rows = a.L * a.H;
     const int rt = rows <= 16 ? 1 : rows <= 32 ? 2 : 4;
     dim3 grid(a.n_splits, (rows + 16 * rt - 1) / (16 * rt), a.B);
-    int err = 0;
-#define PQ_LD1(T, RP, RT)                                                                                            \
-    do {                                                                                                             \
-        using D = DecodeTeams<RP, RT>;                                                                               \
-        auto* kernel = &latent_decode_kernel<T, RP, RT>;                                                             \
-        if (D::BYTES > 64 * 1024)                                                                                    \
-            err = static_cast<int>(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(D::BYTES))); \
-        if (!err) hipLaunchKernelGGL(kernel, grid, dim3(D::THREADS), D::BYTES, st, a);                               \
-    } while (0)
+#define PQ_LD1(T, RP, RT) hipLaunchKernelGGL((latent_decode_kernel<T, RP, RT>), grid, dim3(DecodeTeams<RP, RT>::THREADS), 0, st, a)
 #define PQ_LD(T, RP) do { if (rt == 1) PQ_LD1(T, RP, 1); else if (rt == 2) PQ_LD1(T, RP, 2); else PQ_LD1(T, RP, 4); } while (0)
 #define PQ_LDT(T)                                                                                                    \
     do {                                                                                                             \
@@ -338,7 +330,7 @@ int launch_latent_decode(const LatentDecodeArgs& a, int dtype, hipStream_t st) {
 #undef PQ_LDT
 #undef PQ_LD
 #undef PQ_LD1
-    if (!err) err = static_cast<int>(hipGetLastError());
+    const int err = static_cast<int>(hipGetLastError());
     if (err) return err;
     dim3 mgrid(rows, (a.R + 63) / 64, a.B), mblock(256);
     if (dtype == 0) hipLaunchKernelGGL(latent_merge_kernel<F16>, mgrid, mblock, 0, st, a);
