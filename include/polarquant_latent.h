@@ -15,7 +15,7 @@
  * pq_latent_decode: q [B, L, H, R] already in the latent space, c [B, capacity, R]
  *   shared by all heads, out [B, L, H, R] = softmax over the keys start[b] <= j <=
  *   pos + t of scale * q . c_j (denominator + exp(sink[h])), applied to c.
- *   16-bit dtypes with R % 8 == 0, R <= 512 cut the context into n_splits slices
+ *   16-bit dtypes with R % 8 == 0, R <= 512 cut the context into at most n_splits slices
  *   (pq_latent_decode_plan) through `workspace`; others run a plain kernel.
  *
  * pq_latent_prefill: q [B, L, H, D], k [B, Lk, H, D] (Lk = pos + L), vt

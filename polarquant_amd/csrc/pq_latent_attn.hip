@@ -13,6 +13,7 @@
 // enter the products in the model's 16-bit dtype.
 #include "pq_prompt_attn.h"
 #include "pq_latent_internal.h"
+#include "pq_latent_rules.h"
 
 namespace pq {
 
@@ -24,10 +25,11 @@ namespace pq {
 // only barrier), every wavefront runs the softmax of all rows, and multiplies its channels of V^T, the same LDS tile
 // transposed on the way out, with P^T.  So each key is read from HBM once, and from LDS once per product, for all rows.
 // 16-byte pieces of a key's row are XOR-swizzled by the key so that neither access meets in few banks.
-// Up to 32 rows (their state takes half of a SIMD's registers) a workgroup is two teams of such wavefronts, each with half of the
+// Up to 32 rows (their state takes half of a SIMD's registers) a workgroup may be two teams of such wavefronts, each with half of the
 // slice's tiles, whose states are joined in LDS: a unit holds two sets of wavefronts either way, and one partial of R floats a row
 // goes through memory instead of two (8 sequences of 4096 keys, 32 heads, rank 512, planned for 12288: 33 MB of them written and read
-// beside 34 MB of latents).  Both launches 25.1 -> 21.5 us; of 12000 keys 37.6 -> 32.8; 32 sequences of 8000 74.0 -> 67.1.
+// beside 34 MB of latents).  Both launches 25.1 -> 21.8 us; of 12000 keys 37.4 -> 33.4; 32 sequences of 8000 73 -> 68.  Where they do not
+// pay: pq_latent_rules.h.
 // Workspace: [B, slices, L * H] pairs (maximum in log2 units, sum), then as many rows of R floats.
 constexpr int kDecodeTile = 32;
 __device__ __forceinline__ size_t pairs_floats(const LatentDecodeArgs& a) {     // up to the accumulators' 16-byte boundary
@@ -38,8 +40,8 @@ template <int RP> struct DecodeShape {
     static constexpr int NW = RP / CW;                         // wavefronts
 };
 
-template <int RP, int RT> struct DecodeTeams {
-    static constexpr int N = RT <= 2 ? 2 : 1, NW = DecodeShape<RP>::NW;
+template <int RP, int RT, int N> struct DecodeTeams {
+    static constexpr int NW = DecodeShape<RP>::NW;
     static constexpr int THREADS = kWave * NW * N;
     static constexpr size_t TILES = static_cast<size_t>(N) * NW * kDecodeTile * DecodeShape<RP>::CW * 2;            // bytes of LDS
     static constexpr size_t EXCH = static_cast<size_t>(N) * 2 * NW * 2 * RT * kWave * 16;
@@ -48,14 +50,13 @@ template <int RP, int RT> struct DecodeTeams {
     static_assert(N == 1 || static_cast<size_t>(NW) * kWave * RT * (DecodeShape<RP>::CW / 16 * 16 + 8) <= BYTES, "LDS");
 };
 
-template <typename T, int RP, int RT>
-__global__ __launch_bounds__((DecodeTeams<RP, RT>::THREADS), RT <= 2 ? 2 : 1) void latent_decode_kernel(LatentDecodeArgs a) {
+template <typename T, int RP, int RT, int TEAMS>
+__global__ __launch_bounds__((DecodeTeams<RP, RT, TEAMS>::THREADS), RT <= 2 ? 2 : 1) void latent_decode_kernel(LatentDecodeArgs a) {
     constexpr int CW = DecodeShape<RP>::CW, NW = DecodeShape<RP>::NW, CH = CW / 8, KS = CW / 32, CT = CW / 16;
     constexpr int LPT = kDecodeTile * CH / kWave, RPW = 16 / CH;           // loads per lane; rows per 256 bytes of LDS
-    constexpr int TEAMS = DecodeTeams<RP, RT>::N;
-    __shared__ __attribute__((aligned(16))) uint8_t sm[DecodeTeams<RP, RT>::BYTES];
+    __shared__ __attribute__((aligned(16))) uint8_t sm[DecodeTeams<RP, RT, TEAMS>::BYTES];
     auto tiles = reinterpret_cast<uint16_t(*)[kDecodeTile * CW]>(sm);
-    auto exchs = reinterpret_cast<floatx4_a(*)[2][NW][2 * RT][kWave]>(sm + DecodeTeams<RP, RT>::TILES);
+    auto exchs = reinterpret_cast<floatx4_a(*)[2][NW][2 * RT][kWave]>(sm + DecodeTeams<RP, RT, TEAMS>::TILES);
     const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), team = wave / NW, wv = wave % NW;
     auto& exch = exchs[team];
@@ -99,10 +100,11 @@ __global__ __launch_bounds__((DecodeTeams<RP, RT>::THREADS), RT <= 2 ? 2 : 1) vo
             stage[i] = *reinterpret_cast<const u32x4_a*>(base + (tok <= last ? off[i] : static_cast<uint32_t>(last) * R + col[i]));
         });
     };
-    // A slice of one or two tiles is the first team's alone: joining costs what a tile does.  Otherwise both make the same number of
-    // steps; a tile past the slice is a copy of its first one, every key of it masked.
+    // A slice of up to three tiles is the first team's alone: joining costs what a tile does (8 sequences of 32 slices of three tiles, 32 heads,
+    // rank 512: 19.9 us, joined 22.1).  Otherwise both make the same number of steps; a tile past the slice is a copy of its first one, every
+    // key of it masked.
     const int all = (s1 - s0 + kDecodeTile - 1) / kDecodeTile;
-    const bool alone = TEAMS == 1 || all <= 2;
+    const bool alone = TEAMS == 1 || all <= 3;
     if (alone && team == 1) return;
     const int ntiles = alone ? all : (all + 1) / 2, t0 = s0 + team * ntiles * kDecodeTile;
     fetch(t0);
@@ -315,12 +317,20 @@ __global__ __launch_bounds__(256) void latent_merge_kernel(LatentDecodeArgs a) {
         make_uint2(pack2<T>(sum.x * inv, sum.y * inv), pack2<T>(sum.z * inv, sum.w * inv));
 }
 
-int launch_latent_decode(const LatentDecodeArgs& a, int dtype, hipStream_t st) {
+int launch_latent_decode(const LatentDecodeArgs& asked, int dtype, hipStream_t st) {
+    LatentDecodeArgs a = asked;
     const int rows = a.L * a.H;
-    const int rt = rows <= 16 ? 1 : rows <= 32 ? 2 : 4;
-    dim3 grid(a.n_splits, (rows + 16 * rt - 1) / (16 * rt), a.B);
-#define PQ_LD1(T, RP, RT) hipLaunchKernelGGL((latent_decode_kernel<T, RP, RT>), grid, dim3(DecodeTeams<RP, RT>::THREADS), 0, st, a)
-#define PQ_LD(T, RP) do { if (rt == 1) PQ_LD1(T, RP, 1); else if (rt == 2) PQ_LD1(T, RP, 2); else PQ_LD1(T, RP, 4); } while (0)
+    const int rt = rows <= 16 ? 1 : rows <= 32 ? 2 : 4, tiles = (rows + 16 * rt - 1) / (16 * rt);
+    int teams = 1;
+    if (rt <= 2) {
+        const LatentDecodeLayout lay = latent_decode_layout(a.R <= 64 ? 64 : a.R <= 128 ? 128 : a.R <= 256 ? 256 : 512, static_cast<int64_t>(a.B) * tiles, a.n_splits);
+        teams = lay.teams;
+        a.n_splits = lay.slices;          // (never more than the workspace is for)
+    }
+    dim3 grid(a.n_splits, tiles, a.B);
+#define PQ_LD1(T, RP, RT, N) hipLaunchKernelGGL((latent_decode_kernel<T, RP, RT, N>), grid, dim3(DecodeTeams<RP, RT, N>::THREADS), 0, st, a)
+#define PQ_LD2(T, RP, RT) do { if (teams == 2) PQ_LD1(T, RP, RT, 2); else PQ_LD1(T, RP, RT, 1); } while (0)
+#define PQ_LD(T, RP) do { if (rt == 1) PQ_LD2(T, RP, 1); else if (rt == 2) PQ_LD2(T, RP, 2); else PQ_LD1(T, RP, 4, 1); } while (0)
 #define PQ_LDT(T)                                                                                                    \
     do {                                                                                                             \
         if (a.R <= 64) PQ_LD(T, 64); else if (a.R <= 128) PQ_LD(T, 128);                                             \
@@ -329,6 +339,7 @@ int launch_latent_decode(const LatentDecodeArgs& a, int dtype, hipStream_t st) {
     if (dtype == 0) PQ_LDT(F16); else PQ_LDT(BF16);
 #undef PQ_LDT
 #undef PQ_LD
+#undef PQ_LD2
 #undef PQ_LD1
     const int err = static_cast<int>(hipGetLastError());
     if (err) return err;

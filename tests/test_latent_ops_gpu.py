@@ -180,6 +180,20 @@ def test_latent_decode_halves_of_a_slice(gpu, keys):
             assert err(got, decode_want(q, c, sink, R ** -0.5, keys - 1, None)) < {"bf16": 1.2e-2, "f16": 2e-3}[dt], (dt, at)
 
 
+@pytest.mark.parametrize("B,H,R,S", [(257, 20, 512, 2), (300, 9, 264, 1), (100, 32, 512, 6), (66, 17, 256, 5), (64, 16, 200, 8), (129, 32, 128, 4), (65, 5, 96, 5), (300, 32, 64, 3)])
+@pytest.mark.parametrize("keys", [5, 100, 300])
+def test_latent_decode_of_many_sequences(gpu, B, H, R, S, keys):
+    """One team of wavefronts a workgroup, or two over fewer slices than asked for, with one and two tiles of rows; the first, a middle and the
+    last sequence against the oracle, equal sequences alike."""
+    g = torch.Generator().manual_seed(B + keys)
+    q, sink, c = rand(g, 3, 1, H, R, dt="bf16", s=2.0), rand(g, H), rand(g, 3, keys + 3, R, dt="bf16")
+    c[:, keys:] = 3e4
+    at = torch.tensor([0] + [1] * (B - 2) + [2])
+    got = ops.latent_decode_attention(q[at].to(gpu), c[at].to(gpu), sink.to(gpu), R ** -0.5, keys - 1, n_splits=S)
+    assert err(got[[0, B // 2, B - 1]], decode_want(q, c, sink, R ** -0.5, keys - 1, None)) < 1.2e-2
+    assert torch.equal(got[1:-1], got[1:2].expand(B - 2, -1, -1, -1))
+
+
 def test_latent_decode_positions_in_device_memory_and_stale_rows(gpu):
     """Rows past the sequence hold large finite values from an earlier use; the position comes from the device."""
     g = torch.Generator().manual_seed(3)

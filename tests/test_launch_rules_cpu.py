@@ -1,5 +1,5 @@
 """Which products of up to 16 rows leave the BLAS library for the weight-streaming kernel, how many rows of W its workgroups take, how many
-tokens a strip of the norm with convolution.  The sizes are those both sides were timed at, weights read from memory.  No GPU is needed."""
+tokens a strip of the norm with convolution, how many teams a workgroup of latent decode attention.  The sizes are those both sides were timed at, weights read from memory.  No GPU is needed."""
 import ctypes
 import os
 import subprocess
@@ -32,9 +32,10 @@ def rules():
     os.makedirs(os.path.join(here, "_build"), exist_ok=True)
     so = os.path.join(here, "_build", "liblaunch_rules.so")
     subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-x", "c++", "-", "-o", so, "-I", os.path.join(os.path.dirname(here), "polarquant_amd", "csrc")],
-                   input=b'#include "pq_linear_rules.h"\n#include "pq_steps_rules.h"\nextern "C" {\n'
+                   input=b'#include "pq_linear_rules.h"\n#include "pq_steps_rules.h"\n#include "pq_latent_rules.h"\nextern "C" {\n'
                          b'int tiles(int m, int n, int ks, int mats) { return pq::small_m8_row_tiles(m, n, ks, mats); }\n'
-                         b'int strip(int tokens, int taps, int pieces) { return pq::norm_conv_strip(tokens, taps, pieces); }\n}', check=True)
+                         b'int strip(int tokens, int taps, int pieces) { return pq::norm_conv_strip(tokens, taps, pieces); }\n'
+                         b'int layout(int rank, int groups, int slices) { auto l = pq::latent_decode_layout(rank, groups, slices); return 1000 * l.teams + l.slices; }\n}', check=True)
     return ctypes.CDLL(so)
 
 
@@ -61,3 +62,23 @@ def test_eight_tiles_only_where_x_is_what_costs(row_tiles):
     """32768 and 43136 outputs: 8 tiles gain 7 to 10 % with 8 rows and lose 4 to 5 % with one."""
     for n in (32768, 43136):
         assert row_tiles(8, n, 4, 1) == 8 and all(row_tiles(m, n, 4, 1) < 8 for m in (1, 2, 3, 4))
+
+
+# rank, row tiles of all sequences, the plan's slices -> teams, slices
+LATENT = [(512, 1, 96, 2, 96), (512, 8, 64, 2, 32), (512, 64, 8, 2, 4), (512, 86, 6, 2, 2), (512, 100, 6, 2, 2), (512, 129, 4, 2, 1), (512, 192, 3, 2, 1),
+          (512, 256, 2, 2, 1), (512, 256, 1, 2, 1), (512, 257, 2, 1, 2), (512, 257, 1, 1, 1), (512, 300, 2, 1, 2), (512, 1024, 1, 1, 1),
+          (256, 20, 5, 2, 5), (256, 20, 24, 2, 12), (256, 40, 13, 2, 6), (256, 64, 8, 2, 4), (256, 86, 6, 1, 6), (256, 129, 4, 1, 4), (256, 257, 2, 1, 2),
+          (128, 20, 5, 2, 5), (128, 64, 5, 2, 4), (128, 65, 5, 1, 5), (128, 40, 13, 1, 13), (128, 86, 6, 1, 6), (128, 129, 4, 1, 4), (128, 300, 2, 1, 2),
+          (64, 64, 8, 2, 8), (64, 64, 5, 2, 4), (64, 129, 4, 2, 4), (64, 300, 2, 2, 2), (64, 1024, 1, 2, 1)]
+
+
+@pytest.mark.parametrize("rank,groups,slices,teams,used", LATENT)
+def test_two_teams_only_where_a_round_of_workgroups_holds_them(rules, rank, groups, slices, teams, used):
+    assert divmod(rules.layout(rank, groups, slices), 1000) == (teams, used)
+
+
+def test_latent_plan_fills_the_units_with_workgroups_of_one_team():
+    from polarquant_amd import _ffi
+    plan = _ffi.latent_lib().pq_latent_decode_plan
+    assert [plan(B, 1, 32, 1 << 20, 256) for B in (1, 8, 100, 129, 256, 257, 300, 512, 513)] == [512, 64, 6, 4, 2, 2, 2, 1, 1]
+    assert [plan(8, 1, 32, keys, 256) for keys in (1, 128, 129, 1000)] == [1, 1, 2, 8] and plan(8, 1, 64, 1 << 20, 256) == 32
