@@ -68,13 +68,8 @@ bool pointer(PyObject* o, Arg& a, Also also, void*& p) {
         p = nullptr;
     } else if (plain_tensor(o)) {
         p = THPVariable_Unpack(o).data_ptr();
-    } else if (THPVariable_Check(o)) {              // a subclass says for itself what its pointer is
-        PyObject* at = PyObject_CallMethod(o, "data_ptr", nullptr);
-        uint64_t v = 0;
-        const bool ok = at && integer(at, v);
-        Py_XDECREF(at);
-        if (!ok) return refuse(o, "a pointer");
-        p = reinterpret_cast<void*>(v);
+    } else if (also == Also::kAddress && PyLong_CheckExact(o)) {
+        p = reinterpret_cast<void*>(PyLong_AsUnsignedLongLongMask(o));
     } else if (also == Also::kStrides && PyTuple_Check(o)) {      // for the length of the call
         const Py_ssize_t n = PyTuple_GET_SIZE(o);
         if (n > kListed) return refuse(o, "fewer integers");
@@ -84,6 +79,13 @@ bool pointer(PyObject* o, Arg& a, Also also, void*& p) {
             a.list[i] = static_cast<int64_t>(v);
         }
         p = a.list;
+    } else if (THPVariable_Check(o)) {              // (asks the class; the forms above are the common ones) a subclass says for itself what its pointer is
+        PyObject* at = PyObject_CallMethod(o, "data_ptr", nullptr);
+        uint64_t v = 0;
+        const bool ok = at && integer(at, v);
+        Py_XDECREF(at);
+        if (!ok) return refuse(o, "a pointer");
+        p = reinterpret_cast<void*>(v);
     } else if (also == Also::kAddress) {
         uint64_t v;
         if (!integer(o, v)) return false;
