@@ -345,7 +345,8 @@ int launch_rope_qk(const void* q_lin, int64_t q_stride, const void* k_lin, int64
 static_assert(kStepNormRows < 1024 && kStepNormMax <= 2 * 8 * 512, "what launch_norm has for them");
 static int launch_norm(const void* x, const void* res, const void* w, void* y, void* sum_out, int rows, int hidden, float eps, bool edges,
                        const NormEdges& e, int dtype, hipStream_t st) {
-    // few rows: more threads, fewer pieces one after another; many: the units are full either way
+    // few rows: more threads, fewer pieces one after another; many: the units are full either way.  (The order of a row's float32 sum
+    // goes with the threads: rows longer than 2048 of a call of 1024 rows and of a smaller one may differ in the result's last place.)
     const int nthr = rows < 1024 && hidden > 2048 ? 512 : 256, per = (hidden / 8 + nthr - 1) / nthr;
 #define PQ_RN(KERNEL, THREADS, ...)                                                                                  \
     hipLaunchKernelGGL((KERNEL), dim3(rows), dim3(THREADS), 0, st, (const uint16_t*)x, (const uint16_t*)res,         \

@@ -194,7 +194,7 @@ __global__ __launch_bounds__(256, DKP <= 128 ? 2 : 1) void prompt_attn_kernel(Pr
     // LDS addresses of this lane's reads: row `col` of K, chunk 2 i + hi
     // A row per channel: 8 chunks at VT distances; the chunks' addresses are kept and the distances are offsets (32 or 64 sums do not fit, or
     // are formed again beside every product: 8192 tokens 635 us).
-        uint32_t ka[KS], va[TOKEN_ROWS ? VT : 8];
+    uint32_t ka[KS], va[TOKEN_ROWS ? VT : 8];
     static_for<KS>([&](auto I) { ka[I] = lds0 + col * (DKP * 2) + ((2 * I + hi) ^ k_swz(col)) * 16; });
     static_for<TOKEN_ROWS ? VT : 8>([&](auto I) {
         constexpr int i = decltype(I)::value;

@@ -113,9 +113,10 @@ __device__ __forceinline__ bool angle_radius_fast(float x, float y, float* a_out
     const float r = __builtin_amdgcn_sqrtf(ss);
     const float a = atan2_fast_abs<T>(y, x, r);
     // (bfloat16 only) magnitudes at which the reciprocal or the hardware square root leave their accurate range; half's
-    // finite squares all lie inside (2^-80, 2^80).  Zeros need no test of their own: with one zero operand the estimate is
-    // exactly 0, pi/2 or pi like the exact routine's (0 then fails the kMinNormal test below), and
-    // x == y == 0 gives a NaN angle with radius 0, which fails that test as well.
+    // finite squares all lie inside (2^-80, 2^80).  Zeros need no test of their own: y == 0 gives exactly 0 or pi (0 then fails
+    // the kMinNormal test below); x == 0 gives pi/2 to a few ulps (the polynomials at 1: two below it for half, nine above for bfloat16),
+    // and pi/2 is 37 ulps from a midpoint of half and 28709 from one of bfloat16, so that it rounds like the exact angle;
+    // x == y == 0 gives a NaN angle with radius 0, which fails the kMinNormal test as well.
     // (bitwise | on purpose: one straight-line predicate instead of a chain of exec-mask branches)
     int special = 0;
     if constexpr (!IsHalf<T>::value) special |= static_cast<int>(!(ss > 0x1p-80f));

@@ -72,9 +72,9 @@ __global__ __launch_bounds__(256) void qk_norm_kernel(QkNormArgs a) {
 }
 
 // The same with every piece in registers (NQ of a query row, NK of a key and of a value row a thread): rows, weights and values are
-// requested at once and read once.  The sums' order is the general kernel's, and so are the bits.  8 tokens,
-// 32 query and 8 KV heads of 128 4.0 -> 3.0 us in a chain of launches, 8192 tokens 35 -> 29 (30.6 with the values read all the same).  RING: keys and values go to the ring; a long
-// call's keys go to k_out and its values are not read.
+// requested at once and read once.  RING: keys and values go to the ring; a long call's keys go to k_out and its values are not read.
+// The sums' order is the general kernel's, and so are the bits.  32 query and 8 KV heads of 128, us in a chain of launches: 8 tokens 4.0 ->
+// 3.0, 8192 tokens 35 -> 29 (30.6 with the values read all the same).
 template <typename T, int NQ, int NK, bool RING>
 __global__ __launch_bounds__(256) void qk_norm_row_kernel(QkNormArgs a) {
     constexpr int V = 4, STEP = 256 * V;

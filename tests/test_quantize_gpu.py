@@ -197,7 +197,7 @@ def test_quantizer_math_selftest_exhaustive(gpu, dtype_code, name):
           % (name, bad, 100.0 * slow / 2 ** 32, bad_div, bad_dev, 100.0 * slow_dev / 2 ** 32), flush=True)
     assert bad == 0
     assert bad_dev == 0
-    assert bad_div == 0     # reciprocal + two fused multiply-adds against the fp32 division, every (dividend, scale) pair
+    assert bad_div == 0     # quotients by a two-part inverse and the codes of 7, 4 and 3 bits against the fp32 division, every (dividend, scale) pair
 
 
 @pytest.mark.parametrize("dtype,exponents", [(torch.float16, (-15, -9, 0, 7, 14)), (torch.bfloat16, (-90, -45, -39, 0, 38, 41, 60))])
