@@ -27,7 +27,8 @@
  * pq_stream_add: x_out = x + y + e + v; y in the dtype, e float32, v [width] in the
  *   dtype, each or null; x_out may be x.  pq_embed_rows: out[r] = table[ids[r]] * scale.
  * pq_embed_norm_conv: pq_norm_conv of x' = table[ids] * scale, which goes to x_out, for what
- *   pq_embed_norm_conv_takes says yes to (taps 1 without a convolution).
+ *   pq_embed_norm_conv_takes says yes to (taps 1 without a convolution).  In both, ids outside of the
+ *   table count as its nearest row.
  * pq_softcap: x <- cap * tanh(x * scale / cap) in place (cap <= 0: x * scale).
  *
  * pq_head_linear: y[m, h, :] = epilogue(x[m, h, :] w[h]^T) with w [heads, N, K];

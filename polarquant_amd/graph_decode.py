@@ -80,6 +80,8 @@ class PolarGraphDecoder(GraphDecoder):
         order, so logits agree to rounding.  Off: the BLAS library for every product of the fused step.
         fused_qkv_rope (with small_m_gemm, batch <= 8): the q|k|v projection, the rotation and the two cache
         appends as one launch, `decode_ops.qkv_rope_append`, bit-identical to the projection followed by the rotation.
+        A step's embedding rows are read by the launch of its first norm where the module only looks up; ids outside of the vocabulary then count
+        as its nearest one, as nothing on the GPU checks them.
         fused_prefill: in the prompt pass the residual additions become part of the norms behind them (the eager modules'
         norms and activations are one launch each by themselves); the cache it builds and the logits then agree with the
         eager model to rounding instead of bit for bit."""

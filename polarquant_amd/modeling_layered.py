@@ -72,7 +72,8 @@ class LayeredModel(nn.Module):
     @torch.no_grad()
     def forward(self, input_ids=None, attention_mask=None, past_key_values=None):
         """-> (normed hidden states [B, L, W], tuple of per-layer cache tuples).  Any number of new tokens, with or without
-        a cache.  attention_mask [B, tokens so far] may mark left padding; it is read with the first tokens of a sequence."""
+        a cache.  attention_mask [B, tokens so far] may mark left padding; it is read with the first tokens of a sequence.
+        ids outside of the vocabulary count as its nearest one where a launch reads the embedding's rows itself (they are not checked)."""
         B, L = input_ids.shape
         if past_key_values is None:
             arenas, n = self.new_arenas(B, self.config.cache_capacity or L + 1024), 0
