@@ -242,14 +242,11 @@ __global__ __launch_bounds__(256) void rmsnorm_long_kernel(const uint16_t* __res
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
     __syncthreads();
     const float inv = rsqrtf((part[0] + part[1] + part[2] + part[3]) / static_cast<float>(hidden) + eps);
+    const uint16_t* src = res && sum_out ? sum_out : x;              // (the rounded sums this thread wrote, if there are any)
+    const uint16_t* add = res && !sum_out ? res : nullptr;
     for (int i = threadIdx.x * 8; i < hidden; i += 256 * 8) {
-        uint4 v;
-        if (res && sum_out) {
-            v = load(sum_out + row, i);              // the rounded sums this thread wrote
-        } else {
-            v = load(x + row, i);
-            if (res) v = sum8<T>(v, load(res + row, i));
-        }
+        uint4 v = load(src + row, i);
+        if (add) v = sum8<T>(v, load(add + row, i));
         *reinterpret_cast<uint4*>(y + row + i) = scaled8<T>(v, load(w, i), inv);
     }
 }
