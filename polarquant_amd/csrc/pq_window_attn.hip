@@ -98,14 +98,16 @@ __global__ __launch_bounds__(256) void qk_norm_row_kernel(QkNormArgs a) {
     }
     const int pos = (a.pos_dev ? *a.pos_dev : a.pos) + t;
     float sq = 0.0f, sk = 0.0f;
+    auto squares = [](const float (&x)[V], float sum, bool counts) {
+        float t = sum;
 #pragma unroll
-    for (int p = 0; p < NQ; p++)
+        for (int j = 0; j < V; j++) t = __builtin_fmaf(x[j], x[j], t);
+        return counts ? t : sum;
+    };
 #pragma unroll
-        for (int j = 0; j < V; j++) sq = own(p, nq) ? __builtin_fmaf(q[p][j], q[p][j], sq) : sq;
+    for (int p = 0; p < NQ; p++) sq = squares(q[p], sq, own(p, nq));
 #pragma unroll
-    for (int p = 0; p < NK; p++)
-#pragma unroll
-        for (int j = 0; j < V; j++) sk = own(p, nk) ? __builtin_fmaf(k[p][j], k[p][j], sk) : sk;
+    for (int p = 0; p < NK; p++) sk = squares(k[p], sk, own(p, nk));
     sq = wave_sum(sq);
     sk = wave_sum(sk);
     if ((tid & 63) == 0) { part[0][wv] = sq; part[1][wv] = sk; }
@@ -113,6 +115,7 @@ __global__ __launch_bounds__(256) void qk_norm_row_kernel(QkNormArgs a) {
     sq = part[0][0] + part[0][1] + part[0][2] + part[0][3];
     sk = part[1][0] + part[1][1] + part[1][2] + part[1][3];
     const float rq = 1.0f / sqrtf(sq / static_cast<float>(nq) + a.eps), rk = 1.0f / sqrtf(sk / static_cast<float>(nk) + a.eps);
+    __builtin_amdgcn_s_waitcnt(0x0F70);              // (vmcnt 0: waits for a load behind a store are for the store as well)
 #pragma unroll
     for (int p = 0; p < NQ; p++) {
 #pragma unroll
@@ -127,7 +130,10 @@ __global__ __launch_bounds__(256) void qk_norm_row_kernel(QkNormArgs a) {
 #pragma unroll
     for (int p = 0; p < NK; p++) {
 #pragma unroll
-        for (int j = 0; j < V; j++) k[p][j] = k[p][j] * rk * wk[p][j];
+        for (int j = 0; j < V; j++) {
+            k[p][j] = k[p][j] * rk * wk[p][j];
+            asm("" : "+v"(k[p][j]));                 // (rounded to float32 before the dtype, not once by a multiply that converts)
+        }
         if (!own(p, nk)) continue;
         if constexpr (RING) stv<T, V>(ring(a.k_ring, at(p, nk), a.D), 0, k[p]);
         else stv<T, V>(static_cast<elem_t<T>*>(a.k_out) + static_cast<size_t>(tok) * nk, at(p, nk), k[p]);

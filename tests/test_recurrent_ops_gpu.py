@@ -111,6 +111,24 @@ def test_qk_norm_pieces_in_registers(gpu, H, G, D, Dv):
                 assert err(k, want_k) < TOL[dt]
 
 
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,L", [(64, 1), (3, 16), (2, 300)])
+def test_qk_norm_gives_the_same_bits_with_wider_values(gpu, dt, B, L):
+    """Values of 512 a head are too wide for the kernel that keeps rows in registers: queries and keys, in the ring and as rows, do not depend on
+    which kernel normed them."""
+    H, G, D = 32, 8, 128
+    g = torch.Generator(device=gpu).manual_seed(L)
+    qk = (torch.randn(B * L, (H + G) * D, generator=g, device=gpu) * 2).to(dt)
+    wq, wk = [(1 + 0.2 * torch.randn(n * D, generator=g, device=gpu)).to(dt) for n in (H, G)]
+    got = []
+    for Dv in (128, 512):
+        rows = torch.cat([qk, torch.zeros(B * L, G * Dv, dtype=dt, device=gpu)], 1)
+        ring = ops.WindowRing(B, G, D, Dv, 16, dt, gpu)
+        got.append(list(ops.qk_norm(rows[:, :H * D], rows[:, H * D:(H + G) * D], rows[:, (H + G) * D:], wq, wk, H, 1e-3, ring, Step(B, L, 5))) + [ring.k])
+    for a, b in zip(*got):
+        assert (a is None and b is None) or torch.equal(a, b)
+
+
 @pytest.mark.parametrize("H,G,D,Dv,window", [(4, 2, 32, 64, 40), (6, 1, 64, 32, 33), (2, 2, 128, 128, 150), (20, 1, 40, 24, 64), (1, 1, 136, 256, 17),
                                              (3, 3, 20, 12, 7), (4, 4, 5, 9, 1), (8, 2, 48, 96, 65), (2, 1, 256, 128, 300)])
 def test_window_attention(gpu, H, G, D, Dv, window):
