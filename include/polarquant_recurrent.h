@@ -33,6 +33,13 @@
  *   holds (16-bit dtypes, no pos_dev).
  * pq_head_norm_gate: out = out_scale * rmsnorm(o / den, per head) * w * sigmoid(gate);
  *   w [vdim] for all heads (w_head_stride 0) or [H * vdim] (w_head_stride vdim).
+ *
+ * pq_delta_token, pq_memory_token: a single token a sequence (L = 1), in one launch what
+ *   pq_delta_prep (a = xa wa^T, gate = xg wg^T: [H * dim, a_rank], [H * vdim, g_rank]),
+ *   pq_delta_scan and pq_head_norm_gate, or pq_memory_gates, pq_memory_scan and
+ *   pq_head_norm_gate do.  16-bit dtypes, G = H, row strides multiples of 8, out's of 4;
+ *   delta rule: dim, vdim multiples of 8 in 96 .. 128, taps <= 4, ranks multiples of 8 up to 128;
+ *   matrix memory: dim up to 128, vdim up to 256, multiples of 8.  conv, state and m in place.
  */
 #ifndef POLARQUANT_RECURRENT_H
 #define POLARQUANT_RECURRENT_H
@@ -82,6 +89,19 @@ int pq_memory_scan(const void *q, const void *k, const void *v, int64_t row_stri
 int pq_head_norm_gate(const float *o, const float *den, const void *w, int w_head_stride, const void *gate,
                       int64_t gate_row_stride, void *out, int64_t out_row_stride, int64_t rows, int H, int vdim, float eps,
                       float out_scale, int dtype, void *stream);
+
+int pq_validate_delta_token(int B, int H, int dim, int vdim, int taps, int a_rank, int g_rank, int64_t row_stride,
+                            int64_t out_row_stride, int dtype);
+int pq_delta_token(const void *q, const void *k, const void *v, const void *b, const void *xa, const void *xg,
+                   int64_t row_stride, const void *wa, const void *wg, const void *w_q, const void *w_k, const void *w_v,
+                   const void *A_log, const void *dt_bias, const void *norm, float *conv, float *state, void *out,
+                   int64_t out_row_stride, const int32_t *start, const int32_t *pos_dev, int pos, int B, int H, int dim, int vdim,
+                   int taps, int a_rank, int g_rank, float eps, float out_scale, int dtype, void *stream);
+int pq_validate_memory_token(int B, int H, int dim, int vdim, int64_t row_stride, int64_t out_row_stride, int dtype);
+int pq_memory_token(const void *q, const void *k, const void *v, const void *gate, const void *i, const void *f,
+                    int64_t row_stride, const void *b_i, const void *b_f, const void *norm, int w_head_stride, float *state,
+                    float *m, void *out, int64_t out_row_stride, const int32_t *start, const int32_t *pos_dev, int pos, int B,
+                    int H, int dim, int vdim, float cap, float q_scale, float eps, float out_scale, int dtype, void *stream);
 
 #ifdef __cplusplus
 }

@@ -155,6 +155,11 @@ RECURRENT_SIGNATURES = {
                        + [c_void_p, c_size_t, c_int, c_void_p]),
     "pq_head_norm_gate": (c_int, [c_void_p] * 3 + [c_int, c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int, c_int, c_float, c_float, c_int,
                                   c_void_p]),
+    "pq_validate_delta_token": (c_int, [c_int] * 7 + [c_int64] * 2 + [c_int]),
+    "pq_delta_token": (c_int, [c_void_p] * 6 + [c_int64] + [c_void_p] * 11 + [c_int64, c_void_p, c_void_p] + [c_int] * 8 + [c_float, c_float, c_int, c_void_p]),
+    "pq_validate_memory_token": (c_int, [c_int] * 4 + [c_int64] * 2 + [c_int]),
+    "pq_memory_token": (c_int, [c_void_p] * 6 + [c_int64] + [c_void_p] * 3 + [c_int] + [c_void_p] * 3 + [c_int64, c_void_p, c_void_p] + [c_int] * 5
+                        + [c_float] * 4 + [c_int, c_void_p]),
 }
 
 

@@ -6,20 +6,10 @@
 //   head_norm_gate_kernel  RMS norm per head of what was read out, its weight, the output gate
 //
 // State and everything that enters a recurrence are float32; q, k, v come in the model's dtype.
-#include "pq_elem.h"
+#include "pq_recurrent_device.h"
 #include "pq_recurrent_internal.h"
 
 namespace pq {
-
-// (one instruction each, exact to about a unit in the last place)
-__device__ __forceinline__ float exp_fast(float x) { return __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }
-__device__ __forceinline__ float sigmoid(float z) { return __builtin_amdgcn_rcpf(1.0f + exp_fast(-z)); }
-// max(z, 0) + log(1 + e), e = e^-|z|: for small e by its series, 1 + e would lose it
-__device__ __forceinline__ float softplus(float z) {
-    const float e = exp_fast(-fabsf(z));
-    const float series = e * __builtin_fmaf(e, __builtin_fmaf(e, __builtin_fmaf(e, -0.25f, 0.33333334f), -0.5f), 1.0f);
-    return fmaxf(z, 0.0f) + (e < 0.01f ? series : __builtin_amdgcn_logf(1.0f + e) * 0.6931471805599453f);
-}
 
 // V (1 or 2) consecutive elements at p
 template <typename T, int V> __device__ __forceinline__ void ldvec(const elem_t<T>* p, float (&o)[V]) {
@@ -213,8 +203,7 @@ __global__ __launch_bounds__(256) void memory_gates_kernel(MemoryGateArgs a) {
     const int h = static_cast<int>(n - row * a.H);
     const float i = ld1<T>(static_cast<const elem_t<T>*>(a.i) + row * a.p_row + h) + ld1<T>(static_cast<const elem_t<T>*>(a.b_i) + h);
     const float f = ld1<T>(static_cast<const elem_t<T>*>(a.f) + row * a.p_row + h) + ld1<T>(static_cast<const elem_t<T>*>(a.b_f) + h);
-    a.log_i[n] = a.cap * tanhf(i / a.cap);
-    a.log_f[n] = -softplus(-(a.cap * tanhf(f / a.cap)));
+    capped_gates(i, f, a.cap, a.log_i + n, a.log_f + n);
 }
 
 int launch_memory_gates(const MemoryGateArgs& a, int dtype, hipStream_t st) {
@@ -234,14 +223,6 @@ int launch_memory_gates(const MemoryGateArgs& a, int dtype, hipStream_t st) {
 // QUADS: a lane's rows are quads 64 apart, so that every load and store of the state, of q, k and of the decays moves 16 (8) bytes a lane
 // and whole lines a wavefront.  A single token is a stream of the state in and out and nothing else: 8 sequences, 32 heads of 128 x 128
 // 33.2 -> 9.5 us, 16 heads of 128 x 257 27.6 -> 8.0 us, against element by element, each behind its own bounds check.
-__device__ __forceinline__ float row16_sum(float v) {
-    v += __uint_as_float(row_rotate<8>(__float_as_uint(v)));
-    v += __uint_as_float(row_rotate<4>(__float_as_uint(v)));
-    v += __uint_as_float(row_rotate<2>(__float_as_uint(v)));
-    v += __uint_as_float(row_rotate<1>(__float_as_uint(v)));
-    return v;
-}
-
 template <typename T, bool DELTA, int RPL, bool QUADS>
 __global__ __launch_bounds__(256) void scan_kernel(ScanArgs a) {
     const int lane = threadIdx.x & 63, part = lane & 15, h = blockIdx.y, b = blockIdx.z, H = a.H, L = a.L, dim = a.dim;

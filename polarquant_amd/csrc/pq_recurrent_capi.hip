@@ -200,4 +200,53 @@ int pq_head_norm_gate(const float* o, const float* den, const void* w, int w_hea
     return status(pq::launch_head_norm_gate(a, dtype, S(stream)));
 }
 
+// what the kernels' quads and 16-byte pieces need
+static int check_token(int B, int H, int dim, int least_dim, int vdim, int most_vdim, int64_t row_stride, int64_t out_row_stride, int dtype) {
+    if (dtype != PQ_F16 && dtype != PQ_BF16) return PQ_ERR_BAD_DTYPE;
+    if (B < 1 || B > 65535 || H < 1 || H > 65535 || dim < least_dim || dim > pq::kTokenDim || dim % 8 || vdim < least_dim || vdim > most_vdim || vdim % 8)
+        return PQ_ERR_BAD_SHAPE;
+    const int64_t cols = static_cast<int64_t>(H) * vdim;
+    if (row_stride < cols || row_stride < static_cast<int64_t>(H) * dim || row_stride % 8 || out_row_stride < cols || out_row_stride % 4) return PQ_ERR_BAD_STRIDE;
+    return PQ_OK;
+}
+
+int pq_validate_delta_token(int B, int H, int dim, int vdim, int taps, int a_rank, int g_rank, int64_t row_stride, int64_t out_row_stride, int dtype) {
+    // (from 96 channels on the length of a head's vector is summed as pq_delta_prep sums it)
+    if (int rc = check_token(B, H, dim, 96, vdim, pq::kTokenDim, row_stride, out_row_stride, dtype)) return rc;
+    if (taps < 1 || taps > pq::kTokenTaps || a_rank < 8 || a_rank > 128 || a_rank % 8 || g_rank < 8 || g_rank > 128 || g_rank % 8) return PQ_ERR_BAD_SHAPE;
+    return PQ_OK;
+}
+
+int pq_delta_token(const void* q, const void* k, const void* v, const void* b, const void* xa, const void* xg, int64_t row_stride, const void* wa,
+                   const void* wg, const void* w_q, const void* w_k, const void* w_v, const void* A_log, const void* dt_bias, const void* norm,
+                   float* conv, float* state, void* out, int64_t out_row_stride, const int32_t* start, const int32_t* pos_dev, int pos, int B, int H,
+                   int dim, int vdim, int taps, int a_rank, int g_rank, float eps, float out_scale, int dtype, void* stream) {
+    if (!q || !k || !v || !b || !xa || !xg || !wa || !wg || !w_q || !w_k || !w_v || !A_log || !dt_bias || !norm || (taps > 1 && !conv) || !state || !out)
+        return PQ_ERR_NULL_POINTER;
+    if (int rc = pq_validate_delta_token(B, H, dim, vdim, taps, a_rank, g_rank, row_stride, out_row_stride, dtype)) return rc;
+    if (!aligned(xa, 16) || !aligned(xg, 16) || !aligned(wa, 16) || !aligned(wg, 16) || !aligned(state, 16) || !aligned(norm, 8) || !aligned(out, 8) ||
+        (conv && !aligned(conv, 8)) || !aligned(q, 2) || !aligned(k, 2) || !aligned(v, 2))
+        return PQ_ERR_MISALIGNED;
+    pq::DeltaTokenArgs d{q, k, v, b, xa, xg, row_stride, wa, wg, w_q, w_k, w_v, A_log, dt_bias, norm, conv, state, out, out_row_stride, start, pos_dev,
+                         pos, B, H, dim, vdim, taps, a_rank, g_rank, eps, out_scale};
+    return status(pq::launch_delta_token(d, dtype, S(stream)));
+}
+
+int pq_validate_memory_token(int B, int H, int dim, int vdim, int64_t row_stride, int64_t out_row_stride, int dtype) {
+    return check_token(B, H, dim, 8, vdim, pq::kTokenMemoryVdim, row_stride, out_row_stride, dtype);
+}
+
+int pq_memory_token(const void* q, const void* k, const void* v, const void* gate, const void* i, const void* f, int64_t row_stride, const void* b_i,
+                    const void* b_f, const void* norm, int w_head_stride, float* state, float* m, void* out, int64_t out_row_stride, const int32_t* start,
+                    const int32_t* pos_dev, int pos, int B, int H, int dim, int vdim, float cap, float q_scale, float eps, float out_scale, int dtype,
+                    void* stream) {
+    if (!q || !k || !v || !gate || !i || !f || !b_i || !b_f || !norm || !state || !m || !out) return PQ_ERR_NULL_POINTER;
+    if (int rc = pq_validate_memory_token(B, H, dim, vdim, row_stride, out_row_stride, dtype)) return rc;
+    if (!(cap > 0.0f) || (w_head_stride != 0 && w_head_stride != vdim)) return PQ_ERR_BAD_SHAPE;
+    if (!aligned(q, 8) || !aligned(k, 8) || !aligned(gate, 8) || !aligned(norm, 8) || !aligned(state, 16) || !aligned(out, 8)) return PQ_ERR_MISALIGNED;
+    pq::MemoryTokenArgs a{q, k, v, gate, i, f, row_stride, b_i, b_f, norm, w_head_stride, state, m, out, out_row_stride, start, pos_dev, pos, B, H, dim, vdim,
+                          cap, q_scale, eps, out_scale};
+    return status(pq::launch_memory_token(a, dtype, S(stream)));
+}
+
 }  // extern "C"

@@ -129,4 +129,35 @@ struct HeadNormGateArgs {
 };
 int launch_head_norm_gate(const HeadNormGateArgs& a, int dtype, hipStream_t st);
 
+// One token a sequence, from the input product's columns to the output product's operand (pq_recurrent_token.hip): 16-bit dtypes, as many
+// key as value heads, everything in place.
+struct DeltaTokenArgs {
+    const void *q, *k, *v, *b, *xa, *xg;     // columns of the projection output, rows p_row apart: H * dim, H * dim, H * vdim, H, the ranks
+    int64_t p_row;
+    const void *wa, *wg;                     // [H * dim, a_rank], [H * vdim, g_rank]
+    const void *w_q, *w_k, *w_v, *A_log, *dt_bias, *norm;
+    float *conv, *state;                     // [B, taps - 1, 2 H dim + H vdim], [B, H, vdim, dim]
+    void* out;                               // [B, H * vdim] rows out_row apart
+    int64_t out_row;
+    const int32_t *start, *pos_dev;
+    int pos, B, H, dim, vdim, taps, a_rank, g_rank;
+    float eps, out_scale;
+};
+constexpr int kTokenDim = 128, kTokenTaps = 4, kTokenMemoryVdim = 256;
+int launch_delta_token(const DeltaTokenArgs& a, int dtype, hipStream_t st);
+
+struct MemoryTokenArgs {
+    const void *q, *k, *v, *gate, *i, *f;    // columns of the projection output, rows p_row apart
+    int64_t p_row;
+    const void *b_i, *b_f, *norm;            // [H], [H], [vdim] or [H * vdim] (w_head = 0 or vdim)
+    int w_head;
+    float *state, *m;                        // [B, H, vdim + 1, dim], [B, H, (vdim + 16) / 16]
+    void* out;
+    int64_t out_row;
+    const int32_t *start, *pos_dev;
+    int pos, B, H, dim, vdim;
+    float cap, q_scale, eps, out_scale;
+};
+int launch_memory_token(const MemoryTokenArgs& a, int dtype, hipStream_t st);
+
 }  // namespace pq

@@ -237,7 +237,12 @@ class GatedDelta(Branch):
 
     def forward(self, p, out, state, step):
         q, k, v, b = [x[:, :w.shape[0]] for x, w in zip(p, (self.q, self.k, self.v, self.b))]
-        a, gate = layer_ops.linear(p[4], self._a2.weight()), layer_ops.linear(p[5], self._g2.weight())
+        wa, wg = self._a2.weight(), self._g2.weight()
+        if ops.delta_token_takes(q, k, p[4], p[5], wa, wg, state.S, self.taps, out, step):
+            ops.delta_token(q, k, v, b, p[4], p[5], wa, wg, self.q_conv, self.k_conv, self.v_conv, self.A_log, self.dt_bias, self.norm, state.conv, state.S,
+                            self.eps, out, self.out_scale, step)
+            return
+        a, gate = layer_ops.linear(p[4], wa), layer_ops.linear(p[5], wg)
         x = ops.delta_prep(q, k, v, b, a, self.q_conv, self.k_conv, self.v_conv, self.A_log, self.dt_bias, state.conv, self.dim, self.vdim, step)
         ops.head_norm_gate(ops.delta_scan(x, state.S, step), self.norm, gate, self.heads, self.eps, out, self.out_scale)
 
@@ -269,6 +274,10 @@ class MatrixMemory(Branch):
 
     def forward(self, p, out, state, step):
         q, k, v, g, i, f = [x[:, :w.shape[0]] for x, w in zip(p, (self.q, self.k, self.v, self.g, self.i, self.f))]
+        if ops.memory_token_takes(q, k, g, self.norm, state.S, out, step):
+            ops.memory_token(q, k, v, g, i, f, self.i_b, self.f_b, self.norm, state.S, state.m, self.gate_cap, self.dim ** -0.5, self.eps, out,
+                             self.out_scale, step)
+            return
         log_i, log_f = ops.memory_gates(i, f, self.i_b, self.f_b, self.gate_cap)
         o, den = ops.memory_scan(q, k, v, log_i, log_f, state.S, state.m, self.dim ** -0.5, step)
         ops.head_norm_gate(o, self.norm, g, self.heads, self.eps, out, self.out_scale, den)

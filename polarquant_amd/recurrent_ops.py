@@ -211,3 +211,68 @@ def head_norm_gate(o: torch.Tensor, w: torch.Tensor, gate: torch.Tensor, heads: 
     _run(_ffi.recurrent_lib().call.pq_head_norm_gate, "pq_head_norm_gate", o.device, o, den, w, 0 if w.numel() == vdim else vdim,
          gate, gate.stride(0), out, out.stride(0), M, heads, vdim, float(eps), float(out_scale), dt)
     return out
+
+
+# ----------------------------------------------------------------------------- one token a sequence
+def _one_launch(step: Step, dtype: torch.dtype, *aligned) -> bool:
+    """Whether a call could be the one launch of its mixer's token: a token a sequence, 16-bit dtype, operands at 16 bytes (their rows'
+    strides and the sizes are the library's to judge)."""
+    return step.L == 1 and dtype in (torch.float16, torch.bfloat16) and all(t.data_ptr() % 16 == 0 for t in aligned)
+
+
+# (The one launch is the faster one at any number of sequences, 1 to 64 timed: pq_recurrent_token.hip.)
+def delta_token_takes(q, k, xa, xg, wa, wg, state: torch.Tensor, taps: int, out: torch.Tensor, step: Step) -> bool:
+    B, H, vdim, dim = state.shape
+    return (_one_launch(step, q.dtype, xa, xg, wa, wg, state, out) and q.shape[1] == k.shape[1] == H * dim
+            and _ffi.recurrent_lib().call.pq_validate_delta_token(B, H, dim, vdim, taps, wa.shape[1], wg.shape[1], q.stride(0), out.stride(0),
+                                                                  _DTYPES[q.dtype]) == 0)
+
+
+def delta_token(q, k, v, b, xa, xg, wa, wg, w_q, w_k, w_v, A_log, dt_bias, norm, conv: ConvState, state: torch.Tensor, eps: float, out: torch.Tensor,
+                out_scale: float, step: Step) -> torch.Tensor:
+    """`delta_prep` with a = xa wa^T, `delta_scan` and `head_norm_gate` with the gate xg wg^T, of a token a sequence: rows q, k, v, b, xa,
+    xg of one projection -> out rows [B, H * vdim]."""
+    B, H, vdim, dim = state.shape
+    dt, taps = _code(q), conv.taps
+    assert B == step.B and step.L == 1 and state.is_contiguous() and state.dtype == torch.float32
+    for t, n in ((q, H * dim), (k, H * dim), (v, H * vdim), (b, H), (xa, wa.shape[1]), (xg, wg.shape[1])):
+        _rows(t, B, n, q.dtype)
+        assert t.stride(0) == q.stride(0)
+    _rows(out, B, H * vdim, q.dtype)
+    for w, rows in ((wa, H * dim), (wg, H * vdim)):
+        assert w.shape[0] == rows and w.is_contiguous() and w.dtype == q.dtype
+    for w, n in ((w_q, H * dim), (w_k, H * dim), (w_v, H * vdim)):
+        assert w.shape == (n, taps) and w.is_contiguous() and w.dtype == q.dtype
+    assert A_log.numel() == H and dt_bias.numel() == H * dim and norm.numel() == vdim
+    assert all(t.dtype == q.dtype and t.is_contiguous() for t in (A_log, dt_bias, norm))
+    rows, same = conv.targets(1)
+    assert rows is same and rows.shape == (B, taps - 1, 2 * H * dim + H * vdim)
+    _run(_ffi.recurrent_lib().call.pq_delta_token, "pq_delta_token", q.device, q, k, v, b, xa, xg, q.stride(0), wa, wg, w_q, w_k, w_v, A_log, dt_bias,
+         norm, rows if taps > 1 else None, state, out, out.stride(0), step.start, step.pos_dev, step.pos, B, H, dim, vdim, taps, wa.shape[1], wg.shape[1],
+         float(eps), float(out_scale), dt)
+    return out
+
+
+def memory_token_takes(q, k, gate, norm, state: torch.Tensor, out: torch.Tensor, step: Step) -> bool:
+    B, H, cols, dim = state.shape
+    return (_one_launch(step, q.dtype, q, k, gate, norm, state, out)
+            and _ffi.recurrent_lib().call.pq_validate_memory_token(B, H, dim, cols - 1, q.stride(0), out.stride(0), _DTYPES[q.dtype]) == 0)
+
+
+def memory_token(q, k, v, gate, i, f, b_i, b_f, norm, state: torch.Tensor, m: torch.Tensor, cap: float, q_scale: float, eps: float, out: torch.Tensor,
+                 out_scale: float, step: Step) -> torch.Tensor:
+    """`memory_gates`, `memory_scan` and `head_norm_gate` of a token a sequence: rows of one projection -> out rows [B, H * vdim]."""
+    B, H, cols, dim = state.shape
+    vdim, dt = cols - 1, _code(q)
+    assert B == step.B and step.L == 1 and state.is_contiguous() and m.is_contiguous() and state.dtype == m.dtype == torch.float32
+    assert m.shape == (B, H, (vdim + 16) // 16)
+    for t, n in ((q, H * dim), (k, H * dim), (v, H * vdim), (gate, H * vdim), (i, H), (f, H)):
+        _rows(t, B, n, q.dtype)
+        assert t.stride(0) == q.stride(0)
+    _rows(out, B, H * vdim, q.dtype)
+    assert b_i.numel() == b_f.numel() == H and norm.numel() in (vdim, H * vdim)
+    assert all(t.dtype == q.dtype and t.is_contiguous() for t in (b_i, b_f, norm))
+    _run(_ffi.recurrent_lib().call.pq_memory_token, "pq_memory_token", q.device, q, k, v, gate, i, f, q.stride(0), b_i, b_f, norm,
+         0 if norm.numel() == vdim else vdim, state, m, out, out.stride(0), step.start, step.pos_dev, step.pos, B, H, dim, vdim, float(cap), float(q_scale),
+         float(eps), float(out_scale), dt)
+    return out

@@ -1,0 +1,84 @@
+"""A token a sequence through a recurrent mixer in one launch (pq_recurrent_token.hip) against the launches that take any number of tokens.
+
+Both do the same operations on the same roundings, so that outputs and states are equal bit for bit.  Only the low-rank products add in
+another order: their operands are multiples of 1/8 here, so that every sum is exact."""
+import pytest
+import torch
+
+from polarquant_amd import layer_ops
+from polarquant_amd import recurrent_ops as ops
+from polarquant_amd.recurrent_ops import Step
+
+pytestmark = pytest.mark.gpu
+
+
+def eighths(g, *shape):
+    return torch.randint(-16, 17, shape, generator=g, device="cuda").float() / 8
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,H,dim,vdim,taps,ra,rg,padded", [
+    (1, 1, 128, 128, 4, 128, 128, False), (8, 32, 128, 128, 4, 128, 64, False), (3, 5, 96, 104, 3, 64, 96, True), (2, 3, 112, 128, 1, 8, 128, True),
+    (40, 2, 128, 96, 2, 32, 32, False)])
+def test_delta(B, H, dim, vdim, taps, ra, rg, padded, dtype):
+    g = torch.Generator(device="cuda").manual_seed(dim + B)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    kd, vd = H * dim, H * vdim
+    widths = [kd, kd, vd, -(-H // 8) * 8, ra, rg]
+    p = r(B, sum(widths)).to(dtype)
+    at = [sum(widths[:i]) for i in range(7)]
+    p[:, at[4]:] = eighths(g, B, ra + rg).to(dtype)
+    q, k, v, b, xa, xg = [p[:, at[i]:at[i + 1]] for i in range(6)]
+    b = b[:, :H]
+    wa, wg = (eighths(g, kd, ra) / 16).to(dtype), (eighths(g, vd, rg) / 16).to(dtype)
+    w_q, w_k, w_v = [(0.5 * r(n, taps)).to(dtype) for n in (kd, kd, vd)]
+    A_log, dt_bias, norm = (r(H) - 1).to(dtype), r(kd).to(dtype), (1 + 0.1 * r(vdim)).to(dtype)
+    pos = torch.tensor([5], dtype=torch.int32, device="cuda") if padded else None
+    start = torch.tensor([0, 6, 5][:B], dtype=torch.int32, device="cuda") if padded else None       # (the second sequence has not begun)
+    step = Step(B, 1, 0 if padded else 5, pos, start)
+    conv = [layer_ops.ConvState(B, taps, 2 * kd + vd, "cuda") for _ in range(2)]
+    conv[0].rows.copy_(r(*conv[0].rows.shape))
+    conv[1].rows.copy_(conv[0].rows)
+    S = [r(B, H, vdim, dim)]
+    S.append(S[0].clone())
+    out = [torch.zeros(B, vd + 8, dtype=dtype, device="cuda")[:, 8:] for _ in range(2)]
+    assert ops.delta_token_takes(q, k, xa, xg, wa, wg, S[0], taps, out[0], step)
+    ops.delta_token(q, k, v, b, xa, xg, wa, wg, w_q, w_k, w_v, A_log, dt_bias, norm, conv[0], S[0], 1e-5, out[0], 0.7, step)
+    a, gate = [(x.double() @ w.double().t()).to(dtype) for x, w in ((xa, wa), (xg, wg))]
+    x = ops.delta_prep(q, k, v, b, a, w_q, w_k, w_v, A_log, dt_bias, conv[1], dim, vdim, step)
+    ops.head_norm_gate(ops.delta_scan(x, S[1], step), norm, gate, H, 1e-5, out[1], 0.7)
+    assert torch.equal(conv[0].rows, conv[1].rows) and torch.equal(S[0], S[1]) and torch.equal(out[0], out[1])
+    assert float(out[0].abs().max()) > 0.1
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,H,dim,vdim,per_head,padded", [(1, 1, 8, 8, False, False), (8, 16, 128, 256, True, False), (3, 2, 64, 200, False, True),
+                                                          (2, 5, 40, 72, True, True), (33, 3, 120, 128, True, False)])
+def test_memory(B, H, dim, vdim, per_head, padded, dtype):
+    g = torch.Generator(device="cuda").manual_seed(dim + B)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    up = -(-H // 8) * 8
+    widths = [H * dim, H * dim, H * vdim, H * vdim, up, up]
+    p = r(B, sum(widths)).to(dtype)
+    at = [sum(widths[:i]) for i in range(7)]
+    q, k, v, gate, i, f = [p[:, at[n]:at[n + 1]] for n in range(6)]
+    i, f = 3 * i[:, :H], f[:, :H]
+    p[:, at[4]:at[4] + H] = i
+    i = p[:, at[4]:at[4] + H]
+    b_i, b_f, norm = r(H).to(dtype), (r(H) + 2).to(dtype), (1 + 0.1 * r(H * vdim if per_head else vdim)).to(dtype)
+    pos = torch.tensor([5], dtype=torch.int32, device="cuda") if padded else None
+    start = torch.tensor([0, 6, 5][:B], dtype=torch.int32, device="cuda") if padded else None
+    step = Step(B, 1, 0 if padded else 5, pos, start)
+    state = [ops.memory_state(B, H, dim, vdim, "cuda") for _ in range(2)]
+    state[0][0].copy_(r(*state[0][0].shape))
+    state[0][1].copy_(r(B, H, 1).expand_as(state[0][1]))
+    for a, c in zip(*state):
+        c.copy_(a)
+    out = [torch.zeros(B, H * vdim + 8, dtype=dtype, device="cuda")[:, 8:] for _ in range(2)]
+    assert ops.memory_token_takes(q, k, gate, norm, state[0][0], out[0], step)
+    ops.memory_token(q, k, v, gate, i, f, b_i, b_f, norm, *state[0], 15.0, dim ** -0.5, 1e-5, out[0], 0.7, step)
+    li, lf = ops.memory_gates(i, f, b_i, b_f, 15.0)
+    o, den = ops.memory_scan(q, k, v, li, lf, *state[1], dim ** -0.5, step)
+    ops.head_norm_gate(o, norm, gate, H, 1e-5, out[1], 0.7, den)
+    assert torch.equal(state[0][0], state[1][0]) and torch.equal(state[0][1], state[1][1]) and torch.equal(out[0], out[1])
+    assert float(out[0].abs().max()) > 0.1
