@@ -38,6 +38,9 @@
  *
  * pq_logits: y = cap * tanh(x w^T * scale / cap) in float32 (cap <= 0: x w^T * scale), sizes that stream
  *   only; *advance (or null) is raised by one.
+ * pq_linear_gelu: w [plain + 2 ff, K]; y = x w^T of its first `plain` rows, z = gelu(x w^T of the
+ *   next ff rows) * (x w^T of the last ff), both products rounded first as y is.  Up to 8 rows
+ *   of x, 16-bit dtypes, plain a multiple of 16, ff of 8, K of 64; x and w at 16 bytes, y and z at 8.
  */
 #ifndef POLARQUANT_STEPS_H
 #define POLARQUANT_STEPS_H
@@ -82,6 +85,10 @@ int pq_softcap(float *x, size_t n, float scale, float cap, void *stream);
 int pq_head_linear(const void *x, int64_t x_row_stride, int64_t x_head_stride, const void *w, const void *gate,
                    int64_t gate_row_stride, void *y, int64_t y_row_stride, int64_t y_head_stride, int M, int heads, int N,
                    int K, int epilogue, int dtype, void *stream);
+int pq_validate_linear_gelu(int64_t x_row_stride, int64_t y_row_stride, int64_t z_row_stride, int M, int plain, int ff, int K,
+                            int dtype);
+int pq_linear_gelu(const void *x, int64_t x_row_stride, const void *w, void *y, int64_t y_row_stride, void *z,
+                   int64_t z_row_stride, int M, int plain, int ff, int K, int dtype, void *stream);
 int pq_logits(const void *x, const void *w, float *y, int M, int N, int K, float scale, float cap, int32_t *advance, int dtype,
               void *stream);
 int pq_validate_head_linear(const void *x, int64_t x_row_stride, int64_t x_head_stride, const void *w, const void *gate,

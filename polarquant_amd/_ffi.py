@@ -112,6 +112,8 @@ STEPS_SIGNATURES = {
     "pq_embed_norm_conv_takes": (c_int, [c_int] * 4),
     "pq_embed_norm_conv": (c_int, [c_void_p, c_void_p, c_int64, c_float] + [c_void_p] * 8 + [c_int] * 6 + [c_float, c_int, c_void_p]),
     "pq_logits": (c_int, [c_void_p] * 3 + [c_int] * 3 + [c_float, c_float, c_void_p, c_int, c_void_p]),
+    "pq_validate_linear_gelu": (c_int, [c_int64] * 3 + [c_int] * 5),
+    "pq_linear_gelu": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_int64] + [c_int] * 5 + [c_void_p]),
     "pq_relu_sq": (c_int, [c_void_p] * 2 + [c_size_t] + [c_int] + [c_void_p]),
     "pq_gelu_mul": (c_int, [c_void_p] * 2 + [c_int64, c_void_p, c_int64, c_int64, c_int, c_int, c_void_p]),
     "pq_stream_add": (c_int, [c_void_p] * 5 + [c_int64, c_int, c_int, c_void_p]),

@@ -342,4 +342,10 @@ __device__ __forceinline__ void broadcast_cd(float cdv, float (&cds)[kPairs]) {
     for (int d = 0; d < kPairs; d++) cds[d] = readlane_f(cdv, d);
 }
 
+// gelu in its tanh form: 0.5 z (1 + tanh u) = z / (1 + exp(-2 u)), u = sqrt(2 / pi) (z + 0.044715 z^3)
+__device__ __forceinline__ float gelu_tanh(float z) {
+    const float u2 = 1.5957691216057308f * __builtin_fmaf(0.044715f * z * z, z, z);
+    return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(u2 * -1.4426950408889634f));
+}
+
 }  // namespace pq

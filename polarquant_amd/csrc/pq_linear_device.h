@@ -20,7 +20,9 @@
 //
 // EPI 0 is the kernel as described (bias, or the gated form); EPI 1 + e is the same stream for one of `heads` independent
 // products per launch (blockIdx.y == head, operands `x_head` / N * K / `y_head` elements apart) with epilogue e of
-// pq_steps_internal.h: plain, square of relu, times sigmoid(gate), unrounded float32 output, or that scaled and soft-capped.
+// pq_steps_internal.h: plain, square of relu, times sigmoid(gate), unrounded float32 output, that scaled and soft-capped, or plain rows and
+// behind them pairs of a gate's and another row whose results become gelu(gate) * other (small_m8_linear_kernel only; 8 rows, 18720 plain
+// rows and 14336 pairs of 4096: the step is 2.2 us a layer shorter, which was a launch of its own that moved 0.9 MB).
 #pragma once
 #include "pq_device.h"
 #include "pq_linear_rules.h"
@@ -44,12 +46,25 @@ template <> __device__ __forceinline__ floatx4_l mfma32<BF16>(u32x4_l a, u32x4_l
 template <typename T>
 __device__ __forceinline__ float rnd_l(float f) { return lo2f<T>(f2lo<T>(f)); }
 
+// a * u in the dtype.  Half: rounded once, by the instruction that gelu_mul_kernel's product compiles to (through float32 one result in ten
+// thousand is the other neighbour of a tie).
+template <typename T> __device__ __forceinline__ uint16_t times_rounded(float a, uint16_t u) { return f2lo<T>(a * lo2f<T>(u)); }
+template <> __device__ __forceinline__ uint16_t times_rounded<F16>(float a, uint16_t u) {
+    uint32_t r;
+    asm("v_fma_mixlo_f16 %0, %1, %2, 0 op_sel_hi:[0,1,0]" : "=v"(r) : "v"(a), "v"(static_cast<uint32_t>(u)));
+    return static_cast<uint16_t>(r);
+}
+
 struct HeadEpi {
     int64_t x_head, w_head, y_head;
     const uint16_t* gate;
     int64_t gate_row;
     float scale, cap;
     int32_t* advance;
+    // kEpiGeluPairs: workgroups from this one on take as many rows of the gate as of those `pair_rows` further, and store at z
+    int pair_from, pair_rows;
+    uint16_t* z;
+    int64_t z_row;
 };
 
 // of logits: a counter that nothing in this launch reads is raised by its first thread
@@ -230,7 +245,11 @@ __global__ __launch_bounds__(kWave * KSPLIT) void small_m8_linear_kernel(
     const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
     const int r = lane & 15, g = lane >> 4;
     const int row = r & 7, chunk = (r >> 3) * 4 + g;       // W row inside an 8-row tile == x row; 16-byte piece of the step
-    const int n0 = blockIdx.x * 8 * NT;
+    constexpr bool kGelu = EPI == 1 + kEpiGeluPairs;
+    const bool pairs = kGelu && static_cast<int>(blockIdx.x) >= he.pair_from;
+    // (a workgroup of pairs: the first half of its tiles are rows of the gate, the second those they meet)
+    const int n0 = pairs ? (he.pair_from + static_cast<int>(blockIdx.x)) * 4 * NT : blockIdx.x * 8 * NT;
+    const size_t apart = pairs ? static_cast<size_t>(he.pair_rows - 4 * NT) * K : 0;
     const int klen = K / KSPLIT, steps = klen / 64;
     const int m = row < M ? row : 0;                       // tile columns >= M repeat row 0 and are never stored
     const size_t koff = static_cast<size_t>(wv) * klen + 8 * chunk;
@@ -248,7 +267,7 @@ __global__ __launch_bounds__(kWave * KSPLIT) void small_m8_linear_kernel(
     auto load = [&](Stage8T<GATED, NT, kStage>& st, int s0) {      // branch-free, see small_m_linear_kernel
         static_for<kStage>([&](auto U) {
             constexpr int u = decltype(U)::value;
-            static_for<NT>([&](auto I) { st.w[I][u] = ldw(wp + I * tile + (s0 + u) * 64); });
+            static_for<NT>([&](auto I) { st.w[I][u] = ldw((kGelu && I >= NT / 2 ? wp + apart : wp) + I * tile + (s0 + u) * 64); });
             if constexpr (GATED) static_for<NT>([&](auto I) { st.u[I][u] = ldw(up + I * tile + (s0 + u) * 64); });
             st.x[u] = *reinterpret_cast<const u32x4_l*>(xp + (s0 + u) * 64);
         });
@@ -285,7 +304,7 @@ __global__ __launch_bounds__(kWave * KSPLIT) void small_m8_linear_kernel(
     for (int s1 = full * kStage; s1 < steps; s1++) {
         const u32x4_l xv1 = *reinterpret_cast<const u32x4_l*>(xp + s1 * 64);
         static_for<NT>([&](auto I) {
-            acc[I] = mfma32<T>(ldw(wp + I * tile + s1 * 64), xv1, acc[I]);
+            acc[I] = mfma32<T>(ldw((kGelu && I >= NT / 2 ? wp + apart : wp) + I * tile + s1 * 64), xv1, acc[I]);
             if constexpr (GATED) acu[I] = mfma32<T>(ldw(up + I * tile + s1 * 64), xv1, acu[I]);
         });
     }
@@ -301,6 +320,26 @@ __global__ __launch_bounds__(kWave * KSPLIT) void small_m8_linear_kernel(
     // entry (row 4g + i, column r) and its diagonal partner (row + 8, column + 8), which lane + 40 holds
     if (r >= 8 || r >= M || g >= 2) return;
     for (int h = wv; h < NT; h += KSPLIT) {
+        if constexpr (kGelu) {
+            if (pairs) {
+                if (h >= NT / 2) continue;
+                uint16_t out[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    float s = 0.0f, t = 0.0f;
+#pragma unroll
+                    for (int k = 0; k < KSPLIT; k++) {
+                        s += part[k][h][i][lane] + part[k][h][i][lane + 40];
+                        t += part[k][h + NT / 2][i][lane] + part[k][h + NT / 2][i][lane + 40];
+                    }
+                    out[i] = times_rounded<T>(gelu_tanh(rnd_l<T>(s)), f2lo<T>(t));     // (both rounded as a product of its own leaves them)
+                }
+                const int c = (static_cast<int>(blockIdx.x) - he.pair_from) * 4 * NT + 8 * h + 4 * g;
+                *reinterpret_cast<uint2*>(he.z + static_cast<size_t>(r) * he.z_row + c) =
+                    make_uint2(static_cast<uint32_t>(out[0]) | (static_cast<uint32_t>(out[1]) << 16), static_cast<uint32_t>(out[2]) | (static_cast<uint32_t>(out[3]) << 16));
+                continue;
+            }
+        }
         if constexpr (EPI != 0) {
             float s4[4];
 #pragma unroll

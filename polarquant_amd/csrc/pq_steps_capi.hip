@@ -133,4 +133,21 @@ int pq_logits(const void* x, const void* w, float* y, int M, int N, int K, float
     return status(pq::launch_head_linear_mfma(a, dtype, static_cast<hipStream_t>(stream)));
 }
 
+int pq_validate_linear_gelu(int64_t x_row_stride, int64_t y_row_stride, int64_t z_row_stride, int M, int plain, int ff, int K, int dtype) {
+    if (dtype != PQ_F16 && dtype != PQ_BF16) return PQ_ERR_BAD_DTYPE;
+    if (M < 1 || M > 8 || plain < 16 || plain % 16 || ff < 8 || ff % 8 || K < 64 || K % 64 || static_cast<int64_t>(plain) + 2 * static_cast<int64_t>(ff) > (1 << 30))
+        return PQ_ERR_BAD_SHAPE;
+    if (x_row_stride < K || x_row_stride % 8 || y_row_stride < plain || y_row_stride % 4 || z_row_stride < ff || z_row_stride % 4) return PQ_ERR_BAD_STRIDE;
+    return PQ_OK;
+}
+
+int pq_linear_gelu(const void* x, int64_t x_row_stride, const void* w, void* y, int64_t y_row_stride, void* z, int64_t z_row_stride, int M, int plain, int ff,
+                   int K, int dtype, void* stream) {
+    if (!x || !w || !y || !z) return PQ_ERR_NULL_POINTER;
+    if (int rc = pq_validate_linear_gelu(x_row_stride, y_row_stride, z_row_stride, M, plain, ff, K, dtype)) return rc;
+    if (!aligned(x, 16) || !aligned(w, 16) || !aligned(y, 8) || !aligned(z, 8)) return PQ_ERR_MISALIGNED;
+    pq::LinearGeluArgs a{x, x_row_stride, w, y, z, y_row_stride, z_row_stride, M, plain, ff, K};
+    return status(pq::launch_linear_gelu(a, dtype, static_cast<hipStream_t>(stream)));
+}
+
 }  // extern "C"

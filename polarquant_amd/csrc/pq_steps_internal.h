@@ -59,7 +59,8 @@ int launch_embed_rows(const void* table, const int64_t* ids, float scale, float*
 int launch_softcap(float* x, size_t n, float scale, float cap, hipStream_t st);
 
 // y[m, h, n] = epilogue(sum_k x[m, h, k] w[h, n, k])
-enum { kEpiPlain = 0, kEpiReluSq = 1, kEpiSigmoidGate = 2, kEpiF32 = 3, kEpiLogits = 4 };      // (the last: float32, scaled and soft-capped)
+// (kEpiLogits: float32, scaled and soft-capped; kEpiGeluPairs: LinearGeluArgs)
+enum { kEpiPlain = 0, kEpiReluSq = 1, kEpiSigmoidGate = 2, kEpiF32 = 3, kEpiLogits = 4, kEpiGeluPairs = 5 };
 struct HeadLinearArgs {
     const void* x;
     int64_t x_row, x_head;
@@ -73,6 +74,16 @@ struct HeadLinearArgs {
     int32_t* advance;        // kEpiLogits: raised by one, or null
 };
 int launch_head_linear_any(const HeadLinearArgs& a, int dtype, hipStream_t st);      // pq_steps.hip: any size, any dtype
+// w [plain + 2 ff, K]: y = x w^T of the first `plain` rows, z = gelu(x w^T of the next ff) * (x w^T of the last ff); up to 8 rows of x
+struct LinearGeluArgs {
+    const void* x;
+    int64_t x_row;
+    const void* w;
+    void *y, *z;
+    int64_t y_row, z_row;
+    int M, plain, ff, K;
+};
+int launch_linear_gelu(const LinearGeluArgs& a, int dtype, hipStream_t st);          // pq_head_linear.hip: plain % 16 == 0, ff % 8 == 0, K % 64 == 0
 int launch_head_linear_mfma(const HeadLinearArgs& a, int dtype, hipStream_t st);     // pq_head_linear.hip: M <= 16, N % 16 == 0, K % 32 == 0
 
 }  // namespace pq

@@ -74,12 +74,17 @@ def norm_conv(x: torch.Tensor, w_pre: torch.Tensor, groups: int, eps: float, y: 
     return (x if y is None else x_out), h
 
 
+def runs_plainly(module) -> bool:
+    """Whether nothing hangs onto a module's call (or onto all modules'), so that what it does may run without one."""
+    return (not module._forward_hooks and not module._forward_pre_hooks and "forward" not in module.__dict__
+            and not torch.nn.modules.module._has_any_global_hook())
+
+
 def only_looks_up(embed, dtype: torch.dtype) -> bool:
     """An embedding module without anything of its own or hung onto it (or onto all modules), whose table is a plain tensor that a launch
     can read as it lies."""
     w = getattr(embed, "weight", None)
-    return (type(embed) is torch.nn.Embedding and embed.max_norm is None and not embed._forward_hooks and not embed._forward_pre_hooks
-            and "forward" not in embed.__dict__ and not torch.nn.modules.module._has_any_global_hook()
+    return (type(embed) is torch.nn.Embedding and embed.max_norm is None and runs_plainly(embed)
             and (type(w) is torch.nn.Parameter or type(w) is torch.Tensor)              # (a subclass says for itself what its rows are)
             and w.dtype == dtype and w.is_contiguous() and w.data_ptr() % 16 == 0)
 
@@ -217,6 +222,26 @@ def linear(x: torch.Tensor, w: torch.Tensor, relu_squared: bool = False) -> torc
         return y.view(x.shape[:-1] + (w.shape[0],))
     y = torch.nn.functional.linear(x, w)
     return relu_sq(y) if relu_squared else y
+
+
+def linear_gelu_takes(x: torch.Tensor, w: torch.Tensor, plain: int, ff: int, z: torch.Tensor) -> bool:
+    """Whether `linear_gelu` takes rows x and a w of at least plain + 2 ff rows (more are left alone)."""
+    M, K = x.shape
+    return (x.dtype in (torch.float16, torch.bfloat16) and x.dtype == w.dtype == z.dtype and w.is_contiguous() and w.shape[0] >= plain + 2 * ff
+            and w.shape[1] == K and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and z.data_ptr() % 8 == 0
+            and _ffi.steps_lib().call.pq_validate_linear_gelu(x.stride(0), plain, z.stride(0), M, plain, ff, K, _DTYPES[x.dtype]) == 0)
+
+
+def linear_gelu(x: torch.Tensor, w: torch.Tensor, plain: int, ff: int, z: torch.Tensor) -> torch.Tensor:
+    """Rows x [M, K] -> x w[:plain]^T, and gelu(x w[plain : plain + ff]^T) * (x w[plain + ff : plain + 2 ff]^T) in the rows z [M, ff]: one
+    launch, the same bits as `linear` and `gelu_mul`."""
+    M, K = x.shape
+    assert z.shape == (M, ff) and z.stride(1) == x.stride(1) == 1 and w.device == z.device == x.device
+    y = torch.empty(M, plain, dtype=x.dtype, device=x.device)
+    with _on_device(x.device):
+        rc = _ffi.steps_lib().call.pq_linear_gelu(x, x.stride(0), w, y, plain, z, z.stride(0), M, plain, ff, K, _code(x), _stream_ptr(x.device))
+    _ffi.check(rc, "pq_linear_gelu")
+    return y
 
 
 def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

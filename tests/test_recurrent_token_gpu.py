@@ -82,3 +82,21 @@ def test_memory(B, H, dim, vdim, per_head, padded, dtype):
     ops.head_norm_gate(o, norm, gate, H, 1e-5, out[1], 0.7, den)
     assert torch.equal(state[0][0], state[1][0]) and torch.equal(state[0][1], state[1][1]) and torch.equal(out[0], out[1])
     assert float(out[0].abs().max()) > 0.1
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,plain,ff,K", [(1, 16, 8, 64), (8, 18720, 14336, 4096), (3, 48, 24, 128), (5, 4096, 256, 2048), (8, 64, 40, 8192), (7, 160, 96, 8256),
+                                          (2, 8192, 4096, 512), (6, 2048, 65536, 192)])
+def test_products_with_gelu(M, plain, ff, K, dtype):
+    """Rows of w by the pair; w has rows behind them that are left alone."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x = torch.randn(M, K + 8, generator=g, device="cuda").to(dtype)[:, :K]
+    w = (torch.randn(plain + 2 * ff + 16, K, generator=g, device="cuda") / K ** 0.5).to(dtype)
+    z = torch.full((M, ff + 12), 7.0, dtype=dtype, device="cuda")
+    assert layer_ops.linear_gelu_takes(x, w, plain, ff, z[:, 4:4 + ff])
+    y = layer_ops.linear_gelu(x, w, plain, ff, z[:, 4:4 + ff])
+    p = layer_ops.linear(x, w)
+    want = layer_ops.gelu_mul(p[:, plain:plain + ff], p[:, plain + ff:plain + 2 * ff])
+    assert torch.equal(y, p[:, :plain]) and torch.equal(z[:, 4:4 + ff], want)
+    assert bool((z[:, :4] == 7).all()) and bool((z[:, 4 + ff:] == 7).all())
+    assert not layer_ops.linear_gelu_takes(x, w, plain, ff + 16, z[:, 4:]) and not layer_ops.linear_gelu_takes(x[:, 1:], w, plain, ff, z[:, 4:])
