@@ -202,9 +202,8 @@ __device__ __forceinline__ void attn_piece(const AttnParams& p, const V4Args& v4
             for (int grp = g0; grp < g1; grp++) {
                 PQ_T_MARK();
                 asm volatile("" ::: "memory");
-                const float cdv = build_lut<T, TB, REPP>(lut, lane, qx, qy, mrs, mrm, mts, mtm);
-                float cds[kPairs];
-                broadcast_cd(cdv, cds);
+                Cds<TB, REPP> cds;
+                broadcast_cd(build_lut<T, TB, REPP, true>(lut, lane, qx, qy, mrs, mrm, mts, mtm), cds);
                 asm volatile("" ::: "memory");
                 PQ_T_ADD(0);
                 if (grp + 1 < g1) {
@@ -301,7 +300,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu((V4 && RE
 void attn_kernel(PQ_ATTN_KERNEL_PARAMS) {
     using L = Lut<TB, REPP>;
     // the table region doubles as the staging buffer of the residual block's scores ([REPP][64] fp32)
-    constexpr int kLutBytes = L::BYTES > REPP * kWave * 4 ? L::BYTES : REPP * kWave * 4;
+    constexpr int kLutBytes = L::ALL_BYTES > REPP * kWave * 4 ? L::ALL_BYTES : REPP * kWave * 4;
     __shared__ __attribute__((aligned(16))) char lut_mem[kLutBytes];
     __shared__ __attribute__((aligned(16))) uint16_t p_mem[REPP * kWave];
     const uint32_t lut = lds_addr(lut_mem), pbuf = lds_addr(p_mem);
@@ -342,7 +341,7 @@ template <typename T, int TB, int REPP, bool V4, bool PK6>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu((V4 && REPP <= 4 && TB <= 4) ? 2 : 1, 2)))
 void attn_balanced_kernel(PQ_ATTN_KERNEL_PARAMS) {
     using L = Lut<TB, REPP>;
-    constexpr int kLutBytes = L::BYTES > REPP * kWave * 4 ? L::BYTES : REPP * kWave * 4;
+    constexpr int kLutBytes = L::ALL_BYTES > REPP * kWave * 4 ? L::ALL_BYTES : REPP * kWave * 4;
     __shared__ __attribute__((aligned(16))) char lut_mem[kLutBytes];
     __shared__ __attribute__((aligned(16))) uint16_t p_mem[REPP * kWave];
     __shared__ int walk[kWalkInts];

@@ -63,8 +63,8 @@ __device__ __forceinline__ PairMem pair_mem(uint32_t lut, uint32_t sbuf, uint32_
 
 // A hand-over gave up: tell the host, if it passed a status word.  One lane, an ordinary vector store of a constant
 // (every wavefront that fails writes the same value, so no atomic is needed).  The pointer waits in LDS (stash_status,
-// before the workgroup's barrier) instead of in two scalar registers for the whole kernel: the scorer's group loop holds
-// 64 wave-uniform radius offsets in scalar registers and has none to spare.
+// before the workgroup's barrier) instead of in two scalar registers for the whole kernel: the scorer's group loop may hold
+// 64 wave-uniform radius offsets in scalar registers (one or two heads) and then has none to spare.
 typedef __attribute__((address_space(3))) unsigned long long lds_u64;
 __device__ __forceinline__ void stash_status(unsigned long long* slot, int* status) {
     if (threadIdx.x == 0) *slot = reinterpret_cast<unsigned long long>(status);
@@ -132,7 +132,7 @@ __device__ __forceinline__ bool pair_scorer(const AttnParams& p, const PairMem& 
     const uint16_t* qb = p.q + (static_cast<size_t>(b) * p.N + static_cast<size_t>(kvh) * rep) * kHeadDim;
     // polls a wait may still make: after one wait has given up it is 0, and every later wait falls through at once.  (One
     // scalar register; a separate "all hand-overs succeeded so far" flag would be a second and third, which the group
-    // loop, with its 64 wave-uniform radius offsets, does not have.)
+    // loop does not have where it holds 64 wave-uniform radius offsets.)
     int spin = pm.spin_limit;
     PQ_PAIR_T_MARK(0, false);
     auto publish_begin = [&]() {            // the buffer of tile k is free once tile k - 2 has been consumed
@@ -176,9 +176,8 @@ __device__ __forceinline__ bool pair_scorer(const AttnParams& p, const PairMem& 
         for (int grp = g0; grp < g1; grp++) {
             asm volatile("" ::: "memory");
             PQ_PAIR_T_MARK(1, true);
-            const float cdv = build_lut<T, TB, REPP>(pm.lut, lane, qx, qy, mrs, mrm, mts, mtm);
-            float cds[kPairs];
-            broadcast_cd(cdv, cds);
+            Cds<TB, REPP> cds;
+            broadcast_cd(build_lut<T, TB, REPP, true>(pm.lut, lane, qx, qy, mrs, mrm, mts, mtm), cds);
             asm volatile("" ::: "memory");
             PQ_PAIR_T_MARK(2, false);
             if (grp + 1 < g1) {
@@ -401,7 +400,7 @@ template <typename T, int TB, int REPP, bool PK6>
 __global__ __launch_bounds__(kPairsPerBlock * 2 * kWave) void attn_pair_kernel(PQ_ATTN_KERNEL_PARAMS, int n_slices_total, int silent_scorer,
                                                                               int* __restrict__ status, uint16_t* __restrict__ direct_out) {
     using L = Lut<TB, REPP>;
-    __shared__ __attribute__((aligned(16))) char lut_mem[kPairsPerBlock][L::BYTES];
+    __shared__ __attribute__((aligned(16))) char lut_mem[kPairsPerBlock][L::ALL_BYTES];
     __shared__ __attribute__((aligned(16))) float s_mem[kPairsPerBlock][2 * REPP * kWave];
     __shared__ __attribute__((aligned(16))) uint16_t p_mem[kPairsPerBlock][REPP * kWave];
     __shared__ int flag_mem[kPairsPerBlock][4];
@@ -444,7 +443,7 @@ template <typename T, int TB, int REPP, bool PK6>
 __global__ __launch_bounds__(kPairsPerBlock * 2 * kWave) void attn_pair_balanced_kernel(PQ_ATTN_KERNEL_PARAMS, int n_pairs_total, int silent_scorer,
                                                                                        int* __restrict__ status) {
     using L = Lut<TB, REPP>;
-    __shared__ __attribute__((aligned(16))) char lut_mem[kPairsPerBlock][L::BYTES];
+    __shared__ __attribute__((aligned(16))) char lut_mem[kPairsPerBlock][L::ALL_BYTES];
     __shared__ __attribute__((aligned(16))) float s_mem[kPairsPerBlock][2 * REPP * kWave];
     __shared__ __attribute__((aligned(16))) uint16_t p_mem[kPairsPerBlock][REPP * kWave];
     __shared__ int flag_mem[kPairsPerBlock][4];

@@ -19,6 +19,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 #include <stdint.h>
+#include <type_traits>
 
 namespace pq {
 
@@ -109,6 +110,10 @@ struct Lut {
     static constexpr int PB = NB * EB;            // bytes per pair
     static constexpr int HB = kPairs * PB;        // bytes per half
     static constexpr int BYTES = HALVES * HB;
+    // attention's c_d (score_token): in LDS from three heads on, c_d of pair d in the word of no head if its entries have one (three or
+    // seven heads), else the d-th float behind the table
+    static constexpr bool C_IN_LDS = REPP > 2, SPARE = WORDS > REPP;
+    static constexpr int C0 = BYTES, ALL_BYTES = BYTES + (C_IN_LDS && !SPARE ? kPairs * 4 : 0);
     // theta * EB fits a byte: the four byte offsets of a code word are made by two instructions on the
     // whole word; beyond that (TB 5, 6 with 16-byte entries) each code's offset is shifted into place
     static constexpr bool PACKED_OFFSETS = TB + SH <= 8;
@@ -163,12 +168,8 @@ __device__ __forceinline__ void lds_store_w(uint32_t addr, const float* e) {
     } else if constexpr (W == 2) {
         lds_e2* p = lds_ptr<lds_e2>(addr);
         p->x = e[0]; p->y = e[1];
-    } else if constexpr (W == 3) {
-        lds_e4* p = lds_ptr<lds_e4>(addr);
-        p->x = e[0]; p->y = e[1]; p->z = e[2]; p->w = 0.0f;
     } else {
-        lds_e4* p = lds_ptr<lds_e4>(addr);
-        p->x = e[0]; p->y = e[1]; p->z = e[2]; p->w = e[3];
+        *lds_ptr<lds_f4>(addr) = float4_v{e[0], e[1], e[2], W == 3 ? 0.0f : e[3]};     // (member by member it becomes two ds_write2_b32)
     }
 }
 
@@ -209,20 +210,22 @@ __device__ __forceinline__ void sincos_bin(float x, float* sn, float* cs) {
 
 // Build the table for one group.  lane == pair d.
 //   qx[j], qy[j]: q_j[d], q_j[d+64]
-//   returns c_d for this lane's pair.
-template <typename T, int TB, int REPP>
+//   returns c_d for this lane's pair; for attention (ATTN) it may be left in LDS too (Lut::C_IN_LDS).
+// Attention: the bins lie evenly about an angle m; with A = ax cos m + ay sin m and B = ay cos m - ax sin m the entries at m + phi and m - phi
+// are A cos phi + B sin phi and A cos phi - B sin phi, three instructions a head for two bins instead of four, and one rotation of phi
+// serves both (4-bit values, 4 heads, 8 x 16384, with the c_d in LDS 49.7 -> 48.5 us; half-precision values, 7 heads, 4 x 16384 25.4 -> 24.4).  Scores are results themselves and go from bin to bin: an infinite query's are
+// infinite that way, where A and B would cancel to NaN (in a softmax either ends as NaN).
+template <typename T, int TB, int REPP, bool ATTN>
 __device__ __forceinline__ float build_lut(uint32_t lut, int lane, const float (&qx)[REPP], const float (&qy)[REPP],
                                            uint16_t w_rscale, uint16_t w_rmn, uint16_t w_tscale, uint16_t w_tmn) {
     using L = Lut<TB, REPP>;
     const float ts = lo2f<T>(w_tscale), tm = lo2f<T>(w_tmn);
     const float rs = lo2f<T>(w_rscale), rm = lo2f<T>(w_rmn);
-    float s, c, sd, cd;
-    sincos_bin(__builtin_fmaf(ts, 0.5f, tm), &s, &c);
-    sincos_bin(ts, &sd, &cd);
     const float rmp = __builtin_fmaf(rs, 0.5f, rm);
     float a, cdv;
     if (rs != 0.0f) { a = rs; cdv = rmp / rs; }
     else            { a = rmp * 0x1p-40f; cdv = 0x1p40f; }   // (rho + 2^40) * 2^-40 == 1 exactly
+    if constexpr (ATTN && L::C_IN_LDS && !L::SPARE) *lds_ptr<lds_f1>(lut + L::C0 + lane * 4) = cdv;
     float ax[REPP], ay[REPP];
 #pragma unroll
     for (int j = 0; j < REPP; j++) { ax[j] = qx[j] * a; ay[j] = qy[j] * a; }
@@ -230,29 +233,71 @@ __device__ __forceinline__ float build_lut(uint32_t lut, int lane, const float (
     // pair's base: nothing here depends on how the table is aligned in LDS.
     const uint32_t pair_base = lut + lane * L::PB;
     const uint32_t swz = lane & (L::NB - 1);
-#pragma unroll
-    for (int k = 0; k < L::NB; k++) {
-        float e[REPP];
-#pragma unroll
-        for (int j = 0; j < REPP; j++) e[j] = __builtin_fmaf(ax[j], c, ay[j] * s);
+    auto store = [&](int k, float (&e)[L::WORDS]) {
+        if constexpr (L::SPARE) e[REPP] = ATTN ? cdv : 0.0f;
         const uint32_t off = pair_base + ((swz ^ k) << L::SH);
-        lds_store_w<L::W0>(off, e);
-        if constexpr (L::W1 > 0) lds_store_w<L::W1>(off + L::HB, e + 4);
-        const float c2 = __builtin_fmaf(c, cd, -(s * sd));
-        const float s2 = __builtin_fmaf(s, cd, c * sd);
-        c = c2; s = s2;
+        lds_store_w<(L::WORDS < 4 ? L::WORDS : 4)>(off, e);
+        if constexpr (L::W1 > 0) lds_store_w<L::WORDS - 4>(off + L::HB, e + 4);
+    };
+    float s, c, sd, cd;
+    if constexpr (ATTN) {
+        constexpr int kHalf = L::NB / 2;
+        float sm, cm;
+        sincos_bin(__builtin_fmaf(ts, static_cast<float>(kHalf), tm), &sm, &cm);
+        sincos_bin(ts * 0.5f, &s, &c);
+        cd = __builtin_fmaf(-2.0f * s, s, 1.0f);
+        sd = 2.0f * s * c;
+#pragma unroll
+        for (int j = 0; j < REPP; j++) {
+            const float x = ax[j], y = ay[j];
+            ax[j] = __builtin_fmaf(x, cm, y * sm);
+            ay[j] = __builtin_fmaf(y, cm, -(x * sm));
+        }
+#pragma unroll
+        for (int k = 0; k < kHalf; k++) {
+            float up[L::WORDS], dn[L::WORDS];
+#pragma unroll
+            for (int j = 0; j < REPP; j++) {
+                const float mid = ax[j] * c;
+                up[j] = __builtin_fmaf(ay[j], s, mid);
+                dn[j] = __builtin_fmaf(-ay[j], s, mid);
+            }
+            store(kHalf + k, up);
+            store(kHalf - 1 - k, dn);
+            const float c2 = __builtin_fmaf(c, cd, -(s * sd));
+            const float s2 = __builtin_fmaf(s, cd, c * sd);
+            c = c2; s = s2;
+        }
+    } else {
+        sincos_bin(__builtin_fmaf(ts, 0.5f, tm), &s, &c);
+        sincos_bin(ts, &sd, &cd);
+#pragma unroll
+        for (int k = 0; k < L::NB; k++) {
+            float e[L::WORDS];
+#pragma unroll
+            for (int j = 0; j < REPP; j++) e[j] = __builtin_fmaf(ax[j], c, ay[j] * s);
+            store(k, e);
+            const float c2 = __builtin_fmaf(c, cd, -(s * sd));
+            const float s2 = __builtin_fmaf(s, cd, c * sd);
+            c = c2; s = s2;
+        }
     }
     return cdv;
 }
 
 // Score one token against the table.  `codes` holds the token's 64 pair codes as
-// 16 little-endian words; cds[d] are the wave-uniform c_d.  acc[j] += ...
+// 16 little-endian words.  acc[j] += ...  `cds` says where the c_d are: InLds, as build_lut leaves them (with the entry, or four to a read
+// that all lanes share), or 64 scalar registers.  Attention with three heads and more has them in LDS: its scalar registers hold much
+// else, of which the 64 spilled half, and the 64 readlanes of a group are as many instructions as a tenth of a tile's walk.  For one
+// or two heads the reads cost more than they save (4-bit values, one head, 8 x 4096: 44.2 us, in LDS 44.8).  The score kernel's wavefront walks one group,
+// and 256 bytes more would leave a unit nine tables of four heads instead of ten (8 sequences of 16384, 4 heads 30.6 us, in LDS 34.3).
+struct InLds {};
 // The 64 table reads are issued in batches of 4 or 8 codes, one batch ahead of the
 // FMAs that consume them, so that 4-16 LDS reads are always in flight.
-template <int TB, int REPP>
-__device__ __forceinline__ void score_token(uint32_t lut, const uint32_t (&codes)[16], const float (&cds)[kPairs],
-                                            float (&acc)[REPP]) {
+template <int TB, int REPP, typename C>
+__device__ __forceinline__ void score_token(uint32_t lut, const uint32_t (&codes)[16], const C& cds, float (&acc)[REPP]) {
     using L = Lut<TB, REPP>;
+    constexpr bool kInLds = std::is_same<C, InLds>::value;
     constexpr uint32_t TM4 = ((1u << TB) - 1u) * 0x01010101u;
     constexpr uint32_t RM4 = (0xFFu >> TB) * 0x01010101u;
     constexpr int nbm = L::NB - 1;
@@ -260,12 +305,14 @@ __device__ __forceinline__ void score_token(uint32_t lut, const uint32_t (&codes
     constexpr int NBATCH = 16 / BW;
     float e[2][BW * 4][L::WORDS];
     uint32_t r4s[2][BW];
+    float cs[2][BW][4];
 
     auto load = [&](auto BI) {
         constexpr int bi = decltype(BI)::value, buf = bi & 1;
         static_for<BW>([&](auto CC) {
             constexpr int cc = decltype(CC)::value, c = bi * BW + cc;
             const uint32_t w = codes[c];
+            if constexpr (kInLds && !L::SPARE) lds_load_w<4>(lut + L::C0 + 16 * c, cs[buf][cc]);
             // byte i of ks: XOR pattern (slot swizzle) of pair 4c+i
             constexpr uint32_t ks = ((uint32_t)((4 * c + 0) & nbm)) | ((uint32_t)((4 * c + 1) & nbm) << 8) |
                                     ((uint32_t)((4 * c + 2) & nbm) << 16) | ((uint32_t)((4 * c + 3) & nbm) << 24);
@@ -283,21 +330,25 @@ __device__ __forceinline__ void score_token(uint32_t lut, const uint32_t (&codes
                 uint32_t off = (a4 >> (8 * i)) & 0xFFu;
                 if constexpr (!L::PACKED_OFFSETS) off <<= L::SH;
                 const uint32_t addr = lut + off + d * L::PB;
-                lds_load_w<L::W0>(addr, &e[buf][cc * 4 + i][0]);
-                if constexpr (L::W1 > 0) lds_load_w<L::W1>(addr + L::HB, &e[buf][cc * 4 + i][4]);
+                lds_load_w<(L::WORDS < 4 ? L::WORDS : 4)>(addr, &e[buf][cc * 4 + i][0]);
+                if constexpr (L::W1 > 0) lds_load_w<L::WORDS - 4>(addr + L::HB, &e[buf][cc * 4 + i][4]);
             });
         });
     };
     auto compute = [&](auto BI) {
         constexpr int bi = decltype(BI)::value, buf = bi & 1;
         static_for<BW>([&](auto CC) {
-            constexpr int cc = decltype(CC)::value, c = bi * BW + cc;
+            constexpr int cc = decltype(CC)::value;
             const uint32_t r4 = r4s[buf][cc];
             // consume the batch's reads youngest first: the first use then waits for the whole
             // batch at once (LDS returns in order) and the other three need no wait instruction
             static_for<4>([&](auto II) {
                 constexpr int i = 3 - decltype(II)::value;
-                const float t = static_cast<float>((r4 >> (8 * i)) & 0xFFu) + cds[4 * c + i];
+                float cd;
+                if constexpr (!kInLds) cd = cds[4 * decltype(BI)::value * BW + 4 * cc + i];
+                else if constexpr (L::SPARE) cd = e[buf][cc * 4 + i][REPP];
+                else cd = cs[buf][cc][i];
+                const float t = static_cast<float>((r4 >> (8 * i)) & 0xFFu) + cd;
                 static_for<REPP>([&](auto JJ) {
                     constexpr int j = decltype(JJ)::value;
                     acc[j] = __builtin_fmaf(e[buf][cc * 4 + i][j], t, acc[j]);
@@ -336,6 +387,9 @@ __device__ __forceinline__ void unpack6(const uint32_t (&p)[12], uint32_t (&cw)[
     });
 }
 
+// Where attention's walk looks for the c_d, and how they get there from build_lut's result.
+template <int TB, int REPP> using Cds = std::conditional_t<Lut<TB, REPP>::C_IN_LDS, InLds, float[kPairs]>;
+__device__ __forceinline__ void broadcast_cd(float, InLds&) {}
 // Broadcast the 64 per-pair c_d values (lane d holds c_d) into wave-uniform registers.
 __device__ __forceinline__ void broadcast_cd(float cdv, float (&cds)[kPairs]) {
 #pragma unroll

@@ -40,7 +40,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(Lut<TB, R
         qy[j] = ok ? lo2f<T>(qb[j * kHeadDim + kPairs + lane]) : 0.0f;
     }
     const size_t mi = gidx * kPairs + lane;
-    const float cdv = build_lut<T, TB, REPP>(lut, lane, qx, qy, rscale[mi], rmn[mi], tscale[mi], tmn[mi]);
+    const float cdv = build_lut<T, TB, REPP, false>(lut, lane, qx, qy, rscale[mi], rmn[mi], tscale[mi], tmn[mi]);
     float cds[kPairs];
     broadcast_cd(cdv, cds);
     __syncthreads();

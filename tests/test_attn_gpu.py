@@ -126,6 +126,16 @@ def test_attn_matches_oracle(gpu, dtype, N, Nk, rbits, tbits):
     assert nbad == 0
 
 
+@pytest.mark.parametrize("heads", range(1, 9))
+@pytest.mark.parametrize("tbits", [1, 2, 3, 4])
+def test_attn_every_table(gpu, heads, tbits):
+    """Every width of an entry (the radius offsets are with the entry, behind the table or in scalar registers) and every number of bins, two
+    of them the fewest: the bar of the file against both references."""
+    print("case", heads, tbits, flush=True)
+    out, ref, ref64 = _case(gpu, 1, heads, 1, 2, 1, 4, tbits, torch.float16, seed=10 * heads + tbits)
+    assert _close(out, ref)[0] == 0 and _close(out, ref64)[0] == 0, (_close(out, ref), _close(out, ref64))
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_attn_largest_table(gpu, dtype):
     """8 heads per KV head with 16 angle bins: the largest table (32 KB per slice; 148 KB of LDS for a workgroup of four

@@ -129,6 +129,16 @@ def test_attention_v4_matches_oracle(gpu, N, Nk, n_groups, n_resid):
         assert nbad == 0, (nbad, emax)
 
 
+@pytest.mark.parametrize("heads", [1, 2, 3, 8])
+@pytest.mark.parametrize("rbits,tbits", [(4, 1), (3, 5)])
+def test_attention_v4_every_table(gpu, heads, rbits, tbits):
+    """Widths of an entry with the fewest bins and with more than 16."""
+    out, ref, ref64 = _case(gpu, 1, heads, 1, 3, 1, rbits, tbits, torch.float16, seed=10 * heads + tbits)
+    for r in (ref, ref64):
+        nbad, emax = _close(out, r)
+        assert nbad == 0, (nbad, emax)
+
+
 @pytest.mark.parametrize("rbits,tbits", [(3, 3), (4, 2)])
 def test_attention_v4_other_bit_widths_mask_and_capacity(gpu, rbits, tbits):
     out, ref, ref64 = _case(gpu, 3, 8, 2, 5, 33, rbits, tbits, torch.float16, mask_pad=150, seed=9, caps=(3, 7))
