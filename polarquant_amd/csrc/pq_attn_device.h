@@ -24,6 +24,16 @@ template <> __device__ __forceinline__ floatx4 mfma16<BF16>(uint2 a, uint2 b, fl
     return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(short4_t, a), __builtin_bit_cast(short4_t, b), c, 0, 0, 0);
 }
 
+// 32 deep: k-slots 0 .. 3 of a lane are those of a0 and b0, 4 .. 7 those of a1 and b1
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+template <typename T> __device__ __forceinline__ floatx4 mfma16x2(uint2 a0, uint2 a1, uint2 b0, uint2 b1, floatx4 c) {
+    const u32x4_t a = {a0.x, a0.y, a1.x, a1.y}, b = {b0.x, b0.y, b1.x, b1.y};
+    if constexpr (std::is_same<T, F16>::value) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+
 // 2^x as the bare v_exp_f32: exact to 1 ulp over the normal range and 0 below 2^-126, where the library's exp2f spends
 // five more instructions to return a denormal.  Every use here is a softmax weight relative to a running maximum: a
 // weight below 2^-126 is nothing against the maximum's weight of at least 2^-8.
@@ -40,9 +50,27 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
+// The maximum over the wavefront in a scalar register, by DPP (six trips through the LDS otherwise, whenever a tile raises a maximum): within rows of 16 lanes, then over the rows; lane 63 has it.
+__device__ __forceinline__ float wave_max_dpp(float v) {
+    auto step = [&](auto CTRL) {
+        const float o = __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(__float_as_uint(v)), static_cast<int>(__float_as_uint(v)),
+                                                                                          decltype(CTRL)::value, 0xf, 0xf, false)));
+        v = fmaxf(v, o);
+    };
+    step(IC<0x111>{});       // row_shr 1, 2, 4, 8
+    step(IC<0x112>{});
+    step(IC<0x114>{});
+    step(IC<0x118>{});
+    step(IC<0x142>{});       // row_bcast 15, 31
+    step(IC<0x143>{});
+    return readlane_f(v, 63);
+}
+
 template <int REPP>
 struct AttnState {
     float m[REPP];        // running maximum (log2 units), wave-uniform
+    float ms[REPP];       // what weights are relative to: m, 0 while there is none
+    float thr[REPP];      // a score above this raises m
     float l[REPP];        // per-lane partial sum of probabilities
     floatx4 acc[8];       // lane (g,n): acc[e][i] = out_head_n[dim 8*(4g+i)+e]
     float zp[REPP];       // 4-bit values only: per-lane partial sum of p * zero-point of the token
@@ -60,14 +88,16 @@ __device__ __forceinline__ void softmax_pv_tile(AttnState<REPP>& st, float (&t)[
                                                 uint32_t pbuf, int lane) {
     bool raise = false;
 #pragma unroll
-    for (int j = 0; j < REPP; j++) raise |= t[j] > st.m[j] + kLazyThreshold;
+    for (int j = 0; j < REPP; j++) raise |= t[j] > st.thr[j];
     if (__any(raise)) {
         float alpha[REPP];
 #pragma unroll
         for (int j = 0; j < REPP; j++) {
-            const float mn = fmaxf(st.m[j], wave_max(t[j]));
+            const float mn = fmaxf(st.m[j], wave_max_dpp(t[j]));
             alpha[j] = (mn == -INFINITY) ? 1.0f : exp2_raw(st.m[j] - mn);
             st.m[j] = mn;
+            st.ms[j] = mn == -INFINITY ? 0.0f : mn;
+            st.thr[j] = mn + kLazyThreshold;
             st.l[j] *= alpha[j];
         }
         float a = alpha[0];
@@ -78,8 +108,7 @@ __device__ __forceinline__ void softmax_pv_tile(AttnState<REPP>& st, float (&t)[
     }
 #pragma unroll
     for (int j = 0; j < REPP; j++) {
-        const float ms = (st.m[j] == -INFINITY) ? 0.0f : st.m[j];
-        const float p = exp2_raw(t[j] - ms);
+        const float p = exp2_raw(t[j] - st.ms[j]);
         st.l[j] += p;
         *lds_ptr<__attribute__((address_space(3))) uint16_t>(pbuf + (j * kWave + lane) * 2) = f2lo<T>(p);
     }
@@ -87,18 +116,25 @@ __device__ __forceinline__ void softmax_pv_tile(AttnState<REPP>& st, float (&t)[
     const int g = lane >> 4, n = lane & 15;
     const uint32_t prow = pbuf + ((n < REPP ? n : 0) * kWave + 4 * g) * 2;      // columns past the last head: any row, never stored
 #pragma unroll
-    for (int tb = 0; tb < 4; tb++) {
-        const __attribute__((address_space(3))) uint2* pp = lds_ptr<__attribute__((address_space(3))) uint2>(prow + tb * 32);
-        uint2 pb;
-        pb.x = pp->x; pb.y = pp->y;
+    for (int u = 0; u < 2; u++) {
+        uint2 pb[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const __attribute__((address_space(3))) uint2* pp = lds_ptr<__attribute__((address_space(3))) uint2>(prow + (2 * u + h) * 32);
+            pb[h].x = pp->x; pb[h].y = pp->y;
+        }
 #pragma unroll
         for (int e = 0; e < 8; e++) {
             const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
             auto word = [&](const uint4& v) { return (e >> 1) == 0 ? v.x : (e >> 1) == 1 ? v.y : (e >> 1) == 2 ? v.z : v.w; };
-            uint2 va;
-            va.x = __builtin_amdgcn_perm(word(vv[tb][1]), word(vv[tb][0]), sel);
-            va.y = __builtin_amdgcn_perm(word(vv[tb][3]), word(vv[tb][2]), sel);
-            st.acc[e] = mfma16<T>(va, pb, st.acc[e]);
+            uint2 va[2];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const uint4 (&v)[4] = vv[2 * u + h];
+                va[h].x = __builtin_amdgcn_perm(word(v[1]), word(v[0]), sel);
+                va[h].y = __builtin_amdgcn_perm(word(v[3]), word(v[2]), sel);
+            }
+            st.acc[e] = mfma16x2<T>(va[0], va[1], pb[0], pb[1], st.acc[e]);
         }
     }
     asm volatile("" ::: "memory");
@@ -114,7 +150,7 @@ __device__ __forceinline__ void softmax_pv_tile(AttnState<REPP>& st, float (&t)[
 // and only the first term needs the matrix cores.  Lane (g,n) owns exactly word n of its tokens,
 // so the MFMA row for dim 8n+e is nibble e of that word.  A nibble isolated in a byte and
 // zero-extended to 16 bits IS the half-precision subnormal code * 2^-24 (odd nibbles are left in
-// the high half of their byte: 16 * code * 2^-24), which v_mfma_f32_16x16x16_f16 multiplies
+// the high half of their byte: 16 * code * 2^-24), which v_mfma_f32_16x16x32_f16 multiplies
 // exactly; so the A operand costs two v_and per word and one v_perm per register, like the
 // half-precision rows it replaces, and the accumulators are brought back to real units once,
 // after the last quantized tile (finish_v4).  The probabilities go through half precision for
@@ -140,14 +176,16 @@ __device__ __forceinline__ void softmax_pv_tile_v4(AttnState<REPP>& st, float (&
                                                    float sc, float zp, uint32_t pbuf, int lane) {
     bool raise = false;
 #pragma unroll
-    for (int j = 0; j < REPP; j++) raise |= t[j] > st.m[j] + kLazyThresholdV4;
+    for (int j = 0; j < REPP; j++) raise |= t[j] > st.thr[j];
     if (__any(raise)) {
         float alpha[REPP];
 #pragma unroll
         for (int j = 0; j < REPP; j++) {
-            const float mn = fmaxf(st.m[j], wave_max(t[j]));
+            const float mn = fmaxf(st.m[j], wave_max_dpp(t[j]));
             alpha[j] = (mn == -INFINITY) ? 1.0f : exp2_raw(st.m[j] - mn);
             st.m[j] = mn;
+            st.ms[j] = mn == -INFINITY ? 0.0f : mn;
+            st.thr[j] = mn + kLazyThresholdV4;
             st.l[j] *= alpha[j];
             st.zp[j] *= alpha[j];
         }
@@ -169,8 +207,7 @@ __device__ __forceinline__ void softmax_pv_tile_v4(AttnState<REPP>& st, float (&
     const float zq = zp * __builtin_amdgcn_rcpf(scp);
 #pragma unroll
     for (int j = 0; j < REPP; j++) {
-        const float ms = (st.m[j] == -INFINITY) ? 0.0f : st.m[j];
-        const float p = exp2_raw(t[j] - ms);
+        const float p = exp2_raw(t[j] - st.ms[j]);
         st.l[j] += p;
         const uint16_t wh = f2lo<F16>(p * scp);
         st.zp[j] = __builtin_fmaf(lo2f<F16>(wh), zq, st.zp[j]);
@@ -179,26 +216,37 @@ __device__ __forceinline__ void softmax_pv_tile_v4(AttnState<REPP>& st, float (&
     asm volatile("" ::: "memory");
     const int g = lane >> 4, n = lane & 15;
     const uint32_t prow = pbuf + ((n < REPP ? n : 0) * kWave + 4 * g) * 2;      // columns past the last head: any row, never stored
+    uint2 pb[4];
 #pragma unroll
     for (int tb = 0; tb < 4; tb++) {
         const __attribute__((address_space(3))) uint2* pp = lds_ptr<__attribute__((address_space(3))) uint2>(prow + tb * 32);
-        uint2 pb;
-        pb.x = pp->x; pb.y = pp->y;
-        uint32_t ev[4], od[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) { ev[i] = vq[tb][i] & 0x0f0f0f0fu; od[i] = vq[tb][i] & 0xf0f0f0f0u; }
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-            // byte e/2 of the even / odd words of two tokens -> two zero-extended 16-bit fields
-            const uint32_t by = static_cast<uint32_t>(e >> 1);
-            const uint32_t sel = 0x0c000c00u | ((4u + by) << 16) | by;
-            const uint32_t (&src)[4] = (e & 1) ? od : ev;
-            uint2 va;
-            va.x = __builtin_amdgcn_perm(src[1], src[0], sel);
-            va.y = __builtin_amdgcn_perm(src[3], src[2], sel);
-            st.acc[e] = mfma16<F16>(va, pb, st.acc[e]);
-        }
+        pb[tb].x = pp->x; pb[tb].y = pp->y;
     }
+    // Product 8 u + e: tokens [32 u, 32 u + 32).  It may take its operand two instructions after the permutes at the earliest: those of
+    // the next one are made between, where the compiler would put a wait.
+    uint2 va[2][2];
+    uint32_t ev[2][4], od[2][4];
+    auto operand = [&](auto I) {
+        constexpr int u = decltype(I)::value >> 3, e = decltype(I)::value & 7;
+        static_for<2>([&](auto H) {
+            if constexpr (e == 0) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) { ev[H][i] = vq[2 * u + H][i] & 0x0f0f0f0fu; od[H][i] = vq[2 * u + H][i] & 0xf0f0f0f0u; }
+            }
+            // byte e/2 of the even / odd words of two tokens -> two zero-extended 16-bit fields
+            constexpr uint32_t by = e >> 1, sel = 0x0c000c00u | ((4u + by) << 16) | by;
+            const uint32_t (&src)[4] = (e & 1) ? od[H] : ev[H];
+            va[e & 1][H].x = __builtin_amdgcn_perm(src[1], src[0], sel);
+            va[e & 1][H].y = __builtin_amdgcn_perm(src[3], src[2], sel);
+        });
+    };
+    operand(IC<0>{});
+    static_for<16>([&](auto I) {
+        constexpr int i = decltype(I)::value, e = i & 7, u = i >> 3;
+        if constexpr (i < 15) operand(IC<i + 1>{});
+        __builtin_amdgcn_sched_barrier(0);
+        st.acc[e] = mfma16x2<F16>(va[e & 1][0], va[e & 1][1], pb[2 * u], pb[2 * u + 1], st.acc[e]);
+    });
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
 }
@@ -209,17 +257,19 @@ template <int REPP>
 __device__ __forceinline__ void softmax_sums_only(AttnState<REPP>& st, float (&t)[REPP], float lazy) {
     bool raise = false;
 #pragma unroll
-    for (int j = 0; j < REPP; j++) raise |= t[j] > st.m[j] + lazy;
+    for (int j = 0; j < REPP; j++) raise |= t[j] > st.thr[j];
     if (__any(raise)) {
 #pragma unroll
         for (int j = 0; j < REPP; j++) {
-            const float mn = fmaxf(st.m[j], wave_max(t[j]));
+            const float mn = fmaxf(st.m[j], wave_max_dpp(t[j]));
             st.l[j] *= (mn == -INFINITY) ? 1.0f : exp2_raw(st.m[j] - mn);
             st.m[j] = mn;
+            st.ms[j] = mn == -INFINITY ? 0.0f : mn;
+            st.thr[j] = mn + lazy;
         }
     }
 #pragma unroll
-    for (int j = 0; j < REPP; j++) st.l[j] += exp2_raw(t[j] - ((st.m[j] == -INFINITY) ? 0.0f : st.m[j]));
+    for (int j = 0; j < REPP; j++) st.l[j] += exp2_raw(t[j] - st.ms[j]);
 }
 
 // After the last 4-bit tile: accumulators back to real units, plus the zero-point term (the same

@@ -64,7 +64,7 @@ __device__ __forceinline__ PairMem pair_mem(uint32_t lut, uint32_t sbuf, uint32_
 // A hand-over gave up: tell the host, if it passed a status word.  One lane, an ordinary vector store of a constant
 // (every wavefront that fails writes the same value, so no atomic is needed).  The pointer waits in LDS (stash_status,
 // before the workgroup's barrier) instead of in two scalar registers for the whole kernel: the scorer's group loop may hold
-// 64 wave-uniform radius offsets in scalar registers (one or two heads) and then has none to spare.
+// 64 wave-uniform radius offsets in scalar registers (one head) and then has none to spare.
 typedef __attribute__((address_space(3))) unsigned long long lds_u64;
 __device__ __forceinline__ void stash_status(unsigned long long* slot, int* status) {
     if (threadIdx.x == 0) *slot = reinterpret_cast<unsigned long long>(status);
@@ -275,7 +275,7 @@ __device__ __forceinline__ bool pair_accumulator(const AttnParams& p, const Pair
                                                 has_mask ? static_cast<uint32_t>(sc.n_tokens < p.mask_stride ? sc.n_tokens : p.mask_stride) : 0u);
     AttnState<REPP> st;
 #pragma unroll
-    for (int j = 0; j < REPP; j++) { st.m[j] = -INFINITY; st.l[j] = 0.0f; st.zp[j] = 0.0f; }
+    for (int j = 0; j < REPP; j++) { st.m[j] = st.thr[j] = -INFINITY; st.ms[j] = st.l[j] = st.zp[j] = 0.0f; }
 #pragma unroll
     for (int e = 0; e < 8; e++) st.acc[e] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
     int spin = pm.spin_limit;            // 0 once a wait has given up (see pair_scorer)

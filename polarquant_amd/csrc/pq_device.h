@@ -110,9 +110,9 @@ struct Lut {
     static constexpr int PB = NB * EB;            // bytes per pair
     static constexpr int HB = kPairs * PB;        // bytes per half
     static constexpr int BYTES = HALVES * HB;
-    // attention's c_d (score_token): in LDS from three heads on, c_d of pair d in the word of no head if its entries have one (three or
+    // attention's c_d (score_token): in LDS from two heads on, c_d of pair d in the word of no head if its entries have one (three or
     // seven heads), else the d-th float behind the table
-    static constexpr bool C_IN_LDS = REPP > 2, SPARE = WORDS > REPP;
+    static constexpr bool C_IN_LDS = REPP > 1, SPARE = WORDS > REPP;
     static constexpr int C0 = BYTES, ALL_BYTES = BYTES + (C_IN_LDS && !SPARE ? kPairs * 4 : 0);
     // theta * EB fits a byte: the four byte offsets of a code word are made by two instructions on the
     // whole word; beyond that (TB 5, 6 with 16-byte entries) each code's offset is shifted into place
@@ -287,9 +287,9 @@ __device__ __forceinline__ float build_lut(uint32_t lut, int lane, const float (
 
 // Score one token against the table.  `codes` holds the token's 64 pair codes as
 // 16 little-endian words.  acc[j] += ...  `cds` says where the c_d are: InLds, as build_lut leaves them (with the entry, or four to a read
-// that all lanes share), or 64 scalar registers.  Attention with three heads and more has them in LDS: its scalar registers hold much
+// that all lanes share), or 64 scalar registers.  Attention with two heads and more has them in LDS: its scalar registers hold much
 // else, of which the 64 spilled half, and the 64 readlanes of a group are as many instructions as a tenth of a tile's walk.  For one
-// or two heads the reads cost more than they save (4-bit values, one head, 8 x 4096: 44.2 us, in LDS 44.8).  The score kernel's wavefront walks one group,
+// head the reads cost more than they save (4-bit values, 8 x 4096: 44.2 us, in LDS 44.8).  The score kernel's wavefront walks one group,
 // and 256 bytes more would leave a unit nine tables of four heads instead of ten (8 sequences of 16384, 4 heads 30.6 us, in LDS 34.3).
 struct InLds {};
 // The 64 table reads are issued in batches of 4 or 8 codes, one batch ahead of the
