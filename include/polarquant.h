@@ -143,6 +143,26 @@ int pq_validate_qkv_rope_append(const void *x, int64_t x_row_stride, const void 
                                 const int64_t *pos, const void *q_out, const void *k_dst, int64_t k_rows,
                                 const int64_t *k_row, const void *v_dst, int64_t v_rows, const int64_t *v_row, int N, int Nk);
 
+/* A norm shared by the products around it (bfloat16, M <= 8): norm(x) . w^T = r (x norm_w) . w^T with one number
+ * r = rsqrt(mean(x^2) + eps) a row.  Replaces nn.Linear, the residual addition, the RMS norm and nn.Linear of a decode step
+ * (the decoder layer, models/modeling_llama_polar.py:456-486).
+ *   pq_linear_residual         stream_x [M, N] += x . w^T (+ bias), rounded as the modules do; xw [M, N] = stream_x * norm_w,
+ *                              rounded once; part [M, N / 16] = sums of stream_x^2 over 16 columns.  K a multiple of 256 below 8192, of 512 from there.
+ *   pq_gated_normed            pq_linear_small_m with w_up, of the norm that xw and part [M, K / 16] stand for (xw dense)
+ *   pq_qkv_rope_append_normed  pq_qkv_rope_append likewise.  Both: K a multiple of 256 up to 4096, or 8192; part 16-byte aligned. */
+int pq_linear_residual(const void *x, int64_t x_row_stride, const void *w, const void *bias, int M, int N, int K, int dtype,
+                       void *stream_x, const void *norm_w, void *xw, float *part, void *stream);
+int pq_validate_linear_residual(const void *x, int64_t x_row_stride, const void *w, const void *bias, int M, int N, int K, int dtype,
+                                const void *stream_x, const void *norm_w, const void *xw, const float *part);
+int pq_gated_normed(const void *xw, const float *part, float eps, const void *w, const void *w_up, void *y, int M, int N, int K,
+                    int dtype, void *stream);
+int pq_validate_gated_normed(const void *xw, const float *part, const void *w, const void *w_up, const void *y, int M, int N,
+                             int K, int dtype);
+int pq_qkv_rope_append_normed(const void *xw, const float *part, float eps, const void *w_qkv, const void *bias, int M, int K, int dtype,
+                              const void *cos_table, const void *sin_table, int64_t table_rows, const int64_t *pos, void *q_out,
+                              void *k_dst, int64_t k_rows, const int64_t *k_row, void *v_dst, int64_t v_rows,
+                              const int64_t *v_row, int N, int Nk, void *stream);
+
 /* Layout converter for code rows: pack != 0 turns `n_rows` byte-per-code rows (64 bytes each, every
  * code < 64) into packed 6-bit rows (48 bytes each), pack == 0 the reverse.  For caches built by the
  * reference (always byte-per-code) that are to be kept packed, and back.  No reference counterpart. */

@@ -168,7 +168,7 @@ struct Call<R(A...), STRIDES> {
     X(pq_latent_prefill_takes) X(pq_latent_prefill) X(pq_qk_norm) X(pq_ring_append) X(pq_window_plan) X(pq_window_workspace_bytes)         \
     X(pq_window_attn) X(pq_delta_prep) X(pq_scan_workspace_bytes) X(pq_delta_scan) X(pq_memory_gates) X(pq_memory_scan)                    \
     X(pq_head_norm_gate) X(pq_validate_delta_token) X(pq_delta_token) X(pq_validate_memory_token) X(pq_memory_token)        \
-    X(pq_validate_linear_gelu) X(pq_linear_gelu)
+    X(pq_validate_linear_gelu) X(pq_linear_gelu) X(pq_linear_residual) X(pq_gated_normed) X(pq_qkv_rope_append_normed)
 
 // A prototype as ctypes writes types: the result's letter, then the parameters'.
 template <typename T>

@@ -3,6 +3,7 @@
 // they replace are in include/polarquant.h.
 #include "../../include/polarquant.h"
 #include "pq_internal.h"
+#include "pq_linear_rules.h"
 
 namespace {
 
@@ -519,7 +520,56 @@ int pq_qkv_rope_append(const void* x, int64_t x_row_stride, const void* w_qkv, c
     if (rc != PQ_OK) return rc;
     const int err = pq::launch_qkv_rope_append(x, x_row_stride, w_qkv, bias, M, K, dtype, cos_table, sin_table, table_rows,
                                                pos, q_out, k_dst, k_rows, k_row, v_dst, v_rows, v_row, N, Nk,
-                                               static_cast<hipStream_t>(stream));
+                                               nullptr, 0.0f, static_cast<hipStream_t>(stream));
+    return err == 0 ? PQ_OK : PQ_ERR_LAUNCH;
+}
+
+// ---- a norm shared by the products around it ---------------------------------------------------
+int pq_validate_linear_residual(const void* x, int64_t x_row_stride, const void* w, const void* bias, int M, int N, int K, int dtype,
+                                const void* stream_x, const void* norm_w, const void* xw, const float* part) {
+    if (!stream_x || !norm_w || !xw || !part) return PQ_ERR_NULL_POINTER;
+    if (int rc = pq_validate_linear_small_m(x, x_row_stride, w, nullptr, bias, xw, N, M, N, K, dtype)) return rc;
+    if (dtype != PQ_BF16) return PQ_ERR_BAD_DTYPE;
+    if (M > 8 || !pq::normed_depth(K, false)) return PQ_ERR_BAD_SHAPE;
+    if (!aligned(stream_x, 8) || !aligned(norm_w, 8) || !aligned(part, 4)) return PQ_ERR_MISALIGNED;
+    return PQ_OK;
+}
+
+int pq_linear_residual(const void* x, int64_t x_row_stride, const void* w, const void* bias, int M, int N, int K, int dtype,
+                       void* stream_x, const void* norm_w, void* xw, float* part, void* stream) {
+    if (int rc = pq_validate_linear_residual(x, x_row_stride, w, bias, M, N, K, dtype, stream_x, norm_w, xw, part)) return rc;
+    const int err = pq::launch_linear_residual(x, x_row_stride, w, bias, M, N, K, stream_x, norm_w, xw, part, static_cast<hipStream_t>(stream));
+    return err == 0 ? PQ_OK : PQ_ERR_LAUNCH;
+}
+
+int pq_validate_gated_normed(const void* xw, const float* part, const void* w, const void* w_up, const void* y, int M, int N, int K, int dtype) {
+    if (!part || !w_up) return PQ_ERR_NULL_POINTER;
+    if (int rc = pq_validate_linear_small_m(xw, K, w, w_up, nullptr, y, N, M, N, K, dtype)) return rc;
+    if (dtype != PQ_BF16) return PQ_ERR_BAD_DTYPE;
+    if (M > 8 || !pq::normed_depth(K, true)) return PQ_ERR_BAD_SHAPE;
+    return aligned(part, 16) ? PQ_OK : PQ_ERR_MISALIGNED;
+}
+
+int pq_gated_normed(const void* xw, const float* part, float eps, const void* w, const void* w_up, void* y, int M, int N, int K, int dtype,
+                    void* stream) {
+    if (int rc = pq_validate_gated_normed(xw, part, w, w_up, y, M, N, K, dtype)) return rc;
+    const int err = pq::launch_gated_normed(xw, part, eps, w, w_up, y, M, N, K, static_cast<hipStream_t>(stream));
+    return err == 0 ? PQ_OK : PQ_ERR_LAUNCH;
+}
+
+int pq_qkv_rope_append_normed(const void* xw, const float* part, float eps, const void* w_qkv, const void* bias, int M, int K, int dtype,
+                              const void* cos_table, const void* sin_table, int64_t table_rows, const int64_t* pos, void* q_out,
+                              void* k_dst, int64_t k_rows, const int64_t* k_row, void* v_dst, int64_t v_rows, const int64_t* v_row,
+                              int N, int Nk, void* stream) {
+    if (!part) return PQ_ERR_NULL_POINTER;
+    if (int rc = pq_validate_qkv_rope_append(xw, K, w_qkv, bias, M, K, dtype, cos_table, sin_table, table_rows, pos, q_out, k_dst, k_rows, k_row,
+                                             v_dst, v_rows, v_row, N, Nk))
+        return rc;
+    if (dtype != PQ_BF16) return PQ_ERR_BAD_DTYPE;
+    if (!pq::normed_depth(K, true)) return PQ_ERR_BAD_SHAPE;
+    if (!aligned(part, 16)) return PQ_ERR_MISALIGNED;
+    const int err = pq::launch_qkv_rope_append(xw, K, w_qkv, bias, M, K, dtype, cos_table, sin_table, table_rows, pos, q_out, k_dst, k_rows, k_row,
+                                               v_dst, v_rows, v_row, N, Nk, part, eps, static_cast<hipStream_t>(stream));
     return err == 0 ? PQ_OK : PQ_ERR_LAUNCH;
 }
 

@@ -46,7 +46,10 @@ int launch_small_m_linear(const void* x, int64_t x_stride, const void* w, const 
 int launch_qkv_rope_append(const void* x, int64_t x_stride, const void* w, const void* bias, int M, int K, int dtype,
                            const void* cos_tab, const void* sin_tab, int64_t max_pos, const int64_t* pos, void* q_out,
                            void* k_dst, int64_t k_rows, const int64_t* k_row, void* v_dst, int64_t v_rows,
-                           const int64_t* v_row, int N, int Nk, hipStream_t st);
+                           const int64_t* v_row, int N, int Nk, const float* norm_part, float eps, hipStream_t st);
+int launch_linear_residual(const void* x, int64_t x_stride, const void* w, const void* bias, int M, int N, int K, void* stream_x, const void* norm_w,
+                           void* xw, float* part, hipStream_t st);
+int launch_gated_normed(const void* xw, const float* part, float eps, const void* w, const void* w_up, void* y, int M, int N, int K, hipStream_t st);
 
 struct AttnArgs {
     const void* q;

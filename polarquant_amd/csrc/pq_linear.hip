@@ -25,11 +25,13 @@ struct RopeAppendArgs {
     int N, Nk;
 };
 
-template <typename T, int KSPLIT, int kStage>
+// NORMED: x is one half of a norm (NormedRows, pq_linear_device.h).
+template <typename T, int KSPLIT, int kStage, bool NORMED = false>
 __global__ __launch_bounds__(kWave * KSPLIT) void qkv_rope_append_kernel(
     const uint16_t* __restrict__ x, int64_t x_stride, const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias,
-    int M, int K, RopeAppendArgs ra) {
+    int M, int K, RopeAppendArgs ra, NormedRows normed) {
     __shared__ float part[KSPLIT][2][4][kWave];
+    __shared__ float row_scale[NORMED ? 8 : 1];
     const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
     const int r = lane & 15, g = lane >> 4;
     const int row = r & 7, chunk = (r >> 3) * 4 + g;
@@ -42,6 +44,7 @@ __global__ __launch_bounds__(kWave * KSPLIT) void qkv_rope_append_kernel(
     const uint16_t* xp = x + static_cast<size_t>(m) * x_stride + koff;
     const size_t half_tile = static_cast<size_t>(kPairs) * K;           // rows n0 + 64 .. n0 + 71
 
+    RowScale<KSPLIT> scale;
     floatx4_l acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
     auto ldw = [](const uint16_t* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4_l*>(p)); };
     auto load = [&](Stage8T<false, 2, kStage>& st, int s0) {
@@ -63,7 +66,23 @@ __global__ __launch_bounds__(kWave * KSPLIT) void qkv_rope_append_kernel(
     if (full > 0) {
         Stage8T<false, 2, kStage> sa, sb;
         load(sa, 0);
+        if constexpr (NORMED) scale.load(normed, M);
         int st = 0;
+        if constexpr (NORMED) {
+            if (full > 2) {                        // (the loop's first trip, with the rows' factors in it)
+                load(sb, kStage);
+                __builtin_amdgcn_sched_barrier(0);
+                compute(sa);
+                load(sa, 2 * kStage);
+                __builtin_amdgcn_sched_barrier(0);
+                scale.store(normed, row_scale);
+                __builtin_amdgcn_sched_barrier(0);
+                compute(sb);
+                st = 2;
+            } else {
+                scale.store(normed, row_scale);
+            }
+        }
         while (st + 2 < full) {
             load(sb, (st + 1) * kStage);
             compute(sa);
@@ -106,6 +125,7 @@ __global__ __launch_bounds__(kWave * KSPLIT) void qkv_rope_append_kernel(
             s2 += part[k][1][i][lane] + part[k][1][i][lane + 40];
         }
         const int d = c8 + 4 * g + i;
+        if constexpr (NORMED) { s1 *= row_scale[r]; s2 *= row_scale[r]; }
         if (bias) { s1 += lo2f<T>(bias[n0 + 4 * g + i]); s2 += lo2f<T>(bias[n0 + kPairs + 4 * g + i]); }
         const float x1 = rnd_l<T>(s1), x2 = rnd_l<T>(s2);           // the projection's output in the dtype
         if (is_q || is_k) {
@@ -141,7 +161,7 @@ __global__ __launch_bounds__(kWave * KSPLIT) void qkv_rope_append_kernel(
 int launch_qkv_rope_append(const void* x, int64_t x_stride, const void* w, const void* bias, int M, int K, int dtype,
                            const void* cos_tab, const void* sin_tab, int64_t max_pos, const int64_t* pos, void* q_out,
                            void* k_dst, int64_t k_rows, const int64_t* k_row, void* v_dst, int64_t v_rows,
-                           const int64_t* v_row, int N, int Nk, hipStream_t st) {
+                           const int64_t* v_row, int N, int Nk, const float* norm_part, float eps, hipStream_t st) {
     RopeAppendArgs ra;
     ra.cos_tab = static_cast<const uint16_t*>(cos_tab); ra.sin_tab = static_cast<const uint16_t*>(sin_tab);
     ra.pos = pos; ra.q_out = static_cast<uint16_t*>(q_out); ra.k_dst = static_cast<uint16_t*>(k_dst); ra.k_row = k_row;
@@ -153,7 +173,7 @@ int launch_qkv_rope_append(const void* x, int64_t x_stride, const void* w, const
     dim3 grid((N + 2 * Nk) * 8), block(kWave * ks);
 #define PQ_LAUNCH_R(T, KS, S)                                                                                        \
     hipLaunchKernelGGL((qkv_rope_append_kernel<T, KS, S>), grid, block, 0, st, (const uint16_t*)x, x_stride,        \
-                       (const uint16_t*)w, (const uint16_t*)bias, M, K, ra)
+                       (const uint16_t*)w, (const uint16_t*)bias, M, K, ra, NormedRows{})
 #define PQ_LAUNCH_RK(T)                                                                                              \
     do {                                                                                                             \
         if (ks == 8) PQ_LAUNCH_R(T, 8, 2);                                                                           \
@@ -161,7 +181,11 @@ int launch_qkv_rope_append(const void* x, int64_t x_stride, const void* w, const
         else if (ks == 2) PQ_LAUNCH_R(T, 2, 1);                                                                      \
         else PQ_LAUNCH_R(T, 1, 1);                                                                                   \
     } while (0)
-    if (dtype == 0) PQ_LAUNCH_RK(F16);
+    if (norm_part) {                               // (shapes: normed_width; bfloat16)
+        const NormedRows nr{norm_part, K / 16, eps};
+        if (ks == 8) hipLaunchKernelGGL((qkv_rope_append_kernel<BF16, 8, 2, true>), grid, block, 0, st, (const uint16_t*)x, x_stride, (const uint16_t*)w, (const uint16_t*)bias, M, K, ra, nr);
+        else hipLaunchKernelGGL((qkv_rope_append_kernel<BF16, 4, 1, true>), grid, block, 0, st, (const uint16_t*)x, x_stride, (const uint16_t*)w, (const uint16_t*)bias, M, K, ra, nr);
+    } else if (dtype == 0) PQ_LAUNCH_RK(F16);
     else PQ_LAUNCH_RK(BF16);
 #undef PQ_LAUNCH_RK
 #undef PQ_LAUNCH_R
@@ -210,6 +234,36 @@ int launch_small_m_linear(const void* x, int64_t x_stride, const void* w, const 
 #undef PQ_LAUNCH_M16
 #undef PQ_LAUNCH_N
 #undef PQ_LAUNCH_L
+    return static_cast<int>(hipGetLastError());
+}
+
+// Products before and behind a norm that they share (bfloat16, M <= 8; split of K and row tiles as in launch_small_m_linear).
+int launch_linear_residual(const void* x, int64_t x_stride, const void* w, const void* bias, int M, int N, int K, void* stream_x, const void* norm_w,
+                           void* xw, float* part, hipStream_t st) {
+    HeadEpi he{};
+    he.res = ResidualOut{static_cast<uint16_t*>(stream_x), static_cast<const uint16_t*>(norm_w), static_cast<uint16_t*>(xw), part};
+    const int ks = K >= 8192 ? 8 : 4, nt = small_m8_row_tiles(M, N, ks, 1) > 2 ? 4 : 2;
+    const dim3 grid(N / (8 * nt)), block(kWave * ks);
+#define PQ_LAUNCH_A(KS, S, NT)                                                                                       \
+    hipLaunchKernelGGL((small_m8_linear_kernel<BF16, KS, false, S, 1 + kEpiResidual, NT>), grid, block, 0, st, (const uint16_t*)x, x_stride, \
+                       (const uint16_t*)w, (const uint16_t*)nullptr, (const uint16_t*)bias, (uint16_t*)nullptr, (int64_t)0, M, K, he)
+    if (ks == 8) { if (nt == 4) PQ_LAUNCH_A(8, 1, 4); else PQ_LAUNCH_A(8, 2, 2); }
+    else         { if (nt == 4) PQ_LAUNCH_A(4, 1, 4); else PQ_LAUNCH_A(4, 1, 2); }
+#undef PQ_LAUNCH_A
+    return static_cast<int>(hipGetLastError());
+}
+
+int launch_gated_normed(const void* xw, const float* part, float eps, const void* w, const void* w_up, void* y, int M, int N, int K, hipStream_t st) {
+    HeadEpi he{};
+    he.normed = NormedRows{part, K / 16, eps};
+    const int ks = K >= 8192 ? 8 : 4, nt = small_m8_row_tiles(M, N, ks, 2);
+    const dim3 grid(N / (8 * nt)), block(kWave * ks);
+#define PQ_LAUNCH_G(KS, S, NT)                                                                                       \
+    hipLaunchKernelGGL((small_m8_linear_kernel<BF16, KS, true, S, 0, NT, true>), grid, block, 0, st, (const uint16_t*)xw, (int64_t)K, \
+                       (const uint16_t*)w, (const uint16_t*)w_up, (const uint16_t*)nullptr, (uint16_t*)y, (int64_t)N, M, K, he)
+    if (ks == 8) { if (nt == 4) PQ_LAUNCH_G(8, 1, 4); else PQ_LAUNCH_G(8, 2, 2); }
+    else         { if (nt == 4) PQ_LAUNCH_G(4, 1, 4); else PQ_LAUNCH_G(4, 1, 2); }
+#undef PQ_LAUNCH_G
     return static_cast<int>(hipGetLastError());
 }
 

@@ -22,7 +22,8 @@
 // products per launch (blockIdx.y == head, operands `x_head` / N * K / `y_head` elements apart) with epilogue e of
 // pq_steps_internal.h: plain, square of relu, times sigmoid(gate), unrounded float32 output, that scaled and soft-capped, or plain rows and
 // behind them pairs of a gate's and another row whose results become gelu(gate) * other (small_m8_linear_kernel only; 8 rows, 18720 plain
-// rows and 14336 pairs of 4096: the step is 2.2 us a layer shorter, which was a launch of its own that moved 0.9 MB).
+// rows and 14336 pairs of 4096: the step is 2.2 us a layer shorter, which was a launch of its own that moved 0.9 MB), or added to a residual
+// stream with the first half of the norm behind it (ResidualOut; small_m8_linear_kernel only).
 #pragma once
 #include "pq_device.h"
 #include "pq_linear_rules.h"
@@ -55,6 +56,49 @@ template <> __device__ __forceinline__ uint16_t times_rounded<F16>(float a, uint
     return static_cast<uint16_t>(r);
 }
 
+// A norm cut in two between the products around it (pq_linear_residual, pq_linear_normed).  norm(x) W^T is r (x w) W^T with one number
+// r = rsqrt(mean x^2 + eps) a row: the product before stores x w, rounded once, and the sum of x^2 over every 16 columns; the product behind
+// multiplies its sums by r, which it makes of those.  Its own launch, which the norm had between them, was 4.5 us of a decode step, of which
+// nothing was work; 1.9 of them are saved (8 rows of 4096: the o projection 9.3 -> 10.0 us, gate and up 40.8 -> 42.4, down 24.3 -> 25.0,
+// q, k and v 15.1 -> 15.6).  Every workgroup reads the sums, like x itself.
+struct NormedRows {
+    const float* part;          // [M, n]: sums of squares of a row's 16 n elements
+    int n;
+    float eps;
+};
+struct ResidualOut {
+    uint16_t* x;                // [M, N]: the residual stream; the product is added to it
+    const uint16_t* norm_w;     // [N]
+    uint16_t* xw;               // [M, N]
+    float* part;                // [M, N / 16]
+};
+// The rows' r, by all threads of a workgroup, 8 KSPLIT to a row: requested behind the first weights and made while the next are on their way
+// (behind the last ones they hold registers through the loop, and the fewer workgroups a unit has then cost as much).
+constexpr int kNormedLoads = 2;
+template <int KSPLIT>
+struct RowScale {
+    static constexpr int kThreads = 8 * KSPLIT;
+    float4 v[kNormedLoads];
+    __device__ __forceinline__ void load(const NormedRows& nr, int M) {
+        const int row = threadIdx.x / kThreads, j = threadIdx.x % kThreads;
+        const float* p = nr.part + static_cast<size_t>(row < M ? row : 0) * nr.n;
+#pragma unroll
+        for (int i = 0; i < kNormedLoads; i++) {
+            const int at = (i * kThreads + j) * 4;
+            v[i] = *reinterpret_cast<const float4*>(p + (at < nr.n ? at : 0));
+        }
+    }
+    __device__ __forceinline__ void store(const NormedRows& nr, float* r) const {
+        const int j = threadIdx.x % kThreads;
+        float s = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kNormedLoads; i++) s += (i * kThreads + j) * 4 < nr.n ? (v[i].x + v[i].y) + (v[i].z + v[i].w) : 0.0f;
+#pragma unroll
+        for (int o = kThreads / 2; o > 0; o >>= 1) s += __shfl_xor(s, o);
+        if (j == 0) r[threadIdx.x / kThreads] = rsqrtf(s / static_cast<float>(16 * nr.n) + nr.eps);
+    }
+};
+
 struct HeadEpi {
     int64_t x_head, w_head, y_head;
     const uint16_t* gate;
@@ -65,6 +109,8 @@ struct HeadEpi {
     int pair_from, pair_rows;
     uint16_t* z;
     int64_t z_row;
+    NormedRows normed;           // of x (NORMED)
+    ResidualOut res;             // kEpiResidual
 };
 
 // of logits: a counter that nothing in this launch reads is raised by its first thread
@@ -232,8 +278,8 @@ struct Stage8T {
     u32x4_l w[NT][kStage], x[kStage], u[GATED ? NT : 1][GATED ? kStage : 1];
 };
 
-template <typename T, int KSPLIT, bool GATED, int kStage, int EPI = 0, int NT = 2>
-__global__ __launch_bounds__(kWave * KSPLIT) void small_m8_linear_kernel(
+template <typename T, int KSPLIT, bool GATED, int kStage, int EPI = 0, int NT = 2, bool NORMED = false>
+__global__ __launch_bounds__(kWave * KSPLIT) __attribute__((amdgpu_waves_per_eu(NORMED ? 3 : 1))) void small_m8_linear_kernel(
     const uint16_t* __restrict__ x, int64_t x_stride, const uint16_t* __restrict__ w, const uint16_t* __restrict__ w_up,
     const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, int64_t y_stride, int M, int K, HeadEpi he) {
     advance_once<EPI>(he);
@@ -242,10 +288,11 @@ __global__ __launch_bounds__(kWave * KSPLIT) void small_m8_linear_kernel(
         w += blockIdx.y * he.w_head;
     }
     __shared__ float part[KSPLIT][(GATED ? 2 : 1) * NT][4][kWave];
+    __shared__ float row_scale[NORMED ? 8 : 1];
     const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
     const int r = lane & 15, g = lane >> 4;
     const int row = r & 7, chunk = (r >> 3) * 4 + g;       // W row inside an 8-row tile == x row; 16-byte piece of the step
-    constexpr bool kGelu = EPI == 1 + kEpiGeluPairs;
+    constexpr bool kGelu = EPI == 1 + kEpiGeluPairs, kResidual = EPI == 1 + kEpiResidual;
     const bool pairs = kGelu && static_cast<int>(blockIdx.x) >= he.pair_from;
     // (a workgroup of pairs: the first half of its tiles are rows of the gate, the second those they meet)
     const int n0 = pairs ? (he.pair_from + static_cast<int>(blockIdx.x)) * 4 * NT : blockIdx.x * 8 * NT;
@@ -258,6 +305,16 @@ __global__ __launch_bounds__(kWave * KSPLIT) void small_m8_linear_kernel(
     const uint16_t* xp = x + static_cast<size_t>(m) * x_stride + koff;
     const size_t tile = static_cast<size_t>(8) * K;
 
+    // kResidual: the first wavefront stores, a lane the four columns 4 (g & 1) of tile (r / 8) + 2 (g / 2) of its row, and has requested
+    // what they are added to and multiplied by
+    const int width = static_cast<int>(gridDim.x) * 8 * NT, mine = (r >> 3) + 2 * (g >> 1), rn = n0 + 8 * (mine < NT ? mine : 0) + 4 * (g & 1);
+    uint2 x_old = {0, 0}, norm_w = {0, 0};
+    if constexpr (kResidual) {
+        x_old = *reinterpret_cast<const uint2*>(he.res.x + static_cast<size_t>(m) * width + rn);
+        norm_w = *reinterpret_cast<const uint2*>(he.res.norm_w + rn);
+    }
+
+    RowScale<KSPLIT> scale;
     floatx4_l acc[NT], acu[GATED ? NT : 1];
     static_for<NT>([&](auto I) {
         acc[I] = floatx4_l{0, 0, 0, 0};
@@ -285,7 +342,23 @@ __global__ __launch_bounds__(kWave * KSPLIT) void small_m8_linear_kernel(
     if (full > 0) {
         Stage8T<GATED, NT, kStage> sa, sb;
         load(sa, 0);
+        if constexpr (NORMED) scale.load(he.normed, M);
         int st = 0;
+        if constexpr (NORMED) {
+            if (full > 2) {                        // (the loop's first trip, with the rows' factors in it)
+                load(sb, kStage);
+                __builtin_amdgcn_sched_barrier(0);
+                compute(sa);
+                load(sa, 2 * kStage);
+                __builtin_amdgcn_sched_barrier(0);
+                scale.store(he.normed, row_scale);
+                __builtin_amdgcn_sched_barrier(0);
+                compute(sb);
+                st = 2;
+            } else {
+                scale.store(he.normed, row_scale);
+            }
+        }
         while (st + 2 < full) {
             load(sb, (st + 1) * kStage);
             compute(sa);
@@ -316,6 +389,33 @@ __global__ __launch_bounds__(kWave * KSPLIT) void small_m8_linear_kernel(
         }
     });
     __syncthreads();
+    if constexpr (kResidual) {
+        static_assert(NT <= 4, "a lane for every four columns");
+        if (wv != 0) return;
+        const int at = row + 16 * (g & 1), tile_ = mine < NT ? mine : 0;
+        uint16_t xs[4], us[4];
+        float ss = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float s = 0.0f;
+#pragma unroll
+            for (int k = 0; k < KSPLIT; k++) s += part[k][tile_][i][at] + part[k][tile_][i][at + 40];
+            const uint32_t xw = i < 2 ? x_old.x : x_old.y, ww = i < 2 ? norm_w.x : norm_w.y;
+            if (bias) s += lo2f<T>(bias[rn + i]);
+            xs[i] = f2lo<T>(lo2f<T>(static_cast<uint16_t>(i & 1 ? xw >> 16 : xw)) + rnd_l<T>(s));
+            const float xv = lo2f<T>(xs[i]);
+            us[i] = f2lo<T>(xv * lo2f<T>(static_cast<uint16_t>(i & 1 ? ww >> 16 : ww)));
+            ss = __builtin_fmaf(xv, xv, ss);
+        }
+        ss += __shfl_xor(ss, 16);                            // the row's other four columns of the tile, then the other tile of 16 columns
+        ss += __shfl_xor(ss, 8);
+        if (row >= M || mine >= NT) return;
+        const size_t o = static_cast<size_t>(row) * width + rn;
+        *reinterpret_cast<uint2*>(he.res.x + o) = make_uint2(xs[0] | (static_cast<uint32_t>(xs[1]) << 16), xs[2] | (static_cast<uint32_t>(xs[3]) << 16));
+        *reinterpret_cast<uint2*>(he.res.xw + o) = make_uint2(us[0] | (static_cast<uint32_t>(us[1]) << 16), us[2] | (static_cast<uint32_t>(us[3]) << 16));
+        if (r < 8 && (g & 1) == 0) he.res.part[static_cast<size_t>(row) * (width / 16) + rn / 16] = ss;
+        return;
+    }
     // lane (r < 8, g < 2) owns outputs y[r][n0 + 8h + 4g + i] (h: which 8-row tile), each the sum of the tile's
     // entry (row 4g + i, column r) and its diagonal partner (row + 8, column + 8), which lane + 40 holds
     if (r >= 8 || r >= M || g >= 2) return;
@@ -360,6 +460,7 @@ __global__ __launch_bounds__(kWave * KSPLIT) void small_m8_linear_kernel(
                 s += part[k][h][i][lane] + part[k][h][i][lane + 40];
                 if constexpr (GATED) t += part[k][NT + h][i][lane] + part[k][NT + h][i][lane + 40];
             }
+            if constexpr (NORMED) { s *= row_scale[r]; t *= row_scale[r]; }
             if constexpr (GATED) {
                 const float gv = rnd_l<T>(s), uv = rnd_l<T>(t);
                 const float a = rnd_l<T>(gv / (1.0f + __expf(-gv)));

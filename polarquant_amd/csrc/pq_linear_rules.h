@@ -29,4 +29,12 @@ inline int small_m8_row_tiles(int rows, int N, int ksplit, int matrices) {
     return best;
 }
 
+// Depths that the products around a norm take (launch_linear_residual: `behind` false; the products behind it: true).  K is split four ways,
+// from 8192 on eight, into whole steps of 64; and behind the norm a row's sums, one of 16 elements, have to be two 16-byte loads to a
+// thread at most (8 KSPLIT threads a row): up to 4096, and 8192.
+inline bool normed_depth(int K, bool behind) {
+    const int ks = K >= 8192 ? 8 : 4;
+    return K >= 256 && K % (64 * ks) == 0 && (!behind || K / 16 <= 2 * 4 * 8 * ks);
+}
+
 }  // namespace pq

@@ -60,7 +60,7 @@ int launch_softcap(float* x, size_t n, float scale, float cap, hipStream_t st);
 
 // y[m, h, n] = epilogue(sum_k x[m, h, k] w[h, n, k])
 // (kEpiLogits: float32, scaled and soft-capped; kEpiGeluPairs: LinearGeluArgs)
-enum { kEpiPlain = 0, kEpiReluSq = 1, kEpiSigmoidGate = 2, kEpiF32 = 3, kEpiLogits = 4, kEpiGeluPairs = 5 };
+enum { kEpiPlain = 0, kEpiReluSq = 1, kEpiSigmoidGate = 2, kEpiF32 = 3, kEpiLogits = 4, kEpiGeluPairs = 5, kEpiResidual = 6 };
 struct HeadLinearArgs {
     const void* x;
     int64_t x_row, x_head;

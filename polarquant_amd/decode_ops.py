@@ -157,6 +157,67 @@ def qkv_rope_append(x: torch.Tensor, w_qkv: torch.Tensor, b_qkv: Optional[torch.
     return q_out
 
 
+def normed_depth(K: int, behind: bool) -> bool:
+    """Depths that the products before (`linear_residual`) and behind (`gated_normed`, `qkv_rope_append_normed`) a shared norm take."""
+    return K >= 256 and K % (512 if K >= 8192 else 256) == 0 and (not behind or K <= 4096 or K == 8192)
+
+
+def linear_residual(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], stream: torch.Tensor, norm_weight: torch.Tensor):
+    """`stream += linear_small_m(x, weight, bias)` in place and the first half of the norm of it that follows: `stream * norm_weight` and the
+    sums of squares of every 16 columns, for `gated_normed` or `qkv_rope_append_normed`.  bfloat16, up to 8 rows, `normed_depth(K, False)`."""
+    _gpu(x)
+    N, K = weight.shape
+    x2 = x.reshape(-1, K)
+    M = x2.shape[0]
+    assert weight.is_contiguous() and weight.dtype == x.dtype and x2.stride(1) == 1
+    assert bias is None or (bias.is_contiguous() and bias.numel() == N and bias.dtype == x.dtype)
+    assert stream.is_contiguous() and stream.numel() == M * N and stream.dtype == x.dtype
+    assert norm_weight.is_contiguous() and norm_weight.numel() == N and norm_weight.dtype == x.dtype
+    xw = torch.empty_like(stream)
+    part = torch.empty((M, N // 16), dtype=torch.float32, device=x.device)
+    with _on_device(x.device):
+        rc = _ffi.lib().call.pq_linear_residual(x2, x2.stride(0) if M > 1 else K, weight, bias, M, N, K, _dtype_code(x), stream, norm_weight, xw, part,
+                                                _stream_ptr(x.device))
+    _ffi.check(rc, "pq_linear_residual")
+    return xw, part
+
+
+def gated_normed(half, eps: float, weight: torch.Tensor, up_weight: torch.Tensor) -> torch.Tensor:
+    """`linear_small_m(norm, weight, up_weight=up_weight)` of the norm whose first half `linear_residual` returned: the row's factor is applied
+    to the sums instead of to each element, one rounding less.  `normed_depth(K, True)`."""
+    xw, part = half
+    N, K = weight.shape
+    M = part.shape[0]
+    assert weight.is_contiguous() and up_weight.is_contiguous() and up_weight.shape == weight.shape and weight.dtype == up_weight.dtype == xw.dtype
+    assert xw.is_contiguous() and xw.numel() == M * K and part.is_contiguous() and part.shape[1] * 16 == K and part.dtype == torch.float32
+    y = torch.empty(xw.shape[:-1] + (N,), dtype=xw.dtype, device=xw.device)
+    with _on_device(xw.device):
+        rc = _ffi.lib().call.pq_gated_normed(xw, part, eps, weight, up_weight, y, M, N, K, _dtype_code(xw), _stream_ptr(xw.device))
+    _ffi.check(rc, "pq_gated_normed")
+    return y
+
+
+def qkv_rope_append_normed(half, eps: float, w_qkv: torch.Tensor, b_qkv: Optional[torch.Tensor], cos_table: torch.Tensor,
+                           sin_table: torch.Tensor, pos: torch.Tensor, k_dst: torch.Tensor, k_row: torch.Tensor,
+                           v_dst: torch.Tensor, v_row: torch.Tensor, n_heads: int, n_kv_heads: int) -> torch.Tensor:
+    """`qkv_rope_append` of the norm whose first half `linear_residual` returned, as `gated_normed`."""
+    xw, part = half
+    B, K = part.shape[0], w_qkv.shape[1]
+    assert w_qkv.is_contiguous() and w_qkv.shape == ((n_heads + 2 * n_kv_heads) * 128, K) and w_qkv.dtype == xw.dtype
+    assert xw.is_contiguous() and xw.numel() == B * K and part.is_contiguous() and part.shape[1] * 16 == K and part.dtype == torch.float32
+    assert b_qkv is None or (b_qkv.is_contiguous() and b_qkv.numel() == w_qkv.shape[0] and b_qkv.dtype == xw.dtype)
+    assert k_dst.is_contiguous() and v_dst.is_contiguous() and cos_table.is_contiguous() and sin_table.is_contiguous()
+    assert pos.dtype == k_row.dtype == v_row.dtype == torch.int64
+    assert k_dst.shape[:2] == (B, n_kv_heads) == v_dst.shape[:2] and k_dst.shape[3] == 128 == v_dst.shape[3]
+    q_out = torch.empty((B, n_heads, 1, 128), dtype=xw.dtype, device=xw.device)
+    with _on_device(xw.device):
+        rc = _ffi.lib().call.pq_qkv_rope_append_normed(xw, part, eps, w_qkv, b_qkv, B, K, _dtype_code(xw), cos_table, sin_table, cos_table.shape[0], pos,
+                                                       q_out, k_dst, k_dst.shape[2], k_row, v_dst, v_dst.shape[2], v_row, n_heads, n_kv_heads,
+                                                       _stream_ptr(xw.device))
+    _ffi.check(rc, "pq_qkv_rope_append_normed")
+    return q_out
+
+
 def rope_qk(q_lin: torch.Tensor, k_lin: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, n_heads: int, n_kv_heads: int):
     """`apply_rotary_pos_emb` on projection outputs in one launch, bit-identical to the eager ops: q_lin [B,L,N*128],
     k_lin [B,L,Nk*128] (unit element stride, uniform token stride), cos / sin [1 or B, L, 128] in the same dtype.

@@ -224,8 +224,11 @@ class PolarGraphDecoder(GraphDecoder):
     def _step_body_fused(self):
         """The decode step with one launch per elementwise stage: 2 norms (each with the residual add
         folded in), RoPE + append, SiLU * up, plus the GEMMs and the attention, per layer.  The first norm reads the embedding's
-        rows itself and the last one raises the counters."""
-        from .decode_ops import STEP_NORM_MAX, STEP_NORM_ROWS, embed_rmsnorm, linear_small_m, qkv_rope_append, rmsnorm, rope_append, silu_mul
+        rows itself and the last one raises the counters.  Up to 8 bfloat16 rows the norms between are shared by the products around
+        them (`linear_residual`): a step of 8 sequences of 4096 tokens, two layers of width 4096 with three such norms, 289.7 -> 284.6 us.  (In float16
+        the stream times a norm's weight could overflow.)"""
+        from .decode_ops import (STEP_NORM_MAX, STEP_NORM_ROWS, embed_rmsnorm, gated_normed, linear_residual, linear_small_m, normed_depth, qkv_rope_append,
+                                 qkv_rope_append_normed, rmsnorm, rope_append, silu_mul)
         model, B = self.model, self.B
         product = lambda module, t: module(t, library=True) if isinstance(module, Linear) and not self.small_m_gemm else module(t)
         layers = model.model.layers
@@ -236,15 +239,27 @@ class PolarGraphDecoder(GraphDecoder):
         else:
             x = embed(self.ids).contiguous()
             h = rmsnorm(x, first.weight, first.variance_epsilon)
-        # x: residual stream [B,1,H], updated in place
-        for li, (layer, ar) in enumerate(zip(layers, self.arenas)):
+        # x: residual stream [B,1,H], updated in place; h: its norm, or with `eps` the half of it that `linear_residual` returned
+        eps = None
+        fits = lambda p_, w_: p_.dtype == w_.dtype == torch.bfloat16 and p_.is_contiguous() and normed_depth(w_.shape[1], False) and normed_depth(p_.numel(), True)
+
+        def fusable(layer):
             att, mlp = layer.self_attn, layer.mlp
-            nq, nkv = att.num_heads * att.head_dim, att.num_key_value_heads * att.head_dim
             own = self.small_m_gemm and B <= 16 and all(
                 w_.is_contiguous() and w_.shape[0] % 16 == 0 and w_.shape[1] % 32 == 0
                 for w_ in (att._wqkv, att.o_proj.weight, mlp.gate_proj.weight, mlp.up_proj.weight, mlp.down_proj.weight))
+            return own, own and self.fused_qkv_rope and B <= 8 and att._wqkv.shape[1] % 64 == 0, own and mlp.gate_proj.bias is None and mlp.up_proj.bias is None
+
+        for li, (layer, ar) in enumerate(zip(layers, self.arenas)):
+            att, mlp = layer.self_attn, layer.mlp
+            nq, nkv = att.num_heads * att.head_dim, att.num_key_value_heads * att.head_dim
+            own, qkv_fused, gated = fusable(layer)
             v_dst, v_row = (ar.vres, self.resid_idx) if self.mixed else (ar.v, self.pos)
-            if own and self.fused_qkv_rope and B <= 8 and att._wqkv.shape[1] % 64 == 0:
+            if eps is not None:
+                q = qkv_rope_append_normed(h, eps, att._wqkv, att._bqkv, self.cos_table, self.sin_table, self.pos, ar.kres,
+                                           self.resid_idx, v_dst, v_row, att.num_heads, att.num_key_value_heads)
+                eps = None
+            elif qkv_fused:
                 # projection, rotation and both appends in one launch (bit-identical to the two below)
                 q = qkv_rope_append(h, att._wqkv, att._bqkv, self.cos_table, self.sin_table, self.pos, ar.kres,
                                     self.resid_idx, v_dst, v_row, att.num_heads, att.num_key_value_heads)
@@ -258,18 +273,27 @@ class PolarGraphDecoder(GraphDecoder):
                                 v_dst, v_row, att.num_heads, att.num_key_value_heads)
             o = self._attend(att, ar, q)
             pn = layer.post_attention_layernorm
-            if own and mlp.gate_proj.bias is None and mlp.up_proj.bias is None:
-                a = linear_small_m(o.reshape(B, 1, -1), att.o_proj.weight, att.o_proj.bias)
-                h = rmsnorm(x, pn.weight, pn.variance_epsilon, residual=a, sum_out=x)
-                act = linear_small_m(h, mlp.gate_proj.weight, up_weight=mlp.up_proj.weight)
+            last = li + 1 == len(layers)
+            nn_ = model.model.norm if last else layers[li + 1].input_layernorm
+            if gated:
+                t = o.reshape(B, 1, -1)
+                if B <= 8 and fits(pn.weight, att.o_proj.weight):
+                    half = linear_residual(t, att.o_proj.weight, att.o_proj.bias, x, pn.weight)
+                    act = gated_normed(half, pn.variance_epsilon, mlp.gate_proj.weight, mlp.up_proj.weight)
+                else:
+                    a = linear_small_m(t, att.o_proj.weight, att.o_proj.bias)
+                    h = rmsnorm(x, pn.weight, pn.variance_epsilon, residual=a, sum_out=x)
+                    act = linear_small_m(h, mlp.gate_proj.weight, up_weight=mlp.up_proj.weight)
+                if not last and fits(nn_.weight, mlp.down_proj.weight) and fusable(layers[li + 1])[1]:
+                    eps = nn_.variance_epsilon
+                    h = linear_residual(act, mlp.down_proj.weight, mlp.down_proj.bias, x, nn_.weight)
+                    continue
                 m = linear_small_m(act, mlp.down_proj.weight, mlp.down_proj.bias)
             else:
                 a = product(att.o_proj, o.reshape(B, 1, -1))
                 h = rmsnorm(x, pn.weight, pn.variance_epsilon, residual=a, sum_out=x)
                 # (gate | up as one library GEMM was measured too: no faster than the two, so they stay separate)
                 m = product(mlp.down_proj, silu_mul(product(mlp.gate_proj, h), product(mlp.up_proj, h)))
-            last = li + 1 == len(layers)
-            nn_ = model.model.norm if last else layers[li + 1].input_layernorm
             more = dict(counters=self._counters, increments=self._advance) if last and edges else {}
             h = rmsnorm(x, nn_.weight, nn_.variance_epsilon, residual=m, sum_out=x, **more)
         logits = product(model.lm_head, h)
