@@ -238,7 +238,7 @@ class GatedDelta(Branch):
     def forward(self, p, out, state, step):
         q, k, v, b = [x[:, :w.shape[0]] for x, w in zip(p, (self.q, self.k, self.v, self.b))]
         wa, wg = self._a2.weight(), self._g2.weight()
-        if ops.delta_token_takes(q, k, p[4], p[5], wa, wg, state.S, self.taps, out, step):
+        if ops.delta_token_takes(q, k, p[4], p[5], wa, wg, state.S, self.taps, out, step, self.norm, state.conv):
             ops.delta_token(q, k, v, b, p[4], p[5], wa, wg, self.q_conv, self.k_conv, self.v_conv, self.A_log, self.dt_bias, self.norm, state.conv, state.S,
                             self.eps, out, self.out_scale, step)
             return

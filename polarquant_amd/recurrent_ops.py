@@ -221,9 +221,12 @@ def _one_launch(step: Step, dtype: torch.dtype, *aligned) -> bool:
 
 
 # (The one launch is the faster one at any number of sequences, 1 to 64 timed: pq_recurrent_token.hip.)
-def delta_token_takes(q, k, xa, xg, wa, wg, state: torch.Tensor, taps: int, out: torch.Tensor, step: Step) -> bool:
+def delta_token_takes(q, k, xa, xg, wa, wg, state: torch.Tensor, taps: int, out: torch.Tensor, step: Step, norm: Optional[torch.Tensor] = None,
+                      conv: Optional[ConvState] = None) -> bool:
+    """norm, conv: the norm's weight and the convolutions' state where they are not known to be of one head and at 8 bytes."""
     B, H, vdim, dim = state.shape
     return (_one_launch(step, q.dtype, xa, xg, wa, wg, state, out) and q.shape[1] == k.shape[1] == H * dim
+            and (norm is None or (norm.numel() == vdim and norm.data_ptr() % 8 == 0)) and (conv is None or conv.rows.data_ptr() % 8 == 0)
             and _ffi.recurrent_lib().call.pq_validate_delta_token(B, H, dim, vdim, taps, wa.shape[1], wg.shape[1], q.stride(0), out.stride(0),
                                                                   _DTYPES[q.dtype]) == 0)
 

@@ -7,6 +7,7 @@ import torch
 
 from polarquant_amd import layer_ops
 from polarquant_amd import recurrent_ops as ops
+from polarquant_amd.modeling_recurrent import GatedDelta
 from polarquant_amd.recurrent_ops import Step
 
 pytestmark = pytest.mark.gpu
@@ -100,3 +101,41 @@ def test_products_with_gelu(M, plain, ff, K, dtype):
     assert torch.equal(y, p[:, :plain]) and torch.equal(z[:, 4:4 + ff], want)
     assert bool((z[:, :4] == 7).all()) and bool((z[:, 4 + ff:] == 7).all())
     assert not layer_ops.linear_gelu_takes(x, w, plain, ff + 16, z[:, 4:]) and not layer_ops.linear_gelu_takes(x[:, 1:], w, plain, ff, z[:, 4:])
+
+
+@pytest.mark.parametrize("which", ["norm", "norm per head", "convolution"])
+def test_delta_operands_as_they_lie(which):
+    """A norm's weight and a convolution's state at any address, and a norm a head, go through the launches that take them."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    B, H = 3, 2
+    branch = GatedDelta(64, H, H, 128, 128, 4, 64, 64, 1e-5, 0.7).half().cuda().requires_grad_(False)
+    for p in branch.parameters():
+        p.data = torch.randn(p.shape, generator=g, device="cuda").half() * 0.3
+    states = [branch.new_state(B, torch.float16, "cuda") for _ in range(2)]
+    for t in states[0].tensors():
+        t.copy_(torch.randn(t.shape, generator=g, device="cuda"))
+    for a, c in zip(states[0].tensors(), states[1].tensors()):
+        c.copy_(a)
+    n = [w for _, w in branch.ins()]
+    p = torch.randn(B, sum(n), generator=g, device="cuda").half()
+    rows = [p[:, sum(n[:i]):sum(n[:i + 1])] for i in range(len(n))]
+    rows[4][...], rows[5][...] = eighths(g, B, 64).half(), eighths(g, B, 64).half()         # (products without rounding, as above)
+    for w in (branch.a2, branch.g2):
+        w.copy_((eighths(g, *w.shape) / 16).half())
+    outs = [torch.zeros(B, H * 128, dtype=torch.float16, device="cuda") for _ in range(2)]
+    step = Step(B, 1, 5)
+    branch(rows, outs[0], states[0], step)
+    odd = lambda t: torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)
+    if which == "norm":
+        branch.norm.data = odd(branch.norm.data)
+    elif which == "norm per head":
+        branch.norm.data = branch.norm.data.repeat(H)
+    else:
+        states[1].conv._buf[0] = odd(states[1].conv._buf[0])
+    branch(rows, outs[1], states[1], step)
+    # elsewhere a head's squares are added in another order (channel by channel): some units of float32 (2^-24 each), so outputs are at most
+    # neighbours in half precision; what passes through the convolution and the state is of the size of 1 to 10
+    (c0, s0), (c1, s1) = [s.tensors() for s in states]
+    assert torch.equal(c0, c1) and bool(((s0 - s1).abs() <= 2.0 ** -20 * s0.abs().max()).all())
+    assert bool(((outs[0].float() - outs[1].float()).abs() <= 2.0 ** -10 * outs[0].float().abs() + 2.0 ** -20 * outs[0].abs().max()).all())
+    assert float(outs[0].abs().max()) > 0.05
