@@ -8,7 +8,7 @@
 // memory), 8 rows each in quads, the other operands go through LDS.
 // In a chain of captured calls, bfloat16, against the separate launches (us): delta rule, 32 heads of 128 x 128, ranks 128, 1 / 8 / 64
 // sequences 6.4 / 9.4 / 54.4 against 13.3 / 18.7 / 68.0; matrix memory, 16 heads of 128 x 256, 5.2 / 7.2 / 43.3 against 7.5 / 12.0 / 47.2.
-// (8 sequences: 34 MB of state in and out, 6.7 us at 5 TB/s.)
+// (8 sequences: 34 MB of state in and out, 6.7 us at 5 TB/s.)  Very many heads times sequences go through the separate launches: recurrent_ops.py.
 #include "pq_recurrent_device.h"
 #include "pq_recurrent_internal.h"
 

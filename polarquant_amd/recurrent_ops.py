@@ -220,12 +220,26 @@ def _one_launch(step: Step, dtype: torch.dtype, *aligned) -> bool:
     return step.L == 1 and dtype in (torch.float16, torch.bfloat16) and all(t.data_ptr() % 16 == 0 for t in aligned)
 
 
-# (The one launch is the faster one at any number of sequences, 1 to 64 timed: pq_recurrent_token.hip.)
+# A workgroup of the one launch has a head's whole state and most of a unit's registers, so that it pays while few rounds of workgroups fill
+# the chip; beyond, the separate launches, with a state cut up, stream it faster.  Heads times sequences up to which it is the faster one, and
+# us of the one / the separate launches in a chain of captured calls, bfloat16:
+#   delta rule, 128 x 128, rank 128  4096: 123 / 131, 8192: 255 / 251;  128 x 96, rank 64  4096: 85 / 93, 8192: 218 / 202
+#   memory  8 x 8  256: 5.9 / 7.5, 512: 9.0 / 7.8;  32 x 64  512: 9.1 / 10.9, 1024: 15.6 / 14.7;  64 x 128  1024: 18.6 / 21.9, 2048: 34.8 / 34.4
+#           128 x 128  2048: 46.6 / 49.0, 4096: 98.8 / 93.6;  128 x 256  2048: 81 / 93, 4096: 207 / 184;  64 x 192  4096: 72 / 79, 8192: 178 / 168
+DELTA_TOKEN_HEADS = 4096
+
+
+def memory_token_heads(dim: int, vdim: int) -> int:
+    if vdim >= 160 or dim * vdim >= 16384:
+        return 4096 if dim <= 64 else 2048
+    return 1024 if vdim >= 128 else 512 if vdim >= 64 else 256
+
+
 def delta_token_takes(q, k, xa, xg, wa, wg, state: torch.Tensor, taps: int, out: torch.Tensor, step: Step, norm: Optional[torch.Tensor] = None,
                       conv: Optional[ConvState] = None) -> bool:
     """norm, conv: the norm's weight and the convolutions' state where they are not known to be of one head and at 8 bytes."""
     B, H, vdim, dim = state.shape
-    return (_one_launch(step, q.dtype, xa, xg, wa, wg, state, out) and q.shape[1] == k.shape[1] == H * dim
+    return (_one_launch(step, q.dtype, xa, xg, wa, wg, state, out) and B * H <= DELTA_TOKEN_HEADS and q.shape[1] == k.shape[1] == H * dim
             and (norm is None or (norm.numel() == vdim and norm.data_ptr() % 8 == 0)) and (conv is None or conv.rows.data_ptr() % 8 == 0)
             and _ffi.recurrent_lib().call.pq_validate_delta_token(B, H, dim, vdim, taps, wa.shape[1], wg.shape[1], q.stride(0), out.stride(0),
                                                                   _DTYPES[q.dtype]) == 0)
@@ -258,7 +272,7 @@ def delta_token(q, k, v, b, xa, xg, wa, wg, w_q, w_k, w_v, A_log, dt_bias, norm,
 
 def memory_token_takes(q, k, gate, norm, state: torch.Tensor, out: torch.Tensor, step: Step) -> bool:
     B, H, cols, dim = state.shape
-    return (_one_launch(step, q.dtype, q, k, gate, norm, state, out)
+    return (_one_launch(step, q.dtype, q, k, gate, norm, state, out) and B * H <= memory_token_heads(dim, cols - 1)
             and _ffi.recurrent_lib().call.pq_validate_memory_token(B, H, dim, cols - 1, q.stride(0), out.stride(0), _DTYPES[q.dtype]) == 0)
 
 

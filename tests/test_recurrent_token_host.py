@@ -27,3 +27,20 @@ def test_delta_rule_asks_where_its_operands_lie():
         assert not delta(norm=lambda t: at(t, n))
     assert not delta(conv=lambda t: at(t, 1))
     assert not delta(norm=lambda t: t.repeat(2))                      # a norm a head
+
+
+def memory(B, H, dim, vdim):
+    p = torch.empty(B, H * max(dim, vdim), dtype=torch.float16)
+    q, gate = p[:, :H * dim], p[:, :H * vdim]
+    return ops.memory_token_takes(q, q, gate, torch.empty(H * vdim, dtype=torch.float16), torch.empty(B, H, vdim + 1, dim), torch.empty_like(gate), Step(B, 1, 0))
+
+
+@pytest.mark.parametrize("dim,vdim,heads", [(8, 8, 256), (32, 64, 512), (40, 72, 512), (64, 128, 1024), (96, 128, 1024), (128, 128, 2048), (128, 160, 2048), (64, 192, 4096),
+                                            (8, 256, 4096)])
+def test_memory_takes_the_side_that_is_faster(dim, vdim, heads):
+    assert memory(1, 1, dim, vdim) and memory(8, heads // 8, dim, vdim) and not memory(8, heads // 8 + 1, dim, vdim) and not memory(2 * heads, 1, dim, vdim)
+
+
+@pytest.mark.parametrize("dim,vdim", [(128, 128), (128, 96), (96, 96)])
+def test_delta_rule_takes_the_side_that_is_faster(dim, vdim):
+    assert delta(1, 1, dim, vdim) and delta(128, 32, dim, vdim) and not delta(129, 32, dim, vdim)
