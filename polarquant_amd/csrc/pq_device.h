@@ -213,8 +213,9 @@ __device__ __forceinline__ void sincos_bin(float x, float* sn, float* cs) {
 //   returns c_d for this lane's pair; for attention (ATTN) it may be left in LDS too (Lut::C_IN_LDS).
 // Attention: the bins lie evenly about an angle m; with A = ax cos m + ay sin m and B = ay cos m - ax sin m the entries at m + phi and m - phi
 // are A cos phi + B sin phi and A cos phi - B sin phi, three instructions a head for two bins instead of four, and one rotation of phi
-// serves both (4-bit values, 4 heads, 8 x 16384, with the c_d in LDS 49.7 -> 48.5 us; half-precision values, 7 heads, 4 x 16384 25.4 -> 24.4).  Scores are results themselves and go from bin to bin: an infinite query's are
-// infinite that way, where A and B would cancel to NaN (in a softmax either ends as NaN).
+// serves both (4-bit values, 4 heads, 8 x 16384, with the c_d in LDS 49.7 -> 48.5 us; half-precision values, 7 heads, 4 x 16384 25.4 -> 24.4).
+// Scores go from bin to bin, and so does a group whose A and B could overflow (an infinite query): an entry is infinite that way, where A and
+// B cancel to NaN, and a softmax over scores of minus infinity alone would end as NaN instead of zeros.
 template <typename T, int TB, int REPP, bool ATTN>
 __device__ __forceinline__ float build_lut(uint32_t lut, int lane, const float (&qx)[REPP], const float (&qy)[REPP],
                                            uint16_t w_rscale, uint16_t w_rmn, uint16_t w_tscale, uint16_t w_tmn) {
@@ -240,7 +241,28 @@ __device__ __forceinline__ float build_lut(uint32_t lut, int lane, const float (
         if constexpr (L::W1 > 0) lds_store_w<L::WORDS - 4>(off + L::HB, e + 4);
     };
     float s, c, sd, cd;
+    auto bin_to_bin = [&]() {
+        sincos_bin(__builtin_fmaf(ts, 0.5f, tm), &s, &c);
+        sincos_bin(ts, &sd, &cd);
+#pragma clang loop unroll_count(ATTN ? 1 : L::NB)
+        for (int k = 0; k < L::NB; k++) {
+            float e[L::WORDS];
+#pragma unroll
+            for (int j = 0; j < REPP; j++) e[j] = __builtin_fmaf(ax[j], c, ay[j] * s);
+            store(k, e);
+            const float c2 = __builtin_fmaf(c, cd, -(s * sd));
+            const float s2 = __builtin_fmaf(s, cd, c * sd);
+            c = c2; s = s2;
+        }
+    };
     if constexpr (ATTN) {
+        float most = 0.0f;
+#pragma unroll
+        for (int j = 0; j < REPP; j++) most = fmaxf(fmaxf(most, fabsf(ax[j])), fabsf(ay[j]));
+        if (__builtin_expect(__any(most > 1e38f), 0)) {
+            bin_to_bin();
+            return cdv;
+        }
         constexpr int kHalf = L::NB / 2;
         float sm, cm;
         sincos_bin(__builtin_fmaf(ts, static_cast<float>(kHalf), tm), &sm, &cm);
@@ -269,18 +291,7 @@ __device__ __forceinline__ float build_lut(uint32_t lut, int lane, const float (
             c = c2; s = s2;
         }
     } else {
-        sincos_bin(__builtin_fmaf(ts, 0.5f, tm), &s, &c);
-        sincos_bin(ts, &sd, &cd);
-#pragma unroll
-        for (int k = 0; k < L::NB; k++) {
-            float e[L::WORDS];
-#pragma unroll
-            for (int j = 0; j < REPP; j++) e[j] = __builtin_fmaf(ax[j], c, ay[j] * s);
-            store(k, e);
-            const float c2 = __builtin_fmaf(c, cd, -(s * sd));
-            const float s2 = __builtin_fmaf(s, cd, c * sd);
-            c = c2; s = s2;
-        }
+        bin_to_bin();
     }
     return cdv;
 }

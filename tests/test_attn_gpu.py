@@ -342,3 +342,39 @@ def test_attn_empty_and_fully_masked_sequences(gpu):
     assert bool((out[1] == 0).all()) and bool((out[2] == 0).all())
     ref = po.decode_attention_exact(q[:1], k[:1, :, 256:], *[t[:1] for t in quant], v[:1])
     assert _close(out[:1], ref)[0] == 0
+
+
+@pytest.mark.parametrize("heads", range(1, 9))
+@pytest.mark.parametrize("values4", [False, True])
+def test_attn_scores_of_minus_infinity_alone(gpu, heads, values4):
+    """A query that is infinite where all keys have the same sign: every score is minus infinity and the result zero (of either sign), in
+    the kernels for few and for many groups; the other heads that share the tables are not touched."""
+    from polarquant_amd.attention import polar_decode_attention_v4
+    from polarquant_amd.quantize import quantize_and_pack_nbit
+    from polarquant_amd.values import quantize_values
+
+    for dtype, (B, n_groups, n_resid) in [(d, s) for d in (torch.float16, torch.bfloat16) for s in ((1, 2, 37), (2, 64, 5), (16, 32, 0))]:
+        print("case", heads, values4, dtype, B, n_groups, flush=True)
+        g = torch.Generator(device=gpu).manual_seed(heads)
+        r = lambda *s: torch.randn(*s, generator=g, device=gpu)
+        L = n_groups * 128
+        k = r(B, 2, L + 128, 128)
+        k[..., 0] = k[..., 0].abs() + 4.0                  # (the pair of channels 0 and 64 stays within a few degrees of its first axis)
+        k[..., 64] *= 0.1
+        k, v, q = k.to(dtype), r(B, 2, L + 128, 128).to(dtype), r(B, 2 * heads, 1, 128).to(dtype)
+        cache, kr = quantize_and_pack_nbit(k[:, :, :L].contiguous()), k[:, :, L:].contiguous()
+
+        def attend(t):
+            if values4:
+                return polar_decode_attention_v4(t, *cache, kr, v[:, :, L:].contiguous(), *quantize_values(v[:, :, :L].contiguous()), n_groups, n_resid,
+                                                 single_wavefront=_FORM["single"])
+            return polar_decode_attention(t, *cache, kr, v, n_groups, n_resid)
+
+        plain = attend(q)
+        inf = q.clone()
+        inf[:, ::heads, :, 0] = -float("inf")              # the first head of each KV head
+        out = attend(inf)
+        assert bool((out[:, ::heads] == 0).all())
+        rest = [h for h in range(2 * heads) if h % heads]
+        rtol, atol = (RTOL, ATOL) if dtype == torch.float16 else (BF16_RTOL, BF16_ATOL)
+        assert _close(out[:, rest], plain[:, rest], rtol, atol)[0] == 0 if rest else True
