@@ -279,7 +279,7 @@ struct Stage8T {
 };
 
 template <typename T, int KSPLIT, bool GATED, int kStage, int EPI = 0, int NT = 2, bool NORMED = false>
-__global__ __launch_bounds__(kWave * KSPLIT) __attribute__((amdgpu_waves_per_eu(NORMED ? 3 : 1))) void small_m8_linear_kernel(
+__global__ __launch_bounds__(kWave * KSPLIT) void small_m8_linear_kernel(
     const uint16_t* __restrict__ x, int64_t x_stride, const uint16_t* __restrict__ w, const uint16_t* __restrict__ w_up,
     const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, int64_t y_stride, int M, int K, HeadEpi he) {
     advance_once<EPI>(he);
