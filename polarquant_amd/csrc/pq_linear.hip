@@ -237,7 +237,9 @@ int launch_small_m_linear(const void* x, int64_t x_stride, const void* w, const 
     return static_cast<int>(hipGetLastError());
 }
 
-// Products before and behind a norm that they share (bfloat16, M <= 8; split of K and row tiles as in launch_small_m_linear).
+// Products before and behind a norm that they share (bfloat16, M <= 8; split of K and row tiles as in launch_small_m_linear).  Before it
+// four tiles at most, a lane of the epilogue's wavefront for every four columns: the rule says eight from 28672 columns on, and the norm
+// behind is 8192 wide at most.  Behind it two tiles where K is split eight ways: the rule never says four there for two matrices.
 int launch_linear_residual(const void* x, int64_t x_stride, const void* w, const void* bias, int M, int N, int K, void* stream_x, const void* norm_w,
                            void* xw, float* part, hipStream_t st) {
     HeadEpi he{};
@@ -256,13 +258,14 @@ int launch_linear_residual(const void* x, int64_t x_stride, const void* w, const
 int launch_gated_normed(const void* xw, const float* part, float eps, const void* w, const void* w_up, void* y, int M, int N, int K, hipStream_t st) {
     HeadEpi he{};
     he.normed = NormedRows{part, K / 16, eps};
-    const int ks = K >= 8192 ? 8 : 4, nt = small_m8_row_tiles(M, N, ks, 2);
+    const int ks = K >= 8192 ? 8 : 4, nt = ks == 8 ? 2 : small_m8_row_tiles(M, N, ks, 2);
     const dim3 grid(N / (8 * nt)), block(kWave * ks);
 #define PQ_LAUNCH_G(KS, S, NT)                                                                                       \
     hipLaunchKernelGGL((small_m8_linear_kernel<BF16, KS, true, S, 0, NT, true>), grid, block, 0, st, (const uint16_t*)xw, (int64_t)K, \
                        (const uint16_t*)w, (const uint16_t*)w_up, (const uint16_t*)nullptr, (uint16_t*)y, (int64_t)N, M, K, he)
-    if (ks == 8) { if (nt == 4) PQ_LAUNCH_G(8, 1, 4); else PQ_LAUNCH_G(8, 2, 2); }
-    else         { if (nt == 4) PQ_LAUNCH_G(4, 1, 4); else PQ_LAUNCH_G(4, 1, 2); }
+    if (ks == 8) PQ_LAUNCH_G(8, 2, 2);
+    else if (nt == 4) PQ_LAUNCH_G(4, 1, 4);
+    else PQ_LAUNCH_G(4, 1, 2);
 #undef PQ_LAUNCH_G
     return static_cast<int>(hipGetLastError());
 }

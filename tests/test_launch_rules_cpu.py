@@ -82,3 +82,12 @@ def test_latent_plan_fills_the_units_with_workgroups_of_one_team():
     plan = _ffi.latent_lib().pq_latent_decode_plan
     assert [plan(B, 1, 32, 1 << 20, 256) for B in (1, 8, 100, 129, 256, 257, 300, 512, 513)] == [512, 64, 6, 4, 2, 2, 2, 1, 1]
     assert [plan(8, 1, 32, keys, 256) for keys in (1, 128, 129, 1000)] == [1, 1, 2, 8] and plan(8, 1, 64, 1 << 20, 256) == 32
+
+
+def test_tiles_around_a_shared_norm(row_tiles):
+    """What the launches of the products around a norm rest on: two matrices with K split eight ways are never given four tiles, and one
+    matrix no more than four up to the widest norm (8192)."""
+    for rows in range(1, 9):
+        assert all(row_tiles(rows, n, 8, 2) == 2 for n in range(16, 1 << 19, 16))
+        assert all(row_tiles(rows, n, ks, 1) <= 4 for n in range(16, 8192 + 16, 16) for ks in (4, 8))
+    assert next(n for n in range(16, 1 << 16, 16) if row_tiles(8, n, 4, 1) == 8) >= 28672
