@@ -55,11 +55,9 @@ int launch_head_linear_mfma(const HeadLinearArgs& a, int dtype, hipStream_t st) 
 
 // The rows of a workgroup and the split of K as above: a workgroup of pairs streams as many bytes as one of plain rows.
 int launch_linear_gelu(const LinearGeluArgs& a, int dtype, hipStream_t st) {
-    const int N = a.plain + 2 * a.ff;
     int ks = a.K >= 8192 ? 8 : 4;
     while (ks > 1 && ((a.K % (64 * ks)) != 0 || a.K / (64 * ks) < 2)) ks >>= 1;
-    int nt = N % 16 ? 2 : small_m8_row_tiles(a.M, N, ks, 1);
-    while (nt > 2 && (a.plain % (8 * nt) || a.ff % (4 * nt))) nt >>= 1;
+    const int nt = linear_gelu_row_tiles(a.M, a.plain, a.ff, ks);
     dim3 grid(a.plain / (8 * nt) + a.ff / (4 * nt)), block(kWave * ks);
     const HeadEpi he{0, 0, 0, nullptr, 0, 1.0f, 0.0f, nullptr, a.plain / (8 * nt), a.ff, static_cast<uint16_t*>(a.z), a.z_row};
 #define PQ_G(T, KS, NT)                                                                                              \

@@ -29,6 +29,14 @@ inline int small_m8_row_tiles(int rows, int N, int ksplit, int matrices) {
     return best;
 }
 
+// The same of a product whose last 2 ff rows of W go to workgroups of pairs (launch_linear_gelu): whole workgroups of either kind, two tiles at least.
+inline int linear_gelu_row_tiles(int rows, int plain, int ff, int ksplit) {
+    const int N = plain + 2 * ff;
+    int nt = N % 16 ? 2 : small_m8_row_tiles(rows, N, ksplit, 1);
+    while (nt > 2 && (plain % (8 * nt) || ff % (4 * nt))) nt >>= 1;
+    return nt;
+}
+
 // Depths that the products around a norm take (launch_linear_residual: `behind` false; the products behind it: true).  K is split four ways,
 // from 8192 on eight, into whole steps of 64; and behind the norm a row's sums, one of 16 elements, have to be two 16-byte loads to a
 // thread at most (8 KSPLIT threads a row): up to 4096, and 8192.

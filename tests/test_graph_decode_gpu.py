@@ -256,3 +256,68 @@ def test_options_say_which_launches_a_step_makes(gpu, monkeypatch, options, laun
         monkeypatch.setattr(decode_ops, name, lambda *a, _f=f, _n=name, **k: (made.add(_n), _f(*a, **k))[1])
     dec.step(ids[:, :1])
     assert made == launches | ({"silu_mul"} if bias else set())
+
+
+@pytest.mark.parametrize("B", [1, 2, 8])
+@pytest.mark.parametrize("kind", ["plain", "biases", "values in 4 bits", "one layer's MLP has biases"])
+def test_norms_shared_by_the_products_around_them(gpu, monkeypatch, kind, B):
+    """bfloat16 steps of three layers whose norms are shared (`linear_residual`, `gated_normed`, `qkv_rope_append_normed`): as many of each as the
+    layers allow, logits and caches as with the norms in launches of their own to rounding, replays as the eager step."""
+    from polarquant_amd import decode_ops
+    torch.manual_seed(5)
+    cls = Qwen2PolarForCausalLM if kind == "biases" else LlamaPolarForCausalLM
+    cfg = _tiny(layers=3, **(dict(attention_bias=True) if kind == "biases" else dict(vbits=4) if kind == "values in 4 bits" else {}))
+    model = cls(cfg).to(torch.bfloat16).to(gpu).eval()
+    layers = model.model.layers
+    for layer in layers:                                   # (norm weights that differ, so that one taken for another shows)
+        for norm in (layer.input_layernorm, layer.post_attention_layernorm):
+            norm.weight.data.uniform_(0.5, 1.5)
+    model.model.norm.weight.data.uniform_(0.5, 1.5)
+    if kind == "biases":
+        for layer in layers:
+            layer.mlp.down_proj.bias = torch.nn.Parameter(0.1 * torch.randn(cfg.hidden_size, device=gpu).to(torch.bfloat16))
+            for p in (layer.self_attn.q_proj, layer.self_attn.k_proj, layer.self_attn.v_proj):
+                p.bias.data.normal_(0, 0.1)
+    into, gated, rotated = 5, 3, 2                         # of three layers: before each norm but the first and the last
+    if kind == "one layer's MLP has biases":
+        for p in (layers[1].mlp.gate_proj, layers[1].mlp.up_proj):
+            p.bias = torch.nn.Parameter(0.1 * torch.randn(cfg.intermediate_size, device=gpu).to(torch.bfloat16))
+        into, gated, rotated = 3, 2, 1
+    L, new = 120, 12                                       # (a flush at 128 tokens)
+    ids = torch.randint(0, cfg.vocab_size, (B, L), device=gpu)
+    counts = {}
+
+    def spied(name):
+        plain = getattr(decode_ops, name)
+
+        def call(*args, **kw):
+            counts[name] = counts.get(name, 0) + 1
+            return plain(*args, **kw)
+        monkeypatch.setattr(decode_ops, name, call)
+
+    for name in ("linear_residual", "gated_normed", "qkv_rope_append_normed"):
+        spied(name)
+    with torch.no_grad():
+        dec_g, dec_e, dec_s = [PolarGraphDecoder(model, max_len=L + new + 8, use_graph=u) for u in (True, False, False)]
+        tok = dec_g.prefill(ids).argmax(-1)
+        for d in (dec_e, dec_s):
+            d.prefill(ids)
+        for s in range(new):
+            counts.clear()
+            got = dec_e.step(tok).clone()
+            assert counts == {"linear_residual": into, "gated_normed": gated, "qkv_rope_append_normed": rotated}
+            with monkeypatch.context() as m:
+                m.setattr(decode_ops, "normed_depth", lambda K, behind: False)
+                counts.clear()
+                separate = dec_s.step(tok).clone().float()
+                assert not counts
+            replay = dec_g.step(tok).clone()
+            torch.cuda.synchronize()
+            assert torch.equal(replay, got), s
+            # three layers of bfloat16 that differ in one rounding of each norm: some units (2^-9) of the logits
+            assert float((got.float() - separate).norm() / separate.norm()) <= 16 * 2.0 ** -9, s
+            tok = separate.argmax(-1)
+        for a, b in zip(dec_g.cache(), dec_e.cache()):
+            _same_cache(a, b)
+        for a, b in zip(dec_e.cache()[:1], dec_s.cache()[:1]):         # (no norm stands before the first layer's that is shared)
+            _same_cache(a, b)

@@ -34,6 +34,7 @@ def rules():
     subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-x", "c++", "-", "-o", so, "-I", os.path.join(os.path.dirname(here), "polarquant_amd", "csrc")],
                    input=b'#include "pq_linear_rules.h"\n#include "pq_steps_rules.h"\n#include "pq_latent_rules.h"\nextern "C" {\n'
                          b'int tiles(int m, int n, int ks, int mats) { return pq::small_m8_row_tiles(m, n, ks, mats); }\n'
+                         b'int gelu_tiles(int m, int plain, int ff, int ks) { return pq::linear_gelu_row_tiles(m, plain, ff, ks); }\n'
                          b'int strip(int tokens, int taps, int pieces) { return pq::norm_conv_strip(tokens, taps, pieces); }\n'
                          b'int layout(int rank, int groups, int slices) { auto l = pq::latent_decode_layout(rank, groups, slices); return 1000 * l.teams + l.slices; }\n}', check=True)
     return ctypes.CDLL(so)
@@ -91,3 +92,25 @@ def test_tiles_around_a_shared_norm(row_tiles):
         assert all(row_tiles(rows, n, 8, 2) == 2 for n in range(16, 1 << 19, 16))
         assert all(row_tiles(rows, n, ks, 1) <= 4 for n in range(16, 8192 + 16, 16) for ks in (4, 8))
     assert next(n for n in range(16, 1 << 16, 16) if row_tiles(8, n, 4, 1) == 8) >= 28672
+
+
+def test_cases_of_the_products_around_a_norm_select_their_launches(row_tiles):
+    """The GPU tests' cases run each launch that there is: K split four and eight ways, two and four row tiles."""
+    import test_shared_norm_gpu as t
+    split = lambda k: 8 if k >= 8192 else 4
+    gated = {(split(width), 2 if width >= 8192 else row_tiles(M, ff, 4, 2)) for M, width, ff in t.GATED_VARIANTS}
+    into = {(split(k), min(4, row_tiles(M, width, split(k), 1))) for M, width, k in t.INTO_VARIANTS}
+    assert gated == {(4, 2), (4, 4), (8, 2)} and into == {(4, 2), (4, 4), (8, 2), (8, 4)}
+
+
+def test_cases_of_the_product_with_gelu_select_their_launches(rules):
+    import test_recurrent_token_gpu as t
+    older = [(8, 2, 8, 64, 40, 8192), (4, 4, 8, 18720, 14336, 4096), (4, 2, 5, 4096, 256, 2048), (1, 4, 6, 2048, 65536, 192), (1, 2, 1, 16, 8, 64)]
+    seen = set()
+    for ksplit, tiles, M, plain, ff, K in t.GELU_VARIANTS + older:
+        ks = 8 if K >= 8192 else 4
+        while ks > 1 and (K % (64 * ks) or K // (64 * ks) < 2):
+            ks //= 2
+        assert (ks, rules.gelu_tiles(M, plain, ff, ks)) == (ksplit, tiles)
+        seen.add((ksplit, tiles))
+    assert seen == {(ks, nt) for ks in (1, 2, 4, 8) for nt in (2, 4, 8)}

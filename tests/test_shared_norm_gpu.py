@@ -115,3 +115,68 @@ def test_what_is_not_taken(gpu):
     for K in range(64, 20000, 64):
         assert normed_depth(K, False) == (call.pq_validate_linear_residual(P, K, P, None, 8, 4096, K, 1, P, P, P, P) == 0)
         assert normed_depth(K, True) == (call.pq_validate_gated_normed(P, P, P, P, P, 8, 512, K, 1) == 0)
+
+
+# launches that the cases above leave out: rows, width, and columns of the product behind or depth of the one before
+GATED_VARIANTS = [(1, 4096, 14336), (5, 4096, 14336), (8, 4096, 14336), (8, 512, 16384), (8, 4096, 8192), (8, 8192, 8192)]
+INTO_VARIANTS = [(8, 8192, 8192), (8, 8192, 8704), (8, 5120, 8704), (8, 4096, 14336), (1, 8192, 4096), (8, 8192, 4096), (2, 4096, 4096), (8, 4096, 4096)]
+
+
+@pytest.mark.parametrize("M,width,ff", GATED_VARIANTS)
+def test_gated_product_of_every_launch(gpu, M, width, ff):
+    """(From 60000 results on with the RMS error against the separate launches.)"""
+    test_gated_product(gpu, M, width, ff)
+
+
+@pytest.mark.parametrize("M,width,K", INTO_VARIANTS)
+def test_product_into_the_stream_of_every_launch(gpu, M, width, K):
+    test_product_into_the_stream(gpu, M, width, K)
+
+
+def test_projections_with_rotation_error(gpu):
+    """Enough results for the RMS error, at the widest norm of a depth split four ways and of one split eight ways."""
+    for width in (4096, 8192):
+        test_projections_with_rotation(gpu, 8, width, 56, 4, True)
+
+
+@pytest.mark.parametrize("eps", [1e-5, 1e-3])
+@pytest.mark.parametrize("width", [256, 2048, 4096, 8192])
+def test_factor_of_a_row(gpu, width, eps):
+    """The products' factor of a row by itself.  Rows of weights that hold a single one make every product exact, so that a value is r (x w)
+    rounded once: the same bits as from r in 64 bits unless that lies within float32's error (2^-22) of a tie, one in 2^13.  A row's energy
+    lies in one block of 16 columns, each block in turn, so that a sum that is missed changes everything; the rows are small enough that eps
+    is a good part of the mean square."""
+    g = torch.Generator().manual_seed(width)
+    N, Nk = 1, 4
+    nw = draw(gpu, g, width) + 2.0
+    cols = torch.randint(0, width, ((N + 2 * Nk) * 128,), generator=g)
+    w = torch.zeros((N + 2 * Nk) * 128, width, dtype=torch.bfloat16)
+    w[torch.arange(len(cols)), cols] = 1.0
+    gate, up = torch.zeros(512, width, dtype=torch.bfloat16), torch.zeros(512, width, dtype=torch.bfloat16)
+    gate[torch.arange(512), cols[:512]] = 1.0
+    up[torch.arange(512), cols[512:1024]] = 1.0
+    w, gate, up = w.to(gpu), gate.to(gpu), up.to(gpu)
+    cos = torch.ones(4, 128, dtype=torch.bfloat16, device=gpu)
+    at = torch.zeros(1, dtype=torch.int64, device=gpu)
+    rounded = lambda t: t.to(torch.bfloat16).double()
+    same, total = 0, 0
+    for first in range(0, width // 16, 8):
+        stream = draw(gpu, g, 8, 1, width, scale=1e-3)
+        for m in range(8):
+            block = first + m
+            stream[m, 0, 16 * block:16 * block + 16] = draw(gpu, g, 16, scale=0.2) + 0.3
+        xw, part = linear_residual(torch.zeros(8, 1, 256, dtype=torch.bfloat16, device=gpu), torch.zeros(width, 256, dtype=torch.bfloat16, device=gpu), None,
+                                   stream, nw)
+        r64 = torch.rsqrt(stream.double().square().mean(-1) + eps)
+        n64 = xw.double()[:, 0] * r64
+        k, v = torch.zeros(8, Nk, 1, 128, dtype=torch.bfloat16, device=gpu), torch.zeros(8, Nk, 1, 128, dtype=torch.bfloat16, device=gpu)
+        qkv_rope_append_normed((xw, part), eps, w, None, cos, torch.zeros_like(cos), at, k, at, v, at, N, Nk)
+        got = gated_normed((xw, part), eps, gate, up)[:, 0]
+        gv, uv = rounded(n64[:, cols[:512]]), rounded(n64[:, cols[512:1024]])
+        want = [(k.reshape(8, -1), rounded(n64[:, cols[128:640]])), (v.reshape(8, -1), rounded(n64[:, cols[640:]])),
+                (got, rounded(rounded(torch.nn.functional.silu(gv)) * uv))]
+        for y, e in want:
+            assert bool(((y.double() - e).abs() <= 2.0 ** -6 * e.abs() + 1e-30).all())          # the other neighbour of each rounding
+            same += int((y.double() == e).sum())
+            total += y.numel()
+    assert same >= 0.995 * total, (same, total)
