@@ -37,7 +37,8 @@
  * pq_delta_token, pq_memory_token: a single token a sequence (L = 1), in one launch what
  *   pq_delta_prep (a = xa wa^T, gate = xg wg^T: [H * dim, a_rank], [H * vdim, g_rank]),
  *   pq_delta_scan and pq_head_norm_gate, or pq_memory_gates, pq_memory_scan and
- *   pq_head_norm_gate do.  16-bit dtypes, G = H, row strides multiples of 8, out's of 4;
+ *   pq_head_norm_gate do, bit for bit but for the order of the low-rank products' sums.
+ *   16-bit dtypes, G = H, row strides multiples of 8, out's of 4;
  *   delta rule: dim, vdim multiples of 8 in 96 .. 128, taps <= 4, ranks multiples of 8 up to 128;
  *   matrix memory: dim up to 128, vdim up to 256, multiples of 8.  conv, state and m in place.
  */

@@ -16,8 +16,9 @@
 // flash-style running state (m, l, acc) for the `rep` query heads of its KV
 // head.  P.V runs on the matrix cores: for 32 tokens at a time
 //     D[dim][head] += V^T[dim][token] * P[token][head]
-// with v_mfma_f32_16x16x32 (f16 or bf16), heads padded to the 16 columns.  (16 tokens at a time were twice the products, each as long:
-// 4-bit values, 4 heads, 8 x 16384 47.5 -> 46.9 us, and no difference to the pairs, whose accumulators wait for other things.)
+// with v_mfma_f32_16x16x32 (f16 or bf16), heads padded to the 16 columns.  (16 tokens at a time were twice the products, each as long;
+// with an operand made ahead of each product and maxima by DPP, not timed apart: 4-bit values, 4 heads, 8 x 16384 47.5 -> 46.9 us, and no
+// difference to the pairs, whose accumulators wait for other things.)
 // The V operand is built from plain 16-byte row loads (lane (g,n) loads dims
 // 8n..8n+7 of tokens 4g..4g+3) by a 4x4 in-register transpose with v_perm_b32;
 // P goes through a 1 KiB LDS staging buffer.

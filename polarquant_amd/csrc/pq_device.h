@@ -299,8 +299,9 @@ __device__ __forceinline__ float build_lut(uint32_t lut, int lane, const float (
 // Score one token against the table.  `codes` holds the token's 64 pair codes as
 // 16 little-endian words.  acc[j] += ...  `cds` says where the c_d are: InLds, as build_lut leaves them (with the entry, or four to a read
 // that all lanes share), or 64 scalar registers.  Attention with two heads and more has them in LDS: its scalar registers hold much
-// else, of which the 64 spilled half, and the 64 readlanes of a group are as many instructions as a tenth of a tile's walk.  For one
-// head the reads cost more than they save (4-bit values, 8 x 4096: 44.2 us, in LDS 44.8).  The score kernel's wavefront walks one group,
+// else, of which the 64 spilled half, and the 64 readlanes of a group are as many instructions as a tenth of a tile's walk.  Two heads,
+// 8 x 16384, 4-bit values: registers / LDS 44.2 / 43.1 us (half), 42.9 / 43.0 (bfloat16), 3-bit codes 40.0 / 39.1; ragged, 32 bins 102.8 / 99.6
+// and 102.5 / 99.1, not ragged 34.8 / 35.1.  For one head the reads cost more than they save (4-bit values, 8 x 4096: 44.2 us, in LDS 44.8).  The score kernel's wavefront walks one group,
 // and 256 bytes more would leave a unit nine tables of four heads instead of ten (8 sequences of 16384, 4 heads 30.6 us, in LDS 34.3).
 struct InLds {};
 // The 64 table reads are issued in batches of 4 or 8 codes, one batch ahead of the

@@ -181,7 +181,7 @@ int launch_qkv_rope_append(const void* x, int64_t x_stride, const void* w, const
         else if (ks == 2) PQ_LAUNCH_R(T, 2, 1);                                                                      \
         else PQ_LAUNCH_R(T, 1, 1);                                                                                   \
     } while (0)
-    if (norm_part) {                               // (shapes: normed_width; bfloat16)
+    if (norm_part) {                               // (shapes: normed_depth; bfloat16)
         const NormedRows nr{norm_part, K / 16, eps};
         if (ks == 8) hipLaunchKernelGGL((qkv_rope_append_kernel<BF16, 8, 2, true>), grid, block, 0, st, (const uint16_t*)x, x_stride, (const uint16_t*)w, (const uint16_t*)bias, M, K, ra, nr);
         else hipLaunchKernelGGL((qkv_rope_append_kernel<BF16, 4, 1, true>), grid, block, 0, st, (const uint16_t*)x, x_stride, (const uint16_t*)w, (const uint16_t*)bias, M, K, ra, nr);

@@ -22,7 +22,7 @@
 // products per launch (blockIdx.y == head, operands `x_head` / N * K / `y_head` elements apart) with epilogue e of
 // pq_steps_internal.h: plain, square of relu, times sigmoid(gate), unrounded float32 output, that scaled and soft-capped, or plain rows and
 // behind them pairs of a gate's and another row whose results become gelu(gate) * other (small_m8_linear_kernel only; 8 rows, 18720 plain
-// rows and 14336 pairs of 4096: the step is 2.2 us a layer shorter, which was a launch of its own that moved 0.9 MB), or added to a residual
+// rows and 14336 pairs of 4096, in a chain: 65.1 -> 63.3 us, which was a launch of its own that moved 0.9 MB), or added to a residual
 // stream with the first half of the norm behind it (ResidualOut; small_m8_linear_kernel only).
 #pragma once
 #include "pq_device.h"
@@ -56,11 +56,13 @@ template <> __device__ __forceinline__ uint16_t times_rounded<F16>(float a, uint
     return static_cast<uint16_t>(r);
 }
 
-// A norm cut in two between the products around it (pq_linear_residual, pq_linear_normed).  norm(x) W^T is r (x w) W^T with one number
+// A norm cut in two between the products around it (pq_linear_residual; pq_gated_normed, pq_qkv_rope_append_normed).  norm(x) W^T is r (x w) W^T with one number
 // r = rsqrt(mean x^2 + eps) a row: the product before stores x w, rounded once, and the sum of x^2 over every 16 columns; the product behind
-// multiplies its sums by r, which it makes of those.  Its own launch, which the norm had between them, was 4.5 us of a decode step, of which
-// nothing was work; 1.9 of them are saved (8 rows of 4096: the o projection 9.3 -> 10.0 us, gate and up 40.8 -> 42.4, down 24.3 -> 25.0,
-// q, k and v 15.1 -> 15.6).  Every workgroup reads the sums, like x itself.
+// multiplies its sums by r, which it makes of those.  Every workgroup reads the sums, like x itself.  The norm had a launch of its own, of
+// which nothing was work.  8 rows of 4096, products and norms in a chain of captured calls (us): o projection, norm, gate and up of 14336 50.3
+// -> 49.0, down, norm, q, k and v 39.7 -> 37.2; each by itself norm 3.2, o 9.0 -> 9.5, gate and up 38.9 -> 39.9, down 22.8 -> 23.3, q, k and
+// v 14.8 -> 15.0.  A step with two norms of the first kind and one of the second 289.3 -> 284.3.  Widths 256 to 8192, 1 to 8 rows: 1.00 to 1.21
+// times as fast; from 6 rows on 28672 -> 8192 -> q, k, v takes as long either way.
 struct NormedRows {
     const float* part;          // [M, n]: sums of squares of a row's 16 n elements
     int n;

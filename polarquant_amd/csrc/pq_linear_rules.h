@@ -39,7 +39,7 @@ inline int linear_gelu_row_tiles(int rows, int plain, int ff, int ksplit) {
 
 // Depths that the products around a norm take (launch_linear_residual: `behind` false; the products behind it: true).  K is split four ways,
 // from 8192 on eight, into whole steps of 64; and behind the norm a row's sums, one of 16 elements, have to be two 16-byte loads to a
-// thread at most (8 KSPLIT threads a row): up to 4096, and 8192.
+// thread at most (8 KSPLIT threads a row): up to 4096, and 8192.  (More loads a thread, for the widths between, were not tried.)
 inline bool normed_depth(int K, bool behind) {
     const int ks = K >= 8192 ? 8 : 4;
     return K >= 256 && K % (64 * ks) == 0 && (!behind || K / 16 <= 2 * 4 * 8 * ks);

@@ -1,6 +1,7 @@
 // One token a sequence through a mixer with a matrix-valued state, from its columns of the input product to its columns of the output
 // product's operand: what delta_prep_kernel or memory_gates_kernel, scan_kernel and head_norm_gate_kernel (pq_recurrent.hip) do for any
-// number of tokens, and for the delta rule the two low-rank products before them.
+// number of tokens, the same operations in the same order; for the delta rule also the two low-rank products before them, whose sums are
+// taken in another order (8 elements a lane, then 16 lanes) and rounded to the dtype like theirs.
 //
 // A workgroup per (head, sequence): the norm of what is read out runs over a head, so its state is not cut up.  What bounds it is the
 // stream of the state in and out; everything else is a few hundred elements that each of the separate launches fetched, wrote and waited

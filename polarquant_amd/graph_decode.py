@@ -225,7 +225,7 @@ class PolarGraphDecoder(GraphDecoder):
         """The decode step with one launch per elementwise stage: 2 norms (each with the residual add
         folded in), RoPE + append, SiLU * up, plus the GEMMs and the attention, per layer.  The first norm reads the embedding's
         rows itself and the last one raises the counters.  Up to 8 bfloat16 rows the norms between are shared by the products around
-        them (`linear_residual`): a step of 8 sequences of 4096 tokens, two layers of width 4096 with three such norms, 289.7 -> 284.6 us.  (In float16
+        them (`linear_residual`): a step of 8 sequences of 4096 tokens, two layers of width 4096 with three such norms, 289.3 -> 284.3 us.  (In float16
         the stream times a norm's weight could overflow.)"""
         from .decode_ops import (STEP_NORM_MAX, STEP_NORM_ROWS, embed_rmsnorm, gated_normed, linear_residual, linear_small_m, normed_depth, qkv_rope_append,
                                  qkv_rope_append_normed, rmsnorm, rope_append, silu_mul)

@@ -362,7 +362,7 @@ class ParallelLayer(nn.Module):
 
     def _products_with_gelu(self, h: torch.Tensor, w_in: torch.Tensor, z: torch.Tensor) -> Optional[torch.Tensor]:
         """Rows h of a decode step -> the input product but for the feed-forward's two, whose result goes to z; None where that is not one
-        launch.  (8 rows of 4096: a launch of 3 us less, and the product's own time does not change.)"""
+        launch.  (pq_linear_device.h has both times.)"""
         last = self._branches[-1]
         if type(last) is not GatedGelu or last is not self.mlp or not layer_ops.runs_plainly(last):
             return None
